@@ -112,11 +112,12 @@ int pyseqm_pair_integrals(const pyseqm_layout_t* L, int method, const double* co
                           double* H, double* part, double* enuc_tile, double* enuc_mol,
                           double* enuc_pair, const int* pair_ref, void* stream);
 
-/* Forces -dE/dR (eV/Angstrom, [natoms*3]) at fixed density P: per atom pair, a 4th-order central
- * difference (step h Angstrom) of the pair's Hellmann-Feynman energy 2 P_ij.H_ij + P_ii.e1b +
+/* Forces -dE/dR (eV/Angstrom, [natoms*3]) at fixed density P: per atom pair, the closed-form
+ * gradient of the pair's Hellmann-Feynman energy 2 P_ij.H_ij + P_ii.e1b +
  * P_jj.e2a + P_ii P_jj (ii|jj) - 1/2 P_ij P_ij (ij|ij) + E_nuc(ij) -- the energy the reference
  * differentiates by autograd with scf_backward = 0 (basics.py:1315-1336, scf_loop.py:1996-2031).
- * part: tile partial scratch as in pyseqm_pair_integrals. */
+ * h: must be positive; the step of an earlier finite-difference form, kept in the signature, without
+ * effect on the result.  part: tile partial scratch as in pyseqm_pair_integrals. */
 int pyseqm_pair_forces(const pyseqm_layout_t* L, int method, const double* coords, const double* atom_par,
                        const double* P, double h, double* part, double* forces, void* stream);
 

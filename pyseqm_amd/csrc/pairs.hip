@@ -74,11 +74,90 @@ __global__ void k_atom_setup(pyseqm_layout_t L, double* par) {
   derive_atom(par + (size_t)a * PYSEQM_NPAR, L.atom_Z[a]);
 }
 
+// ------------------------------------------------------------------ value + derivative
+// A function of the pair distance together with its derivative: the force kernels evaluate the
+// formulas below once on Duals instead of at displaced geometries.  On plain doubles every helper
+// is the operation the integral kernels have always used.
+struct Dual {
+  double v, d;
+};
+__device__ inline Dual operator+(Dual a, Dual b) { return {a.v + b.v, a.d + b.d}; }
+__device__ inline Dual operator-(Dual a, Dual b) { return {a.v - b.v, a.d - b.d}; }
+__device__ inline Dual operator-(Dual a) { return {-a.v, -a.d}; }
+__device__ inline Dual operator+(Dual a, double b) { return {a.v + b, a.d}; }
+__device__ inline Dual operator+(double a, Dual b) { return {a + b.v, b.d}; }
+__device__ inline Dual operator-(Dual a, double b) { return {a.v - b, a.d}; }
+__device__ inline Dual operator-(double a, Dual b) { return {a - b.v, -b.d}; }
+__device__ inline Dual operator*(double a, Dual b) { return {a * b.v, a * b.d}; }
+__device__ inline Dual operator*(Dual a, double b) { return {a.v * b, a.d * b}; }
+__device__ inline Dual operator*(Dual a, Dual b) { return {a.v * b.v, fma(a.v, b.d, a.d * b.v)}; }
+__device__ inline Dual operator/(Dual a, double b) { return a * (1.0 / b); }
+// 1 / x from v_rcp_f64 and two Newton steps, 1 / sqrt(x) from v_rsq_f64 and two (x normal, positive for
+// the root): the arguments here are distances and squared distances of atom pairs
+__device__ inline double rcp_nr(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+__device__ inline double rsq_nr(double x) {
+  double r = __builtin_amdgcn_rsq(x);
+  r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+  return fma(0.5 * r, fma(-x * r, r, 1.0), r);
+}
+__device__ inline double inv_root(double x) { return 1.0 / sqrt(x); }
+__device__ inline Dual inv_root(Dual x) {
+  const double r = rsq_nr(x.v);
+  return {r, -0.5 * (r * r * r) * x.d};
+}
+// a / sqrt(x)
+__device__ inline double quot_root(double a, double x) { return a / sqrt(x); }
+__device__ inline Dual quot_root(double a, Dual x) { return a * inv_root(x); }
+__device__ inline double exp_of(double x) { return exp(x); }
+__device__ inline Dual exp_of(Dual x) {
+  const double e = exp(x.v);
+  return {e, e * x.d};
+}
+__device__ inline double value_of(double x) { return x; }
+__device__ inline double value_of(Dual x) { return x.v; }
+__device__ inline double recip(double) { return 0.0; }  // unused: over() divides
+__device__ inline Dual recip(Dual x) {
+  const double r = rcp_nr(x.v);
+  return {r, -(r * r) * x.d};
+}
+// a / x, given recip(x)
+__device__ inline double over(double a, double x, double) { return a / x; }
+__device__ inline Dual over(Dual a, Dual, Dual rx) { return a * rx; }
+__device__ inline double quot(double a, double x) { return a / x; }
+__device__ inline Dual quot(double a, Dual x) { return a * recip(x); }
+// x^(k + 1/2) of a constant, in a formula on doubles / on Duals
+__device__ inline double half_pow(double, double x, int k) { return pow(x, k + 0.5); }
+__device__ inline double half_pow(Dual, double x, int k) {
+  double p = sqrt(x);
+  for (int t = 0; t < k; ++t) p *= x;
+  return p;
+}
+__device__ inline double pow_3_2(double x) { return pow(x, 1.5); }
+__device__ inline Dual pow_3_2(Dual x) {
+  const double q = sqrt(x.v);
+  return {x.v * q, 1.5 * q * x.d};
+}
+template <class S>
+__device__ inline S constant(double x);
+template <>
+__device__ inline double constant<double>(double x) {
+  return x;
+}
+template <>
+__device__ inline Dual constant<Dual>(double x) {
+  return {x, 0.0};
+}
+
 // ------------------------------------------------------------ local-frame integrals
 // 22 heavy-heavy integrals in MOPAC storage order (SS/SS)=0 ... (P*P/P*P)=21, local axis
 // sigma pointing from atom j to atom i (two_elec_two_center_int_local_frame.py:126-262).
-__device__ void local_xx(double r, double da, double db, double qa1, double qb1, double r0a,
-                         double r0b, double r1a, double r1b, double r2a, double r2b, double ri[22]) {
+template <class S>
+__device__ inline void local_xx(S r, double da, double db, double qa1, double qb1, double r0a,
+                         double r0b, double r1a, double r1b, double r2a, double r2b, S ri[22]) {
   const double e1 = kEV * 0.5, e2 = kEV * 0.25, e3 = kEV * 0.125, e4 = kEV * 0.0625;
   const double qa = 2.0 * qa1, qb = 2.0 * qb1;
   const double aee = (r0a + r0b) * (r0a + r0b), ade = (r1a + r0b) * (r1a + r0b);
@@ -86,23 +165,23 @@ __device__ void local_xx(double r, double da, double db, double qa1, double qb1,
   const double aeq = (r0a + r2b) * (r0a + r2b), axx = (r1a + r1b) * (r1a + r1b);
   const double adq = (r1a + r2b) * (r1a + r2b), aqd = (r2a + r1b) * (r2a + r1b);
   const double aqq = (r2a + r2b) * (r2a + r2b);
-  const double r2 = r * r;
-  auto inv = [](double x) { return 1.0 / sqrt(x); };
-  const double ee = kEV * inv(r2 + aee);
-  const double dze = -e1 * inv((r + da) * (r + da) + ade) + e1 * inv((r - da) * (r - da) + ade);
-  const double c6 = e1 * inv(r2 + aqe);
-  const double qzze = e2 * inv((r - qa) * (r - qa) + aqe) + e2 * inv((r + qa) * (r + qa) + aqe) - c6;
-  const double qxxe = e1 * inv(r2 + qa * qa + aqe) - c6;
-  const double edz = -e1 * inv((r - db) * (r - db) + aed) + e1 * inv((r + db) * (r + db) + aed);
-  const double c12 = e1 * inv(r2 + aeq);
-  const double eqzz = e2 * inv((r - qb) * (r - qb) + aeq) + e2 * inv((r + qb) * (r + qb) + aeq) - c12;
-  const double eqxx = e1 * inv(r2 + qb * qb + aeq) - c12;
-  const double t20 = e2 * inv((r + da) * (r + da) + adq), t22 = e2 * inv((r - da) * (r - da) + adq);
-  const double t24 = e2 * inv((r - db) * (r - db) + aqd), t26 = e2 * inv((r + db) * (r + db) + aqd);
-  const double t36 = e2 * inv(r2 + aqq), t39 = e2 * inv(r2 + qa * qa + aqq), t40 = e2 * inv(r2 + qb * qb + aqq);
-  const double t42 = e3 * inv((r - qb) * (r - qb) + aqq), t44 = e3 * inv((r + qb) * (r + qb) + aqq);
-  const double t46 = e3 * inv((r + qa) * (r + qa) + aqq), t48 = e3 * inv((r - qa) * (r - qa) + aqq);
-  auto sq = [](double x) { return x * x; };
+  const S r2 = r * r;
+  auto inv = [](S x) { return inv_root(x); };
+  const S ee = kEV * inv(r2 + aee);
+  const S dze = -e1 * inv((r + da) * (r + da) + ade) + e1 * inv((r - da) * (r - da) + ade);
+  const S c6 = e1 * inv(r2 + aqe);
+  const S qzze = e2 * inv((r - qa) * (r - qa) + aqe) + e2 * inv((r + qa) * (r + qa) + aqe) - c6;
+  const S qxxe = e1 * inv(r2 + qa * qa + aqe) - c6;
+  const S edz = -e1 * inv((r - db) * (r - db) + aed) + e1 * inv((r + db) * (r + db) + aed);
+  const S c12 = e1 * inv(r2 + aeq);
+  const S eqzz = e2 * inv((r - qb) * (r - qb) + aeq) + e2 * inv((r + qb) * (r + qb) + aeq) - c12;
+  const S eqxx = e1 * inv(r2 + qb * qb + aeq) - c12;
+  const S t20 = e2 * inv((r + da) * (r + da) + adq), t22 = e2 * inv((r - da) * (r - da) + adq);
+  const S t24 = e2 * inv((r - db) * (r - db) + aqd), t26 = e2 * inv((r + db) * (r + db) + aqd);
+  const S t36 = e2 * inv(r2 + aqq), t39 = e2 * inv(r2 + qa * qa + aqq), t40 = e2 * inv(r2 + qb * qb + aqq);
+  const S t42 = e3 * inv((r - qb) * (r - qb) + aqq), t44 = e3 * inv((r + qb) * (r + qb) + aqq);
+  const S t46 = e3 * inv((r + qa) * (r + qa) + aqq), t48 = e3 * inv((r - qa) * (r - qa) + aqq);
+  auto sq = [](auto x) { return x * x; };
   ri[0] = ee;
   ri[1] = -dze;
   ri[2] = ee + qzze;
@@ -129,31 +208,32 @@ __device__ void local_xx(double r, double da, double db, double qa1, double qb1,
            t42 - t44 - t39 + t36;
   ri[17] = ee + eqxx + qzze + e3 * inv(sq(r + qa) + qb * qb + aqq) + e3 * inv(sq(r - qa) + qb * qb + aqq) -
            t46 - t48 - t40 + t36;
-  const double qxxqxx = e3 * inv(r2 + sq(qa - qb) + aqq) + e3 * inv(r2 + sq(qa + qb) + aqq) - t39 - t40 + t36;
+  const S qxxqxx = e3 * inv(r2 + sq(qa - qb) + aqq) + e3 * inv(r2 + sq(qa + qb) + aqq) - t39 - t40 + t36;
   ri[18] = ee + eqxx + qxxe + qxxqxx;
   const double dm = sq(qa1 - qb1), dp = sq(qa1 + qb1);
   ri[19] = e3 * inv(sq(r + qa1 - qb1) + dm + aqq) - e3 * inv(sq(r + qa1 + qb1) + dm + aqq) -
            e3 * inv(sq(r - qa1 - qb1) + dm + aqq) + e3 * inv(sq(r - qa1 + qb1) + dm + aqq) -
            e3 * inv(sq(r + qa1 - qb1) + dp + aqq) + e3 * inv(sq(r + qa1 + qb1) + dp + aqq) +
            e3 * inv(sq(r - qa1 - qb1) + dp + aqq) - e3 * inv(sq(r - qa1 + qb1) + dp + aqq);
-  const double qxxqyy = e2 * inv(r2 + qa * qa + qb * qb + aqq) - t39 - t40 + t36;
+  const S qxxqyy = e2 * inv(r2 + qa * qa + qb * qb + aqq) - t39 - t40 + t36;
   ri[20] = ee + eqxx + qxxe + qxxqyy;
   ri[21] = 0.5 * (qxxqxx - qxxqyy);
 }
 
 // 4 heavy-H integrals (two_elec_two_center_int_local_frame.py:90-107)
-__device__ void local_xh(double r, double da, double qa1, double r0a, double r1a, double r2a,
-                         double r0b, double ri[4]) {
+template <class S>
+__device__ inline void local_xh(S r, double da, double qa1, double r0a, double r1a, double r2a,
+                         double r0b, S ri[4]) {
   const double e1 = kEV * 0.5, e2 = kEV * 0.25;
   const double qa = 2.0 * qa1;
   const double aee = (r0a + r0b) * (r0a + r0b), ade = (r1a + r0b) * (r1a + r0b);
   const double aqe = (r2a + r0b) * (r2a + r0b);
-  const double ee = kEV / sqrt(r * r + aee);
-  const double c = e1 / sqrt(r * r + aqe);
+  const S ee = quot_root(kEV, r * r + aee);
+  const S c = quot_root(e1, r * r + aqe);
   ri[0] = ee;
-  ri[1] = e1 / sqrt((r + da) * (r + da) + ade) - e1 / sqrt((r - da) * (r - da) + ade);
-  ri[2] = ee + e2 / sqrt((r + qa) * (r + qa) + aqe) + e2 / sqrt((r - qa) * (r - qa) + aqe) - c;
-  ri[3] = ee + e1 / sqrt(r * r + qa * qa + aqe) - c;
+  ri[1] = quot_root(e1, (r + da) * (r + da) + ade) - quot_root(e1, (r - da) * (r - da) + ade);
+  ri[2] = ee + quot_root(e2, (r + qa) * (r + qa) + aqe) + quot_root(e2, (r - qa) * (r - qa) + aqe) - c;
+  ri[3] = ee + quot_root(e1, r * r + qa * qa + aqe) - c;
 }
 
 // Rotation with R v = e_x built from the quaternion of v (two_elec_two_center_int.py:1576-1631),
@@ -227,15 +307,17 @@ __device__ inline void local_tensor(const double ri[22], double Lm[10][10]) {
 // ------------------------------------------------------------------- STO overlaps
 // A_k(x) = int_1^inf t^k e^{-xt} dt and B_k(x) = int_-1^1 t^k e^{-xt} dt, k = 0..6, with the
 // reference's recurrences / truncated series (diat_overlap_PM6_SP.py:464-670).
-__device__ inline void aint7(double x, double a[7]) {
-  if (x == 0.0) {
+template <class S>
+__device__ inline void aint7(S x, S a[7]) {
+  if (value_of(x) == 0.0) {
 #pragma unroll
-    for (int k = 0; k < 7; ++k) a[k] = 0.0;
+    for (int k = 0; k < 7; ++k) a[k] = constant<S>(0.0);
     return;
   }
-  a[0] = exp(-x) / x;
+  const S rx = recip(x);
+  a[0] = over(exp_of(-x), x, rx);
 #pragma unroll
-  for (int k = 1; k < 7; ++k) a[k] = a[0] + k * a[k - 1] / x;
+  for (int k = 1; k < 7; ++k) a[k] = a[0] + over((double)k * a[k - 1], x, rx);
 }
 
 // Branch of bint7 at argument x: 2 recurrence (|x| > 0.5), 1 truncated series, 0 x ~ 0.
@@ -246,15 +328,17 @@ __device__ inline int bint_branch(double x) {
 
 // forced >= 0 evaluates that branch regardless of x (finite differences of a pair energy keep the
 // branch of the geometry they differentiate, as the reference's autograd does).
-__device__ inline void bint7(double x, double b[7], int forced = -1) {
-  const int br = forced >= 0 ? forced : bint_branch(x);
+template <class S>
+__device__ inline void bint7(S x, S b[7], int forced = -1) {
+  const int br = forced >= 0 ? forced : bint_branch(value_of(x));
   if (br == 2) {
-    const double tx = exp(x) / x, tmx = -exp(-x) / x;
+    const S rx = recip(x);
+    const S tx = over(exp_of(x), x, rx), tmx = over(-exp_of(-x), x, rx);
     b[0] = tx + tmx;
 #pragma unroll
-    for (int k = 1; k < 7; ++k) b[k] = ((k & 1) ? -tx : tx) + tmx + k * b[k - 1] / x;
+    for (int k = 1; k < 7; ++k) b[k] = ((k & 1) ? -tx : tx) + tmx + over((double)k * b[k - 1], x, rx);
   } else if (br == 1) {
-    const double x2 = x * x, x3 = x2 * x, x4 = x2 * x2, x5 = x4 * x, x6 = x4 * x2;
+    const S x2 = x * x, x3 = x2 * x, x4 = x2 * x2, x5 = x4 * x, x6 = x4 * x2;
     b[0] = 2.0 + x2 / 3.0 + x4 / 60.0 + x6 / 2520.0;
     b[2] = 2.0 / 3.0 + x2 / 5.0 + x4 / 84.0 + x6 / 3240.0;
     b[4] = 2.0 / 5.0 + x2 / 7.0 + x4 / 108.0 + x6 / 3960.0;
@@ -263,7 +347,9 @@ __device__ inline void bint7(double x, double b[7], int forced = -1) {
     b[3] = -2.0 / 5.0 * x - x3 / 21.0 - x5 / 540.0;
     b[5] = -2.0 / 7.0 * x - x3 / 27.0 - x5 / 660.0;
   } else {
-    b[0] = 2.0; b[1] = 0.0; b[2] = 2.0 / 3.0; b[3] = 0.0; b[4] = 2.0 / 5.0; b[5] = 0.0; b[6] = 2.0 / 7.0;
+    const double at0[7] = {2.0, 0.0, 2.0 / 3.0, 0.0, 2.0 / 5.0, 0.0, 2.0 / 7.0};
+#pragma unroll
+    for (int k = 0; k < 7; ++k) b[k] = constant<S>(at0[k]);
   }
 }
 
@@ -287,72 +373,73 @@ __device__ inline int overlap_branches(double r, double zas, double zap, double 
 // S[0..4] = S111 (s|s), S211 (p_sig(i)|s(j)), S121, S221, S222 in the diatomic frame
 // (diat_overlap_PM6_SP.py:84-345).  za/zb = (zeta_s, zeta_p) of atoms i / j.
 // bsel >= 0: B-integral branches (overlap_branches) to use instead of those of r.
-__device__ void overlap_local(int jc, double r, double zas, double zap, double zbs, double zbp,
-                              bool need_p_i, bool need_p_j, double S[5], int bsel = -1) {
-  S[0] = S[1] = S[2] = S[3] = S[4] = 0.0;
-  double A[7], B[7];
+template <class T>
+__device__ inline void overlap_local(int jc, T r, double zas, double zap, double zbs, double zbp,
+                              bool need_p_i, bool need_p_j, T S[5], int bsel = -1) {
+  S[0] = S[1] = S[2] = S[3] = S[4] = constant<T>(0.0);
+  T A[7], B[7];
   const double s3 = 1.7320508075688772;
   const double s10 = 3.1622776601683795, s30 = 5.477225575051661;
   auto AB = [&](double z1, double z2) {
     const int ci = (z1 == zas ? 0 : 1) | (z2 == zbs ? 0 : 2);
-    aint7(0.5 * r * (z1 + z2), A);
-    bint7(0.5 * r * (z1 - z2), B, bsel >= 0 ? (bsel >> (2 * ci)) & 3 : -1);
+    aint7<T>(0.5 * r * (z1 + z2), A);
+    bint7<T>(0.5 * r * (z1 - z2), B, bsel >= 0 ? (bsel >> (2 * ci)) & 3 : -1);
   };
   if (jc == 2) {
     AB(zas, zbs);
-    S[0] = pow(zas * zbs * r * r, 1.5) * (A[2] * B[0] - B[2] * A[0]) / 4.0;
+    S[0] = pow_3_2(zas * zbs * r * r) * (A[2] * B[0] - B[2] * A[0]) / 4.0;
   } else if (jc == 3) {
-    const double r4 = r * r * r * r;
+    const T r4 = r * r * r * r;
     AB(zas, zbs);
-    S[0] = pow(zbs, 1.5) * pow(zas, 2.5) * r4 * (A[3] * B[0] - B[3] * A[0] + A[2] * B[1] - B[2] * A[1]) / (s3 * 8.0);
+    S[0] = half_pow(r, zbs, 1) * half_pow(r, zas, 2) * r4 * (A[3] * B[0] - B[3] * A[0] + A[2] * B[1] - B[2] * A[1]) / (s3 * 8.0);
     if (need_p_i) {
       AB(zap, zbs);
-      S[1] = pow(zbs, 1.5) * pow(zap, 2.5) * r4 * (A[2] * B[0] - B[2] * A[0] + A[3] * B[1] - B[3] * A[1]) / 8.0;
+      S[1] = half_pow(r, zbs, 1) * half_pow(r, zap, 2) * r4 * (A[2] * B[0] - B[2] * A[0] + A[3] * B[1] - B[3] * A[1]) / 8.0;
     }
   } else if (jc == 4) {
-    const double r5 = r * r * r * r * r;
+    const T r5 = r * r * r * r * r;
     AB(zas, zbs);
-    S[0] = pow(zbs * zas, 2.5) * r5 * (A[4] * B[0] + B[4] * A[0] - 2.0 * A[2] * B[2]) / 48.0;
+    S[0] = half_pow(r, zbs * zas, 2) * r5 * (A[4] * B[0] + B[4] * A[0] - 2.0 * A[2] * B[2]) / 48.0;
     AB(zap, zbs);
-    S[1] = pow(zbs * zap, 2.5) * r5 *
+    S[1] = half_pow(r, zbs * zap, 2) * r5 *
            (A[3] * (B[0] - B[2]) - A[1] * (B[2] - B[4]) + B[3] * (A[0] - A[2]) - B[1] * (A[2] - A[4])) /
            (16.0 * s3);
     AB(zas, zbp);
-    S[2] = pow(zbp * zas, 2.5) * r5 *
+    S[2] = half_pow(r, zbp * zas, 2) * r5 *
            (A[3] * (B[0] - B[2]) - A[1] * (B[2] - B[4]) - B[3] * (A[0] - A[2]) + B[1] * (A[2] - A[4])) /
            (16.0 * s3);
     AB(zap, zbp);
-    const double w = pow(zbp * zap, 2.5) * r5 / 16.0;
+    const T w = half_pow(r, zbp * zap, 2) * r5 / 16.0;
     S[3] = -w * (B[2] * (A[4] + A[0]) - A[2] * (B[4] + B[0]));
     S[4] = 0.5 * w * (A[4] * (B[0] - B[2]) - B[4] * (A[0] - A[2]) - A[2] * B[0] + B[2] * A[0]);
   } else if (jc == 431) {
-    const double r5 = r * r * r * r * r;
+    const T r5 = r * r * r * r * r;
     AB(zas, zbs);
-    S[0] = pow(zbs, 1.5) * pow(zas, 3.5) * r5 *
+    S[0] = half_pow(r, zbs, 1) * half_pow(r, zas, 3) * r5 *
            (A[4] * B[0] + 2.0 * B[1] * A[3] - 2.0 * A[1] * B[3] - B[4] * A[0]) / (s10 * 24.0);
     if (need_p_i) {
       AB(zap, zbs);
-      S[1] = pow(zbs, 1.5) * pow(zap, 3.5) * r5 *
+      S[1] = half_pow(r, zbs, 1) * half_pow(r, zap, 3) * r5 *
              (A[3] * (B[0] + B[2]) - A[1] * (B[4] + B[2]) + B[1] * (A[2] + A[4]) - B[3] * (A[2] + A[0])) /
              (8.0 * s30);
     }
   } else if (jc == 5) {
-    const double r6 = r * r * r * r * r * r;
+    const T r6 = r * r * r * r * r * r;
     AB(zas, zbs);
-    S[0] = pow(zbs, 2.5) * pow(zas, 3.5) * r6 *
+    S[0] = half_pow(r, zbs, 2) * half_pow(r, zas, 3) * r6 *
            (A[5] * B[0] + B[1] * A[4] - 2.0 * B[2] * A[3] - 2.0 * A[2] * B[3] + B[4] * A[1] + B[5] * A[0]) /
            (s30 * 48.0);
     AB(zap, zbs);
-    S[1] = pow(zbs, 2.5) * pow(zap, 3.5) * r6 *
+    S[1] = half_pow(r, zbs, 2) * half_pow(r, zap, 3) * r6 *
            (A[4] * B[0] + B[1] * A[5] - 2.0 * B[3] * A[3] - 2.0 * A[2] * B[2] + A[1] * B[5] + A[0] * B[4]) /
            (48.0 * s10);
     AB(zas, zbp);
-    S[2] = pow(zbp, 2.5) * pow(zas, 3.5) * r6 *
+    S[2] = half_pow(r, zbp, 2) * half_pow(r, zas, 3) * r6 *
            ((A[4] * B[0] - A[5] * B[1]) + 2.0 * (A[3] * B[1] - A[4] * B[2]) - 2.0 * (A[1] * B[3] - A[2] * B[4]) -
             (A[0] * B[4] - A[1] * B[5])) /
            (48.0 * s10);
     AB(zap, zbp);
-    const double pre = pow(zbp, 2.5) * pow(zap, 3.5) * r6;
+    const T pre = half_pow(r, zbp, 2) * half_pow(r, zap, 3) * r6;
     S[3] = pre *
            ((A[3] * B[0] - A[5] * B[2]) + (A[2] * B[1] - A[4] * B[3]) - (A[1] * B[2] - A[3] * B[4]) -
             (A[0] * B[3] - A[2] * B[5])) /
@@ -362,21 +449,21 @@ __device__ void overlap_local(int jc, double r, double zas, double zap, double z
             (A[2] - A[0]) * (B[3] - B[5])) /
            (32.0 * s30);
   } else if (jc == 6) {
-    const double r7 = r * r * r * r * r * r * r;
+    const T r7 = r * r * r * r * r * r * r;
     AB(zas, zbs);
-    S[0] = pow(zbs * zas, 3.5) * r7 * (A[6] * B[0] - 3.0 * B[2] * A[4] + 3.0 * A[2] * B[4] - A[0] * B[6]) / 1440.0;
+    S[0] = half_pow(r, zbs * zas, 3) * r7 * (A[6] * B[0] - 3.0 * B[2] * A[4] + 3.0 * A[2] * B[4] - A[0] * B[6]) / 1440.0;
     AB(zap, zbs);
-    S[1] = pow(zbs * zap, 3.5) * r7 *
+    S[1] = half_pow(r, zbs * zap, 3) * r7 *
            ((A[5] * B[0] + A[6] * B[1]) + (-A[4] * B[1] - A[5] * B[2]) - 2.0 * (A[3] * B[2] + A[4] * B[3]) -
             2.0 * (-A[2] * B[3] - A[3] * B[4]) + (A[1] * B[4] + A[2] * B[5]) + (-A[0] * B[5] - A[1] * B[6])) /
            (480.0 * s3);
     AB(zas, zbp);
-    S[2] = pow(zbp * zas, 3.5) * r7 *
+    S[2] = half_pow(r, zbp * zas, 3) * r7 *
            ((A[5] * B[0] - A[6] * B[1]) + (A[4] * B[1] - A[5] * B[2]) - 2.0 * (A[3] * B[2] - A[4] * B[3]) -
             2.0 * (A[2] * B[3] - A[3] * B[4]) + (A[1] * B[4] - A[2] * B[5]) + (A[0] * B[5] - A[1] * B[6])) /
            (480.0 * s3);
     AB(zap, zbp);
-    const double pre = pow(zbp, 3.5) * pow(zap, 3.5) * r7;
+    const T pre = half_pow(r, zbp, 3) * half_pow(r, zap, 3) * r7;
     S[3] = pre * ((A[4] * B[0] - A[6] * B[2]) - 2.0 * (A[2] * B[2] - A[4] * B[4]) + (A[0] * B[4] - A[2] * B[6])) / 480.0;
     S[4] = pre *
            ((A[6] - A[4]) * (B[0] - B[2]) - 2.0 * (A[4] - A[2]) * (B[2] - B[4]) + (A[2] - A[0]) * (B[4] - B[6])) /
@@ -386,25 +473,26 @@ __device__ void overlap_local(int jc, double r, double zas, double zap, double z
 }
 
 // --------------------------------------------------------------- core-core repulsion
-__device__ double core_repulsion(int method, int Zi, int Zj, double rbohr, double gam, const double* pi,
-                            const double* pj) {
-  const double ra = rbohr * kA0;
+template <class S>
+__device__ inline S core_repulsion(int method, int Zi, int Zj, S rbohr, S gam, const double* pi,
+                           const double* pj) {
+  const S ra = rbohr * kA0;
   const double ti = pi[PAR_TORE], tj = pj[PAR_TORE];
-  const double t1 = ti * tj * gam;
-  double t2 = exp(-pi[PAR_ALPHA] * ra);
-  if ((Zi == 7 || Zi == 8) && Zj == 1) t2 *= ra;
-  const double t3 = exp(-pj[PAR_ALPHA] * ra);
-  double e = t1 * (1.0 + t2 + t3);
+  const S t1 = ti * tj * gam;
+  S t2 = exp_of(-pi[PAR_ALPHA] * ra);
+  if ((Zi == 7 || Zi == 8) && Zj == 1) t2 = t2 * ra;
+  const S t3 = exp_of(-pj[PAR_ALPHA] * ra);
+  S e = t1 * (1.0 + t2 + t3);
   const int ng = method == PYSEQM_AM1 ? 4 : (method == PYSEQM_PM3 ? 2 : 0);
   if (ng) {
-    double g = 0.0;
+    S g = constant<S>(0.0);
     for (int k = 0; k < ng; ++k) {
       const double* ki = pi + PAR_GAUSS + 3 * k;
       const double* kj = pj + PAR_GAUSS + 3 * k;
-      g += ki[0] * exp(-ki[1] * (ra - ki[2]) * (ra - ki[2]));
-      g += kj[0] * exp(-kj[1] * (ra - kj[2]) * (ra - kj[2]));
+      g = g + ki[0] * exp_of(-ki[1] * (ra - ki[2]) * (ra - ki[2]));
+      g = g + kj[0] * exp_of(-kj[1] * (ra - kj[2]) * (ra - kj[2]));
     }
-    e += ti * tj / ra * g;
+    e = e + quot(ti * tj, ra) * g;
   }
   return e;
 }
@@ -691,15 +779,272 @@ __device__ void load_pair_density(const double* Pm, int n, int ai, int aj, PairD
     for (int b = 0; b < 4; ++b) D.pab[a][b] = (a < NI && b < NJ) ? Pm[(size_t)(ai + a) * n + aj + b] : 0.0;
 }
 
-// Forces: dE_pair/dR (R = r_j - r_i, Angstrom) by a 4th-order central difference of the pair
-// energy at fixed density (step h); +dE/dR on atom i, -dE/dR on atom j, reduced per tile.
+// The nonzero elements of the local tensor (local_tensor): local pair of atom i, of atom j, integral.
+__device__ constexpr int kLocP[34] = {0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 2, 2, 2, 2, 2, 5, 5, 5, 5, 5, 9, 9, 9, 9, 9,
+                                      3, 3, 4, 4, 6, 6, 7, 7, 8};
+__device__ constexpr int kLocQ[34] = {0, 1, 2, 5, 9, 0, 1, 2, 5, 9, 0, 1, 2, 5, 9, 0, 1, 2, 5, 9, 0, 1, 2, 5, 9,
+                                      3, 4, 3, 4, 6, 7, 6, 7, 8};
+__device__ constexpr int kLocM[34] = {0,  4,  10, 11, 11, 1,  5,  12, 13, 13, 2,  7,  15, 17, 17, 3,  8,
+                                      16, 18, 20, 3,  8,  16, 20, 18, 6,  14, 9,  19, 6,  14, 9,  19, 21};
+
+// Density blocks of a pair in its local frame (orbitals s, sigma, pi, pi'; a hydrogen has s only).
+struct LocalDensity {
+  double a[10], b[10];  // diagonal blocks, tril, plain
+  double c[4][4];       // block (i, j)
+};
+
+template <int NI, int NJ>
+__device__ inline void to_local(const PairDensity& P, const double R[3][3], LocalDensity& out) {
+  auto tri = [&](const double (&v)[10], double (&o)[10]) {  // v: off-diagonal entries doubled
+    o[0] = v[0];
+    double m[3][3];
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+#pragma unroll
+      for (int y = 0; y < 3; ++y) m[x][y] = (x == y ? 1.0 : 0.5) * v[tri_index(1 + x, 1 + y)];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      o[tri_index(1 + x, 0)] = 0.5 * (R[x][0] * v[1] + R[x][1] * v[3] + R[x][2] * v[6]);
+      double t[3];
+#pragma unroll
+      for (int y = 0; y < 3; ++y) t[y] = R[x][0] * m[0][y] + R[x][1] * m[1][y] + R[x][2] * m[2][y];
+#pragma unroll
+      for (int y = 0; y <= x; ++y) o[tri_index(1 + x, 1 + y)] = t[0] * R[y][0] + t[1] * R[y][1] + t[2] * R[y][2];
+    }
+  };
+  if constexpr (NI == 4) tri(P.pa, out.a);
+  if constexpr (NJ == 4) tri(P.pb, out.b);
+  if constexpr (NI == 1) out.a[0] = P.pa[0];
+  if constexpr (NJ == 1) out.b[0] = P.pb[0];
+  double t[4][4];
+#pragma unroll
+  for (int y = 0; y < NJ; ++y) {
+    t[0][y] = P.pab[0][y];
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+      if (NI == 4) t[1 + x][y] = R[x][0] * P.pab[1][y] + R[x][1] * P.pab[2][y] + R[x][2] * P.pab[3][y];
+  }
+#pragma unroll
+  for (int x = 0; x < NI; ++x) {
+    out.c[x][0] = t[x][0];
+#pragma unroll
+    for (int y = 0; y < 3; ++y)
+      if (NJ == 4) out.c[x][1 + y] = R[y][0] * t[x][1] + R[y][1] * t[x][2] + R[y][2] * t[x][3];
+  }
+}
+
+// The change of a local block element when the axis turns towards local orbital K (2: pi, 3: pi'):
+// d sigma = orbital K, d (orbital K) = - sigma, on the first (second) index where the atom has p orbitals.
+template <int K>
+__device__ inline double turn_tri(const double (&m)[10], int x, int y) {
+  double d = 0.0;
+  if (x == 1) d += m[tri_index(K, y)];
+  if (x == K) d -= m[tri_index(1, y)];
+  if (y == 1) d += m[tri_index(x, K)];
+  if (y == K) d -= m[tri_index(x, 1)];
+  return d;
+}
+template <int K, int NI, int NJ>
+__device__ inline double turn_ab(const double (&m)[4][4], int x, int y) {
+  double d = 0.0;
+  if (NI == 4 && x == 1) d += m[K][y];
+  if (NI == 4 && x == K) d -= m[1][y];
+  if (NJ == 4 && y == 1) d += m[x][K];
+  if (NJ == 4 && y == K) d -= m[x][1];
+  return d;
+}
+
+// Two-electron (and, with ELCORE, electron-core) potential of the local density M, contracted with
+// the change of the local density X as the axis turns towards pi (t[0]) and pi' (t[1]).
+template <int KIND, bool ELCORE>
+__device__ inline void axis_torque(const Dual* ri, const LocalDensity& M, const LocalDensity& X, double ti, double tj,
+                                   double (&t)[2]) {
+  constexpr int NJ = KIND == XX ? 4 : 1;
+  constexpr int NE = KIND == XX ? 34 : 5;
+  double ja[10], jb[10], K[4][4];
+#pragma unroll
+  for (int k = 0; k < 10; ++k) ja[k] = jb[k] = 0.0;
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) K[x][y] = 0.0;
+  constexpr int xhP[5] = {0, 1, 2, 5, 9}, xhM[5] = {0, 1, 2, 3, 3};
+#pragma unroll
+  for (int q = 0; q < NE; ++q) {
+    const int p = KIND == XX ? kLocP[q] : xhP[q], o = KIND == XX ? kLocQ[q] : 0;
+    const double w = ri[KIND == XX ? kLocM[q] : xhM[q]].v;
+    const int mu = kTriI[p], nu = kTriJ[p], la = kTriI[o], si = kTriJ[o];
+    ja[p] += (la == si ? w : 2.0 * w) * M.b[o];
+    if (ELCORE && o == 0) ja[p] -= tj * w;
+    if (KIND == XX) {
+      jb[o] += (mu == nu ? w : 2.0 * w) * M.a[p];
+      if (ELCORE && p == 0) jb[o] -= ti * w;
+    }
+    K[mu][la] += w * M.c[nu][si];
+    if (mu != nu) K[nu][la] += w * M.c[mu][si];
+    if (la != si) K[mu][si] += w * M.c[nu][la];
+    if (mu != nu && la != si) K[nu][si] += w * M.c[mu][la];
+  }
+#pragma unroll
+  for (int p = 1; p < 10; ++p) {
+    const int mu = kTriI[p], nu = kTriJ[p];
+    const double f = mu == nu ? 1.0 : 2.0;
+    t[0] += f * ja[p] * turn_tri<2>(X.a, mu, nu);
+    t[1] += f * ja[p] * turn_tri<3>(X.a, mu, nu);
+    if (KIND == XX) {
+      t[0] += f * jb[p] * turn_tri<2>(X.b, mu, nu);
+      t[1] += f * jb[p] * turn_tri<3>(X.b, mu, nu);
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+#pragma unroll
+    for (int y = 0; y < NJ; ++y) {
+      t[0] -= K[x][y] * turn_ab<2, 4, NJ>(X.c, x, y);
+      t[1] -= K[x][y] * turn_ab<3, 4, NJ>(X.c, x, y);
+    }
+}
+
+// dE_pair/dR (R = r_j - r_i, Angstrom) of pair_energy (MODE 0, or 1 with XL) at fixed densities, in
+// closed form.  In the frame of the pair axis the energy is sum_m c_m ri_m(r) (22 local integrals, c_m
+// bilinear in the local densities) + sum_m o_m S_m(r) (5 overlaps) + core repulsion(r): the
+// derivative along the axis takes each of those functions of r once with its derivative (Dual), and the
+// two derivatives across the axis are the turns of the local densities under the local potential.
+// Inside the antipodal fallback cone a frame is constant (the reference's autograd gives it no
+// derivative), which drops that frame's part across the axis; the overlaps keep their B-integral branch.
+// Bound: FP64 VALU and its latencies (about 64 inverse roots and 8 exponentials per heavy-heavy pair),
+// one wave per SIMD in the heavy-heavy kernel (256 VGPRs and as many accumulation registers).  Against
+// 12 displaced energies per pair (4th-order differences, each rotating all 100 integrals) on 512
+// alkanes of 2-30 carbons: heavy-heavy 1156 -> 42 us, heavy-H 393 -> 35 us, H-H 187 -> 24 us; one
+// ethane 311 -> 17 us.  The differences agree with it to 2e-10 of the force norm, their rounding.
+template <int KIND, bool XL>
+__device__ inline void pair_gradient(int method, const double (&R0)[3], const double* pi, const double* pj,
+                                     const PairDensity& P, const PairDensity& D, double (&G)[3]) {
+  constexpr int NI = KIND == HH ? 1 : 4;
+  constexpr int NJ = KIND == XX ? 4 : 1;
+  const PairGeom g = geom_from_vector(R0[0], R0[1], R0[2]);
+  const Dual r = {g.r, 1.0};
+  const double ti = pi[PAR_TORE], tj = pj[PAR_TORE];
+  double along = 0.0;                  // dE/dr, eV/bohr
+  double across[3] = {0.0, 0.0, 0.0};  // dE/d(unit vector i -> j), before projection off the axis
+  // resonance: sum 2 D_ab H_ab
+  if (g.r <= kOverlapCut) {
+    const bool fixed = quat_flips(g.x[0]);
+    double Rp[3][3];
+    quat_frame(g.x[0], g.x[1], g.x[2], Rp, fixed ? 2 : 1);
+    const double u[3] = {Rp[0][0], Rp[0][1], Rp[0][2]};
+    Dual S[5];
+    overlap_local<Dual>(jcall_of((int)pi[PAR_QN], (int)pj[PAR_QN]), r, pi[PAR_ZS], pi[PAR_ZP], pj[PAR_ZS],
+                        pj[PAR_ZP], NI == 4, NJ == 4, S);
+    along += D.pab[0][0] * (pi[PAR_BS] + pj[PAR_BS]) * S[0].d;
+    if constexpr (NI == 4) {
+      const double bps = pi[PAR_BP] + pj[PAR_BS];
+      along += bps * (D.pab[1][0] * u[0] + D.pab[2][0] * u[1] + D.pab[3][0] * u[2]) * S[1].d;
+      if (!fixed)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) across[m] += bps * S[1].v * D.pab[1 + m][0];
+    }
+    if constexpr (NJ == 4) {
+      const double bsp = pi[PAR_BS] + pj[PAR_BP], bpp = pi[PAR_BP] + pj[PAR_BP];
+      along -= bsp * (D.pab[0][1] * u[0] + D.pab[0][2] * u[1] + D.pab[0][3] * u[2]) * S[2].d;
+      double du[3], duu = 0.0;
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        du[m] = 0.0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) du[m] += (D.pab[1 + m][1 + k] + D.pab[1 + k][1 + m]) * u[k];
+        duu += 0.5 * du[m] * u[m];
+      }
+      const double tr = D.pab[1][1] + D.pab[2][2] + D.pab[3][3];
+      along += bpp * ((tr - duu) * S[4].d - duu * S[3].d);
+      if (!fixed)
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+          across[m] -= bsp * S[2].v * D.pab[0][1 + m] + bpp * (S[3].v + S[4].v) * du[m];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);  // the overlaps' registers are free again below
+  // two-electron, electron-core and core-core terms
+  Dual gam;
+  if constexpr (KIND == HH) {
+    const double rho = pi[PAR_RHO0] + pj[PAR_RHO0];
+    gam = quot_root(kEV, r * r + rho * rho);
+    const double cw = XL ? D.pa[0] * P.pb[0] + P.pa[0] * D.pb[0] - P.pa[0] * P.pb[0] : P.pa[0] * P.pb[0];
+    const double xw = XL ? D.pab[0][0] - 0.5 * P.pab[0][0] : 0.5 * P.pab[0][0];
+    along += (cw - tj * D.pa[0] - ti * D.pb[0] - xw * P.pab[0][0]) * gam.d;
+  } else {
+    const bool fixed = quat_flips(-g.x[0]);
+    double R[3][3];
+    quat_frame(-g.x[0], -g.x[1], -g.x[2], R, fixed ? 2 : 1);
+    LocalDensity Pl, Dl;
+    to_local<NI, NJ>(P, R, Pl);
+    if constexpr (XL) to_local<NI, NJ>(D, R, Dl);
+    Dual ri[22];
+    if constexpr (KIND == XX)
+      local_xx<Dual>(r, pi[PAR_DD], pj[PAR_DD], pi[PAR_QQ], pj[PAR_QQ], pi[PAR_RHO0], pj[PAR_RHO0], pi[PAR_RHO1],
+                     pj[PAR_RHO1], pi[PAR_RHO2], pj[PAR_RHO2], ri);
+    else
+      local_xh<Dual>(r, pi[PAR_DD], pi[PAR_QQ], pi[PAR_RHO0], pi[PAR_RHO1], pi[PAR_RHO2], pj[PAR_RHO0], ri);
+    gam = ri[0];
+    const LocalDensity& E = XL ? Dl : Pl;
+    constexpr int NE = KIND == XX ? 34 : 5;
+    constexpr int xhP[5] = {0, 1, 2, 5, 9}, xhM[5] = {0, 1, 2, 3, 3};
+    auto xw = [&](int x, int y) { return XL ? Dl.c[x][y] - 0.5 * Pl.c[x][y] : 0.5 * Pl.c[x][y]; };
+#pragma unroll
+    for (int q = 0; q < NE; ++q) {
+      const int p = KIND == XX ? kLocP[q] : xhP[q], o = KIND == XX ? kLocQ[q] : 0;
+      const int mu = kTriI[p], nu = kTriJ[p], la = kTriI[o], si = kTriJ[o];
+      double c = XL ? Dl.a[p] * Pl.b[o] + Pl.a[p] * (Dl.b[o] - Pl.b[o]) : Pl.a[p] * Pl.b[o];
+      if (o == 0) c -= tj * E.a[p];
+      if (mu != nu) c *= 2.0;
+      double cb = 0.0;
+      if (p == 0) cb = ti * E.b[o];
+      if (la != si) {
+        c *= 2.0;
+        cb *= 2.0;
+      }
+      c -= cb;
+      c -= xw(mu, la) * Pl.c[nu][si];
+      if (mu != nu) c -= xw(nu, la) * Pl.c[mu][si];
+      if (la != si) c -= xw(mu, si) * Pl.c[nu][la];
+      if (mu != nu && la != si) c -= xw(nu, si) * Pl.c[mu][la];
+      along += c * ri[KIND == XX ? kLocM[q] : xhM[q]].d;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (!fixed) {
+      double t[2] = {0.0, 0.0};
+      axis_torque<KIND, true>(ri, Pl, E, ti, tj, t);
+      if constexpr (XL) {  // the potential of D - P on the turn of P
+#pragma unroll
+        for (int k = 0; k < 10; ++k) {
+          Dl.a[k] -= Pl.a[k];
+          if (NJ == 4 || k == 0) Dl.b[k] -= Pl.b[k];
+        }
+#pragma unroll
+        for (int x = 0; x < NI; ++x)
+#pragma unroll
+          for (int y = 0; y < NJ; ++y) Dl.c[x][y] -= Pl.c[x][y];
+        axis_torque<KIND, false>(ri, Dl, Pl, ti, tj, t);
+      }
+      // the frame's sigma points from j to i: turning it towards pi moves the unit vector i -> j by -pi
+#pragma unroll
+      for (int m = 0; m < 3; ++m) across[m] -= t[0] * R[1][m] + t[1] * R[2][m];
+    }
+  }
+  along += core_repulsion<Dual>(method, (int)pi[PAR_Z], (int)pj[PAR_Z], r, gam, pi, pj).d;
+  const double off = across[0] * g.x[0] + across[1] * g.x[1] + across[2] * g.x[2];
+  const double rd = 1.0 / (g.r * kA0);
+#pragma unroll
+  for (int m = 0; m < 3; ++m) G[m] = along * (1.0 / kA0) * g.x[m] + rd * (across[m] - off * g.x[m]);
+}
+
+// Forces: +dE/dR on atom i, -dE/dR on atom j, reduced per tile.
 // XL: Dm is the density contracted with H (the XL-BOMD D), P the propagated field.
 template <int KIND, bool XL>
 __global__ __launch_bounds__(64) void k_pair_forces(pyseqm_layout_t L, int method, int tile_base,
                                                      const double* __restrict__ coords,
                                                      const double* __restrict__ par, const double* __restrict__ P,
-                                                     const double* __restrict__ Dm, double h,
-                                                     double* __restrict__ part) {
+                                                     const double* __restrict__ Dm, double* __restrict__ part) {
   const int tile = tile_base + xcd_run(blockIdx.x, gridDim.x);
   const int lane = threadIdx.x;
   const Tile t = load_tile(L.tiles, tile);
@@ -717,30 +1062,11 @@ __global__ __launch_bounds__(64) void k_pair_forces(pyseqm_layout_t L, int metho
     PairDensity Pd, Dd;
     load_pair_density<NI, NJ>(P + mo, n, ai, aj, Pd);
     if constexpr (XL) load_pair_density<NI, NJ>(Dm + mo, n, ai, aj, Dd);
-    const PairDensity& Dr = XL ? Dd : Pd;
     const double R0[3] = {coords[3 * j] - coords[3 * i], coords[3 * j + 1] - coords[3 * i + 1],
                           coords[3 * j + 2] - coords[3 * i + 2]};
-    const double c1 = 8.0 / (12.0 * h), c2 = -1.0 / (12.0 * h);
-    const PairGeom g0 = geom_from_vector(R0[0], R0[1], R0[2]);
-    const int wmode = quat_flips(-g0.x[0]) ? 2 : 1;  // frame of -x_ij (integrals)
-    const int smode = quat_flips(g0.x[0]) ? 2 : 1;   // frame of +x_ij (overlaps)
-    const int bsel = overlap_branches(g0.r, pi[PAR_ZS], pi[PAR_ZP], pj[PAR_ZS], pj[PAR_ZP]);
-#pragma unroll 1
-    for (int x = 0; x < 3; ++x) {
-      double gx = 0.0;
-#pragma unroll 1
-      for (int sgn = -2; sgn <= 2; ++sgn) {
-        if (sgn == 0) continue;
-        double R[3] = {R0[0], R0[1], R0[2]};
-        R[x] += sgn * h;
-        const double e =
-            pair_energy<KIND, XL>(method, geom_from_vector(R[0], R[1], R[2]), pi, pj, Pd, Dr, wmode, smode, bsel);
-        const double c = (sgn == 1 || sgn == -1) ? c1 : c2;
-        gx += (sgn > 0 ? c : -c) * e;
-      }
-      rowv[x] = gx;    // force on i = -dE/dr_i = +dE/dR
-      colv[x] = -gx;   // force on j
-    }
+    pair_gradient<KIND, XL>(method, R0, pi, pj, Pd, XL ? Dd : Pd, rowv);
+#pragma unroll
+    for (int x = 0; x < 3; ++x) colv[x] = -rowv[x];
   }
   write_partials(part, tile, lane, rowv, colv);
 }
@@ -1061,13 +1387,13 @@ int launch_pair_forces(const pyseqm_layout_t* L, int method, const double* coord
   hipStream_t s = (hipStream_t)stream;
   int base = 0;
   if (L->ntile[0])
-    k_pair_forces<XX, XL><<<L->ntile[0], 64, 0, s>>>(*L, method, base, coords, atom_par, P, D, h, part);
+    k_pair_forces<XX, XL><<<L->ntile[0], 64, 0, s>>>(*L, method, base, coords, atom_par, P, D, part);
   base += L->ntile[0];
   if (L->ntile[1])
-    k_pair_forces<XH, XL><<<L->ntile[1], 64, 0, s>>>(*L, method, base, coords, atom_par, P, D, h, part);
+    k_pair_forces<XH, XL><<<L->ntile[1], 64, 0, s>>>(*L, method, base, coords, atom_par, P, D, part);
   base += L->ntile[1];
   if (L->ntile[2])
-    k_pair_forces<HH, XL><<<L->ntile[2], 64, 0, s>>>(*L, method, base, coords, atom_par, P, D, h, part);
+    k_pair_forces<HH, XL><<<L->ntile[2], 64, 0, s>>>(*L, method, base, coords, atom_par, P, D, part);
   if (L->natoms) {
     if (lanes_per_atom(L) == 64)
       k_atom_forces<64><<<(L->natoms + 3) / 4, 256, 0, s>>>(*L, part, forces);

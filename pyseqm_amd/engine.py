@@ -453,7 +453,8 @@ class SCFEngine:
 
     def forces(self, P, h=1.0e-3):
         """Forces (natoms, 3) in eV/Angstrom at fixed density P (Hellmann-Feynman, the reference's
-        autograd force with scf_backward = 0, basics.py:1315-1336)."""
+        autograd force with scf_backward = 0, basics.py:1315-1336).  The pair gradients are closed-form:
+        `h` (a step length once) has to be positive and has no other effect."""
         b = self.b
         out = torch.zeros(max(b.natoms, 1), 3, dtype=torch.float64, device=self.device)
         nat.call("pyseqm_pair_forces", b.L, nat.METHODS[self.method], nat.ptr(self.coords), nat.ptr(self.atom_par),
