@@ -17,6 +17,8 @@ using namespace pyseqm;
 
 namespace {
 
+enum { XX = 0, XH = 1, HH = 2 };  // tile kinds: heavy-heavy, heavy-H, H-H
+
 __device__ constexpr double kTore[19] = {0, 1, 0, 1, 2, 3, 4, 5, 6, 7, 0, 1, 2, 3, 4, 5, 6, 7, 0};
 __device__ constexpr int kQn[19] = {0, 1, 1, 2, 2, 2, 2, 2, 2, 2, 2, 3, 3, 3, 3, 3, 3, 3, 3};
 
@@ -129,17 +131,34 @@ __device__ inline double over(double a, double x, double) { return a / x; }
 __device__ inline Dual over(Dual a, Dual, Dual rx) { return a * rx; }
 __device__ inline double quot(double a, double x) { return a / x; }
 __device__ inline Dual quot(double a, Dual x) { return a * recip(x); }
-// x^(k + 1/2) of a constant, in a formula on doubles / on Duals
+// x^(k + 1/2), k >= 1, of an exponent product at distance r: on doubles, and where r or x is a Dual
 __device__ inline double half_pow(double, double x, int k) { return pow(x, k + 0.5); }
 __device__ inline double half_pow(Dual, double x, int k) {
   double p = sqrt(x);
   for (int t = 0; t < k; ++t) p *= x;
   return p;
 }
+__device__ inline Dual half_pow(double, Dual x, int k) {
+  double p = sqrt(x.v);
+  for (int t = 1; t < k; ++t) p *= x.v;
+  return {p * x.v, (k + 0.5) * p * x.d};
+}
 __device__ inline double pow_3_2(double x) { return pow(x, 1.5); }
 __device__ inline Dual pow_3_2(Dual x) {
   const double q = sqrt(x.v);
   return {x.v * q, 1.5 * q * x.d};
+}
+// r as a value of its own at each use in a formula on Duals: the A and B integrals of the four exponent
+// pairs are then evaluated where they are used, one pair's after another's, and not all together ahead
+// of the branches that share them (112 doubles alive, which spilled)
+template <class T>
+__device__ inline double once(double r) {
+  if constexpr (sizeof(T) == sizeof(Dual)) asm volatile("" : "+v"(r));
+  return r;
+}
+template <class T>
+__device__ inline Dual once(Dual r) {
+  return {once<T>(r.v), r.d};
 }
 template <class S>
 __device__ inline S constant(double x);
@@ -239,8 +258,8 @@ __device__ inline void local_xh(S r, double da, double qa1, double r0a, double r
 // Rotation with R v = e_x built from the quaternion of v (two_elec_two_center_int.py:1576-1631),
 // including its antipodal fallback (|1 + v_x| < 1e-7 -> constant 180 deg turn about z).
 // mode 0: as the reference; 1: never take the fallback (smooth in v); 2: always the fallback.
-// Finite differences use 1 or 2 chosen from the undisplaced geometry, which reproduces the
-// reference's autograd derivative (zero frame derivative inside the fallback cone).
+// Gradients take 1 or 2 by quat_flips, which reproduces the reference's autograd derivative (zero
+// frame derivative inside the fallback cone).
 __device__ inline bool quat_flips(double vx) { return fabs(1.0 + vx) < 1.0e-7; }
 
 __device__ inline void quat_frame(double vx, double vy, double vz, double R[3][3], int mode = 0) {
@@ -326,11 +345,9 @@ __device__ inline int bint_branch(double x) {
   return ax > 0.5 ? 2 : (ax > 1.0e-6 ? 1 : 0);
 }
 
-// forced >= 0 evaluates that branch regardless of x (finite differences of a pair energy keep the
-// branch of the geometry they differentiate, as the reference's autograd does).
 template <class S>
-__device__ inline void bint7(S x, S b[7], int forced = -1) {
-  const int br = forced >= 0 ? forced : bint_branch(value_of(x));
+__device__ inline void bint7(S x, S b[7]) {
+  const int br = bint_branch(value_of(x));
   if (br == 2) {
     const S rx = recip(x);
     const S tx = over(exp_of(x), x, rx), tmx = over(-exp_of(-x), x, rx);
@@ -363,41 +380,34 @@ __device__ inline int jcall_of(int qi, int qj) {
   return 0;
 }
 
-// Branches of the B integrals for the four exponent pairs (s_i s_j, p_i s_j, s_i p_j, p_i p_j),
-// 2 bits each.
-__device__ inline int overlap_branches(double r, double zas, double zap, double zbs, double zbp) {
-  return bint_branch(0.5 * r * (zas - zbs)) | (bint_branch(0.5 * r * (zap - zbs)) << 2) |
-         (bint_branch(0.5 * r * (zas - zbp)) << 4) | (bint_branch(0.5 * r * (zap - zbp)) << 6);
-}
-
 // S[0..4] = S111 (s|s), S211 (p_sig(i)|s(j)), S121, S221, S222 in the diatomic frame
 // (diat_overlap_PM6_SP.py:84-345).  za/zb = (zeta_s, zeta_p) of atoms i / j.
-// bsel >= 0: B-integral branches (overlap_branches) to use instead of those of r.
-template <class T>
-__device__ inline void overlap_local(int jc, T r, double zas, double zap, double zbs, double zbp,
-                              bool need_p_i, bool need_p_j, T S[5], int bsel = -1) {
+// T is the type of the results: Dual where r or the exponents are.  KIND (XX, XH, HH) limits the code
+// to the formulas that a tile of that kind can meet.
+template <class T, int KIND, class Rt, class Zt>
+__device__ inline void overlap_local(int jc, Rt r, Zt zas, Zt zap, Zt zbs, Zt zbp, bool need_p_i, T S[5]) {
   S[0] = S[1] = S[2] = S[3] = S[4] = constant<T>(0.0);
   T A[7], B[7];
   const double s3 = 1.7320508075688772;
   const double s10 = 3.1622776601683795, s30 = 5.477225575051661;
-  auto AB = [&](double z1, double z2) {
-    const int ci = (z1 == zas ? 0 : 1) | (z2 == zbs ? 0 : 2);
-    aint7<T>(0.5 * r * (z1 + z2), A);
-    bint7<T>(0.5 * r * (z1 - z2), B, bsel >= 0 ? (bsel >> (2 * ci)) & 3 : -1);
+  auto AB = [&](Zt z1, Zt z2) {
+    const Rt h = 0.5 * once<T>(r);
+    aint7<T>(h * (z1 + z2), A);
+    bint7<T>(h * (z1 - z2), B);
   };
-  if (jc == 2) {
+  if (KIND == HH && jc == 2) {
     AB(zas, zbs);
     S[0] = pow_3_2(zas * zbs * r * r) * (A[2] * B[0] - B[2] * A[0]) / 4.0;
-  } else if (jc == 3) {
-    const T r4 = r * r * r * r;
+  } else if (KIND == XH && jc == 3) {
+    const Rt r4 = r * r * r * r;
     AB(zas, zbs);
     S[0] = half_pow(r, zbs, 1) * half_pow(r, zas, 2) * r4 * (A[3] * B[0] - B[3] * A[0] + A[2] * B[1] - B[2] * A[1]) / (s3 * 8.0);
     if (need_p_i) {
       AB(zap, zbs);
       S[1] = half_pow(r, zbs, 1) * half_pow(r, zap, 2) * r4 * (A[2] * B[0] - B[2] * A[0] + A[3] * B[1] - B[3] * A[1]) / 8.0;
     }
-  } else if (jc == 4) {
-    const T r5 = r * r * r * r * r;
+  } else if (KIND == XX && jc == 4) {
+    const Rt r5 = r * r * r * r * r;
     AB(zas, zbs);
     S[0] = half_pow(r, zbs * zas, 2) * r5 * (A[4] * B[0] + B[4] * A[0] - 2.0 * A[2] * B[2]) / 48.0;
     AB(zap, zbs);
@@ -412,8 +422,8 @@ __device__ inline void overlap_local(int jc, T r, double zas, double zap, double
     const T w = half_pow(r, zbp * zap, 2) * r5 / 16.0;
     S[3] = -w * (B[2] * (A[4] + A[0]) - A[2] * (B[4] + B[0]));
     S[4] = 0.5 * w * (A[4] * (B[0] - B[2]) - B[4] * (A[0] - A[2]) - A[2] * B[0] + B[2] * A[0]);
-  } else if (jc == 431) {
-    const T r5 = r * r * r * r * r;
+  } else if (KIND == XH && jc == 431) {
+    const Rt r5 = r * r * r * r * r;
     AB(zas, zbs);
     S[0] = half_pow(r, zbs, 1) * half_pow(r, zas, 3) * r5 *
            (A[4] * B[0] + 2.0 * B[1] * A[3] - 2.0 * A[1] * B[3] - B[4] * A[0]) / (s10 * 24.0);
@@ -423,8 +433,8 @@ __device__ inline void overlap_local(int jc, T r, double zas, double zap, double
              (A[3] * (B[0] + B[2]) - A[1] * (B[4] + B[2]) + B[1] * (A[2] + A[4]) - B[3] * (A[2] + A[0])) /
              (8.0 * s30);
     }
-  } else if (jc == 5) {
-    const T r6 = r * r * r * r * r * r;
+  } else if (KIND == XX && jc == 5) {
+    const Rt r6 = r * r * r * r * r * r;
     AB(zas, zbs);
     S[0] = half_pow(r, zbs, 2) * half_pow(r, zas, 3) * r6 *
            (A[5] * B[0] + B[1] * A[4] - 2.0 * B[2] * A[3] - 2.0 * A[2] * B[3] + B[4] * A[1] + B[5] * A[0]) /
@@ -448,8 +458,8 @@ __device__ inline void overlap_local(int jc, T r, double zas, double zap, double
            ((A[5] - A[3]) * (B[0] - B[2]) + (A[4] - A[2]) * (B[1] - B[3]) - (A[3] - A[1]) * (B[2] - B[4]) -
             (A[2] - A[0]) * (B[3] - B[5])) /
            (32.0 * s30);
-  } else if (jc == 6) {
-    const T r7 = r * r * r * r * r * r * r;
+  } else if (KIND == XX && jc == 6) {
+    const Rt r7 = r * r * r * r * r * r * r;
     AB(zas, zbs);
     S[0] = half_pow(r, zbs * zas, 3) * r7 * (A[6] * B[0] - 3.0 * B[2] * A[4] + 3.0 * A[2] * B[4] - A[0] * B[6]) / 1440.0;
     AB(zap, zbs);
@@ -469,7 +479,6 @@ __device__ inline void overlap_local(int jc, T r, double zas, double zap, double
            ((A[6] - A[4]) * (B[0] - B[2]) - 2.0 * (A[4] - A[2]) * (B[2] - B[4]) + (A[2] - A[0]) * (B[4] - B[6])) /
            960.0;
   }
-  (void)need_p_j;
 }
 
 // --------------------------------------------------------------- core-core repulsion
@@ -520,12 +529,12 @@ __device__ inline PairGeom pair_geom(const double* coords, int i, int j) {
 // Molecular-frame two-electron integrals of a heavy-heavy pair, column by column:
 // fn(k, l, (mu nu|la si)) for k = tril(mu, nu) on atom i and l = tril(la, si) on atom j.
 template <class Fn>
-__device__ inline void xx_integrals(const PairGeom& g, const double* pi, const double* pj, Fn&& fn, int fmode = 0) {
+__device__ inline void xx_integrals(const PairGeom& g, const double* pi, const double* pj, Fn&& fn) {
   double ri[22];
   local_xx(g.r, pi[PAR_DD], pj[PAR_DD], pi[PAR_QQ], pj[PAR_QQ], pi[PAR_RHO0], pj[PAR_RHO0], pi[PAR_RHO1],
            pj[PAR_RHO1], pi[PAR_RHO2], pj[PAR_RHO2], ri);
   double R[3][3];
-  quat_frame(-g.x[0], -g.x[1], -g.x[2], R, fmode);
+  quat_frame(-g.x[0], -g.x[1], -g.x[2], R);
   double T[10][10], Lm[10][10];
   pair_map(R, T);
   local_tensor(ri, Lm);
@@ -551,11 +560,11 @@ __device__ inline void xx_integrals(const PairGeom& g, const double* pi, const d
 
 // Heavy-H integrals (mu nu|s s), k = tril(mu, nu) on the heavy atom i.
 template <class Fn>
-__device__ inline void xh_integrals(const PairGeom& g, const double* pi, const double* pj, Fn&& fn, int fmode = 0) {
+__device__ inline void xh_integrals(const PairGeom& g, const double* pi, const double* pj, Fn&& fn) {
   double ri[4];
   local_xh(g.r, pi[PAR_DD], pi[PAR_QQ], pi[PAR_RHO0], pi[PAR_RHO1], pi[PAR_RHO2], pj[PAR_RHO0], ri);
   double R[3][3];
-  quat_frame(-g.x[0], -g.x[1], -g.x[2], R, fmode);
+  quat_frame(-g.x[0], -g.x[1], -g.x[2], R);
   double T[10][10];
   pair_map(R, T);
 #pragma unroll
@@ -568,8 +577,7 @@ __device__ inline double hh_integral(const PairGeom& g, const double* pi, const 
 
 // Off-diagonal core block H_ij[a][b] = S_ij[a][b] (beta_a(i) + beta_b(j)) / 2 for NI x NJ orbitals.
 template <int NI, int NJ>
-__device__ inline void core_block(const PairGeom& g, const double* pi, const double* pj, double Hb[4][4],
-                                  int fmode = 0, int bsel = -1) {
+__device__ inline void core_block(const PairGeom& g, const double* pi, const double* pj, double Hb[4][4]) {
   double di[4][4];
 #pragma unroll
   for (int a = 0; a < 4; ++a)
@@ -578,9 +586,10 @@ __device__ inline void core_block(const PairGeom& g, const double* pi, const dou
   if (g.r <= kOverlapCut) {
     const int jc = jcall_of((int)pi[PAR_QN], (int)pj[PAR_QN]);  // validated on the host
     double S[5];
-    overlap_local(jc, g.r, pi[PAR_ZS], pi[PAR_ZP], pj[PAR_ZS], pj[PAR_ZP], NI == 4, NJ == 4, S, bsel);
+    overlap_local<double, NJ == 4 ? XX : NI == 4 ? XH : HH>(jc, g.r, pi[PAR_ZS], pi[PAR_ZP], pj[PAR_ZS], pj[PAR_ZP],
+                                                             NI == 4, S);
     double Rp[3][3];
-    quat_frame(g.x[0], g.x[1], g.x[2], Rp, fmode);
+    quat_frame(g.x[0], g.x[1], g.x[2], Rp);
     di[0][0] = S[0];
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
@@ -605,7 +614,6 @@ __device__ inline void core_block(const PairGeom& g, const double* pi, const dou
 }
 
 // ------------------------------------------------------------------- tile kernels
-enum { XX = 0, XH = 1, HH = 2 };
 
 template <int KIND>
 __global__ __launch_bounds__(64) void k_pair_tiles(pyseqm_layout_t L, int method, int tile_base,
@@ -693,76 +701,6 @@ struct PairDensity {
   double pa[10], pb[10];  // diagonal blocks, tril, off-diagonal entries doubled
   double pab[4][4];       // block (i, j)
 };
-
-// MODE 0: the pair's share of Eelec(P) + E_nuc; 1 (XL-BOMD): of sum D F(P) - 1/2 sum (F(P) - H) P +
-// E_nuc; 2 (linear): of sum D F(P), no core repulsion (rep_out = 0).
-template <int KIND, int MODE>
-__device__ double pair_energy(int method, const PairGeom& g, const double* pi, const double* pj,
-                              const PairDensity& P, const PairDensity& D, int wmode, int smode, int bsel,
-                              double* rep_out = nullptr) {
-  constexpr int NI = KIND == HH ? 1 : 4;
-  constexpr int NJ = KIND == XX ? 4 : 1;
-  const double ti = pi[PAR_TORE], tj = pj[PAR_TORE];
-  double e = 0.0, gam = 0.0;
-  // Coulomb weight of w_kl: P_a P_b (plain), D_a P_b + P_a D_b - P_a P_b (XL), D_a P_b + P_a D_b (linear)
-  auto coul = [&](int k, int l) {
-    return MODE == 1   ? D.pa[k] * P.pb[l] + P.pa[k] * D.pb[l] - P.pa[k] * P.pb[l]
-           : MODE == 2 ? D.pa[k] * P.pb[l] + P.pa[k] * D.pb[l]
-                       : P.pa[k] * P.pb[l];
-  };
-  // exchange weight: 1/2 P_ab (plain), D_ab - 1/2 P_ab (XL), D_ab (linear), times K(P)_ab
-  auto xw = [&](int a, int b) {
-    return MODE == 1 ? D.pab[a][b] - 0.5 * P.pab[a][b] : MODE == 2 ? D.pab[a][b] : 0.5 * P.pab[a][b];
-  };
-  if constexpr (KIND == XX) {
-    double K[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) K[a][b] = 0.0;
-    xx_integrals(g, pi, pj, [&](int k, int l, double w) {
-      const int mu = kTriI[k], nu = kTriJ[k], la = kTriI[l], si = kTriJ[l];
-      e += coul(k, l) * w;
-      if (l == 0) e -= tj * D.pa[k] * w;
-      if (k == 0) e -= ti * D.pb[l] * w;
-      if (k == 0 && l == 0) gam = w;
-      K[mu][la] += w * P.pab[nu][si];
-      if (mu != nu) K[nu][la] += w * P.pab[mu][si];
-      if (la != si) K[mu][si] += w * P.pab[nu][la];
-      if (mu != nu && la != si) K[nu][si] += w * P.pab[mu][la];
-    }, wmode);
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) e -= xw(a, b) * K[a][b];
-  } else if constexpr (KIND == XH) {
-    double K[4] = {0.0, 0.0, 0.0, 0.0};
-    xh_integrals(g, pi, pj, [&](int k, double w) {
-      const int mu = kTriI[k], nu = kTriJ[k];
-      e += coul(k, 0) * w - tj * D.pa[k] * w;
-      if (k == 0) {
-        gam = w;
-        e -= ti * D.pb[0] * w;
-      }
-      K[mu] += w * P.pab[nu][0];
-      if (mu != nu) K[nu] += w * P.pab[mu][0];
-    }, wmode);
-#pragma unroll
-    for (int a = 0; a < 4; ++a) e -= xw(a, 0) * K[a];
-  } else {
-    gam = hh_integral(g, pi, pj);
-    e = (coul(0, 0) - tj * D.pa[0] - ti * D.pb[0] - xw(0, 0) * P.pab[0][0]) * gam;
-  }
-  double Hb[4][4];
-  core_block<NI, NJ>(g, pi, pj, Hb, smode, bsel);
-#pragma unroll
-  for (int a = 0; a < NI; ++a)
-#pragma unroll
-    for (int b = 0; b < NJ; ++b) e += 2.0 * D.pab[a][b] * Hb[a][b];
-  const double rep = MODE == 2 ? 0.0 : core_repulsion(method, (int)pi[PAR_Z], (int)pj[PAR_Z], g.r, gam, pi, pj);
-  if (rep_out) *rep_out = rep;
-  return e + rep;
-}
 
 template <int NI, int NJ>
 __device__ void load_pair_density(const double* Pm, int n, int ai, int aj, PairDensity& D) {
@@ -905,8 +843,7 @@ __device__ inline void axis_torque(const Dual* ri, const LocalDensity& M, const 
     }
 }
 
-// dE_pair/dR (R = r_j - r_i, Angstrom) of pair_energy (MODE 0, or 1 with XL) at fixed densities, in
-// closed form.  In the frame of the pair axis the energy is sum_m c_m ri_m(r) (22 local integrals, c_m
+// dE_pair/dR (R = r_j - r_i, Angstrom) of the pair energy above at fixed densities, in closed form.  In the frame of the pair axis the energy is sum_m c_m ri_m(r) (22 local integrals, c_m
 // bilinear in the local densities) + sum_m o_m S_m(r) (5 overlaps) + core repulsion(r): the
 // derivative along the axis takes each of those functions of r once with its derivative (Dual), and the
 // two derivatives across the axis are the turns of the local densities under the local potential.
@@ -934,8 +871,8 @@ __device__ inline void pair_gradient(int method, const double (&R0)[3], const do
     quat_frame(g.x[0], g.x[1], g.x[2], Rp, fixed ? 2 : 1);
     const double u[3] = {Rp[0][0], Rp[0][1], Rp[0][2]};
     Dual S[5];
-    overlap_local<Dual>(jcall_of((int)pi[PAR_QN], (int)pj[PAR_QN]), r, pi[PAR_ZS], pi[PAR_ZP], pj[PAR_ZS],
-                        pj[PAR_ZP], NI == 4, NJ == 4, S);
+    overlap_local<Dual, KIND>(jcall_of((int)pi[PAR_QN], (int)pj[PAR_QN]), r, pi[PAR_ZS], pi[PAR_ZP], pj[PAR_ZS],
+                              pj[PAR_ZP], NI == 4, S);
     along += D.pab[0][0] * (pi[PAR_BS] + pj[PAR_BS]) * S[0].d;
     if constexpr (NI == 4) {
       const double bps = pi[PAR_BP] + pj[PAR_BS];
@@ -1086,126 +1023,395 @@ __global__ __launch_bounds__(256) void k_atom_forces(pyseqm_layout_t L, const do
 // At a converged closed-shell SCF density the energy is stationary in P, so dE/dtheta is the
 // derivative at fixed P: the gradient the reference's autograd returns through H, the integrals and
 // the core repulsion when the SCF density is detached (scf_backward = 0, scf_loop.py:1996-2031;
-// learned parameters re-packed per call, basics.py:781-789).  Each pair's energy (its Eelec share and
-// its core repulsion) depends on the input slots below of its two atoms, through the multipoles
-// (dd, qq, rho0/1/2), the overlaps, the resonance integrals and the core-repulsion terms; a
-// 4th-order central difference of the pair energy in each slot, with the overlap branches pinned at
-// the unperturbed values, gives that pair's share.  U_ss, U_pp and g_sp reach the one-center terms
-// only, which k_param_onecenter differentiates in closed form.
-__device__ constexpr int kPairParams[21] = {PAR_ZS,        PAR_ZP,        PAR_BS,        PAR_BP,        PAR_GSS,
-                                            PAR_GPP,       PAR_GP2,       PAR_HSP,       PAR_ALPHA,     PAR_GAUSS,
-                                            PAR_GAUSS + 1, PAR_GAUSS + 2, PAR_GAUSS + 3, PAR_GAUSS + 4, PAR_GAUSS + 5,
-                                            PAR_GAUSS + 6, PAR_GAUSS + 7, PAR_GAUSS + 8, PAR_GAUSS + 9,
-                                            PAR_GAUSS + 10, PAR_GAUSS + 11};
-constexpr int kParamGroup = 5;  // slots per pass: 2 values (Eelec, core repulsion) each in a 10-wide partial
-__host__ __device__ inline int pair_param_count(int method) {
-  return method == PYSEQM_AM1 ? 21 : (method == PYSEQM_PM3 ? 15 : 9);
-}
-// Step of slot k of a record: hrel * max(|value|, 0.1).
-__device__ inline double param_step(const double* p, int k, double hrel) { return hrel * fmax(fabs(p[k]), 0.1); }
-__device__ constexpr int kStencil[4] = {-2, -1, 1, 2};
-__device__ constexpr double kStencilW[4] = {1.0 / 12.0, -8.0 / 12.0, 8.0 / 12.0, -1.0 / 12.0};
+// learned parameters re-packed per call, basics.py:781-789).  A pair's energy depends on the inputs of
+// its two atoms through few quantities per atom (kPV below), and its derivatives in them are closed:
+//   * the multipoles dd, qq, rho0, rho1, rho2: the two-electron and electron-core terms are
+//     sum_m c_m ri_m, with c_m bilinear in the densities rotated to the pair's frame and every ri_m a
+//     sum of inverse roots, which are differentiated one by one (charge_terms);
+//   * rho0 once more through the core repulsion's (ss|ss);
+//   * the exponents, through the 5 overlaps (Dual, on the B-integral branch of the pair);
+//   * the resonance integrals, which enter linearly, alpha and the Gaussians.
+// k_param_jacobian has the derivative of each atom's multipoles in its inputs (4th-order differences of
+// derive_atom, whose secant iterations have no short closed form), and k_param_gather joins the two.
+// U_ss, U_pp and g_sp reach the one-center terms only, which k_param_onecenter differentiates.
+// One pass over the pairs with 23 values per side, where displaced energies took 4 x 2 x 21 pair energies
+// in 5 passes: on 32 alkanes of 1-8 carbons 6760 -> 37 us (+ 42 us
+// for the Jacobian).
+constexpr int kPV = 23;  // dd qq rho0 rho1 rho2 | core repulsion's rho0 | zs zp bs bp | alpha | 12 Gaussian
+enum { PV_DD = 0, PV_QQ, PV_R0, PV_R1, PV_R2, PV_REP, PV_ZS, PV_ZP, PV_BS, PV_BP, PV_ALPHA, PV_GAUSS };
+constexpr int kJacSlots = 6;
+__device__ constexpr int kJacParam[kJacSlots] = {PAR_ZS, PAR_ZP, PAR_GSS, PAR_GPP, PAR_GP2, PAR_HSP};
+__device__ constexpr int kJacOut[5] = {PAR_DD, PAR_QQ, PAR_RHO0, PAR_RHO1, PAR_RHO2};
 
-// rec[((a * kParamGroup + g) * 4 + s) * NPAR ...]: atom a's record with slot kPairParams[p0 + g]
-// moved by kStencil[s] steps and the derived slots recomputed.  One thread per (atom, g, s).
-__global__ void k_param_records(pyseqm_layout_t L, const double* __restrict__ par, int p0, int np, double hrel,
-                                double* __restrict__ rec) {
+// jac[(a * 6 + k) * 5 + y]: d(multipole kJacOut[y])/d(input kJacParam[k]) of atom a, by 4th-order central
+// differences with step hrel * max(|value|, 0.1).  One thread per (atom, input).
+__global__ void k_param_jacobian(pyseqm_layout_t L, const double* __restrict__ par, double hrel,
+                                 double* __restrict__ jac) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int s = t & 3, g = (t >> 2) % kParamGroup, a = (t >> 2) / kParamGroup;
-  if (a >= L.natoms || g >= np) return;
+  const int a = t / kJacSlots, k = t - a * kJacSlots;
+  if (a >= L.natoms) return;
   const double* src = par + (size_t)a * PYSEQM_NPAR;
-  double* q = rec + ((size_t)(a * kParamGroup + g) * 4 + s) * PYSEQM_NPAR;
-  for (int k = 0; k < PYSEQM_NPAR; ++k) q[k] = src[k];
-  const int slot = kPairParams[p0 + g];
-  q[slot] = src[slot] + kStencil[s] * param_step(src, slot, hrel);
-  derive_atom(q, L.atom_Z[a]);
+  const int slot = kJacParam[k], Z = L.atom_Z[a];
+  const double h = hrel * fmax(fabs(src[slot]), 0.1);
+  double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  for (int s = -2; s <= 2; ++s) {
+    if (s == 0) continue;
+    double q[PYSEQM_NPAR];
+    for (int i = 0; i < PYSEQM_NPAR; ++i) q[i] = src[i];
+    q[slot] = src[slot] + s * h;
+    derive_atom(q, Z);
+    const double w = s == -2 ? 1.0 : (s == -1 ? -8.0 : (s == 1 ? 8.0 : -1.0));
+    for (int y = 0; y < 5; ++y) acc[y] += w * q[kJacOut[y]];
+  }
+  for (int y = 0; y < 5; ++y) jac[(size_t)t * 5 + y] = acc[y] / (12.0 * h);
 }
 
-// Per pair and slot of the pass: d(pair Eelec share)/d(slot) and d(core repulsion)/d(slot) for
-// atom i (row partial values 2g, 2g + 1) and for atom j (column partial); MODE 2: the pair's share
-// of d(sum Y F(P))/d(slot) (no core repulsion) for a symmetric Y.
+// d(sum_m c_m ri_m)/d(multipoles) of a heavy-heavy pair (local_xx): ga for atom i, gb for atom j, in the
+// order dd, qq, rho0, rho1, rho2.  Every term is A / sqrt(u^2 + v^2 + (rho_a + rho_b)^2) with u, v
+// linear in r, da, db, qa, qb; g = -A / root^3 times u, v or the rho sum gives its derivatives.
+struct ChargeTerms {
+  double da, db, qa, qb;        // the charge offsets (qa, qb: local_xx's qa1, qb1)
+  double ra[3], rb[3];          // rho0, rho1, rho2
+  double gda, gdb, gqa, gqb;    // derivatives in the offsets
+  double gra[3], grb[3];        // derivatives in the rhos
+  // A / sqrt((r + s_da da + ..)^2 + (t_da da + ..)^2 + (rho_I + rho_J)^2)
+  template <int I, int J>
+  __device__ inline void term(double r, double A, double sda, double sdb, double sqa, double sqb, double tda = 0.0,
+                              double tdb = 0.0, double tqa = 0.0, double tqb = 0.0) {
+    const double u = r + sda * da + sdb * db + sqa * qa + sqb * qb;
+    const double v = tda * da + tdb * db + tqa * qa + tqb * qb;
+    const double w = ra[I] + rb[J];
+    const double q = rsq_nr(u * u + v * v + w * w);
+    const double g = -A * (q * q * q);
+    gda += g * (sda * u + tda * v);
+    gdb += g * (sdb * u + tdb * v);
+    gqa += g * (sqa * u + tqa * v);
+    gqb += g * (sqb * u + tqb * v);
+    gra[I] += g * w;
+    grb[J] += g * w;
+  }
+};
+
+__device__ inline void charge_terms_xx(double r, const double (&c)[22], ChargeTerms& t) {
+  const double e1 = kEV * 0.5, e2 = kEV * 0.25, e3 = kEV * 0.125, e4 = kEV * 0.0625;
+  const double ee = c[0] + c[2] + c[3] + c[10] + c[11] + c[15] + c[16] + c[17] + c[18] + c[20];
+  t.term<0, 0>(r, kEV * ee, 0, 0, 0, 0);
+  const double dze = -(c[1] + c[12] + c[13]);
+  t.term<1, 0>(r, -e1 * dze, 1, 0, 0, 0);
+  t.term<1, 0>(r, e1 * dze, -1, 0, 0, 0);
+  const double edz = -(c[4] + c[7] + c[8]);
+  t.term<0, 1>(r, -e1 * edz, 0, -1, 0, 0);
+  t.term<0, 1>(r, e1 * edz, 0, 1, 0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  const double qzze = c[2] + c[15] + c[17], qxxe = c[3] + c[16] + c[18] + c[20];
+  t.term<2, 0>(r, e2 * qzze, 0, 0, -2, 0);
+  t.term<2, 0>(r, e2 * qzze, 0, 0, 2, 0);
+  t.term<2, 0>(r, -e1 * (qzze + qxxe), 0, 0, 0, 0);
+  t.term<2, 0>(r, e1 * qxxe, 0, 0, 0, 0, 0, 0, 2, 0);
+  const double eqzz = c[10] + c[15] + c[16], eqxx = c[11] + c[17] + c[18] + c[20];
+  t.term<0, 2>(r, e2 * eqzz, 0, 0, 0, -2);
+  t.term<0, 2>(r, e2 * eqzz, 0, 0, 0, 2);
+  t.term<0, 2>(r, -e1 * (eqzz + eqxx), 0, 0, 0, 0);
+  t.term<0, 2>(r, e1 * eqxx, 0, 0, 0, 0, 0, 0, 0, 2);
+  // dipole-dipole
+  __builtin_amdgcn_sched_barrier(0);
+  t.term<1, 1>(r, e2 * c[5], 1, -1, 0, 0);
+  t.term<1, 1>(r, e2 * c[5], -1, 1, 0, 0);
+  t.term<1, 1>(r, -e2 * c[5], -1, -1, 0, 0);
+  t.term<1, 1>(r, -e2 * c[5], 1, 1, 0, 0);
+  t.term<1, 1>(r, e1 * c[6], 0, 0, 0, 0, 1, -1, 0, 0);
+  t.term<1, 1>(r, -e1 * c[6], 0, 0, 0, 0, 1, 1, 0, 0);
+  // quadrupole (i) - dipole (j)
+  __builtin_amdgcn_sched_barrier(0);
+  const double c78 = c[7] + c[8];
+  t.term<2, 1>(r, -e2 * c78, 0, -1, 0, 0);
+  t.term<2, 1>(r, e2 * c78, 0, 1, 0, 0);
+  t.term<2, 1>(r, e3 * c[7], 0, -1, 2, 0);
+  t.term<2, 1>(r, -e3 * c[7], 0, 1, 2, 0);
+  t.term<2, 1>(r, e3 * c[7], 0, -1, -2, 0);
+  t.term<2, 1>(r, -e3 * c[7], 0, 1, -2, 0);
+  t.term<2, 1>(r, e2 * c[8], 0, -1, 0, 0, 0, 0, 2, 0);
+  t.term<2, 1>(r, -e2 * c[8], 0, 1, 0, 0, 0, 0, 2, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  t.term<2, 1>(r, e2 * c[9], 0, 0, 1, 0, 0, -1, 1, 0);
+  t.term<2, 1>(r, -e2 * c[9], 0, 0, -1, 0, 0, -1, 1, 0);
+  t.term<2, 1>(r, -e2 * c[9], 0, 0, 1, 0, 0, 1, 1, 0);
+  t.term<2, 1>(r, e2 * c[9], 0, 0, -1, 0, 0, 1, 1, 0);
+  // dipole (i) - quadrupole (j)
+  __builtin_amdgcn_sched_barrier(0);
+  const double c1213 = c[12] + c[13];
+  t.term<1, 2>(r, -e2 * c1213, 1, 0, 0, 0);
+  t.term<1, 2>(r, e2 * c1213, -1, 0, 0, 0);
+  t.term<1, 2>(r, e3 * c[12], 1, 0, 0, -2);
+  t.term<1, 2>(r, -e3 * c[12], -1, 0, 0, -2);
+  t.term<1, 2>(r, e3 * c[12], 1, 0, 0, 2);
+  t.term<1, 2>(r, -e3 * c[12], -1, 0, 0, 2);
+  t.term<1, 2>(r, e2 * c[13], 1, 0, 0, 0, 0, 0, 0, 2);
+  t.term<1, 2>(r, -e2 * c[13], -1, 0, 0, 0, 0, 0, 0, 2);
+  __builtin_amdgcn_sched_barrier(0);
+  t.term<1, 2>(r, e2 * c[14], 0, 0, 0, -1, 1, 0, 0, -1);
+  t.term<1, 2>(r, -e2 * c[14], 0, 0, 0, 1, 1, 0, 0, -1);
+  t.term<1, 2>(r, -e2 * c[14], 0, 0, 0, -1, 1, 0, 0, 1);
+  t.term<1, 2>(r, e2 * c[14], 0, 0, 0, 1, 1, 0, 0, 1);
+  // quadrupole-quadrupole
+  __builtin_amdgcn_sched_barrier(0);
+  t.term<2, 2>(r, e4 * c[15], 0, 0, 2, -2);
+  t.term<2, 2>(r, e4 * c[15], 0, 0, 2, 2);
+  t.term<2, 2>(r, e4 * c[15], 0, 0, -2, -2);
+  t.term<2, 2>(r, e4 * c[15], 0, 0, -2, 2);
+  t.term<2, 2>(r, -e3 * (c[15] + c[16]), 0, 0, 0, -2);
+  t.term<2, 2>(r, -e3 * (c[15] + c[16]), 0, 0, 0, 2);
+  t.term<2, 2>(r, -e3 * (c[15] + c[17]), 0, 0, 2, 0);
+  t.term<2, 2>(r, -e3 * (c[15] + c[17]), 0, 0, -2, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  t.term<2, 2>(r, e2 * (c[15] + c[16] + c[17] + c[18] + c[20]), 0, 0, 0, 0);
+  t.term<2, 2>(r, -e2 * (c[16] + c[18] + c[20]), 0, 0, 0, 0, 0, 0, 2, 0);
+  t.term<2, 2>(r, -e2 * (c[17] + c[18] + c[20]), 0, 0, 0, 0, 0, 0, 0, 2);
+  t.term<2, 2>(r, e3 * c[16], 0, 0, 0, -2, 0, 0, 2, 0);
+  t.term<2, 2>(r, e3 * c[16], 0, 0, 0, 2, 0, 0, 2, 0);
+  t.term<2, 2>(r, e3 * c[17], 0, 0, 2, 0, 0, 0, 0, 2);
+  t.term<2, 2>(r, e3 * c[17], 0, 0, -2, 0, 0, 0, 0, 2);
+  __builtin_amdgcn_sched_barrier(0);
+  const double cxx = c[18] + 0.5 * c[21], cxy = c[20] - 0.5 * c[21];
+  t.term<2, 2>(r, e3 * cxx, 0, 0, 0, 0, 0, 0, 2, -2);
+  t.term<2, 2>(r, e3 * cxx, 0, 0, 0, 0, 0, 0, 2, 2);
+  {  // e2 cxy / sqrt(r^2 + (2 qa)^2 + (2 qb)^2 + ..): two offsets across the axis
+    const double w = t.ra[2] + t.rb[2];
+    const double q = rsq_nr(r * r + 4.0 * t.qa * t.qa + 4.0 * t.qb * t.qb + w * w);
+    const double g = -e2 * cxy * (q * q * q);
+    t.gqa += 4.0 * g * t.qa;
+    t.gqb += 4.0 * g * t.qb;
+    t.gra[2] += g * w;
+    t.grb[2] += g * w;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  t.term<2, 2>(r, e3 * c[19], 0, 0, 1, -1, 0, 0, 1, -1);
+  t.term<2, 2>(r, -e3 * c[19], 0, 0, 1, 1, 0, 0, 1, -1);
+  t.term<2, 2>(r, -e3 * c[19], 0, 0, -1, -1, 0, 0, 1, -1);
+  t.term<2, 2>(r, e3 * c[19], 0, 0, -1, 1, 0, 0, 1, -1);
+  t.term<2, 2>(r, -e3 * c[19], 0, 0, 1, -1, 0, 0, 1, 1);
+  t.term<2, 2>(r, e3 * c[19], 0, 0, 1, 1, 0, 0, 1, 1);
+  t.term<2, 2>(r, e3 * c[19], 0, 0, -1, -1, 0, 0, 1, 1);
+  t.term<2, 2>(r, -e3 * c[19], 0, 0, -1, 1, 0, 0, 1, 1);
+}
+
+// the same for a heavy-H pair (local_xh)
+__device__ inline void charge_terms_xh(double r, const double (&c)[4], ChargeTerms& t) {
+  const double e1 = kEV * 0.5, e2 = kEV * 0.25;
+  t.term<0, 0>(r, kEV * (c[0] + c[2] + c[3]), 0, 0, 0, 0);
+  t.term<1, 0>(r, e1 * c[1], 1, 0, 0, 0);
+  t.term<1, 0>(r, -e1 * c[1], -1, 0, 0, 0);
+  t.term<2, 0>(r, e2 * c[2], 0, 0, 2, 0);
+  t.term<2, 0>(r, e2 * c[2], 0, 0, -2, 0);
+  t.term<2, 0>(r, -e1 * (c[2] + c[3]), 0, 0, 0, 0);
+  t.term<2, 0>(r, e1 * c[3], 0, 0, 0, 0, 0, 0, 2, 0);
+}
+
+// A pair's derivatives in the quantities of atom i (row partial) and of atom j (column partial), MODE 0
+// of Eelec(P) and of the core repulsion, MODE 2 of sum Y F(P) for a symmetric Y (no core repulsion).
 template <int KIND, int MODE>
 __global__ __launch_bounds__(64) void k_pair_param_grad(pyseqm_layout_t L, int method, int tile_base,
                                                         const double* __restrict__ coords,
                                                         const double* __restrict__ par, const double* __restrict__ P,
-                                                        const double* __restrict__ Y,
-                                                        const double* __restrict__ rec, int p0, int np, double hrel,
-                                                        double* __restrict__ part) {
+                                                        const double* __restrict__ Y, double* __restrict__ part) {
   const int tile = tile_base + xcd_run(blockIdx.x, gridDim.x);
   const int lane = threadIdx.x;
   const Tile t = load_tile(L.tiles, tile);
   int i, j;
   const bool valid = lane_pair(t, lane, i, j);
-  double rowv[10], colv[10];
+  // lanes without a pair take the tile's first row and column (both exist) and add zeros below
+  if (!valid) {
+    i = t.row0;
+    j = t.col0 + t.ncol - 1;
+  }
+  const double* pi = par + (size_t)i * PYSEQM_NPAR;
+  const double* pj = par + (size_t)j * PYSEQM_NPAR;
+  const int r8 = lane >> 3, c8 = lane & 7;
+  double* prow = part + ((size_t)tile * 16 + r8) * kPV;
+  double* pcol = part + ((size_t)tile * 16 + 8 + c8) * kPV;
+  // value k of the tile's row and column partials, written as soon as it is known (every lane active)
+  auto put = [&](int k, double row, double col) {
+    const double rs = row8(valid ? row : 0.0), cs = col8(valid ? col : 0.0);
+    if (c8 == 0) prow[k] = rs;
+    if (r8 == 0) pcol[k] = cs;
+  };
+  const long long mo = L.mol_mat_off[t.mol];
+  const int n = L.mol_norb[t.mol];
+  constexpr int NI = KIND == HH ? 1 : 4;
+  constexpr int NJ = KIND == XX ? 4 : 1;
+  PairDensity Pd, Yd;
+  load_pair_density<NI, NJ>(P + mo, n, L.atom_ao[i], L.atom_ao[j], Pd);
+  if constexpr (MODE == 2) load_pair_density<NI, NJ>(Y + mo, n, L.atom_ao[i], L.atom_ao[j], Yd);
+  const PairDensity& D = MODE == 2 ? Yd : Pd;  // contracted with H and the electron-core terms
+  const PairGeom g = pair_geom(coords, i, j);
+  const double ti = pi[PAR_TORE], tj = pj[PAR_TORE];
+  {
+    double zr[4] = {0.0, 0.0, 0.0, 0.0}, zc[4] = {0.0, 0.0, 0.0, 0.0};
+    // overlaps: exponents and resonance integrals
+    if (g.r <= kOverlapCut) {
+      double Rp[3][3];
+      quat_frame(g.x[0], g.x[1], g.x[2], Rp, quat_flips(g.x[0]) ? 2 : 1);
+      const double d0 = D.pab[0][0];
+      double d1 = 0.0, d2 = 0.0, duu = 0.0, tr = 0.0;
+      if constexpr (NI == 4) d1 = D.pab[1][0] * Rp[0][0] + D.pab[2][0] * Rp[0][1] + D.pab[3][0] * Rp[0][2];
+      if constexpr (NJ == 4) {
+        d2 = -(D.pab[0][1] * Rp[0][0] + D.pab[0][2] * Rp[0][1] + D.pab[0][3] * Rp[0][2]);
 #pragma unroll
-  for (int k = 0; k < 10; ++k) rowv[k] = colv[k] = 0.0;
-  if (valid) {
-    const double* pi = par + (size_t)i * PYSEQM_NPAR;
-    const double* pj = par + (size_t)j * PYSEQM_NPAR;
-    const long long mo = L.mol_mat_off[t.mol];
-    const int n = L.mol_norb[t.mol];
-    constexpr int NI = KIND == HH ? 1 : 4;
-    constexpr int NJ = KIND == XX ? 4 : 1;
-    PairDensity Pd, Yd;
-    load_pair_density<NI, NJ>(P + mo, n, L.atom_ao[i], L.atom_ao[j], Pd);
-    if constexpr (MODE == 2) load_pair_density<NI, NJ>(Y + mo, n, L.atom_ao[i], L.atom_ao[j], Yd);
-    const PairDensity& Dr = MODE == 2 ? Yd : Pd;
-    const PairGeom g0 = pair_geom(coords, i, j);
-    const int wmode = quat_flips(-g0.x[0]) ? 2 : 1;
-    const int smode = quat_flips(g0.x[0]) ? 2 : 1;
-    const int bsel = overlap_branches(g0.r, pi[PAR_ZS], pi[PAR_ZP], pj[PAR_ZS], pj[PAR_ZP]);
-#pragma unroll 1
-    for (int g = 0; g < np; ++g) {
-      const int slot = kPairParams[p0 + g];
+        for (int m = 0; m < 3; ++m) {
+          tr += D.pab[1 + m][1 + m];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) duu += Rp[0][m] * D.pab[1 + m][1 + k] * Rp[0][k];
+        }
+      }
+      const int jc = jcall_of((int)pi[PAR_QN], (int)pj[PAR_QN]);
+      const double bss = pi[PAR_BS] + pj[PAR_BS], bps = pi[PAR_BP] + pj[PAR_BS], bsp = pi[PAR_BS] + pj[PAR_BP],
+                   bpp = pi[PAR_BP] + pj[PAR_BP];
+      // each overlap depends on one exponent per side, so one pass per side serves s and p
 #pragma unroll 1
       for (int side = 0; side < 2; ++side) {
-        const int a = side == 0 ? i : j;
-        const double inv = 1.0 / param_step(side == 0 ? pi : pj, slot, hrel);
-        double de = 0.0, dn = 0.0;
-#pragma unroll 1
-        for (int s = 0; s < 4; ++s) {
-          const double* q = rec + ((size_t)(a * kParamGroup + g) * 4 + s) * PYSEQM_NPAR;
-          double rep = 0.0;
-          const double e = pair_energy<KIND, MODE>(method, g0, side == 0 ? q : pi, side == 0 ? pj : q, Pd, Dr,
-                                                   wmode, smode, bsel, &rep);
-          de += kStencilW[s] * (e - rep);
-          dn += kStencilW[s] * rep;
-        }
+        const double sa = side == 0 ? 1.0 : 0.0, sb = 1.0 - sa;
+        Dual S[5];
+        overlap_local<Dual, KIND>(jc, g.r, Dual{pi[PAR_ZS], sa}, Dual{pi[PAR_ZP], sa}, Dual{pj[PAR_ZS], sb},
+                                  Dual{pj[PAR_ZP], sb}, NI == 4, S);
+        const double ss = bss * d0 * S[0].d, ps = bps * d1 * S[1].d, sp = bsp * d2 * S[2].d;
+        const double pp = bpp * ((tr - duu) * S[4].d - duu * S[3].d);
+        const double vss = d0 * S[0].v, vps = d1 * S[1].v, vsp = d2 * S[2].v;
+        const double vpp = (tr - duu) * S[4].v - duu * S[3].v;
         if (side == 0) {
-          rowv[2 * g] = de * inv;
-          rowv[2 * g + 1] = dn * inv;
+          zr[0] = ss + sp;
+          zr[1] = ps + pp;
+          zr[2] = vss + vsp;
+          zr[3] = vps + vpp;
         } else {
-          colv[2 * g] = de * inv;
-          colv[2 * g + 1] = dn * inv;
+          zc[0] = ss + ps;
+          zc[1] = sp + pp;
+          zc[2] = vss + vps;
+          zc[3] = vsp + vpp;
         }
       }
     }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) put(PV_ZS + k, zr[k], zc[k]);
   }
-  write_partials(part, tile, lane, rowv, colv);
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    // two-electron and electron-core terms: the multipoles
+    ChargeTerms q = {pi[PAR_DD], pj[PAR_DD], pi[PAR_QQ], pj[PAR_QQ],
+                     {pi[PAR_RHO0], pi[PAR_RHO1], pi[PAR_RHO2]}, {pj[PAR_RHO0], pj[PAR_RHO1], pj[PAR_RHO2]},
+                     0.0, 0.0, 0.0, 0.0, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+    if constexpr (KIND == HH) {
+      const double cw = MODE == 2 ? D.pa[0] * Pd.pb[0] + Pd.pa[0] * D.pb[0] : Pd.pa[0] * Pd.pb[0];
+      const double xw = MODE == 2 ? D.pab[0][0] : 0.5 * Pd.pab[0][0];
+      q.term<0, 0>(g.r, kEV * (cw - tj * D.pa[0] - ti * D.pb[0] - xw * Pd.pab[0][0]), 0, 0, 0, 0);
+    } else {
+      double R[3][3];
+      quat_frame(-g.x[0], -g.x[1], -g.x[2], R, quat_flips(-g.x[0]) ? 2 : 1);
+      LocalDensity Pl, Yl;
+      to_local<NI, NJ>(Pd, R, Pl);
+      if constexpr (MODE == 2) to_local<NI, NJ>(Yd, R, Yl);
+      const LocalDensity& E = MODE == 2 ? Yl : Pl;
+      constexpr int NM = KIND == XX ? 22 : 4, NE = KIND == XX ? 34 : 5;
+      constexpr int xhP[5] = {0, 1, 2, 5, 9}, xhM[5] = {0, 1, 2, 3, 3};
+      const double xf = MODE == 2 ? 1.0 : 0.5;
+      double cm[NM];
+#pragma unroll
+      for (int k = 0; k < NM; ++k) cm[k] = 0.0;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const int p = KIND == XX ? kLocP[e] : xhP[e], o = KIND == XX ? kLocQ[e] : 0;
+        const int mu = kTriI[p], nu = kTriJ[p], la = kTriI[o], si = kTriJ[o];
+        const double fp = mu == nu ? 1.0 : 2.0, fo = la == si ? 1.0 : 2.0;
+        double c = MODE == 2 ? Yl.a[p] * Pl.b[o] + Pl.a[p] * Yl.b[o] : Pl.a[p] * Pl.b[o];
+        c *= fp * fo;
+        if (o == 0) c -= tj * fp * E.a[p];
+        if (p == 0) c -= ti * fo * E.b[o];
+        double x = E.c[mu][la] * Pl.c[nu][si];
+        if (mu != nu) x += E.c[nu][la] * Pl.c[mu][si];
+        if (la != si) x += E.c[mu][si] * Pl.c[nu][la];
+        if (mu != nu && la != si) x += E.c[nu][si] * Pl.c[mu][la];
+        cm[KIND == XX ? kLocM[e] : xhM[e]] += c - xf * x;
+      }
+      if constexpr (KIND == XX)
+        charge_terms_xx(g.r, cm, q);
+      else
+        charge_terms_xh(g.r, cm, q);
+    }
+    put(PV_DD, q.gda, q.gdb);
+    put(PV_QQ, q.gqa, q.gqb);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) put(PV_R0 + k, q.gra[k], q.grb[k]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // core repulsion (core_repulsion) in rho0, alpha and the Gaussians; zeros where there is none
+  if constexpr (MODE == 0) {
+    const double ra = g.r * kA0, w = pi[PAR_RHO0] + pj[PAR_RHO0];
+    const double inv = rsq_nr(g.r * g.r + w * w);
+    const double tt = ti * tj;
+    const int Zi = (int)pi[PAR_Z], Zj = (int)pj[PAR_Z];
+    double t2 = exp(-pi[PAR_ALPHA] * ra);
+    if ((Zi == 7 || Zi == 8) && Zj == 1) t2 *= ra;
+    const double t3 = exp(-pj[PAR_ALPHA] * ra);
+    const double dg = -tt * (1.0 + t2 + t3) * kEV * (inv * inv * inv) * w;
+    put(PV_REP, dg, dg);
+    put(PV_ALPHA, -tt * kEV * inv * t2 * ra, -tt * kEV * inv * t3 * ra);
+    const int ng = method == PYSEQM_AM1 ? 4 : (method == PYSEQM_PM3 ? 2 : 0);
+    const double pre = tt / ra;
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) {
+      double v[2][3];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const double* p = (s == 0 ? pi : pj) + PAR_GAUSS + 3 * k;
+        const double dm = ra - p[2], e = k < ng ? pre * exp(-p[1] * dm * dm) : 0.0;
+        v[s][0] = e;
+        v[s][1] = -p[0] * dm * dm * e;
+        v[s][2] = 2.0 * p[0] * p[1] * dm * e;
+      }
+#pragma unroll
+      for (int x = 0; x < 3; ++x) put(PV_GAUSS + 3 * k + x, v[0][x], v[1][x]);
+    }
+  } else {
+    put(PV_REP, 0.0, 0.0);
+#pragma unroll
+    for (int k = PV_ALPHA; k < kPV; ++k) put(k, 0.0, 0.0);
+  }
 }
 
-// out[a][0][k] += sum of atom a's pair shares of dEelec/d(slot k), out[a][1][k] += the core
-// repulsion's, for the pass's slots (fixed gather order).
-template <int G>
-__global__ __launch_bounds__(256) void k_param_gather(pyseqm_layout_t L, const double* __restrict__ part, int p0,
-                                                      int np, double* __restrict__ out) {
-  const int a = blockIdx.x * (256 / G) + threadIdx.x / G;
-  const int lane = threadIdx.x % G;
-  if (a >= L.natoms) return;  // uniform over the lane group
-  double acc[10];
-  gather_slots<G>(part, L.csr_idx, L.csr_off[a], L.csr_off[a + 1], lane, acc);
-  if (lane < np) {
-    double de = acc[0], dn = acc[1];
+// out[a][0][slot] += atom a's pair shares of dEelec/d(slot), out[a][1][slot] += the core repulsion's: the
+// sums of its partial slots (fixed order), through its multipoles' Jacobian.  One wave per atom.
+__global__ __launch_bounds__(256) void k_param_gather(pyseqm_layout_t L, int method, const double* __restrict__ part,
+                                                      const double* __restrict__ jac, double* __restrict__ out) {
+  const int a = blockIdx.x * 4 + threadIdx.x / 64;
+  const int lane = threadIdx.x % 64;
+  if (a >= L.natoms) return;  // uniform over the wave
+  double acc[kPV];
 #pragma unroll
-    for (int g = 1; g < kParamGroup; ++g)
-      if (lane == g) {
-        de = acc[2 * g];
-        dn = acc[2 * g + 1];
-      }
-    const int slot = kPairParams[p0 + lane];
-    out[(size_t)a * 48 + slot] += de;
-    out[(size_t)a * 48 + 24 + slot] += dn;
+  for (int k = 0; k < kPV; ++k) acc[k] = 0.0;
+  for (int e = L.csr_off[a] + lane; e < L.csr_off[a + 1]; e += 64) {
+    const double* src = part + (size_t)L.csr_idx[e] * kPV;
+#pragma unroll
+    for (int k = 0; k < kPV; ++k) acc[k] += src[k];
   }
+#pragma unroll
+  for (int k = 0; k < kPV; ++k) acc[k] = wave64(acc[k]);
+  if (lane != 0) return;
+  double* oe = out + (size_t)a * 48;
+  double* on = oe + 24;
+#pragma unroll
+  for (int k = 0; k < kJacSlots; ++k) {
+    const double* J = jac + ((size_t)a * kJacSlots + k) * 5;
+    oe[kJacParam[k]] += acc[PV_DD] * J[0] + acc[PV_QQ] * J[1] + acc[PV_R0] * J[2] + acc[PV_R1] * J[3] + acc[PV_R2] * J[4];
+    on[kJacParam[k]] += acc[PV_REP] * J[2];
+  }
+  oe[PAR_ZS] += acc[PV_ZS];
+  oe[PAR_ZP] += acc[PV_ZP];
+  oe[PAR_BS] += acc[PV_BS];
+  oe[PAR_BP] += acc[PV_BP];
+  on[PAR_ALPHA] += acc[PV_ALPHA];
+  const int ng = method == PYSEQM_AM1 ? 12 : (method == PYSEQM_PM3 ? 6 : 0);
+#pragma unroll
+  for (int k = 0; k < 12; ++k)
+    if (k < ng) on[PAR_GAUSS + k] += acc[PV_GAUSS + k];
 }
 
 // The closed-form one-center part: E_A = sum_mu P_mumu U_mu + 1/2 sum P G1(P) over the atom's
@@ -1419,40 +1625,33 @@ extern "C" int pyseqm_pair_forces_xl(const pyseqm_layout_t* L, int method, const
 
 extern "C" long long pyseqm_param_grad_workspace(const pyseqm_layout_t* L) {
   if (!L || L->natoms < 0) return -1;
-  return (long long)L->natoms * kParamGroup * 4 * PYSEQM_NPAR;
+  const long long nt = (long long)L->ntile[0] + L->ntile[1] + L->ntile[2];
+  return nt * 16 * kPV + (long long)L->natoms * kJacSlots * 5;
 }
 
 namespace {
+// ws: the tiles' 23-wide partials, then the atoms' Jacobians (pyseqm_param_grad_workspace)
 template <int MODE>
 int launch_param_grad(const pyseqm_layout_t* L, int method, const double* coords, const double* atom_par,
-                      const double* P, const double* Y, double hrel, double* rec, double* part, double* out,
-                      void* stream) {
+                      const double* P, const double* Y, double hrel, double* ws, double* out, void* stream) {
   if (!L || method < PYSEQM_MNDO || method > PYSEQM_PM3 || !(hrel > 0.0)) return PYSEQM_EINVAL;
   if (L->natoms == 0) return PYSEQM_OK;
   hipStream_t s = (hipStream_t)stream;
+  const size_t nt = (size_t)L->ntile[0] + L->ntile[1] + L->ntile[2];
+  double* part = ws;
+  double* jac = ws + nt * 16 * kPV;
   k_param_onecenter<<<(L->natoms + 127) / 128, 128, 0, s>>>(*L, P, Y, out);
-  const int npp = pair_param_count(method);
-  for (int p0 = 0; p0 < npp; p0 += kParamGroup) {
-    const int np = npp - p0 < kParamGroup ? npp - p0 : kParamGroup;
-    const long long nthr = (long long)L->natoms * kParamGroup * 4;
-    k_param_records<<<(unsigned)((nthr + 255) / 256), 256, 0, s>>>(*L, atom_par, p0, np, hrel, rec);
-    int base = 0;
-    if (L->ntile[0])
-      k_pair_param_grad<XX, MODE><<<L->ntile[0], 64, 0, s>>>(*L, method, base, coords, atom_par, P, Y, rec, p0, np,
-                                                             hrel, part);
-    base += L->ntile[0];
-    if (L->ntile[1])
-      k_pair_param_grad<XH, MODE><<<L->ntile[1], 64, 0, s>>>(*L, method, base, coords, atom_par, P, Y, rec, p0, np,
-                                                             hrel, part);
-    base += L->ntile[1];
-    if (L->ntile[2])
-      k_pair_param_grad<HH, MODE><<<L->ntile[2], 64, 0, s>>>(*L, method, base, coords, atom_par, P, Y, rec, p0, np,
-                                                             hrel, part);
-    if (lanes_per_atom(L) == 64)
-      k_param_gather<64><<<(L->natoms + 3) / 4, 256, 0, s>>>(*L, part, p0, np, out);
-    else
-      k_param_gather<16><<<(L->natoms + 15) / 16, 256, 0, s>>>(*L, part, p0, np, out);
-  }
+  k_param_jacobian<<<(L->natoms * kJacSlots + 127) / 128, 128, 0, s>>>(*L, atom_par, hrel, jac);
+  int base = 0;
+  if (L->ntile[0])
+    k_pair_param_grad<XX, MODE><<<L->ntile[0], 64, 0, s>>>(*L, method, base, coords, atom_par, P, Y, part);
+  base += L->ntile[0];
+  if (L->ntile[1])
+    k_pair_param_grad<XH, MODE><<<L->ntile[1], 64, 0, s>>>(*L, method, base, coords, atom_par, P, Y, part);
+  base += L->ntile[1];
+  if (L->ntile[2])
+    k_pair_param_grad<HH, MODE><<<L->ntile[2], 64, 0, s>>>(*L, method, base, coords, atom_par, P, Y, part);
+  k_param_gather<<<(L->natoms + 3) / 4, 256, 0, s>>>(*L, method, part, jac, out);
   return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
 }
 }  // namespace
@@ -1460,14 +1659,16 @@ int launch_param_grad(const pyseqm_layout_t* L, int method, const double* coords
 extern "C" int pyseqm_param_grad(const pyseqm_layout_t* L, int method, const double* coords, const double* atom_par,
                                  const double* P, double hrel, double* rec, double* part, double* out,
                                  void* stream) {
-  return launch_param_grad<0>(L, method, coords, atom_par, P, nullptr, hrel, rec, part, out, stream);
+  (void)part;
+  return launch_param_grad<0>(L, method, coords, atom_par, P, nullptr, hrel, rec, out, stream);
 }
 
 extern "C" int pyseqm_fock_param_vjp(const pyseqm_layout_t* L, int method, const double* coords,
                                      const double* atom_par, const double* P, const double* Y, double hrel,
                                      double* rec, double* part, double* out, void* stream) {
   if (!Y) return PYSEQM_EINVAL;
-  return launch_param_grad<2>(L, method, coords, atom_par, P, Y, hrel, rec, part, out, stream);
+  (void)part;
+  return launch_param_grad<2>(L, method, coords, atom_par, P, Y, hrel, rec, out, stream);
 }
 
 extern "C" int pyseqm_atom_setup(const pyseqm_layout_t* L, double* atom_par, void* stream) {

@@ -466,9 +466,9 @@ class SCFEngine:
         parameters (COLUMNS order): (natoms, 2, 24), [:, 0] for Eelec and [:, 1] for the core
         repulsion Enuc.  At a converged SCF density this is the exact gradient of Etot (the energy is
         stationary in P), the one the reference's autograd returns for learned parameters with
-        scf_backward = 0 (basics.py:781-789, scf_loop.py:1996-2031).  Pair terms by 4th-order
-        central differences of each pair's energy (step hrel * max(|value|, 0.1)), one-center terms
-        in closed form.  atom_par / coords default to the engine's current ones."""
+        scf_backward = 0 (basics.py:781-789, scf_loop.py:1996-2031).  Pair and one-center terms in
+        closed form; the derivatives of each atom's multipoles in its inputs are 4th-order central
+        differences (step hrel * max(|value|, 0.1)).  atom_par / coords default to the engine's current ones."""
         b = self.b
         out = torch.zeros(max(b.natoms, 1), 2, 24, dtype=torch.float64, device=self.device)
         rec = torch.empty(max(int(nat.lib().pyseqm_param_grad_workspace(nat.ctypes.byref(b.L))), 1),
