@@ -3,11 +3,7 @@
 // as the SCF's make_Pnew uses it, scf_loop.py:55-103), without padding the block to a batch size.
 //
 //   1. Householder reduction of the block to tridiagonal form T = Q^T F Q (dsytd2 order), with the
-//      matrix in registers: a GR x 16 grid of threads, thread (tr, tc) holding the RR x RC elements
-//      (tr + GR a, tc + 16 b); row sums of the symmetric product reduce over the 16 lanes of a row
-//      group (one 16-lane DPP row) by DPP moves, and only vectors pass through LDS.  The
-//      reflectors go to the global workspace.  4 x 16 threads with 12 x 3 slots for blocks of up
-//      to 48 orbitals, 16 x 16 with 6 x 6 up to 96, 32 x 16 with 6 x 12 up to 192 (64, 256, 512).
+//      matrix in registers (tridiagonalise below).  The reflectors go to the global workspace.
 //   2. The nocc lowest eigenvalues of T by multisection on Sturm counts: a group of lanes per
 //      eigenvalue evaluates the count at evenly spaced points of its bracket each round.
 //   3. Their eigenvectors by inverse iteration (tridiagonal LU with partial pivoting, three solves
@@ -17,28 +13,46 @@
 //      eigenvalues further apart orthogonal to eps |T| / gap < 3e-11; a degenerate eigenvalue's
 //      vectors come from different start vectors, so they span its subspace and the passes make
 //      them orthonormal inside it (P depends on the occupied subspace only).
-//   5. Back-transformation C = Q Z in LDS (groups of lanes per column of Z), then P = 2 C C^T.
+//   5. Back-transformation C = Q Z by blocks of 16 reflectors and P = 2 C C^T, both on FP64 MFMA
+//      tiles.
 // Every reduction runs in a fixed order: reruns are bitwise identical.
 #include "common.h"
 
 using namespace pyseqm;
 
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
 namespace {
 
 constexpr int kEighMaxN = 192;      // largest block this solver takes
 constexpr int kLdsDoubles = 20480;  // 160 KiB of LDS
-constexpr int kRed = 128;           // doubles of reduction scratch (two halves of 64)
+constexpr int kTPanel = 256;        // doubles of one panel's 16 x 16 T factor
 
 // workspace per listed molecule, in doubles, at slot * 4 * nmax^2:
-//   [0, nmax^2)          reflectors: row i holds v_i (v_i[i+1] = 1) and tau_i at [i][i]
+//   [0, nmax^2)          reflectors: row i holds u_i (zero at columns <= i of its panel of 16)
 //   [nmax^2, 4 nmax^2)   the U factor of each inverse-iteration LU (reciprocal diagonal and two
-//                        superdiagonals), element k of vector j at k * nmax + j
-// LDS: eigenvectors n x nocc, then d, e, eigenvalues (n each), two reflector buffers and p (S each,
-// S = the variant's 48 / 96 / 192 register-grid rows, zero-padded past n), kRed of scratch.  The
-// variant, and so S, follows the launch's largest block nmax.
+//                        superdiagonals), element k of vector j at k * nmax + j; the panels' T
+//                        factors of the back-transformation afterwards (blocks above 48 orbitals)
+// LDS: eigenvectors n x ldz (the Householder vectors before them, in the same place), then
+// (d, e^2) pairs, e, eigenvalues, reflector scales and vector scales (n each), and the panels' T
+// factors of blocks of up to 48 orbitals.  The variant follows the launch's largest block nmax.
 __host__ __device__ inline int grid_slots(int nmax) { return nmax <= 48 ? 48 : (nmax <= 96 ? 96 : 192); }
-__host__ __device__ inline int lds_doubles(int nmax, int nocc) {
-  return nmax * nocc + 3 * nmax + 3 * grid_slots(nmax) + kRed;
+// The size rule of the entry points: n nocc + 3 n + 3 S + 128 doubles (S: the variant's 48 / 96 /
+// 192 grid rows).  lds_doubles, what a launch asks for, stays within it for every accepted block.
+__host__ __device__ inline int rule_doubles(int n, int nv) { return n * nv + 3 * n + 3 * grid_slots(n) + 128; }
+// Row stride of the eigenvectors: odd where that fits (rows of 16 lanes then fall on distinct LDS
+// banks), else nv.
+__host__ __device__ inline int zstride(int n, int nv) { return n * (nv | 1) + 6 * n + 1 <= kLdsDoubles ? (nv | 1) : nv; }
+// Doubles of the eigenvector region: also holds the Householder vectors (2 S) before.
+__host__ __device__ inline int zregion(int n, int nv, int S) {
+  const int z = n * zstride(n, nv);
+  return z > 2 * S ? z : 2 * S;
+}
+inline int lds_doubles(int nmax, int nv) {
+  const int S = grid_slots(nmax);
+  // where the odd stride does not fit the largest block it may still fit a smaller one of the launch
+  if (zstride(nmax, nv) != (nv | 1)) return kLdsDoubles;
+  return zregion(nmax, nv, S) + 1 + 6 * nmax + (S == 48 ? 3 * kTPanel : 0);
 }
 
 template <int NT>
@@ -79,7 +93,7 @@ __device__ inline double rcp_f64(double q) {
 }
 
 // number of eigenvalues of the tridiagonal (d, e) below x: the negative pivots q_k of the LDL^T
-// factorisation of T - x I (e2[k] = e[k]^2), counted as sign changes of the Sturm sequence
+// factorisation of T - x I (de[k] = (d_k, e_k^2)), counted as sign changes of the Sturm sequence
 // p_0 = 1, p_k = (d_k - x) p_{k-1} - e2_{k-1} p_{k-2} (q_k = p_k / p_{k-1}), whose dependent chain
 // is one FMA per step instead of a reciprocal.  |q_k| < pivmin is floored to q_k = -pivmin, as in
 // the ratio form: |p_k| < pivmin |p_{k-1}| -> p_k = -pivmin p_{k-1}.  Every 8 steps both terms are
@@ -91,20 +105,20 @@ __device__ inline void sturm_step(double dk, double e2k, double x, double pivmin
   p0 = p1;
   p1 = p2;
 }
-__device__ inline int sturm_count(const double* d, const double* e2, int n, double x, double pivmin) {
-  double p0 = 1.0, p1 = d[0] - x;
+__device__ inline int sturm_count(const double2* de, int n, double x, double pivmin) {
+  double p0 = 1.0, p1 = de[0].x - x;
   if (fabs(p1) < pivmin) p1 = -pivmin;
   int cnt = p1 < 0.0;
   int k = 1;
   for (; k + 8 <= n; k += 8) {
 #pragma unroll
-    for (int t = 0; t < 8; ++t) sturm_step(d[k + t], e2[k + t - 1], x, pivmin, p0, p1, cnt);
+    for (int t = 0; t < 8; ++t) sturm_step(de[k + t].x, de[k + t - 1].y, x, pivmin, p0, p1, cnt);
     int ex;
     frexp(fmax(fabs(p0), fabs(p1)), &ex);
     p0 = ldexp(p0, -ex);
     p1 = ldexp(p1, -ex);
   }
-  for (; k < n; ++k) sturm_step(d[k], e2[k - 1], x, pivmin, p0, p1, cnt);
+  for (; k < n; ++k) sturm_step(de[k].x, de[k - 1].y, x, pivmin, p0, p1, cnt);
   return cnt;
 }
 
@@ -117,24 +131,6 @@ __device__ inline double dpp_f64(double v) {
   const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, false);
   const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, false);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// Sum over the 16 lanes of a DPP row, in every lane: partners at xor 1, xor 2 (quad
-// permutations), then the other quad (half-row mirror) and the other half-row (row mirror).
-// Additions are commutative, so every lane ends with the same bits.
-__device__ inline double row16_sum(double v) {
-  v += dpp_f64<0xB1>(v);
-  v += dpp_f64<0x4E>(v);
-  v += dpp_f64<0x141>(v);
-  v += dpp_f64<0x140>(v);
-  return v;
-}
-
-// Sum of 32 values held by lanes 0..31 (and again by lanes 32..63): each 16-lane row sums by DPP,
-// then the two rows of each half add (a + b in one lane, b + a in its partner: the same bits).
-__device__ inline double sum32(double v) {
-  v = row16_sum(v);
-  return v + __shfl_xor(v, 16);
 }
 
 // Sum / max / min over aligned groups of t lanes (t a power of two, the same in every lane):
@@ -176,287 +172,400 @@ __device__ inline double start_value(int j, int k) {
   return (double)h * (2.0 / 4294967296.0) - 1.0;
 }
 
-// C = Q Z on the register block (thread (tr, tc) holds C[tc + 16 b][tr + GR c]): the reflectors
-// last to first, C -= v (tau v^T C).  Only the first CMAX column slots hold vectors (a compile-time
-// count, so the work follows nv).  Every row slot takes part in every step: v is zero at rows <= i
-// and beyond the block, so those products and updates are exact no-ops, and the loops stay free
-// of per-slot selects; the CMAX column chains run interleaved.  The next reflector is read from
-// the workspace while the current one is applied.  C (in LDS, n x nv, over Z) is written after a
-// barrier that follows every thread's read of Z.
-template <int GR, int RR, int RC, int CMAX>
-__device__ __forceinline__ void back_transform(double (&Ar)[RR][RC], const double* __restrict__ HH, int nmax, int n,
-                                               int nv, int tr, int tc, double* C) {
-  double vcur[RC], vnext[RC];
-  double tcur = 0.0, tnext = 0.0;
-  auto load_v = [&](int i, double* v, double& t) {
-    t = HH[(size_t)i * nmax + i];
+
+// ---- the thread grid of the Householder phase.  The lanes of a wave form 4 rows x 16 columns:
+// column tc = lane bits 5 4 1 0, row rl = lane bits 3 2; thread row tr = 4 wave + rl.
+// Sum over the 16 columns of a thread row: the two high bits by permlane swaps, the two low ones by
+// quad permutations (VALU only).  Every lane of the row ends with the same bits.
+__device__ inline double cols16_sum(double v) {
+  v = swap32_sum(v);
+  v = swap16_sum(v);
+  v += dpp_f64<0xB1>(v);
+  v += dpp_f64<0x4E>(v);
+  return v;
+}
+// lanes 0-31: the sum over bit 5 of a; lanes 32-63: of b
+__device__ inline double fold32(double a, double b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a);
+  const unsigned long long y = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+         __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+// lanes with bit 4 clear: the sum over bit 4 of a; set: of b
+__device__ inline double fold16(double a, double b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a);
+  const unsigned long long y = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+         __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+
+// Workgroup barrier for LDS alone: the reflector stores to the workspace stay in flight (a full
+// barrier waits for each of them).  One wave needs none: its LDS accesses execute in order.
+template <int NW>
+__device__ inline void lds_barrier() {
+  if constexpr (NW == 1)
+    asm volatile("" ::: "memory");
+  else
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+struct TriState {
+  double* xb;   // reflector column, S rows (LDS)
+  double* pb;   // p = tau A u, S rows (LDS)
+  double2* de;  // diagonal in .x
+  double* e;
+  double* tau;
+  double* HH;  // reflectors, row i - off, column c - off
+  int off, nmax, tr, tc, lane, wave;
+};
+
+// Householder steps whose first live row j lies in row slot A0 (so that slots below A0, rows and
+// columns alike, are finished: their work is left out at compile time), then those of A0 + 1.
+//
+// Step j eliminates column j - 1.  x = A[j:, j-1] is in LDS (zero below row j).  With
+// beta = -sign(x_j) |x| and u = x - beta e_j: H = I - tau u u^T, tau = 1 / (|x|^2 + |x_j| |x|),
+// p = tau A u, w = p - (tau / 2)(p.u) u, A -= u w^T + w u^T.  The vectors need no scaling pass, and
+// A u = A x - beta A[:, j] starts before beta is known.  Two barriers per step: x, then p.  Every
+// wave holds all columns of x and p, so |x|^2 and p.u are summed in each wave without LDS.
+// What bounds it: instruction issue and the latency of this chain, not arithmetic (a wave's
+// vector instruction takes 4 cycles whatever it does), hence the few instructions per step:
+// row sums folded two values at a time by permlane swaps, no range tests (the block sits at the
+// high end of the grid, rows and columns below `off` are zero), column j updated first.  One block of
+// 182 orbitals: 630 -> 235 us; of 92 (4 waves) 210 -> 71; of 14 (one wave) 34 -> 8.
+template <int NW, int RR, int RC, int A0>
+__device__ __forceinline__ void tri_steps(double (&A)[RR][RC], int& j, const TriState& t) {
+  constexpr int GR = 4 * NW, S = GR * RR;
+  constexpr int B0 = A0 * GR / 16, B1 = ((A0 + 1) * GR - 1) / 16;  // column slots that may hold j
+  constexpr int R = RR - A0, C = RC - B0;
+  constexpr int R1 = (R + 1) / 2, R2 = (R1 + 1) / 2;  // row sums left after each fold
+  const int last = min((A0 + 1) * GR - 1, S - 2);
+  const int b5 = t.lane >> 5, b4 = (t.lane >> 4) & 1, quad = t.lane & 3;
+  // quad lane q writes folded value q: row slot of that value in this lane
+  const int i1 = min(2 * min(quad, R2 - 1) + b4, R1 - 1);
+  const int prow = (A0 + min(2 * i1 + b5, R - 1)) * GR + t.tr;
+  const double* xcol = t.xb + t.tc + 16 * B0;
+  const double* xrow = t.xb + t.tr + GR * A0;
+  const double* pcol = t.pb + t.tc + 16 * B0;
+  const double* prw = t.pb + t.tr + GR * A0;
+  for (; j <= last; ++j) {
+    lds_barrier<NW>();
+    double uc[C], ur[R];
 #pragma unroll
-    for (int b = 0; b < RC; ++b) {
-      const int k = tc + 16 * b;
-      v[b] = (k > i && k < n) ? HH[(size_t)i * nmax + k] : 0.0;
+    for (int b = 0; b < C; ++b) uc[b] = xcol[16 * b];
+#pragma unroll
+    for (int a = 0; a < R; ++a) ur[a] = xrow[GR * a];
+    const double alpha = t.xb[j];
+    double s[R];
+#pragma unroll
+    for (int a = 0; a < R; ++a) s[a] = 0.0;
+#pragma unroll
+    for (int b = 0; b < C; ++b)
+#pragma unroll
+      for (int a = 0; a < R; ++a) s[a] = fma(A[A0 + a][B0 + b], uc[b], s[a]);
+    double q0 = 0.0, q1 = 0.0;
+#pragma unroll
+    for (int b = 0; b < C; ++b) {
+      if (b & 1)
+        q1 = fma(uc[b], uc[b], q1);
+      else
+        q0 = fma(uc[b], uc[b], q0);
     }
-  };
-  if (n >= 3) load_v(n - 3, vcur, tcur);
-  for (int i = n - 3; i >= 0; --i) {
-    if (i >= 1) load_v(i - 1, vnext, tnext);
-    if (tcur != 0.0) {  // the same in every thread
-      double sd[CMAX];
-#pragma unroll
-      for (int c = 0; c < CMAX; ++c) sd[c] = 0.0;
-#pragma unroll
-      for (int b = 0; b < RC; ++b)
-#pragma unroll
-        for (int c = 0; c < CMAX; ++c) sd[c] = fma(Ar[c][b], vcur[b], sd[c]);
-#pragma unroll
-      for (int c = 0; c < CMAX; ++c) sd[c] = tcur * row16_sum(sd[c]);
-#pragma unroll
-      for (int b = 0; b < RC; ++b)
-#pragma unroll
-        for (int c = 0; c < CMAX; ++c) Ar[c][b] = fma(-vcur[b], sd[c], Ar[c][b]);
+    const double x2 = cols16_sum(q0 + q1);
+    double tau = 0.0, beta = alpha;
+    if (!(x2 <= 1.0e-280)) {  // |x| below 1e-140 counts as zero; a NaN goes on
+      double r = __builtin_amdgcn_rsq(x2);
+      r = fma(0.5 * r, fma(-x2 * r, r, 1.0), r);
+      r = fma(0.5 * r, fma(-x2 * r, r, 1.0), r);
+      double nx = x2 * r;
+      nx = fma(0.5 * r, fma(-nx, nx, x2), nx);
+      beta = -copysign(nx, alpha);
+      tau = rcp_f64(fma(fabs(alpha), nx, x2));
     }
+    // x -> u, and the sums' share of it
+    const double pt = t.tc == (j & 15) ? -beta : 0.0;
+    const int bn = j >> 4;
 #pragma unroll
-    for (int b = 0; b < RC; ++b) vcur[b] = vnext[b];
-    tcur = tnext;
+    for (int b = B0; b <= B1; ++b)
+      if (b == bn) {  // uniform
+#pragma unroll
+        for (int a = 0; a < R; ++a) s[a] = fma(A[A0 + a][b], pt, s[a]);
+        uc[b - B0] += pt;
+      }
+    ur[0] += t.tr + GR * A0 == j ? -beta : 0.0;
+    // row sums: fold over column bit 5, then 4, then sum over the quad
+    double f[R1], g[R2];
+#pragma unroll
+    for (int i = 0; i < R1; ++i) f[i] = fold32(s[2 * i], s[min(2 * i + 1, R - 1)]);
+#pragma unroll
+    for (int i = 0; i < R2; ++i) {
+      g[i] = fold16(f[2 * i], f[min(2 * i + 1, R1 - 1)]);
+      g[i] += dpp_f64<0xB1>(g[i]);
+      g[i] += dpp_f64<0x4E>(g[i]);
+    }
+    double pval = g[0];
+#pragma unroll
+    for (int i = 1; i < R2; ++i) pval = quad == i ? g[i] : pval;
+    if (quad < R2) t.pb[prow] = prow >= j ? tau * pval : 0.0;
+    if (t.wave == j % NW && (t.lane & 12) == 0) {  // one wave stores u
+      double* h = t.HH + (size_t)(j - 1 - t.off) * t.nmax - t.off + t.tc + 16 * B0;
+#pragma unroll
+      for (int b = 0; b < C; ++b)
+        if (b > B1 - B0 || t.tc + 16 * (B0 + b) >= j) h[16 * b] = uc[b];
+      if (t.lane == 0) {
+        t.e[j - 1 - t.off] = beta;
+        t.tau[j - 1 - t.off] = tau;
+      }
+    }
+    lds_barrier<NW>();
+    double wc[C], wr[R];
+#pragma unroll
+    for (int b = 0; b < C; ++b) wc[b] = pcol[16 * b];
+#pragma unroll
+    for (int a = 0; a < R; ++a) wr[a] = prw[GR * a];
+    q0 = q1 = 0.0;
+#pragma unroll
+    for (int b = 0; b < C; ++b) {
+      if (b & 1)
+        q1 = fma(uc[b], wc[b], q1);
+      else
+        q0 = fma(uc[b], wc[b], q0);
+    }
+    const double K = -0.5 * tau * cols16_sum(q0 + q1);
+#pragma unroll
+    for (int a = 0; a < R; ++a) wr[a] = fma(K, ur[a], wr[a]);
+#pragma unroll
+    for (int b = 0; b < C; ++b) {
+      const double wb = fma(K, uc[b], wc[b]);
+#pragma unroll
+      for (int a = 0; a < R; ++a) A[A0 + a][B0 + b] = fma(-ur[a], wb, fma(-wr[a], uc[b], A[A0 + a][B0 + b]));
+      if (b <= B1 - B0 && B0 + b == bn && t.tc == (j & 15)) {  // column j: the next x, and d_j
+#pragma unroll
+        for (int a = 0; a < R; ++a) {
+          const double val = A[A0 + a][B0 + b];
+          if (a == 0) {
+            const int r = t.tr + GR * A0;
+            t.xb[r] = r > j ? val : 0.0;
+            if (r == j) t.de[j - t.off].x = val;
+          } else {
+            t.xb[t.tr + GR * (A0 + a)] = val;
+          }
+        }
+      }
+    }
   }
-  __syncthreads();  // every thread has read Z
+  if constexpr (A0 + 1 < RR) tri_steps<NW, RR, RC, A0 + 1>(A, j, t);
+}
+
+// Householder tridiagonalisation of the n x n block Fm, held in registers at the high end of the
+// S x S grid: thread (tr, tc) holds A[tr + GR a][tc + 16 b], a < RR, b < RC, row r of the grid being
+// row r - off of the block.
+template <int NW, int RR, int RC>
+__device__ __forceinline__ void tridiagonalise(const double* __restrict__ Fm, int n, const TriState& t) {
+  constexpr int GR = 4 * NW, S = GR * RR, NT = 64 * NW;
+  static_assert(16 * RC == S, "square register grid");
+  double A[RR][RC];
 #pragma unroll
-  for (int c = 0; c < CMAX; ++c)
+  for (int a = 0; a < RR; ++a)
 #pragma unroll
     for (int b = 0; b < RC; ++b) {
-      const int k = tc + 16 * b, a = tr + GR * c;
-      if (k < n && a < nv) C[k * nv + a] = Ar[c][b];
+      const int r = t.tr + GR * a - t.off, c = t.tc + 16 * b - t.off;
+      A[a][b] = (r >= 0 && c >= 0) ? Fm[(size_t)r * n + c] : 0.0;
     }
+  // reflector i is zero at the columns <= i of its panel
+  for (int k = threadIdx.x; k < n * 16; k += NT) {
+    const int i = k / 16 + t.off, c = (i & ~15) + (k & 15);
+    if (c <= i && c >= t.off) t.HH[(size_t)(i - t.off) * t.nmax + c - t.off] = 0.0;
+  }
+#pragma unroll
+  for (int b = 0; b < RC; ++b)
+    if (b == t.off / 16 && t.tc == (t.off & 15)) {
+#pragma unroll
+      for (int a = 0; a < RR; ++a) {
+        const int r = t.tr + GR * a;
+        t.xb[r] = r > t.off ? A[a][b] : 0.0;
+        if (r == t.off) t.de[0].x = A[a][b];
+      }
+    }
+  int j = t.off + 1;
+  tri_steps<NW, RR, RC, 0>(A, j, t);
+  lds_barrier<NW>();
+  if (n >= 2 && t.tr == GR - 1 && t.tc == 15) {
+    t.e[n - 2] = t.xb[S - 1];
+    t.de[n - 1].x = A[RR - 1][RC - 1];
+  }
+  __syncthreads();
+}
+
+// T of the block reflector H_16q ... H_16q+15 = I - V T V^T (V's columns the reflectors u of panel
+// q), T = (diag(1/tau) + strict upper triangle of V^T V)^-1, by back substitution: lane c of the
+// wave computes column c.  Written row-major to Tq.  Reflectors outside off .. S - 3 have tau = 0.
+template <int S>
+__device__ void panel_t(const double* __restrict__ HH, const double* tau, int nmax, int n, int q, double* Tq) {
+  const int off = S - n, lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  const int refl = min(max(16 * q + m - off, 0), n - 3);
+  const double* v = HH + (size_t)refl * nmax;
+  doublex4 G = {0.0, 0.0, 0.0, 0.0};
+  for (int r = 16 * q; r < S; r += 16) {
+    double a[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int c = r + 4 * s + g - off;
+      a[s] = c >= 0 ? v[c] : 0.0;
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) G = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], a[s], G, 0, 0, 0);
+  }
+  // G[r][c] sits in register r / 4 of lane 16 (r % 4) + c
+  const int im = 16 * q + m - off;
+  const double tm = (im >= 0 && im <= n - 3) ? tau[im] : 0.0;
+  double T[16];
+#pragma unroll
+  for (int i = 15; i >= 0; --i) {
+    double acc = 0.0;
+#pragma unroll
+    for (int k = i + 1; k < 16; ++k) {
+      const long long w = __double_as_longlong(G[i >> 2]);
+      const int src = 16 * (i & 3) + k;
+      const unsigned lo = __builtin_amdgcn_readlane((int)w, src), hi = __builtin_amdgcn_readlane((int)(w >> 32), src);
+      acc = fma(__longlong_as_double(((long long)hi << 32) | lo), T[k], acc);
+    }
+    const long long w = __double_as_longlong(tm);
+    const unsigned lo = __builtin_amdgcn_readlane((int)w, i), hi = __builtin_amdgcn_readlane((int)(w >> 32), i);
+    const double ti = __longlong_as_double(((long long)hi << 32) | lo);
+    T[i] = m == i ? ti : (m > i ? -ti * acc : 0.0);
+  }
+  if (g == 0) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) Tq[16 * i + m] = T[i];
+  }
+}
+
+// Panels q, q - 1, ..., 0 of the back-transformation on one wave's 16 columns of Z: C -= V T V^T C.
+// Cr[t] holds rows 16 t + 4 s + lane / 16 (element s), column lane % 16: the MFMA result layout,
+// which is also the layout of its right operand, so C needs no move between the three products.
+// V and T come from the workspace (the waves read the same panel: L1 / L2).  One reflector at a
+// time on vector instructions took 201 us for 91 vectors of 182 orbitals (each step waited for its
+// reflector); blocks of 16 take 71 us, bounded by those reads and the chain of products.
+template <int S, int Q>
+__device__ __forceinline__ void back_panels(doublex4 (&Cr)[S / 16], const double* __restrict__ HH,
+                                            const double* __restrict__ T, int nmax, int n) {
+  constexpr int NTL = S / 16;
+  const int off = S - n;
+  if (16 * Q + 15 >= off) {  // uniform
+    int m = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    asm volatile("" : "+v"(m), "+v"(g));  // keeps every panel's addresses from being held at once (they spill)
+    // V's operands are read one tile ahead of their products; the scheduler, left alone, reads whole
+    // panels ahead and spills
+    const int o1 = min(max(16 * Q + m - off, 0), n - 3) * nmax - off + g;
+    int o2[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) o2[s] = min(max(16 * Q + 4 * s + g - off, 0), n - 3) * nmax - off + m;
+    const double* tq = T + kTPanel * Q + 16 * m + g;
+    doublex4 y0 = {0.0, 0.0, 0.0, 0.0}, y1 = {0.0, 0.0, 0.0, 0.0};
+    double a[2][4], tv[4];
+    // rows below off (first tile only) are zero in C; their V is read at the block's first row
+#pragma unroll
+    for (int s = 0; s < 4; ++s) a[0][s] = HH[o1 + max(16 * Q + 4 * s, off - g)];
+#pragma unroll
+    for (int t = Q; t < NTL; ++t) {
+      const int k = (t - Q) & 1;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (t + 1 < NTL)
+          a[k ^ 1][s] = HH[o1 + 16 * t + 16 + 4 * s];
+        else
+          tv[s] = tq[4 * s];
+      }
+      y0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k][0], Cr[t][0], y0, 0, 0, 0);
+      y1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k][1], Cr[t][1], y1, 0, 0, 0);
+      y0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k][2], Cr[t][2], y0, 0, 0, 0);
+      y1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k][3], Cr[t][3], y1, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) a[0][s] = HH[o2[s] + max(16 * Q, off - m)];
+    y0 += y1;
+    doublex4 y = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) y = __builtin_amdgcn_mfma_f64_16x16x4f64(-tv[s], y0[s], y, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = Q; t < NTL; ++t) {
+      const int k = (t - Q) & 1;
+      if (t + 1 < NTL) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) a[k ^ 1][s] = HH[o2[s] + 16 * t + 16];
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) Cr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k][s], y[s], Cr[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if constexpr (Q > 0) back_panels<S, Q - 1>(Cr, HH, T, nmax, n);
 }
 
 // EVEC = false: the density P = 2 C_occ C_occ^T of the nocc lowest vectors.  EVEC = true: every
 // eigenpair (nv = n vectors), written as Qout (packed layout, column j = eigenvector j) and evals
 // (orb_off[m] + j, the Rayleigh quotients of the final vectors: exact to rounding whatever the
 // multisection bracket width).
-// CM: column slots of the back-transformation that hold vectors (GR CM >= nv of every listed block,
-// chosen per launch from the launch's largest nv).
-template <int GR, int GC, int RR, int RC, bool EVEC, int CM>
-__global__ __launch_bounds__(GR* GC) void k_eigh_density(pyseqm_layout_t L, const int* __restrict__ idx,
+template <int NW, int RR, int RC, bool EVEC>
+__global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, const int* __restrict__ idx,
                                                        const double* __restrict__ F, double* __restrict__ P,
                                                        double* __restrict__ ws, int nmax,
                                                        int* __restrict__ fail, const long long* __restrict__ orb_off,
                                                        double* __restrict__ evals) {
-  constexpr int NT = GR * GC;
-  static_assert(GC == 16, "row groups are DPP rows");
-  extern __shared__ double lds[];
+  constexpr int NT = 64 * NW, S = 16 * RC;
+  extern __shared__ __align__(16) double lds[];
   const int slot = blockIdx.x;
   const int m = idx[slot];
   const int n = L.mol_norb[m];
   const int nv = EVEC ? n : L.mol_nocc[m];  // vectors computed
   const size_t mo = L.mol_mat_off[m];
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const size_t nm2 = (size_t)nmax * nmax;
   double* HH = ws + (size_t)slot * 4 * nm2;
   double* U0 = HH + nm2;
   double* U1 = HH + 2 * nm2;
   double* U2 = HH + 3 * nm2;
-  double* Z = lds;  // eigenvectors, n x nv: Z[k * nv + j]
-  double* d = Z + n * nv;
-  double* e = d + n;
+  const int ldz = zstride(n, nv);
+  double* Z = lds;  // eigenvectors: Z[k * ldz + j]
+  double2* de = reinterpret_cast<double2*>(Z + ((zregion(n, nv, S) + 1) & ~1));  // (d, e^2)
+  double* e = reinterpret_cast<double*>(de + n);
   double* lam = e + n;
-  constexpr int S = GR * RR;  // = GC * RC: register-grid rows / columns
-  static_assert(GR * RR == GC * RC, "square register grid");
-  double* xs0 = lam + n;  // reflector columns of even / odd steps, zero at indices <= i + 1 and >= n
-  double* xs1 = xs0 + S;
-  double* pp = xs1 + S;
-  double* red = pp + S;  // kRed
-  double* red1 = red;  // GR <= 64 partials each
-  double* red2 = red + kRed / 2;
-  const double* Fm = F + mo;
+  double* tau = lam + n;
+  double* red = tau + n;  // n doubles: block reductions' scratch
+  double* T = S == 48 ? red + n : U0;  // the panels' T factors
 
-  // ---- 1. Householder tridiagonalisation (dsytd2, lower) in registers, two barriers per step.
-  // Thread (tr, tc) of the GR x GC grid holds A[tr + GR a][tc + GC b], a < RR, b < RC.
-  // Step i: x = A[i+1:, i] is in LDS with partial sums of |x[1:]|^2 (written by the owners of
-  // column i, tc == i mod GC, during the previous step's update); every thread forms tau, beta
-  // and v = (1, x[1:] / (alpha - beta)) at its columns;
-  // p = tau A v (row sums over the lanes of each row group, rows <= i masked by v = 0), with
-  // partial sums of p.v; then A -= v w^T + w v^T, w = p - (tau / 2)(p.v) v, on every slot (v = w
-  // = 0 at indices <= i leave the finished rows and columns alone).
-  const int tr = tid / GC, tc = tid - (tid / GC) * GC;
-  double Ar[RR][RC];
-#pragma unroll
-  for (int a = 0; a < RR; ++a)
-#pragma unroll
-    for (int b = 0; b < RC; ++b) {
-      const int r = tr + GR * a, c = tc + GC * b;
-      Ar[a][b] = (r < n && c < n) ? Fm[(size_t)r * n + c] : 0.0;
-    }
-  // the reflector buffers and p start at zero (their entries past n stay zero), then column 0
-  // (the owners of column 0, tc == 0, slot b = 0); later columns are written by the rank-2
-  // update of the step before, which computes them
-  for (int t = tid; t < 3 * S; t += NT) xs0[t] = 0.0;
-  __syncthreads();
-  if (tc == 0) {
-    double part = 0.0;
-#pragma unroll
-    for (int a = 0; a < RR; ++a) {
-      const int r = tr + GR * a;
-      const double val = Ar[a][0];
-      if (r == 0) {
-        d[0] = val;
-      } else if (r < n) {
-        xs0[r] = val;
-        if (r > 1) part += val * val;
-      }
-    }
-    red1[tr] = part;
+  // ---- 1. tridiagonal form
+  {
+    TriState t;
+    t.xb = Z;
+    t.pb = Z + S;
+    t.de = de;
+    t.e = e;
+    t.tau = tau;
+    t.HH = HH;
+    t.off = S - n;
+    t.nmax = nmax;
+    t.tc = (lane & 3) | ((lane >> 4) << 2);
+    t.tr = 4 * wave + ((lane >> 2) & 3);
+    t.lane = lane;
+    t.wave = wave;
+    tridiagonalise<NW, RR, RC>(F + mo, n, t);
   }
-  const int lane32 = tid & 31;
-  for (int i = 0; i + 2 < n; ++i) {
-    const double* x = (i & 1) ? xs1 : xs0;
-    double* xnext = (i & 1) ? xs0 : xs1;
-    __syncthreads();
-    // every LDS read of the step's first half is issued here, unconditionally, so that they travel
-    // together instead of one round trip per slot (x holds S entries, zero past the live range)
-    double xc[RC], xr[RR];
-#pragma unroll
-    for (int b = 0; b < RC; ++b) xc[b] = x[tc + GC * b];
-#pragma unroll
-    for (int a = 0; a < RR; ++a) xr[a] = x[tr + GR * a];
-    const double alpha = x[i + 1];
-    // |x[1:]|^2 from the GR partials: lane k of every wave takes partial k mod 32, then a fixed
-    // tree (16-lane DPP row, then the row pair): the same bits in every thread
-    const double r1 = red1[lane32];  // red1 holds kRed / 2 = 64 doubles: in bounds
-    const double xn2 = sum32(lane32 < GR ? r1 : 0.0);
-    double tau = 0.0, beta = alpha, scal = 0.0;
-    if (xn2 > 0.0) {
-      beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
-      const double am = alpha - beta;
-      scal = rcp_f64(am);
-      tau = -am * rcp_f64(beta);
-    }
-    // tau = 0 (column already zero) runs the same steps with p = w = 0: A unchanged
-    if (tid == 0) {
-      e[i] = beta;
-      HH[(size_t)i * nmax + i] = tau;
-    }
-    // v at this thread's columns and rows: 1 at i + 1, else x scal (x is zero at indices <= i and
-    // >= n, so no range test is needed)
-    double vc[RC], vr[RR];
-#pragma unroll
-    for (int b = 0; b < RC; ++b) vc[b] = (tc + GC * b == i + 1) ? 1.0 : xc[b] * scal;
-#pragma unroll
-    for (int a = 0; a < RR; ++a) vr[a] = (tr + GR * a == i + 1) ? 1.0 : xr[a] * scal;
-    if (tr == 0) {
-#pragma unroll
-      for (int b = 0; b < RC; ++b) {
-        const int c = tc + GC * b;
-        if (c > i && c < n) HH[(size_t)i * nmax + c] = vc[b];
-      }
-    }
-    // p = tau A v.  Column slots whose columns are all finished (v = 0) or all beyond the block are
-    // skipped (a uniform test); every row of a live slot is summed: finished rows and rows beyond
-    // the block give values that are never used (p is kept at live rows only).
-    double s[RR];
-#pragma unroll
-    for (int a = 0; a < RR; ++a) s[a] = 0.0;
-#pragma unroll
-    for (int b = 0; b < RC; ++b) {
-      if (GC * b + GC - 1 <= i || GC * b >= n) continue;
-#pragma unroll
-      for (int a = 0; a < RR; ++a) s[a] = fma(Ar[a][b], vc[b], s[a]);
-    }
-    // p is written at every row (zero off the live range, finished slots included), so that w
-    // below needs no range test
-    double q = 0.0;
-#pragma unroll
-    for (int a = 0; a < RR; ++a) {
-      double pa = 0.0;
-      if (GR * a + GR - 1 > i) {  // some row of the slot still live (uniform)
-        pa = tau * row16_sum(s[a]);
-        q = fma(pa, vr[a], q);  // vr = 0 off the live rows
-      }
-      const int r = tr + GR * a;
-      if (tc == 0) pp[r] = (r > i && r < n) ? pa : 0.0;
-    }
-    if (tc == 0) red2[tr] = q;
-    __syncthreads();
-    // p at this thread's rows and at the first chunk of its columns are read with the partials;
-    // each later chunk's columns are read while the chunk before it is applied
-    constexpr int kUpdChunk = 4;
-    constexpr int kChunks = (RC + kUpdChunk - 1) / kUpdChunk;
-    double wr[RR], wc[2][kUpdChunk];
-#pragma unroll
-    for (int a = 0; a < RR; ++a) wr[a] = pp[tr + GR * a];
-#pragma unroll
-    for (int j = 0; j < kUpdChunk; ++j)
-      if (j < RC) wc[0][j] = pp[tc + GC * j];
-    const double r2 = red2[lane32];
-    const double pv = sum32(lane32 < GR ? r2 : 0.0);
-    const double a2 = -0.5 * tau * pv;
-#pragma unroll
-    for (int a = 0; a < RR; ++a) wr[a] = fma(a2, vr[a], wr[a]);  // p = v = 0 off the live rows
-    // A -= v w^T + w v^T on the live column slots, every row (v = w = 0 at finished rows and rows
-    // beyond the block leave them exactly unchanged).  Column i + 1 (slot bn, a uniform index) is
-    // then copied out and handed to the next step by its owners (tc == tn): the reflector input x,
-    // its partial squared norm and the diagonal element.
-    const int bn = (i + 1) / GC, tn = (i + 1) - bn * GC;
-    double coln[RR];
-#pragma unroll
-    for (int a = 0; a < RR; ++a) coln[a] = 0.0;
-#pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch) {
-      const int b0 = ch * kUpdChunk;
-      if (ch + 1 < kChunks) {
-#pragma unroll
-        for (int j = 0; j < kUpdChunk; ++j)
-          if (b0 + kUpdChunk + j < RC) wc[(ch + 1) & 1][j] = pp[tc + GC * (b0 + kUpdChunk + j)];
-      }
-      if (GC * min(b0 + kUpdChunk, RC) - 1 <= i || GC * b0 >= n) continue;  // whole chunk idle (uniform)
-#pragma unroll
-      for (int j = 0; j < kUpdChunk; ++j) {
-        const int b = b0 + j;
-        if (b >= RC) break;
-        if (GC * b + GC - 1 <= i || GC * b >= n) continue;
-        const double vb = vc[b];
-        const double wb = fma(a2, vb, wc[ch & 1][j]);  // p = v = 0 off the live columns
-#pragma unroll
-        for (int a = 0; a < RR; ++a) Ar[a][b] = fma(-vr[a], wb, fma(-wr[a], vb, Ar[a][b]));
-      }
-    }
-#pragma unroll
-    for (int b = 0; b < RC; ++b)
-      if (b == bn) {  // uniform
-#pragma unroll
-        for (int a = 0; a < RR; ++a) coln[a] = Ar[a][b];
-      }
-    double partn = 0.0;
-    if (tc == tn) {
-#pragma unroll
-      for (int a = 0; a < RR; ++a) {
-        const int r = tr + GR * a;
-        if (r == i + 1) d[i + 1] = coln[a];
-        xnext[r] = (r > i + 1 && r < n) ? coln[a] : 0.0;  // every row: zero off the live range
-        if (r > i + 2 && r < n) partn = fma(coln[a], coln[a], partn);
-      }
-    }
-    if (tc == tn) red1[tr] = partn;
-  }
-  // the trailing 2 x 2 block (or the 1 x 1 of a one-orbital block)
-#pragma unroll
-  for (int a = 0; a < RR; ++a)
-#pragma unroll
-    for (int b = 0; b < RC; ++b) {
-      const int r = tr + GR * a, c = tc + GC * b;
-      if (r == n - 2 && c == n - 2) d[n - 2] = Ar[a][b];
-      if (r == n - 1 && c == n - 2) e[n - 2] = Ar[a][b];
-      if (r == n - 1 && c == n - 1) d[n - 1] = Ar[a][b];
-    }
-  __syncthreads();
-
   // ---- 2. the nv lowest eigenvalues: multisection, a group of tb lanes per eigenvalue
   double lo_p = 1.0e300, hi_p = -1.0e300, e2max = 0.0;
   for (int k = tid; k < n; k += NT) {
     const double el = k > 0 ? fabs(e[k - 1]) : 0.0, er = k + 1 < n ? fabs(e[k]) : 0.0;
-    lo_p = fmin(lo_p, d[k] - el - er);
-    hi_p = fmax(hi_p, d[k] + el + er);
+    lo_p = fmin(lo_p, de[k].x - el - er);
+    hi_p = fmax(hi_p, de[k].x + el + er);
     if (k + 1 < n) {
-      pp[k] = e[k] * e[k];  // e^2 for the Sturm counts (pp is free after the reduction)
-      e2max = fmax(e2max, pp[k]);
+      de[k].y = e[k] * e[k];  // e^2 for the Sturm counts 
+      e2max = fmax(e2max, de[k].y);
     }
   }
   double glo = eig_block_min<NT>(lo_p, red);
@@ -482,7 +591,7 @@ __global__ __launch_bounds__(GR* GC) void k_eigh_density(pyseqm_layout_t L, cons
         for (int round = 0; round < 64; ++round) {
           if (!(hi - lo > fmax(4.4e-16 * fmax(fabs(lo), fabs(hi)), btol) + 2.0 * pivmin)) break;
           const double x = lo + (hi - lo) * (double)(gl + 1) / (double)(tb + 1);
-          const int cnt = (x > lo && x < hi) ? sturm_count(d, pp, n, x, pivmin) : -1;
+          const int cnt = (x > lo && x < hi) ? sturm_count(de, n, x, pivmin) : -1;
           const double nlo = group_max_t(cnt >= 0 && cnt <= j ? x : lo, tb);
           const double nhi = group_min_t(cnt > j ? x : hi, tb);
           if (nlo == lo && nhi == hi) break;  // no representable interior point left
@@ -495,10 +604,10 @@ __global__ __launch_bounds__(GR* GC) void k_eigh_density(pyseqm_layout_t L, cons
   }
   __syncthreads();
 
-  // ---- 3. inverse iteration, one thread per eigenvector; vector j in LDS at Z[k * nv + j]
+  // ---- 3. inverse iteration, one thread per eigenvector; vector j in LDS at Z[k * ldz + j]
   const double tiny = 2.2e-16 * fmax(tnorm, 1.0e-300);
   for (int j = tid; j < nv; j += NT) {
-    for (int k = 0; k < n; ++k) Z[k * nv + j] = start_value(j, k);
+    for (int k = 0; k < n; ++k) Z[k * ldz + j] = start_value(j, k);
     const double sig = lam[j];
     for (int rep = 0; rep < 3; ++rep) {
       // LU of T - sig I with partial pivoting, the right-hand side eliminated alongside; the
@@ -506,17 +615,17 @@ __global__ __launch_bounds__(GR* GC) void k_eigh_density(pyseqm_layout_t L, cons
       // keeps one of two rows as the pivot row (its diagonal and sub-diagonal entries compared)
       // and eliminates the other, both cases as one select-based update (lanes differ in their
       // choices); the next step's d, e and right-hand side are read from LDS one step ahead.
-      double diag = d[0] - sig, sup = n > 1 ? e[0] : 0.0;
+      double diag = de[0].x - sig, sup = n > 1 ? e[0] : 0.0;
       double yk = Z[j];
-      double sub_n = n > 1 ? e[0] : 0.0, dn_n = n > 1 ? d[1] : 0.0, ns_n = n > 2 ? e[1] : 0.0;
-      double y_n = n > 1 ? Z[nv + j] : 0.0;
+      double sub_n = n > 1 ? e[0] : 0.0, dn_n = n > 1 ? de[1].x : 0.0, ns_n = n > 2 ? e[1] : 0.0;
+      double y_n = n > 1 ? Z[ldz + j] : 0.0;
       for (int k = 0; k + 1 < n; ++k) {
         const double sub = sub_n, nd = dn_n - sig, ns = ns_n, yk1 = y_n;
         if (k + 2 < n) {
           sub_n = ns_n;
-          dn_n = d[k + 2];
+          dn_n = de[k + 2].x;
           ns_n = k + 3 < n ? e[k + 2] : 0.0;
-          y_n = Z[(k + 2) * nv + j];
+          y_n = Z[(k + 2) * ldz + j];
         }
         const size_t o = (size_t)k * nmax + j;
         const bool keep = fabs(diag) >= fabs(sub);  // no row exchange
@@ -528,14 +637,14 @@ __global__ __launch_bounds__(GR* GC) void k_eigh_density(pyseqm_layout_t L, cons
         U0[o] = rp;
         U1[o] = p1;
         U2[o] = p2;
-        Z[k * nv + j] = py;
+        Z[k * ldz + j] = py;
         yk = fma(-mlt, py, oy);
         diag = fma(-mlt, p1, o1);
         sup = fma(-mlt, p2, o2);
       }
       const double rlast = 1.0 / (fabs(diag) < tiny ? copysign(tiny, diag) : diag);
       double x1 = yk * rlast, x2 = 0.0, xmax = fabs(x1);
-      Z[(n - 1) * nv + j] = x1;
+      Z[(n - 1) * ldz + j] = x1;
       // back substitution in blocks of kPF rows: the U factors of the next block are loaded while
       // this block is solved (the loads come from L2; one row ahead left each row waiting on one)
       constexpr int kPF = 8;
@@ -562,8 +671,8 @@ __global__ __launch_bounds__(GR* GC) void k_eigh_density(pyseqm_layout_t L, cons
         for (int t = 0; t < kPF; ++t) {
           const int k = k0 - t;
           if (k >= 0) {
-            const double x = (Z[k * nv + j] - c1[t] * x1 - c2[t] * x2) * c0[t];
-            Z[k * nv + j] = x;
+            const double x = (Z[k * ldz + j] - c1[t] * x1 - c2[t] * x2) * c0[t];
+            Z[k * ldz + j] = x;
             xmax = fmax(xmax, fabs(x));
             x2 = x1;
             x1 = x;
@@ -577,7 +686,7 @@ __global__ __launch_bounds__(GR* GC) void k_eigh_density(pyseqm_layout_t L, cons
         }
       }
       const double sc = xmax > 0.0 ? 1.0 / xmax : 1.0;
-      for (int k = 0; k < n; ++k) Z[k * nv + j] *= sc;
+      for (int k = 0; k < n; ++k) Z[k * ldz + j] *= sc;
     }
   }
   __syncthreads();
@@ -593,100 +702,107 @@ __global__ __launch_bounds__(GR* GC) void k_eigh_density(pyseqm_layout_t L, cons
       for (int pass = 0; pass < 2; ++pass)
         for (int p = j; p < q; ++p) {
           double dot = 0.0;
-          for (int k = 0; k < n; ++k) dot += Z[k * nv + p] * Z[k * nv + q];
-          for (int k = 0; k < n; ++k) Z[k * nv + q] -= dot * Z[k * nv + p];
+          for (int k = 0; k < n; ++k) dot += Z[k * ldz + p] * Z[k * ldz + q];
+          for (int k = 0; k < n; ++k) Z[k * ldz + q] -= dot * Z[k * ldz + p];
         }
       double nr = 0.0;
-      for (int k = 0; k < n; ++k) nr += Z[k * nv + q] * Z[k * nv + q];
+      for (int k = 0; k < n; ++k) nr += Z[k * ldz + q] * Z[k * ldz + q];
       if (!(nr > 1.0e-200)) {  // a vector lost to its cluster's span: flagged, left unscaled
         atomicAdd(fail, 1);
         continue;
       }
       const double sc = 1.0 / sqrt(nr);
-      for (int k = 0; k < n; ++k) Z[k * nv + q] *= sc;
+      for (int k = 0; k < n; ++k) Z[k * ldz + q] *= sc;
     }
   }
   __syncthreads();
 
   if (EVEC) {  // Rayleigh quotients z^T T z of the normalised vectors (ascending to rounding)
     for (int j = tid; j < nv; j += NT) {
-      double rq = d[0] * Z[j] * Z[j];
+      double rq = de[0].x * Z[j] * Z[j];
       for (int k = 1; k < n; ++k) {
-        const double zk = Z[k * nv + j], zk1 = Z[(k - 1) * nv + j];
-        rq += d[k] * zk * zk + 2.0 * e[k - 1] * zk * zk1;
+        const double zk = Z[k * ldz + j], zk1 = Z[(k - 1) * ldz + j];
+        rq += de[k].x * zk * zk + 2.0 * e[k - 1] * zk * zk1;
       }
       lam[j] = rq;
     }
     __syncthreads();
   }
-  // ---- 5. C = Q Z in registers: thread (tr, tc) holds C[tc + 16 b][tr + GR c] (b < RC rows
-  //         over the lanes of its DPP row, c < RR columns), so each column's product v^T C reduces
-  //         inside one DPP row and the reflectors (last to first) need no barrier; each thread
-  //         reads its RC elements of the next reflector from the workspace while applying one.
-  double* C = Z;
-  {
+  // ---- 5. C = Q Z: 16 columns per wave in registers, blocks of 16 reflectors last to first, each
+  //         as C -= V (T (V^T C)) on FP64 MFMA; C goes back over Z
+  if (n >= 3) {
+    constexpr int NTL = S / 16;
+    for (int q = wave + (S - n) / 16; q < NTL; q += NW) panel_t<S>(HH, tau, nmax, n, q, T + kTPanel * q);
+    __syncthreads();
+    const int off = S - n;
+    for (int vt = wave; 16 * vt < nv; vt += NW) {
+      const int col = 16 * vt + (lane & 15), g = lane >> 4;
+      doublex4 Cr[NTL];
 #pragma unroll
-    for (int c = 0; c < RR; ++c)
+      for (int t = 0; t < NTL; ++t)
 #pragma unroll
-      for (int b = 0; b < RC; ++b) {
-        const int k = tc + 16 * b, a = tr + GR * c;
-        Ar[c][b] = (k < n && a < nv) ? Z[k * nv + a] : 0.0;
-      }
-    back_transform<GR, RR, RC, CM>(Ar, HH, nmax, n, nv, tr, tc, C);
+        for (int s = 0; s < 4; ++s) {
+          const int k = 16 * t + 4 * s + g - off;
+          const double z = Z[max(k, 0) * ldz + min(col, nv - 1)];
+          Cr[t][s] = (k >= 0 && col < nv) ? z : 0.0;
+        }
+      const double* hh = HH;
+      const double* tt = T;
+      asm volatile("" : "+s"(hh));  // keep the panels' loads inside the loop (hoisted, they spill)
+      if constexpr (S != 48) asm volatile("" : "+s"(tt));
+      back_panels<S, NTL - 1>(Cr, hh, tt, nmax, n);
+#pragma unroll
+      for (int t = 0; t < NTL; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int k = 16 * t + 4 * s + g - off;
+          if (k >= 0 && col < nv) Z[k * ldz + col] = Cr[t][s];
+        }
+    }
     __syncthreads();
   }
   if (EVEC) {
     double* Qm = P + mo;
-    for (int t = tid; t < n * n; t += NT) Qm[t] = C[t];  // C is n x n, row k = orbital, column j = vector
+    for (int t = tid; t < n * n; t += NT) Qm[t] = Z[(t / n) * ldz + t % n];  // row = orbital, column = vector
     for (int j = tid; j < n; j += NT) evals[orb_off[m] + j] = lam[j];
     return;
   }
-  // ---- P = 2 C C^T, 4 x 4 output blocks per thread over the upper triangle of blocks (tasks
-  //      enumerated over the triangle only), both triangles written; every element sums over the
-  //      vectors in order, and the two copies of a diagonal block's element are the same bits
+  // ---- P = 2 C C^T, a 16 x 16 tile of the upper triangle per wave at a time (two chains over the
+  //      vectors, added); elements r <= c are written to both triangles: the two copies are the
+  //      same bits.  91 vectors of 182 orbitals: 58 us as 4 x 4 blocks per thread, 21 us as MFMA tiles
   double* Pm = P + mo;
-  const int nb4 = (n + 3) / 4;
-  const int ntask = nb4 * (nb4 + 1) / 2;
-  for (int t = tid; t < ntask; t += NT) {
-    int bi = 0, rem = t;
-    while (rem >= nb4 - bi) {
-      rem -= nb4 - bi;
+  const int nt = (n + 15) / 16, ntask = nt * (nt + 1) / 2;
+  const int mr = lane & 15, g = lane >> 4, nfull = nv / 4;
+  for (int task = wave; task < ntask; task += NW) {
+    int bi = 0, rem = task;
+    while (rem >= nt - bi) {
+      rem -= nt - bi;
       ++bi;
     }
     const int bj = bi + rem;
-    int ro[4], co[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      ro[q] = min(4 * bi + q, n - 1) * nv;
-      co[q] = min(4 * bj + q, n - 1) * nv;
+    const double* ca = Z + min(16 * bi + mr, n - 1) * ldz + g;
+    const double* cb = Z + min(16 * bj + mr, n - 1) * ldz + g;
+    doublex4 a0 = {0.0, 0.0, 0.0, 0.0}, a1 = {0.0, 0.0, 0.0, 0.0};
+    int k = 0;
+    for (; k + 1 < nfull; k += 2) {
+      a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(ca[4 * k], cb[4 * k], a0, 0, 0, 0);
+      a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(ca[4 * k + 4], cb[4 * k + 4], a1, 0, 0, 0);
     }
-    double acc[4][4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc[p][q] = 0.0;
-    for (int a = 0; a < nv; ++a) {
-      double x[4], y[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        x[q] = C[ro[q] + a];
-        y[q] = C[co[q] + a];
-      }
-#pragma unroll
-      for (int p = 0; p < 4; ++p)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc[p][q] += x[p] * y[q];
+    if (k < nfull) a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(ca[4 * k], cb[4 * k], a0, 0, 0, 0);
+    if (4 * nfull < nv) {
+      const bool in = 4 * nfull + g < nv;
+      const double x = in ? ca[4 * nfull] : 0.0, y = in ? cb[4 * nfull] : 0.0;
+      a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, a1, 0, 0, 0);
     }
+    a0 += a1;
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int r = 4 * bi + p, c = 4 * bj + q;
-        if (r < n && c < n) {
-          Pm[(size_t)r * n + c] = 2.0 * acc[p][q];
-          Pm[(size_t)c * n + r] = 2.0 * acc[p][q];
-        }
+    for (int s = 0; s < 4; ++s) {
+      const int r = 16 * bi + 4 * s + g, c = 16 * bj + mr;
+      if (r <= c && c < n) {
+        Pm[(size_t)r * n + c] = 2.0 * a0[s];
+        Pm[(size_t)c * n + r] = 2.0 * a0[s];
       }
+    }
   }
 }
 
@@ -697,36 +813,21 @@ extern "C" long long pyseqm_eigh_density_workspace(int nact, int nmax) {
   return 4LL * nact * nmax * nmax;
 }
 
-// thread grid GR x 16 with RR x RC register slots per thread: GR RR and 16 RC cover nmax
-// (the back-transformation's column slots: half of them when every listed block's vector count
-// nvmax fits, which the density step's nocc usually does)
-template <int GR, int RR, int RC, bool EVEC>
-void launch_variant(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, int nvmax, const double* F,
-                    double* out, double* ws, int* fail, const long long* orb_off, double* evals, size_t lds,
-                    hipStream_t s) {
-  if (nvmax <= GR * (RR / 2))
-    k_eigh_density<GR, 16, RR, RC, EVEC, RR / 2><<<nact, GR * 16, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off,
-                                                                         evals);
-  else
-    k_eigh_density<GR, 16, RR, RC, EVEC, RR><<<nact, GR * 16, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off,
-                                                                      evals);
-}
-
+// waves per workgroup and register slots per thread: the 4 NW x 16 thread grid covers 48, 96 or 192
 template <bool EVEC>
-void launch_eigh(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, int nvmax, const double* F,
-                 double* out, double* ws, int* fail, const long long* orb_off, double* evals, size_t lds,
-                 hipStream_t s) {
+void launch_eigh(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const double* F, double* out,
+                 double* ws, int* fail, const long long* orb_off, double* evals, size_t lds, hipStream_t s) {
   if (nmax <= 48)
-    launch_variant<4, 12, 3, EVEC>(L, idx, nact, nmax, nvmax, F, out, ws, fail, orb_off, evals, lds, s);
+    k_eigh_density<1, 12, 3, EVEC><<<nact, 64, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
   else if (nmax <= 96)
-    launch_variant<16, 6, 6, EVEC>(L, idx, nact, nmax, nvmax, F, out, ws, fail, orb_off, evals, lds, s);
+    k_eigh_density<4, 6, 6, EVEC><<<nact, 256, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
   else
-    launch_variant<32, 6, 12, EVEC>(L, idx, nact, nmax, nvmax, F, out, ws, fail, orb_off, evals, lds, s);
+    k_eigh_density<8, 6, 12, EVEC><<<nact, 512, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
 }
 
 extern "C" int pyseqm_eigh_density_lds_ok(int norb, int nocc) {
   if (norb < 1 || norb > kEighMaxN || nocc < 0 || nocc > norb) return 0;
-  return lds_doubles(norb, nocc) <= kLdsDoubles;
+  return rule_doubles(norb, nocc) <= kLdsDoubles;
 }
 
 extern "C" int pyseqm_eigh_density(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, int nocc_max,
@@ -737,7 +838,7 @@ extern "C" int pyseqm_eigh_density(const pyseqm_layout_t* L, const int* idx, int
   if (nact == 0) return PYSEQM_OK;
   const size_t lds = (size_t)lds_doubles(nmax, nocc_max) * sizeof(double);
   hipStream_t s = (hipStream_t)stream;
-  launch_eigh<false>(L, idx, nact, nmax, nocc_max, F, P, ws, fail, nullptr, nullptr, lds, s);
+  launch_eigh<false>(L, idx, nact, nmax, F, P, ws, fail, nullptr, nullptr, lds, s);
   return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
 }
 
@@ -748,6 +849,6 @@ extern "C" int pyseqm_eigh_vectors(const pyseqm_layout_t* L, const int* idx, int
   if (!pyseqm_eigh_density_lds_ok(nmax, nmax)) return PYSEQM_EINVAL;
   if (nact == 0) return PYSEQM_OK;
   const size_t lds = (size_t)lds_doubles(nmax, nmax) * sizeof(double);
-  launch_eigh<true>(L, idx, nact, nmax, nmax, F, Q, ws, fail, orb_off, evals, lds, (hipStream_t)stream);
+  launch_eigh<true>(L, idx, nact, nmax, F, Q, ws, fail, orb_off, evals, lds, (hipStream_t)stream);
   return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
 }

@@ -1,0 +1,81 @@
+"""The workgroup eigensolver at the edges of its register grids (48, 96, 192 rows), of its 16-wide panels and
+of its occupations, against numpy's float64 eigh.
+
+Bars: the density within 1e-10 of the reference's (levels of 1..40 eV and a gap of 11 eV: n eps |F| / gap < 1e-12,
+and eps |F| / gap < 1e-11 between levels of the nearest spacing drawn), exactly symmetric;
+reruns bitwise equal.
+"""
+import numpy as np
+import pytest
+import torch
+
+from pyseqm_amd.engine import SCFEngine, eigh_wg_ok
+from pyseqm_amd.layout import PackedBatch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _blocks(sizes, noccs, kind, seed):
+    rng = np.random.default_rng(seed)
+    out = []
+    for n, o in zip(sizes, noccs):
+        lam = np.concatenate([-np.sort(rng.uniform(10.0, 40.0, o)), np.sort(rng.uniform(1.0, 20.0, n - o))])
+        if kind == "degenerate":  # pairs of equal levels
+            for i in range(1, o, 2):
+                lam[i] = lam[i - 1]
+        elif kind == "close":  # clusters: spacings of 1e-6, 1e-9 and 1e-12 of the spectrum's width
+            for i in range(1, o):
+                if i % 7 < 3:
+                    lam[i] = lam[i - 1] + (4e-5, 4e-8, 4e-11)[i % 7]
+        Q, _ = np.linalg.qr(rng.normal(size=(n, n)))
+        f = (Q * lam) @ Q.T
+        if kind == "diagonal":
+            f = np.diag(rng.permutation(lam))
+        elif kind == "blocks":  # two decoupled halves
+            f[:n // 2, n // 2:] = 0.0
+            f[n // 2:, :n // 2] = 0.0
+            f[np.arange(n), np.arange(n)] -= 30.0 * (np.arange(n) < o)
+        out.append(0.5 * (f + f.T))
+    return out
+
+
+def _engine(sizes, noccs):
+    nh = [n // 4 for n in sizes]
+    nH = [n - 4 * k for n, k in zip(sizes, nh)]
+    molsize = max(a + b for a, b in zip(nh, nH))
+    b = PackedBatch.from_counts(nh, nH, noccs, molsize, DEV)
+    return SCFEngine(None, None, "AM1", DEV, batch=b)
+
+
+SETS = {48: [1, 2, 3, 4, 15, 16, 17, 31, 33, 47, 48], 96: [1, 3, 16, 49, 50, 64, 65, 80, 95, 96],
+        192: [1, 2, 5, 97, 98, 112, 113, 128, 129, 160, 161, 182, 191, 192]}
+
+
+@pytest.mark.parametrize("grid", sorted(SETS))
+@pytest.mark.parametrize("kind", ["spread", "degenerate", "close", "diagonal", "blocks"])
+def test_density_at_grid_edges(grid, kind):
+    sizes = SETS[grid]
+    noccs = [min([n // 2, n, 0, (2 * n) // 3, 1][k % 5] if n < 97 else n // 2 - k % 3, n) for k, n in enumerate(sizes)]
+    eng = _engine(sizes, noccs)
+    assert eigh_wg_ok(max(sizes), max(noccs))
+    fs = _blocks(sizes, noccs, kind, grid)
+    F = torch.as_tensor(np.concatenate([f.reshape(-1) for f in fs]), device=DEV)
+    Ps = []
+    for _ in range(2):
+        P = torch.full_like(F, float("nan"))
+        eng._eigh_wg(F, np.arange(len(sizes)), P)
+        Ps.append(P)
+    torch.cuda.synchronize()
+    assert torch.equal(*Ps)
+    o = 0
+    for f, n, nocc in zip(fs, sizes, noccs):
+        p = P[o:o + n * n].view(n, n).cpu().numpy()
+        o += n * n
+        w, U = np.linalg.eigh(f)
+        if 0 < nocc < n and w[nocc] - w[nocc - 1] < 1.0:
+            continue  # no gap in this block: its density is undetermined
+        ref = 2.0 * U[:, :nocc] @ U[:, :nocc].T
+        assert np.array_equal(p, p.T), n
+        assert np.abs(p - ref).max() < 1e-10, (n, nocc, np.abs(p - ref).max())
+    assert int(eng.eigh_fail.item()) == 0
