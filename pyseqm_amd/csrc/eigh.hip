@@ -4,15 +4,17 @@
 //
 //   1. Householder reduction of the block to tridiagonal form T = Q^T F Q (dsytd2 order), with the
 //      matrix in registers (tridiagonalise below).  The reflectors go to the global workspace.
-//   2. The nocc lowest eigenvalues of T by multisection on Sturm counts: a group of lanes per
-//      eigenvalue evaluates the count at evenly spaced points of its bracket each round.
-//   3. Their eigenvectors by inverse iteration (tridiagonal LU with partial pivoting, three solves
-//      from a fixed pseudo-random start), one thread per vector, the vectors in LDS.
-//   4. Vectors of eigenvalues closer than 1e-5 |T| (a cluster) orthogonalised against each other
-//      by two Gram-Schmidt passes, every vector normalised.  Inverse iteration leaves vectors of
-//      eigenvalues further apart orthogonal to eps |T| / gap < 3e-11; a degenerate eigenvalue's
-//      vectors come from different start vectors, so they span its subspace and the passes make
-//      them orthonormal inside it (P depends on the occupied subspace only).
+//   2. The nocc lowest eigenvalues of T by Sturm counts: one evenly spaced grid over the whole
+//      spectrum for all of them, then multisection (a group of lanes per eigenvalue) to 1e-11 |T|,
+//      to rounding where a neighbour is closer than 1e-9 |T|.
+//   3. Their eigenvectors from twisted factorisations of T - lambda I, two lanes per vector (one from
+//      each end), the vectors in LDS: one factorisation at the bracket's middle, whose Rayleigh
+//      correction is kept unrounded beside lambda, and one there.
+//   4. Vectors of eigenvalues closer than 1e-3 |T| (a cluster) orthogonalised against each other,
+//      a cluster per wave.  Vectors further apart come out orthogonal to eps |T| / gap.  Where a
+//      neighbour is closer than 1e-10 |T| (a degenerate level, which a twisted factorisation would
+//      give the same vector twice) the vectors come from inverse iteration with different starts
+//      instead: they span the level's subspace (P depends on the occupied subspace only).
 //   5. Back-transformation C = Q Z by blocks of 16 reflectors and P = 2 C C^T, both on FP64 MFMA
 //      tiles.
 // Every reduction runs in a fixed order: reruns are bitwise identical.
@@ -27,32 +29,36 @@ namespace {
 constexpr int kEighMaxN = 192;      // largest block this solver takes
 constexpr int kLdsDoubles = 20480;  // 160 KiB of LDS
 constexpr int kTPanel = 256;        // doubles of one panel's 16 x 16 T factor
+constexpr int kLdsExtra = 25;       // doubles of the twist rows and of an alignment gap
 
 // workspace per listed molecule, in doubles, at slot * 4 * nmax^2:
 //   [0, nmax^2)          reflectors: row i holds u_i (zero at columns <= i of its panel of 16)
-//   [nmax^2, 4 nmax^2)   the U factor of each inverse-iteration LU (reciprocal diagonal and two
-//                        superdiagonals), element k of vector j at k * nmax + j; the panels' T
-//                        factors of the back-transformation afterwards (blocks above 48 orbitals)
-// LDS: eigenvectors n x ldz (the Householder vectors before them, in the same place), then
-// (d, e^2) pairs, e, eigenvalues, reflector scales and vector scales (n each), and the panels' T
-// factors of blocks of up to 48 orbitals.  The variant follows the launch's largest block nmax.
+//   [nmax^2, 4 nmax^2)   element k of vector j at k * nmax + j: the lower multipliers of the twisted
+//                        factorisations (blocks above 48 orbitals), the U factor of each
+//                        inverse-iteration LU (reciprocal diagonal and two superdiagonals); then
+//                        the panels' T factors of the back-transformation (above 48 orbitals)
+// LDS: eigenvectors n x ldz (before them, in the same place, the Householder vectors, then the grid's
+// counts), (d, e^2) pairs, e, eigenvalues, reflector scales and vector scales (n each), the twist
+// rows (a byte each), and for blocks of up to 48 orbitals the panels' T factors and the lower
+// multipliers.  The variant follows the launch's largest block nmax.
 __host__ __device__ inline int grid_slots(int nmax) { return nmax <= 48 ? 48 : (nmax <= 96 ? 96 : 192); }
 // The size rule of the entry points: n nocc + 3 n + 3 S + 128 doubles (S: the variant's 48 / 96 /
 // 192 grid rows).  lds_doubles, what a launch asks for, stays within it for every accepted block.
 __host__ __device__ inline int rule_doubles(int n, int nv) { return n * nv + 3 * n + 3 * grid_slots(n) + 128; }
 // Row stride of the eigenvectors: odd where that fits (rows of 16 lanes then fall on distinct LDS
 // banks), else nv.
-__host__ __device__ inline int zstride(int n, int nv) { return n * (nv | 1) + 6 * n + 1 <= kLdsDoubles ? (nv | 1) : nv; }
-// Doubles of the eigenvector region: also holds the Householder vectors (2 S) before.
+__host__ __device__ inline int zstride(int n, int nv) { return n * (nv | 1) + 6 * n + kLdsExtra <= kLdsDoubles ? (nv | 1) : nv; }
+// Doubles of the eigenvector region: also holds the Householder vectors (2 S) and the grid's counts
+// (two ints per thread) before.
 __host__ __device__ inline int zregion(int n, int nv, int S) {
-  const int z = n * zstride(n, nv);
-  return z > 2 * S ? z : 2 * S;
+  const int z = n * zstride(n, nv), least = S == 192 ? 512 : (S == 96 ? 256 : 96);
+  return z > least ? z : least;
 }
 inline int lds_doubles(int nmax, int nv) {
   const int S = grid_slots(nmax);
   // where the odd stride does not fit the largest block it may still fit a smaller one of the launch
   if (zstride(nmax, nv) != (nv | 1)) return kLdsDoubles;
-  return zregion(nmax, nv, S) + 1 + 6 * nmax + (S == 48 ? 3 * kTPanel : 0);
+  return zregion(nmax, nv, S) + 6 * nmax + kLdsExtra + (S == 48 ? 3 * kTPanel + nmax * (nv | 1) : 0);
 }
 
 template <int NT>
@@ -92,34 +98,66 @@ __device__ inline double rcp_f64(double q) {
   return r;
 }
 
-// number of eigenvalues of the tridiagonal (d, e) below x: the negative pivots q_k of the LDL^T
-// factorisation of T - x I (de[k] = (d_k, e_k^2)), counted as sign changes of the Sturm sequence
+// cnt[i] = number of eigenvalues of the tridiagonal de[k] = (d_k, e_k^2) below x[i]: the negative
+// pivots q_k of the LDL^T factorisation of T - x I, counted as sign changes of the Sturm sequence
 // p_0 = 1, p_k = (d_k - x) p_{k-1} - e2_{k-1} p_{k-2} (q_k = p_k / p_{k-1}), whose dependent chain
-// is one FMA per step instead of a reciprocal.  |q_k| < pivmin is floored to q_k = -pivmin, as in
-// the ratio form: |p_k| < pivmin |p_{k-1}| -> p_k = -pivmin p_{k-1}.  Every 8 steps both terms are
-// scaled by the same power of two (exact; signs and ratios unchanged), which keeps them in range.
-__device__ inline void sturm_step(double dk, double e2k, double x, double pivmin, double& p0, double& p1, int& cnt) {
-  double p2 = fma(dk - x, p1, -(e2k * p0));
-  if (fabs(p2) < pivmin * fabs(p1)) p2 = -pivmin * p1;
-  cnt += (__double_as_longlong(p2) ^ __double_as_longlong(p1)) < 0;  // sign bits differ
-  p0 = p1;
-  p1 = p2;
-}
-__device__ inline int sturm_count(const double2* de, int n, double x, double pivmin) {
-  double p0 = 1.0, p1 = de[0].x - x;
-  if (fabs(p1) < pivmin) p1 = -pivmin;
-  int cnt = p1 < 0.0;
-  int k = 1;
-  for (; k + 8 <= n; k += 8) {
+// is one FMA per step instead of a reciprocal.  Every e2 is above zero (the caller floors it at
+// (1e-30 |T|)^2), so a p_k of exactly zero is followed by one of the sign opposite to p_{k-1}: one
+// sign change over the two steps whichever sign bit the zero carries.  Signs collect in the bits of
+// one register (one instruction a step); every 8 steps they are counted and both terms scaled
+// by the same power of two (exact; signs and ratios unchanged), which keeps them in range.
+template <int K>
+__device__ inline void sturm_counts(const double2* de, int n, const double (&x)[K], int (&cnt)[K]) {
+  double p0[K], p1[K];
+  unsigned m[K];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) sturm_step(de[k + t].x, de[k + t - 1].y, x, pivmin, p0, p1, cnt);
-    int ex;
-    frexp(fmax(fabs(p0), fabs(p1)), &ex);
-    p0 = ldexp(p0, -ex);
-    p1 = ldexp(p1, -ex);
+  for (int i = 0; i < K; ++i) {
+    p0[i] = 1.0;
+    p1[i] = de[0].x - x[i];
+    m[i] = (unsigned)__double2hiint(p1[i]) >> 31;
+    cnt[i] = (int)m[i];
   }
-  for (; k < n; ++k) sturm_step(de[k].x, de[k - 1].y, x, pivmin, p0, p1, cnt);
-  return cnt;
+  auto step = [&](double dk, double e2k) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const double p2 = fma(dk - x[i], p1[i], -(e2k * p0[i]));
+      m[i] = __builtin_amdgcn_alignbit(m[i], (unsigned)__double2hiint(p2), 31);  // m << 1 | sign
+      p0[i] = p1[i];
+      p1[i] = p2;
+    }
+  };
+  // the next eight rows are read while eight are used (reads past row n - 1 fall into the arrays
+  // that follow de and are not used)
+  int k = 1;
+  double prev = de[0].y;
+  double2 w[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) w[t] = de[1 + t];
+#pragma unroll 2
+  for (; k + 8 <= n; k += 8) {
+    double2 wn[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) wn[t] = de[k + 8 + t];
+    step(w[0].x, prev);
+#pragma unroll
+    for (int t = 1; t < 8; ++t) step(w[t].x, w[t - 1].y);
+    prev = w[7].y;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) w[t] = wn[t];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      cnt[i] += __popc((m[i] ^ (m[i] >> 1)) & 0xffu);
+      const int ex = max(__builtin_amdgcn_frexp_exp(p0[i]), __builtin_amdgcn_frexp_exp(p1[i]));
+      p0[i] = __builtin_amdgcn_ldexp(p0[i], -ex);
+      p1[i] = __builtin_amdgcn_ldexp(p1[i], -ex);
+    }
+  }
+  const unsigned rest = (1u << (n - k)) - 1u;
+#pragma unroll
+  for (int t = 0; t < 7; ++t)
+    if (k + t < n) step(w[t].x, t == 0 ? prev : w[t > 0 ? t - 1 : 0].y);
+#pragma unroll
+  for (int i = 0; i < K; ++i) cnt[i] += __popc((m[i] ^ (m[i] >> 1)) & rest);
 }
 
 // One DPP lane permutation of a double (two 32-bit DPP moves; VALU, no LDS round trip).
@@ -172,6 +210,151 @@ __device__ inline double start_value(int j, int k) {
   return (double)h * (2.0 / 4294967296.0) - 1.0;
 }
 
+
+// One end's multipliers L_k = e_k / q_k of T - (hi + lo) I for the vector of this lane, q_k = p_k /
+// p_{k-1} with p_k the Sturm sequence from that end (DIR 1: from the top, -1: from the bottom), so
+// that the chain has no division.  out walks by os per row.  A p_k of zero is floored at tiny
+// p_{k-1}.  d and e point at this end's first entries; rows are read eight ahead of their use (at
+// most eight past the other end, into the LDS arrays around; not used there).
+template <int DIR, class P>
+__device__ __forceinline__ void twisted_sweep(const double2* d, const double* e, int n, double hi, double lo,
+                                              double tiny, P out, int os) {
+  double p0 = 1.0, p1 = (d[0].x - hi) - lo;
+  if (fabs(p1) < tiny) p1 = tiny;
+  auto step = [&](double dk, double ek) {
+    const double ep0 = ek * p0;
+    *out = ep0 * rcp_f64(p1);
+    out += os;
+    double p2 = fma((dk - hi) - lo, p1, -(ek * ep0));
+    const double f = tiny * p1;
+    p2 = fabs(p2) < fabs(f) ? f : p2;
+    p0 = p1;
+    p1 = p2;
+  };
+  double w[8], x[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    w[t] = d[DIR * (t + 1)].x;
+    x[t] = e[DIR * t];
+  }
+  int k = 0;
+#pragma unroll 2
+  for (; k + 8 < n; k += 8) {
+    double wn[8], xn[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      wn[t] = d[DIR * (k + 9 + t)].x;
+      xn[t] = e[DIR * (k + 8 + t)];
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) step(w[t], x[t]);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      w[t] = wn[t];
+      x[t] = xn[t];
+    }
+    const int ex = max(__builtin_amdgcn_frexp_exp(p0), __builtin_amdgcn_frexp_exp(p1));
+    p0 = __builtin_amdgcn_ldexp(p0, -ex);
+    p1 = __builtin_amdgcn_ldexp(p1, -ex);
+  }
+#pragma unroll
+  for (int t = 0; t < 8; ++t)
+    if (k + t + 1 < n) step(w[t], x[t]);
+}
+
+// Inverse iteration on T - sig I: three solves from a fixed pseudo-random start (of vector j), one
+// thread; z (stride ldz) ends scaled to a largest element of 1.  Returns 1 / |z|.
+__device__ __forceinline__ double inverse_iteration(const double2* de, const double* e, double* z, int ldz, double* U0,
+                                                 double* U1, double* U2, int ldu, int n, int j, double sig,
+                                                 double tiny) {
+  double nrm = 0.0;
+  for (int k = 0; k < n; ++k) z[k * ldz] = start_value(j, k);
+  for (int rep = 0; rep < 3; ++rep) {
+    // LU of T - sig I with partial pivoting, the right-hand side eliminated alongside; the
+    // running row and right-hand side stay in registers, U goes to the workspace.  Each step
+    // keeps one of two rows as the pivot row (its diagonal and sub-diagonal entries compared)
+    // and eliminates the other, both cases as one select-based update (lanes differ in their
+    // choices); the next step's d, e and right-hand side are read from LDS one step ahead.
+    double diag = de[0].x - sig, sup = n > 1 ? e[0] : 0.0;
+    double yk = z[0];
+    double sub_n = n > 1 ? e[0] : 0.0, dn_n = n > 1 ? de[1].x : 0.0, ns_n = n > 2 ? e[1] : 0.0;
+    double y_n = n > 1 ? z[ldz] : 0.0;
+    for (int k = 0; k + 1 < n; ++k) {
+      const double sub = sub_n, nd = dn_n - sig, ns = ns_n, yk1 = y_n;
+      if (k + 2 < n) {
+        sub_n = ns_n;
+        dn_n = de[k + 2].x;
+        ns_n = k + 3 < n ? e[k + 2] : 0.0;
+        y_n = z[(k + 2) * ldz];
+      }
+      const size_t o = (size_t)k * ldu;
+      const bool keep = fabs(diag) >= fabs(sub);  // no row exchange
+      const double piv = keep ? (fabs(diag) < tiny ? copysign(tiny, diag) : diag) : sub;
+      const double rp = rcp_f64(piv);
+      const double mlt = (keep ? sub : diag) * rp;
+      const double p1 = keep ? sup : nd, p2 = keep ? 0.0 : ns, py = keep ? yk : yk1;
+      const double o1 = keep ? nd : sup, o2 = keep ? ns : 0.0, oy = keep ? yk1 : yk;
+      U0[o] = rp;
+      U1[o] = p1;
+      U2[o] = p2;
+      z[k * ldz] = py;
+      yk = fma(-mlt, py, oy);
+      diag = fma(-mlt, p1, o1);
+      sup = fma(-mlt, p2, o2);
+    }
+    const double rlast = 1.0 / (fabs(diag) < tiny ? copysign(tiny, diag) : diag);
+    double x1 = yk * rlast, x2 = 0.0, xmax = fabs(x1);
+    z[(n - 1) * ldz] = x1;
+    // back substitution in blocks of kPF rows: the U factors of the next block are loaded while
+    // this block is solved (the loads come from L2; one row ahead left each row waiting on one)
+    constexpr int kPF = 8;
+    double c0[kPF], c1[kPF], c2[kPF];
+#pragma unroll
+    for (int t = 0; t < kPF; ++t) {
+      const int kk = n - 2 - t;
+      const size_t o = (size_t)(kk >= 0 ? kk : 0) * ldu;
+      c0[t] = U0[o];
+      c1[t] = U1[o];
+      c2[t] = U2[o];
+    }
+    for (int k0 = n - 2; k0 >= 0; k0 -= kPF) {
+      double n0[kPF], n1[kPF], n2[kPF];
+#pragma unroll
+      for (int t = 0; t < kPF; ++t) {
+        const int kk = k0 - kPF - t;
+        const size_t o = (size_t)(kk >= 0 ? kk : 0) * ldu;
+        n0[t] = U0[o];
+        n1[t] = U1[o];
+        n2[t] = U2[o];
+      }
+#pragma unroll
+      for (int t = 0; t < kPF; ++t) {
+        const int k = k0 - t;
+        if (k >= 0) {
+          const double x = (z[k * ldz] - c1[t] * x1 - c2[t] * x2) * c0[t];
+          z[k * ldz] = x;
+          xmax = fmax(xmax, fabs(x));
+          x2 = x1;
+          x1 = x;
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < kPF; ++t) {
+        c0[t] = n0[t];
+        c1[t] = n1[t];
+        c2[t] = n2[t];
+      }
+    }
+    const double sc = xmax > 0.0 ? 1.0 / xmax : 1.0;
+    nrm = 0.0;
+    for (int k = 0; k < n; ++k) {
+      const double v = z[k * ldz] * sc;
+      z[k * ldz] = v;
+      nrm = fma(v, v, nrm);
+    }
+  }
+  return 1.0 / sqrt(nrm);
+}
 
 // ---- the thread grid of the Householder phase.  The lanes of a wave form 4 rows x 16 columns:
 // column tc = lane bits 5 4 1 0, row rl = lane bits 3 2; thread row tr = 4 wave + rl.
@@ -537,8 +720,10 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
   double* e = reinterpret_cast<double*>(de + n);
   double* lam = e + n;
   double* tau = lam + n;
-  double* red = tau + n;  // n doubles: block reductions' scratch
-  double* T = S == 48 ? red + n : U0;  // the panels' T factors
+  double* aux = tau + n;  // block reductions' scratch; the vectors' scales
+  double* red = aux;
+  unsigned char* twist = reinterpret_cast<unsigned char*>(aux + n);
+  double* T = S == 48 ? aux + n + 24 : U0;  // the panels' T factors (and the lower multipliers after them)
 
   // ---- 1. tridiagonal form
   {
@@ -557,162 +742,322 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
     t.wave = wave;
     tridiagonalise<NW, RR, RC>(F + mo, n, t);
   }
-  // ---- 2. the nv lowest eigenvalues: multisection, a group of tb lanes per eigenvalue
-  double lo_p = 1.0e300, hi_p = -1.0e300, e2max = 0.0;
+  // ---- 2. the nv lowest eigenvalues, and the next one above (its distance says how sharp the
+  //         highest of them has to be).  What bounds it: instruction issue, some 7 per row and
+  //         point, so the rounds after the grid run one wave per SIMD.  91 of 182: 144 -> 73 us
+  const int nvx = EVEC ? n : min(nv + 1, n);
+  double lo_p = 1.0e300, hi_p = -1.0e300;
   for (int k = tid; k < n; k += NT) {
     const double el = k > 0 ? fabs(e[k - 1]) : 0.0, er = k + 1 < n ? fabs(e[k]) : 0.0;
     lo_p = fmin(lo_p, de[k].x - el - er);
     hi_p = fmax(hi_p, de[k].x + el + er);
-    if (k + 1 < n) {
-      de[k].y = e[k] * e[k];  // e^2 for the Sturm counts 
-      e2max = fmax(e2max, de[k].y);
-    }
   }
   double glo = eig_block_min<NT>(lo_p, red);
   double ghi = eig_block_max<NT>(hi_p, red);
-  e2max = eig_block_max<NT>(e2max, red);
   const double tnorm = fmax(fabs(glo), fabs(ghi));
-  const double pivmin = 1.0e-300 * fmax(1.0, e2max);
-  glo -= 2.2e-16 * tnorm * 4.0 + 2.0 * pivmin;
-  ghi += 2.2e-16 * tnorm * 4.0 + 2.0 * pivmin;
-  // Bracket width at which an eigenvalue is final: 1e-11 |T| (or the rounding floor).  Inverse
-  // iteration only needs the shift that close: with eigenvalues further apart than the cluster
-  // threshold 1e-5 |T| each solve shrinks the other components by 1e-6 or more, and the vectors
-  // of a cluster are orthogonalised as a set.
-  const double btol = 1.0e-11 * tnorm;
-  {
-    int tb = 64;
-    while (tb > 1 && nv * tb > NT) tb >>= 1;
-    const int ngrp = NT / tb, gi = tid / tb, gl = tid % tb;
-    for (int j0 = 0; j0 < nv; j0 += ngrp) {
-      const int j = j0 + gi;
-      if (j < nv) {  // uniform over the lane group
-        double lo = glo, hi = ghi;
-        for (int round = 0; round < 64; ++round) {
-          if (!(hi - lo > fmax(4.4e-16 * fmax(fabs(lo), fabs(hi)), btol) + 2.0 * pivmin)) break;
-          const double x = lo + (hi - lo) * (double)(gl + 1) / (double)(tb + 1);
-          const int cnt = (x > lo && x < hi) ? sturm_count(de, n, x, pivmin) : -1;
-          const double nlo = group_max_t(cnt >= 0 && cnt <= j ? x : lo, tb);
-          const double nhi = group_min_t(cnt > j ? x : hi, tb);
-          if (nlo == lo && nhi == hi) break;  // no representable interior point left
-          lo = nlo;
-          hi = nhi;
-        }
-        if (gl == 0) lam[j] = 0.5 * (lo + hi);
-      }
-    }
-  }
+  const double slack = 2.2e-16 * tnorm * 4.0 + 2.0e-300 * fmax(1.0, tnorm);
+  glo -= slack;
+  ghi += slack;
+  for (int k = tid; k + 1 < n; k += NT) de[k].y = fmax(e[k] * e[k], fmax(1.0e-60 * tnorm * tnorm, 1.0e-300));
   __syncthreads();
+  const double btol = 1.0e-11 * tnorm, ctol = 1.0e-9 * tnorm, dtol = 1.0e-10 * tnorm, gtol = 1.0e-3 * tnorm;
+  {
+    constexpr int M = 2 * NT;  // grid points
+    int* counts = reinterpret_cast<int*>(Z);
+    const double step = (ghi - glo) / (double)(M + 1);
+    {
+      const double x[2] = {fma((double)(tid + 1), step, glo), fma((double)(tid + NT + 1), step, glo)};
+      int c[2];
+      sturm_counts<2>(de, n, x, c);
+      counts[tid] = c[0];
+      counts[tid + NT] = c[1];
+    }
+    __syncthreads();
+    constexpr int kLanes = NT > 256 ? 256 : NT;  // one wave per SIMD
+    int tb = 64;
+    while (tb > 1 && nvx * tb > kLanes) tb >>= 1;  // nvx <= NT in every variant
+    const int j = tid / tb, gl = tid % tb;
+    double lo = glo, hi = ghi;
+    auto narrow = [&](double tol) {  // uniform over the lane group
+      for (int round = 0; round < 64; ++round) {
+        if (!(hi - lo > fmax(4.4e-16 * fmax(fabs(lo), fabs(hi)), tol) + 2.0e-300)) break;
+        const double x[1] = {lo + (hi - lo) * (double)(gl + 1) / (double)(tb + 1)};
+        int c[1];
+        sturm_counts<1>(de, n, x, c);
+        const bool in = x[0] > lo && x[0] < hi;
+        const double nlo = group_max_t(in && c[0] <= j ? x[0] : lo, tb);
+        const double nhi = group_min_t(in && c[0] > j ? x[0] : hi, tb);
+        if (nlo == lo && nhi == hi) break;  // no representable interior point left
+        lo = nlo;
+        hi = nhi;
+      }
+    };
+    if (j < nvx) {
+      int a = -1, b = M;  // counts[a] <= j < counts[b]
+      while (b - a > 1) {
+        const int c = (a + b) >> 1;
+        if (counts[c] > j)
+          b = c;
+        else
+          a = c;
+      }
+      if (a >= 0) lo = fma((double)(a + 1), step, glo);
+      if (b < M) hi = fma((double)(b + 1), step, glo);
+      narrow(btol);
+      if (gl == 0) lam[j] = 0.5 * (lo + hi);
+    }
+    __syncthreads();
+    const bool near = j < nvx && ((j > 0 && lam[j] - lam[j - 1] <= ctol) || (j + 1 < nvx && lam[j + 1] - lam[j] <= ctol));
+    __syncthreads();
+    if (near) {
+      narrow(0.0);
+      if (gl == 0) lam[j] = 0.5 * (lo + hi);
+    }
+    __syncthreads();
+  }
+  // e^2 is done with: .y carries the part of each eigenvalue below lam's rounding
+  for (int k = tid; k < n; k += NT) de[k].y = 0.0;
+  auto degenerate = [&](int j) {
+    return (j > 0 && lam[j] - lam[j - 1] <= dtol) || (j + 1 < nvx && lam[j + 1] - lam[j] <= dtol);
+  };
+  bool mine = false;
+  for (int j = tid; j < nv; j += NT) mine = mine || degenerate(j);
+  const bool any_degenerate = __syncthreads_or(mine);
 
-  // ---- 3. inverse iteration, one thread per eigenvector; vector j in LDS at Z[k * ldz + j]
-  const double tiny = 2.2e-16 * fmax(tnorm, 1.0e-300);
-  for (int j = tid; j < nv; j += NT) {
-    for (int k = 0; k < n; ++k) Z[k * ldz + j] = start_value(j, k);
-    const double sig = lam[j];
-    for (int rep = 0; rep < 3; ++rep) {
-      // LU of T - sig I with partial pivoting, the right-hand side eliminated alongside; the
-      // running row and right-hand side stay in registers, U goes to the workspace.  Each step
-      // keeps one of two rows as the pivot row (its diagonal and sub-diagonal entries compared)
-      // and eliminates the other, both cases as one select-based update (lanes differ in their
-      // choices); the next step's d, e and right-hand side are read from LDS one step ahead.
-      double diag = de[0].x - sig, sup = n > 1 ? e[0] : 0.0;
-      double yk = Z[j];
-      double sub_n = n > 1 ? e[0] : 0.0, dn_n = n > 1 ? de[1].x : 0.0, ns_n = n > 2 ? e[1] : 0.0;
-      double y_n = n > 1 ? Z[ldz + j] : 0.0;
-      for (int k = 0; k + 1 < n; ++k) {
-        const double sub = sub_n, nd = dn_n - sig, ns = ns_n, yk1 = y_n;
-        if (k + 2 < n) {
-          sub_n = ns_n;
-          dn_n = de[k + 2].x;
-          ns_n = k + 3 < n ? e[k + 2] : 0.0;
-          y_n = Z[(k + 2) * ldz + j];
+  // ---- 3. eigenvectors: NT / 2 vectors at a time, lane `side` 0 from the top, 1 from the bottom.
+  // L and U: the two ends' multipliers (twisted_sweep).  The twist row r has the least |gamma_k|, gamma_k = d_k - lambda - e_{k-1} L_{k-1} - e_k U_k.  z_r = 1, outwards z = -L z
+  // (products only), and gamma_r / |z|^2 corrects lambda.  Kept unrounded as lam + .y: rounded, it
+  // would tilt the vectors of neighbours at a gap by eps |T| / gap.
+  constexpr int kHalf = NT / 2;
+  {
+    // waves 0 1 and 2 3 (a SIMD each), then 4 5 and 6 7; the halves of a lone wave
+    const int side = NW == 1 ? lane >> 5 : (wave >> 1) & 1;
+    const int vec = NW == 1 ? lane & 31 : lane + 64 * ((wave & 1) + 2 * (wave >> 2));
+    double* U = S == 48 ? T + 3 * kTPanel : U0;
+    const int ldu = S == 48 ? ldz : nmax;
+    const double tiny = 1.0e-40 * fmax(tnorm, 1.0e-200);
+    for (int c0 = 0; c0 < nv; c0 += kHalf) {
+      const int j = c0 + vec;
+      const int nc = min(kHalf, nv - c0);
+      const bool live = j < nv;
+      int r = 0;  // the twist row, of the first factorisation for both
+      for (int pass = 0; pass < 2; ++pass) {
+        if (live) {
+          const double hi = lam[j], lo = de[j].y;
+          if (side == 0)
+            twisted_sweep<1>(de, e, n, hi, lo, tiny, Z + j, ldz);
+          else
+            twisted_sweep<-1>(de + n - 1, e + n - 2, n, hi, lo, tiny, U + (n - 2) * ldu + j, -ldu);
         }
-        const size_t o = (size_t)k * nmax + j;
-        const bool keep = fabs(diag) >= fabs(sub);  // no row exchange
-        const double piv = keep ? (fabs(diag) < tiny ? copysign(tiny, diag) : diag) : sub;
-        const double rp = rcp_f64(piv);
-        const double mlt = (keep ? sub : diag) * rp;
-        const double p1 = keep ? sup : nd, p2 = keep ? 0.0 : ns, py = keep ? yk : yk1;
-        const double o1 = keep ? nd : sup, o2 = keep ? ns : 0.0, oy = keep ? yk1 : yk;
-        U0[o] = rp;
-        U1[o] = p1;
-        U2[o] = p2;
-        Z[k * ldz + j] = py;
-        yk = fma(-mlt, py, oy);
-        diag = fma(-mlt, p1, o1);
-        sup = fma(-mlt, p2, o2);
-      }
-      const double rlast = 1.0 / (fabs(diag) < tiny ? copysign(tiny, diag) : diag);
-      double x1 = yk * rlast, x2 = 0.0, xmax = fabs(x1);
-      Z[(n - 1) * ldz + j] = x1;
-      // back substitution in blocks of kPF rows: the U factors of the next block are loaded while
-      // this block is solved (the loads come from L2; one row ahead left each row waiting on one)
-      constexpr int kPF = 8;
-      double c0[kPF], c1[kPF], c2[kPF];
-#pragma unroll
-      for (int t = 0; t < kPF; ++t) {
-        const int kk = n - 2 - t;
-        const size_t o = (size_t)(kk >= 0 ? kk : 0) * nmax + j;
-        c0[t] = U0[o];
-        c1[t] = U1[o];
-        c2[t] = U2[o];
-      }
-      for (int k0 = n - 2; k0 >= 0; k0 -= kPF) {
-        double n0[kPF], n1[kPF], n2[kPF];
-#pragma unroll
-        for (int t = 0; t < kPF; ++t) {
-          const int kk = k0 - kPF - t;
-          const size_t o = (size_t)(kk >= 0 ? kk : 0) * nmax + j;
-          n0[t] = U0[o];
-          n1[t] = U1[o];
-          n2[t] = U2[o];
+        __syncthreads();
+        double gam = 0.0;
+        if (pass == 0) {  // twist rows: tg lanes per vector, rows part, part + tg, ...
+          int tg = 64;
+          while (nc * tg > NT) tg >>= 1;
+          const int v = tid / tg, part = tid % tg, jv = c0 + v;
+          if (v < nc) {
+            const double hi = lam[jv], lo = de[jv].y;
+            double best = 0.0;
+            int rb = -1;
+            auto take = [&](double g, int k) {
+              if (rb < 0 || fabs(g) < fabs(best)) {
+                best = g;
+                rb = k;
+              }
+            };
+            const double* zl = Z + jv - ldz;
+            const double* ul = U + jv;
+            int k = part;
+            if (k == 0) {
+              take(n > 1 ? fma(-e[0], ul[0], (de[0].x - hi) - lo) : (de[0].x - hi) - lo, 0);
+              k += tg;
+            }
+#pragma unroll 4
+            for (; k + 1 < n; k += tg)
+              take(fma(-e[k], ul[k * ldu], fma(-e[k - 1], zl[k * ldz], (de[k].x - hi) - lo)), k);
+            if (k + 1 == n) take(fma(-e[k - 1], zl[k * ldz], (de[k].x - hi) - lo), k);
+            for (int o = 1; o < tg; o <<= 1) {
+              const double og = __shfl_xor(best, o);
+              const int orow = __shfl_xor(rb, o);
+              if (orow >= 0 && (rb < 0 || fabs(og) < fabs(best) || (fabs(og) == fabs(best) && orow < rb))) {
+                best = og;
+                rb = orow;
+              }
+            }
+            if (part == 0) {
+              aux[jv] = best;
+              twist[jv] = (unsigned char)max(rb, 0);
+            }
+          }
+          __syncthreads();
+          if (live) {
+            gam = aux[j];
+            r = twist[j];
+          }
+          __syncthreads();  // every lane has its gamma: aux takes the norms
         }
+        double nrm = 0.0;
+        if (live) {
+          double z = 0.0;
+          if (side == 0) {
+            auto row = [&](double* zk, double l, int k) {
+              z = k == r ? 1.0 : -l * z;  // zero above the twist row, until it
+              if (k <= r) {
+                *zk = z;
+                nrm = fma(z, z, nrm);
+              }
+            };
+            const int n8 = n & ~7;
+            if (n > n8) row(Z + (n - 1) * ldz + j, 0.0, n - 1);
+            for (int k = n - 2; k >= n8; --k) row(Z + k * ldz + j, Z[k * ldz + j], k);
+            if (n8) {
+              double* zk = Z + (n8 - 8) * ldz + j;
+              double l[8];
 #pragma unroll
-        for (int t = 0; t < kPF; ++t) {
-          const int k = k0 - t;
-          if (k >= 0) {
-            const double x = (Z[k * ldz + j] - c1[t] * x1 - c2[t] * x2) * c0[t];
-            Z[k * ldz + j] = x;
-            xmax = fmax(xmax, fabs(x));
-            x2 = x1;
-            x1 = x;
+              for (int t = 0; t < 8; ++t) l[t] = zk[t * ldz];
+              if (n8 == n) l[7] = 0.0;  // row n - 1 has no multiplier
+#pragma unroll 2
+              for (int k0 = n8 - 8; k0 >= 0; k0 -= 8) {
+                double ln[8];
+                if (k0 >= 8) {
+#pragma unroll
+                  for (int t = 0; t < 8; ++t) ln[t] = zk[(t - 8) * ldz];
+                }
+#pragma unroll
+                for (int t = 7; t >= 0; --t) row(zk + t * ldz, l[t], k0 + t);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) l[t] = ln[t];
+                zk -= 8 * ldz;
+              }
+            }
+            aux[j] = nrm;
+          } else {
+            auto row = [&](double* zk, double u, int k) {
+              z = k == r ? 1.0 : -u * z;
+              if (k > r) {
+                *zk = z;
+                nrm = fma(z, z, nrm);
+              }
+            };
+            if (r == 0) z = 1.0;
+            constexpr int kB = 16;  // the multipliers come from the workspace (L2): rows read ahead
+            double* zk = Z + ldz + j;
+            const double* uk = U + j;
+            int k0 = 1;
+            if (n > kB) {
+              double u[kB];
+#pragma unroll
+              for (int t = 0; t < kB; ++t) u[t] = uk[t * ldu];
+#pragma unroll 2
+              for (; k0 + kB <= n; k0 += kB) {
+                double un[kB];
+                if (k0 + 2 * kB <= n) {
+#pragma unroll
+                  for (int t = 0; t < kB; ++t) un[t] = uk[(kB + t) * ldu];
+                }
+#pragma unroll
+                for (int t = 0; t < kB; ++t) row(zk + t * ldz, u[t], k0 + t);
+#pragma unroll
+                for (int t = 0; t < kB; ++t) u[t] = un[t];
+                zk += kB * ldz;
+                uk += kB * ldu;
+              }
+            }
+#pragma unroll 4
+            for (; k0 < n; ++k0) {
+              row(zk, *uk, k0);
+              zk += ldz;
+              uk += ldu;
+            }
           }
         }
-#pragma unroll
-        for (int t = 0; t < kPF; ++t) {
-          c0[t] = n0[t];
-          c1[t] = n1[t];
-          c2[t] = n2[t];
+        __syncthreads();
+        if (live && side == 1) {
+          nrm += aux[j];
+          aux[j] = 1.0 / sqrt(nrm);  // the vector's scale
+          if (pass == 0) {
+            const double corr = fmin(fmax(gam / nrm, -btol), btol);
+            const double s = lam[j] + corr;
+            de[j].y = corr - (s - lam[j]);
+            lam[j] = s;
+          }
         }
+        __syncthreads();
       }
-      const double sc = xmax > 0.0 ? 1.0 / xmax : 1.0;
-      for (int k = 0; k < n; ++k) Z[k * ldz + j] *= sc;
     }
   }
-  __syncthreads();
+  if (any_degenerate) {  // inverse iteration for the vectors of degenerate levels, one thread each
+    const double tiny = 2.2e-16 * fmax(tnorm, 1.0e-300);
+    for (int j = tid; j < nv; j += NT)
+      if (degenerate(j)) aux[j] = inverse_iteration(de, e, Z + j, ldz, U0 + j, U1 + j, U2 + j, nmax, n, j, lam[j], tiny);
+    __syncthreads();
+  }
 
-  // ---- 4. clusters (eigenvalues closer than ctol) orthogonalised by the thread of their first
-  //         member, two Gram-Schmidt passes; every vector normalised
-  const double ctol = 1.0e-5 * fmax(tnorm, 1.0e-300);
-  for (int j = tid; j < nv; j += NT) {
-    if (j > 0 && lam[j] - lam[j - 1] <= ctol) continue;  // inside a cluster: its first thread works
-    int jend = j + 1;
-    while (jend < nv && lam[jend] - lam[jend - 1] <= ctol) ++jend;
-    for (int q = j; q < jend; ++q) {
-      for (int pass = 0; pass < 2; ++pass)
-        for (int p = j; p < q; ++p) {
-          double dot = 0.0;
-          for (int k = 0; k < n; ++k) dot += Z[k * ldz + p] * Z[k * ldz + q];
-          for (int k = 0; k < n; ++k) Z[k * ldz + q] -= dot * Z[k * ldz + p];
+  // ---- 4. clusters (runs of eigenvalues closer than gtol): chain after chain per wave, each vector
+  //         against those before it within gtol, four at a time (their products are small, so that is
+  //         the same to rounding as one by one); a second time where it lost half of its length.
+  //         182 orbitals: 15-61 us by one thread per cluster at 1e-5 |T|, 13-26 here at 1e-3
+  {
+    constexpr int E = (S + 63) / 64;
+    int chain = 0;
+    for (int base = 0; base < nv; base += 64) {
+      const int jl = base + lane;
+      const bool starts = jl + 1 < nv && (jl == 0 || lam[jl] - lam[jl - 1] > gtol) && lam[jl + 1] - lam[jl] <= gtol;
+      unsigned long long todo = __ballot(starts);
+      for (; todo; todo &= todo - 1, ++chain) {
+        if (chain % NW != wave) continue;
+        const int first = base + __ffsll(todo) - 1;
+        int p0 = first;
+        for (int q = first; q < nv && (q == first || lam[q] - lam[q - 1] <= gtol); ++q) {
+          double zq[E];
+          const double sc = aux[q];
+#pragma unroll
+          for (int i = 0; i < E; ++i) {
+            const int k = lane + 64 * i;
+            zq[i] = k < n ? sc * Z[k * ldz + q] : 0.0;
+          }
+          while (lam[q] - lam[p0] > gtol) ++p0;
+          for (int rep = 0; rep < 2; ++rep) {
+            for (int p = p0; p < q; p += 4) {
+              double zp[4][E], dot[4];
+#pragma unroll
+              for (int c = 0; c < 4; ++c) {
+                dot[c] = 0.0;
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                  const int k = lane + 64 * i;
+                  zp[c][i] = k < n && p + c < q ? Z[min(k, n - 1) * ldz + min(p + c, q)] : 0.0;
+                  dot[c] = fma(zp[c][i], zq[i], dot[c]);
+                }
+              }
+#pragma unroll
+              for (int c = 0; c < 4; ++c) dot[c] = wave64(dot[c]);
+#pragma unroll
+              for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int i = 0; i < E; ++i) zq[i] = fma(-dot[c], zp[c][i], zq[i]);
+            }
+            double nr = 0.0;
+#pragma unroll
+            for (int i = 0; i < E; ++i) nr = fma(zq[i], zq[i], nr);
+            nr = wave64(nr);
+            if (!(nr > 1.0e-200)) {  // lost to its cluster's span: flagged, left unscaled
+              if (lane == 0) atomicAdd(fail, 1);
+              break;
+            }
+            const double s = 1.0 / sqrt(nr);
+#pragma unroll
+            for (int i = 0; i < E; ++i) zq[i] *= s;
+            if (nr > 0.5) break;
+          }
+#pragma unroll
+          for (int i = 0; i < E; ++i) {
+            const int k = lane + 64 * i;
+            if (k < n) Z[k * ldz + q] = zq[i];
+          }
+          if (lane == 0) aux[q] = 1.0;
         }
-      double nr = 0.0;
-      for (int k = 0; k < n; ++k) nr += Z[k * ldz + q] * Z[k * ldz + q];
-      if (!(nr > 1.0e-200)) {  // a vector lost to its cluster's span: flagged, left unscaled
-        atomicAdd(fail, 1);
-        continue;
       }
-      const double sc = 1.0 / sqrt(nr);
-      for (int k = 0; k < n; ++k) Z[k * ldz + q] *= sc;
     }
   }
   __syncthreads();
@@ -724,7 +1069,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
         const double zk = Z[k * ldz + j], zk1 = Z[(k - 1) * ldz + j];
         rq += de[k].x * zk * zk + 2.0 * e[k - 1] * zk * zk1;
       }
-      lam[j] = rq;
+      lam[j] = rq * aux[j] * aux[j];
     }
     __syncthreads();
   }
@@ -737,6 +1082,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
     const int off = S - n;
     for (int vt = wave; 16 * vt < nv; vt += NW) {
       const int col = 16 * vt + (lane & 15), g = lane >> 4;
+      const double scale = aux[min(col, nv - 1)];
       doublex4 Cr[NTL];
 #pragma unroll
       for (int t = 0; t < NTL; ++t)
@@ -744,7 +1090,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
         for (int s = 0; s < 4; ++s) {
           const int k = 16 * t + 4 * s + g - off;
           const double z = Z[max(k, 0) * ldz + min(col, nv - 1)];
-          Cr[t][s] = (k >= 0 && col < nv) ? z : 0.0;
+          Cr[t][s] = (k >= 0 && col < nv) ? z * scale : 0.0;
         }
       const double* hh = HH;
       const double* tt = T;
@@ -759,6 +1105,9 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
           if (k >= 0 && col < nv) Z[k * ldz + col] = Cr[t][s];
         }
     }
+    __syncthreads();
+  } else {  // no reflectors
+    for (int t = tid; t < n * nv; t += NT) Z[(t / nv) * ldz + t % nv] *= aux[t % nv];
     __syncthreads();
   }
   if (EVEC) {

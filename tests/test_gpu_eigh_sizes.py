@@ -2,8 +2,8 @@
 of its occupations, against numpy's float64 eigh.
 
 Bars: the density within 1e-10 of the reference's (levels of 1..40 eV and a gap of 11 eV: n eps |F| / gap < 1e-12,
-and eps |F| / gap < 1e-11 between levels of the nearest spacing drawn), exactly symmetric;
-reruns bitwise equal.
+and eps |F| / gap < 1e-11 between levels of the nearest spacing drawn), exactly symmetric; eigenpairs
+with residual and orthogonality below 1e-9 |F| (clusters are orthogonalised as a set); reruns bitwise equal.
 """
 import numpy as np
 import pytest
@@ -79,3 +79,30 @@ def test_density_at_grid_edges(grid, kind):
         assert np.array_equal(p, p.T), n
         assert np.abs(p - ref).max() < 1e-10, (n, nocc, np.abs(p - ref).max())
     assert int(eng.eigh_fail.item()) == 0
+
+
+@pytest.mark.parametrize("grid", sorted(SETS))
+@pytest.mark.parametrize("kind", ["spread", "degenerate", "close", "diagonal"])
+def test_eigenpairs_at_grid_edges(grid, kind):
+    sizes = [n for n in SETS[grid] + [139] if n <= min(grid, 139)]
+    eng = _engine(sizes, [n // 2 for n in sizes])
+    fs = _blocks(sizes, [n // 2 for n in sizes], kind, grid + 1)
+    F = torch.as_tensor(np.concatenate([f.reshape(-1) for f in fs]), device=DEV)
+    Q = torch.full_like(F, float("nan"))
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    evals = torch.full((int(off[-1]),), float("nan"), dtype=torch.float64, device=DEV)
+    ws = torch.empty(4 * len(sizes) * max(sizes) ** 2, dtype=torch.float64, device=DEV)
+    fail = torch.zeros(1, dtype=torch.int32, device=DEV)
+    orb_off = torch.as_tensor(off[:-1].astype(np.int64), device=DEV)
+    eng.eigenpairs(F, orb_off, evals, Q, ws, fail)
+    torch.cuda.synchronize()
+    o = 0
+    for k, (f, n) in enumerate(zip(fs, sizes)):
+        q = Q[o:o + n * n].view(n, n).cpu().numpy()
+        o += n * n
+        e = evals[int(off[k]):int(off[k]) + n].cpu().numpy()
+        scale = np.abs(f).max() * np.sqrt(n)
+        assert np.abs(e - np.linalg.eigvalsh(f)).max() < 1e-10 * scale, n
+        assert np.abs(q.T @ q - np.eye(n)).max() < 1e-9, n
+        assert np.abs(f @ q - q * e).max() < 1e-9 * scale, n
+    assert int(fail.item()) == 0
