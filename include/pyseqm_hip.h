@@ -362,6 +362,25 @@ int pyseqm_ksa_max_rank(void);
 int pyseqm_small_solve(const int* idx, int nact, int r, const double* O, const double* rhs, double* alpha,
                        void* stream);
 
+/* ------------------------------------------------------------------ reference layouts
+ * Views of the packed batch in the reference's padded layouts (rows of a molecule's 4 molsize x
+ * 4 molsize matrix: 4 per atom, hydrogens and padding with zeros); molsize >= every molecule's atoms.
+ * pyseqm_to_padded: packed matrices X -> out [nmol][4 molsize][4 molsize]; mode 0 every element, 1 the
+ *   upper triangle, 2 the upper triangle as the block array (hcore.py:155-179)
+ *   out [nmol molsize^2][4][4].  pyseqm_from_padded: the inverse of mode 0.
+ * pair_base [nmol]: pairs before each molecule.  pyseqm_pair_ref: reference pair index of every tile
+ *   lane, -1 without a pair, out [ntiles_total*64].
+ * pyseqm_w_reference: out [npairs][10][10], the dense integrals (hcore.py:9-179).
+ * pyseqm_orbital_charges (scf_loop.py:2376-2387): out [nmol][4 molsize][molsize] from eigenvectors V with
+ *   the given strides (doubles). */
+int pyseqm_to_padded(const pyseqm_layout_t* L, int molsize, int mode, const double* X, double* out, void* stream);
+int pyseqm_from_padded(const pyseqm_layout_t* L, int molsize, const double* Xp, double* out, void* stream);
+int pyseqm_pair_ref(const pyseqm_layout_t* L, const long long* pair_base, int* out, void* stream);
+int pyseqm_w_reference(const pyseqm_layout_t* L, const long long* pair_base, const double* w_xx, const double* w_xh,
+                       const double* w_hh, double* out, void* stream);
+int pyseqm_orbital_charges(const pyseqm_layout_t* L, int molsize, const double* V, long long stride_mol,
+                           long long stride_row, long long stride_col, double* out, void* stream);
+
 /* ------------------------------------------------------------------ XL-BOMD / MD
  * Density propagation of XL_BOMD._propagate_P (seqm/MolecularDynamics.py:1418-1427) plus the
  * ring update Pt[m-1-cindx] = P (1461) over `total` packed elements:

@@ -84,6 +84,11 @@ _SIGS = {
                            c_void_p, c_void_p],
     "pyseqm_pair_forces_xl": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_double, c_void_p, c_void_p,
                               c_void_p],
+    "pyseqm_to_padded": [c_int, c_int, c_void_p, c_void_p, c_void_p],
+    "pyseqm_from_padded": [c_int, c_void_p, c_void_p, c_void_p],
+    "pyseqm_pair_ref": [c_void_p, c_void_p, c_void_p],
+    "pyseqm_w_reference": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
+    "pyseqm_orbital_charges": [c_int, c_void_p, c_longlong, c_longlong, c_longlong, c_void_p, c_void_p],
     "pyseqm_xl_energy": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
 }
 # entry points without a layout argument: name -> full argtypes

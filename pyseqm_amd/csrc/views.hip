@@ -1,0 +1,200 @@
+// The packed batch in the reference's layouts: padded matrices (nmol, 4 molsize, 4 molsize), the
+// block array of the core Hamiltonian (hcore.py:155-179), dense two-center integrals (npairs, 10, 10)
+// and per-orbital atomic charges (scf_loop.py:2376-2387).  Every index follows from the molecule's
+// atom counts, so no index arrays are built or read, and every output element is written (zeros
+// included): each kernel moves its input and its output once.  What bounds them is HBM; the index
+// lists they stand in for took the host 25 ms per batch of 128 alkanes of 2-30 carbons.
+#include "common.h"
+
+using namespace pyseqm;
+
+namespace {
+
+// orbital of padded row p (component p % 4 of atom p / 4) in a molecule of nat atoms, nh of them heavy,
+// or -1: hydrogens carry one orbital, the last atoms of a row are padding
+__device__ inline int orbital_of(int p, int nat, int nh) {
+  const int a = p >> 2;
+  if (a < nh) return p;
+  return (a < nat && (p & 3) == 0) ? 4 * nh + a - nh : -1;
+}
+__device__ inline void counts_of(const pyseqm_layout_t& L, int m, int& nat, int& nh, int& n) {
+  nat = L.mol_atom_off[m + 1] - L.mol_atom_off[m];
+  n = L.mol_norb[m];
+  nh = (n - nat) / 3;  // n = 4 nh + (nat - nh)
+}
+
+constexpr int kViewRows = 8;  // padded rows per block
+
+// MODE 0: every element; 1: the upper triangle of the padded matrix, zero below; 2: that triangle as
+// 4 x 4 blocks (atom i, atom j)
+template <int MODE>
+__global__ __launch_bounds__(256) void k_to_padded(pyseqm_layout_t L, int molsize, const double* __restrict__ X,
+                                                   double* __restrict__ out) {
+  const int m = blockIdx.x, w = 4 * molsize;
+  int nat, nh, n;
+  counts_of(L, m, nat, nh, n);
+  const double* x = X + L.mol_mat_off[m];
+  double* o = out + (size_t)m * w * w;
+  const int r1 = min(w, (int)(blockIdx.y + 1) * kViewRows);
+  for (int r = blockIdx.y * kViewRows; r < r1; ++r) {
+    const int ro = orbital_of(r, nat, nh);
+    for (int c = threadIdx.x; c < w; c += 256) {
+      const int co = orbital_of(c, nat, nh);
+      double v = 0.0;
+      if (ro >= 0 && co >= 0 && (MODE == 0 || r <= c)) v = x[(size_t)ro * n + co];
+      if (MODE == 2)
+        o[((size_t)(r >> 2) * molsize + (c >> 2)) * 16 + (r & 3) * 4 + (c & 3)] = v;
+      else
+        o[(size_t)r * w + c] = v;
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void k_from_padded(pyseqm_layout_t L, int molsize, const double* __restrict__ Xp,
+                                                     double* __restrict__ out) {
+  const int m = blockIdx.x, w = 4 * molsize;
+  int nat, nh, n;
+  counts_of(L, m, nat, nh, n);
+  const double* x = Xp + (size_t)m * w * w;
+  double* o = out + L.mol_mat_off[m];
+  const int r1 = min(n, (int)(blockIdx.y + 1) * kViewRows);
+  for (int r = blockIdx.y * kViewRows; r < r1; ++r) {
+    const int rp = r < 4 * nh ? r : 4 * (r - 3 * nh);
+    for (int c = threadIdx.x; c < n; c += 256) o[(size_t)r * n + c] = x[(size_t)rp * w + (c < 4 * nh ? c : 4 * (c - 3 * nh))];
+  }
+}
+
+// index of pair (i, j), i < j local, in the reference's order within a molecule of nat atoms
+__device__ inline long long pair_index(int i, int j, int nat) {
+  return (long long)i * nat - (long long)i * (i + 1) / 2 + (j - i - 1);
+}
+
+__global__ __launch_bounds__(64) void k_pair_ref(pyseqm_layout_t L, const long long* __restrict__ pair_base,
+                                                 int* __restrict__ out) {
+  const Tile t = load_tile(L.tiles, blockIdx.x);
+  int i, j;
+  const bool ok = lane_pair(t, threadIdx.x, i, j);
+  const int a0 = L.mol_atom_off[t.mol], nat = L.mol_atom_off[t.mol + 1] - a0;
+  out[(size_t)blockIdx.x * 64 + threadIdx.x] = ok ? (int)(pair_base[t.mol] + pair_index(i - a0, j - a0, nat)) : -1;
+}
+
+// One block per tile.  The tile's integrals (rows of packed lanes) are read in order into LDS and written
+// a pair's 100 values at a time; heavy-H pairs fill column 0, H-H pairs element 0 (the rest is
+// zero).  The LDS row stride is odd, so a pair's values lie on distinct banks.
+template <int KIND>
+__global__ __launch_bounds__(256) void k_w_reference(pyseqm_layout_t L, int tile0, const long long* __restrict__ pair_base,
+                                                     const double* __restrict__ w, double* __restrict__ out) {
+  constexpr int NW = KIND == 0 ? 100 : (KIND == 1 ? 10 : 1);
+  __shared__ double buf[NW * 65];
+  __shared__ long long ref[64];
+  const int tile = tile0 + blockIdx.x;
+  const Tile t = load_tile(L.tiles, tile);
+  const int S = tile_wstride(t), nv = t.diag ? t.nrow * (t.nrow - 1) / 2 : t.nrow * t.ncol;
+  if (threadIdx.x < 64) {
+    int i, j;
+    if (lane_pair(t, threadIdx.x, i, j)) {
+      const int a0 = L.mol_atom_off[t.mol], nat = L.mol_atom_off[t.mol + 1] - a0;
+      ref[lane_rank(t, threadIdx.x)] = pair_base[t.mol] + pair_index(i - a0, j - a0, nat);
+    }
+  }
+  const double* src = w + L.tile_woff[tile];
+  for (int e = threadIdx.x; e < NW * S; e += 256) {
+    const int q = e / S, p = e - q * S;
+    if (p < nv) buf[q * 65 + p] = src[e];
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < nv * 100; e += 256) {
+    const int p = e / 100, q = e - p * 100;
+    double v = 0.0;
+    if (KIND == 0)
+      v = buf[q * 65 + p];
+    else if (KIND == 1)
+      v = q % 10 == 0 ? buf[(q / 10) * 65 + p] : 0.0;
+    else
+      v = q == 0 ? buf[p] : 0.0;
+    out[ref[p] * 100 + q] = v;
+  }
+}
+
+// charge[i][a] of the reference's per-orbital charges: with v row i of V squared, heavy atom a takes
+// v[a], v[nh + a], v[2 nh + a], v[3 nh + a] (the reference's reshape), hydrogen a takes its orbital
+__global__ __launch_bounds__(256) void k_orbital_charges(pyseqm_layout_t L, int molsize, const double* __restrict__ V,
+                                                         long long sm, long long sr, long long sc,
+                                                         double* __restrict__ out) {
+  const int m = blockIdx.x, w = 4 * molsize;
+  int nat, nh, n;
+  counts_of(L, m, nat, nh, n);
+  const double* v = V + m * sm;
+  double* o = out + (size_t)m * w * molsize;
+  const int i1 = min(w, (int)(blockIdx.y + 1) * kViewRows);
+  for (int i = blockIdx.y * kViewRows; i < i1; ++i)
+    for (int a = threadIdx.x; a < molsize; a += 256) {
+      double q = 0.0;
+      if (i < n && a < nh) {
+        for (int c = 0; c < 4; ++c) {
+          const double x = v[i * sr + (long long)(c * nh + a) * sc];
+          q += x * x;
+        }
+      } else if (i < n && a < nat) {
+        const double x = v[i * sr + (long long)(3 * nh + a) * sc];
+        q = x * x;
+      }
+      o[(size_t)i * molsize + a] = q;
+    }
+}
+
+dim3 view_grid(const pyseqm_layout_t& L, int molsize) { return dim3(L.nmol, (4 * molsize + kViewRows - 1) / kViewRows); }
+int launched() { return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH; }
+
+}  // namespace
+
+extern "C" int pyseqm_to_padded(const pyseqm_layout_t* L, int molsize, int mode, const double* X, double* out,
+                                void* stream) {
+  if (!L || molsize < 1 || mode < 0 || mode > 2) return PYSEQM_EINVAL;
+  if (L->nmol == 0) return PYSEQM_OK;
+  const dim3 g = view_grid(*L, molsize);
+  hipStream_t s = (hipStream_t)stream;
+  if (mode == 0)
+    k_to_padded<0><<<g, 256, 0, s>>>(*L, molsize, X, out);
+  else if (mode == 1)
+    k_to_padded<1><<<g, 256, 0, s>>>(*L, molsize, X, out);
+  else
+    k_to_padded<2><<<g, 256, 0, s>>>(*L, molsize, X, out);
+  return launched();
+}
+
+extern "C" int pyseqm_from_padded(const pyseqm_layout_t* L, int molsize, const double* Xp, double* out, void* stream) {
+  if (!L || molsize < 1) return PYSEQM_EINVAL;
+  if (L->nmol == 0) return PYSEQM_OK;
+  k_from_padded<<<view_grid(*L, molsize), 256, 0, (hipStream_t)stream>>>(*L, molsize, Xp,
+                                                                                                         out);
+  return launched();
+}
+
+extern "C" int pyseqm_pair_ref(const pyseqm_layout_t* L, const long long* pair_base, int* out, void* stream) {
+  if (!L) return PYSEQM_EINVAL;
+  const int nt = L->ntile[0] + L->ntile[1] + L->ntile[2];
+  if (nt == 0) return PYSEQM_OK;
+  k_pair_ref<<<nt, 64, 0, (hipStream_t)stream>>>(*L, pair_base, out);
+  return launched();
+}
+
+extern "C" int pyseqm_w_reference(const pyseqm_layout_t* L, const long long* pair_base, const double* w_xx,
+                                  const double* w_xh, const double* w_hh, double* out, void* stream) {
+  if (!L) return PYSEQM_EINVAL;
+  hipStream_t s = (hipStream_t)stream;
+  const int t1 = L->ntile[0], t2 = t1 + L->ntile[1];
+  if (L->ntile[0]) k_w_reference<0><<<L->ntile[0], 256, 0, s>>>(*L, 0, pair_base, w_xx, out);
+  if (L->ntile[1]) k_w_reference<1><<<L->ntile[1], 256, 0, s>>>(*L, t1, pair_base, w_xh, out);
+  if (L->ntile[2]) k_w_reference<2><<<L->ntile[2], 256, 0, s>>>(*L, t2, pair_base, w_hh, out);
+  return launched();
+}
+
+extern "C" int pyseqm_orbital_charges(const pyseqm_layout_t* L, int molsize, const double* V, long long stride_mol,
+                                      long long stride_row, long long stride_col, double* out, void* stream) {
+  if (!L || molsize < 1) return PYSEQM_EINVAL;
+  if (L->nmol == 0) return PYSEQM_OK;
+  k_orbital_charges<<<view_grid(*L, molsize), 256, 0, (hipStream_t)stream>>>(
+      *L, molsize, V, stride_mol, stride_row, stride_col, out);
+  return launched();
+}

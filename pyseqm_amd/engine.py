@@ -544,17 +544,16 @@ class SCFEngine:
     def w_reference(self):
         """Two-center integrals as the reference's dense (npairs, 10, 10) array (hcore.py:9-179)."""
         b = self.b
-        dev = self.device
-        w = torch.zeros(max(b.npairs, 1), 10, 10, dtype=torch.float64, device=dev)
-        for kind, buf in enumerate((self.w_xx, self.w_xh, self.w_hh)):
-            ref, idx = b.w_gather_index(kind, dev)
-            if ref is None:
-                continue
-            rows = buf[idx]
-            if kind == 0:
-                w[ref] = rows.view(-1, 10, 10)
-            elif kind == 1:
-                w[ref, :, 0] = rows
-            else:
-                w[ref, 0, 0] = rows[:, 0]
-        return w[:b.npairs]
+        w = torch.empty(b.npairs, 10, 10, dtype=torch.float64, device=self.device)
+        nat.call("pyseqm_w_reference", b.L, nat.ptr(b.pair_base_device()), nat.ptr(self.w_xx), nat.ptr(self.w_xh),
+                 nat.ptr(self.w_hh), nat.ptr(w), nat.stream_ptr(self.device))
+        return w
+
+    def orbital_charges(self, V):
+        """Per-orbital charge on each atom (nmol, 4 molsize, molsize) from the eigenvectors (nmol, n, n)
+        (scf_loop.py:2376-2387)."""
+        b = self.b
+        out = torch.empty(b.nmol, 4 * b.molsize, b.molsize, dtype=torch.float64, device=self.device)
+        nat.call("pyseqm_orbital_charges", b.L, b.molsize, nat.ptr(V), V.stride(0), V.stride(1), V.stride(2),
+                 nat.ptr(out), nat.stream_ptr(self.device))
+        return out

@@ -315,10 +315,20 @@ class PackedBatch:
 
     def pair_ref_device(self):
         """Device copy of pair_ref_host (int32), made on first use."""
-        if "pair_ref" not in self.d:
+        if "pair_ref" not in self.d and self.device.type == "cuda":
+            self.d["pair_ref"] = torch.empty(max(64 * self.ntiles, 1), dtype=torch.int32, device=self.device)
+            _native.call("pyseqm_pair_ref", self.L, _native.ptr(self.pair_base_device()),
+                         _native.ptr(self.d["pair_ref"]), _native.stream_ptr(self.device))
+        elif "pair_ref" not in self.d:
             self.d["pair_ref"] = torch.as_tensor(np.ascontiguousarray(self.pair_ref_host), dtype=torch.int32,
                                                  device=self.device)
         return self.d["pair_ref"]
+
+    def pair_base_device(self):
+        """Pairs before each molecule (int64) on the device, uploaded on first use."""
+        if "pair_base" not in self.d:
+            self.d["pair_base"] = torch.as_tensor(self.pair_base[:-1].copy(), dtype=torch.int64, device=self.device)
+        return self.d["pair_base"]
 
     # ----------------------------------------------------------------- device
     def _to_device(self, device_tiles=False):
@@ -453,14 +463,43 @@ class PackedBatch:
         k = np.arange(len(mol)) - first[mol]
         return self.mol_mat_off[mol] + k * (self.norb[mol] + 1), mol
 
+    def _plain(self, X):
+        """Whether a tensor can go to the view kernels as it is: FP64 on this batch's device, outside
+        autograd.  Others (host tensors, other types, tracked tensors) take index arrays."""
+        return self.device.type == "cuda" and X.device == self.d["mol_norb"].device and X.dtype == torch.float64 \
+            and not X.requires_grad
+
     def to_padded(self, X):
         """Packed matrices (flat) -> reference layout (nmol, 4*molsize, 4*molsize) on the device."""
+        if self._plain(X) and X.dim() == 1 and X.numel() >= self.total:
+            return self._view(X, 0, (self.nmol, 4 * self.molsize, 4 * self.molsize))
         flat, mm, rr, cc = (torch.as_tensor(a, device=X.device) for a in self.matrix_index())
         out = torch.zeros(self.nmol, 4 * self.molsize, 4 * self.molsize, dtype=X.dtype, device=X.device)
         out[mm, rr, cc] = X[flat]
         return out
 
+    def _view(self, X, mode, shape):
+        X = X.contiguous()
+        out = torch.empty(shape, dtype=torch.float64, device=X.device)
+        _native.call("pyseqm_to_padded", self.L, self.molsize, mode, _native.ptr(X), _native.ptr(out),
+                     _native.stream_ptr(X.device))
+        return out
+
+    def to_padded_upper(self, X):
+        """The upper triangle of to_padded (zero below), FP64 on the device."""
+        return self._view(X, 1, (self.nmol, 4 * self.molsize, 4 * self.molsize))
+
+    def to_blocks(self, X):
+        """That upper triangle as the reference's block array (nmol molsize^2, 4, 4) (hcore.py:155-179)."""
+        return self._view(X, 2, (self.nmol * self.molsize * self.molsize, 4, 4))
+
     def from_padded(self, Xp):
+        if self._plain(Xp) and tuple(Xp.shape) == (self.nmol, 4 * self.molsize, 4 * self.molsize):
+            Xp = Xp.contiguous()
+            out = torch.empty(self.total, dtype=torch.float64, device=Xp.device)
+            _native.call("pyseqm_from_padded", self.L, self.molsize, _native.ptr(Xp), _native.ptr(out),
+                         _native.stream_ptr(Xp.device))
+            return out
         flat, mm, rr, cc = (torch.as_tensor(a, device=Xp.device) for a in self.matrix_index())
         out = torch.zeros(self.total, dtype=Xp.dtype, device=Xp.device)
         out[flat] = Xp[mm, rr, cc]

@@ -2,16 +2,13 @@
 values (seqm/seqm_functions/hcore.py:9-179), computed by the pair-integral kernel of the
 molecule's device engine.  riXH / ri (local-frame intermediates kept by the reference for its
 analytic gradient) are not materialised and are returned as None."""
-import torch
-
-from .fock import matrix_to_blocks
 
 
 def hcore(molecule, doTETCI=True):
     eng = molecule.engine()
     eng.set_coordinates(molecule.coordinates.detach())
     b = eng.b
-    M = matrix_to_blocks(b.to_padded(eng.H), b.nmol, b.molsize)
+    M = b.to_blocks(eng.H)
     if not doTETCI:
         return M, None, None, None, None, None
     rho0 = eng.atom_par[:b.natoms, 26]

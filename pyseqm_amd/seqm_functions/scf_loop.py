@@ -18,20 +18,6 @@ def _converger(scf_converger):
     raise NotImplementedError("scf_converger [3] (KSA) is outside the closed-shell sp SCF path")
 
 
-def orbital_charges(molecule, v):
-    """Per-orbital charge on each atom from the eigenvectors (scf_loop.py:2376-2387)."""
-    nmol = molecule.nmol
-    m = molecule.molsize
-    charge = torch.zeros(nmol, 4 * m, m, dtype=v.dtype, device=v.device)
-    v2 = v * v
-    for i in range(nmol):
-        nh, nH = int(molecule.nHeavy[i]), int(molecule.nHydro[i])
-        n = 4 * nh + nH
-        charge[i, :n, :nh] = v2[i][:n, :4 * nh].reshape(n, 4, nh).sum(dim=1)
-        charge[i, :n, nh:nh + nH] = v2[i][:n, 4 * nh:4 * nh + nH]
-    return charge
-
-
 def _check_pair_cutoff(molecule):
     """The device engine couples every atom pair of a molecule; a pair_outer_cutoff that would drop
     pairs (the reference's Parser keeps only r < cutoff, basics.py:313-328) is refused."""
@@ -71,7 +57,7 @@ def scf_loop(molecule, eps=1.0e-4, P=None, sp2=[False], scf_converger=[1], eig=F
     en = eng.energies(r.P)
     F = b.to_padded(en["F"])
     Ppad = b.to_padded(r.P)
-    Hcore = torch.triu(b.to_padded(eng.H))  # the reference fills only the upper triangle
+    Hcore = b.to_padded_upper(eng.H)  # the reference fills only the upper triangle
     w = eng.w_reference()
     rho0 = eng.atom_par[:, 26]
     rho0xi = rho0[molecule.idxi]
@@ -79,7 +65,7 @@ def scf_loop(molecule, eps=1.0e-4, P=None, sp2=[False], scf_converger=[1], eig=F
     e = V = charge = None
     if eig:
         e, V = eng.eig(en["F"])
-        charge = orbital_charges(molecule, V)
+        charge = eng.orbital_charges(V)
     if scf_backward >= 1:
         # the density (and the orbital energies) carry the gradient of the SCF fixed point with
         # respect to the learned parameters (scf_loop.py:1779-1993); 2 (the reference's unrolled
