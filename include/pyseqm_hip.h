@@ -323,7 +323,8 @@ int pyseqm_sp2_mcweeny(const pyseqm_layout_t* L, const int* idx, int nact, int n
  * Every eigenpair of the listed blocks (the eigen-decomposition of Fermi_Q, fermi_q.py:27-30, via
  * sym_eig_trunc(eig_only=True), diag.py:110-241): Q in the packed layout (column j = eigenvector
  * j, ascending eigenvalues), evals[orb_off[m] + j].  The workgroup eigensolver with all n vectors:
- * nmax <= 192 and pyseqm_eigh_density_lds_ok(nmax, nmax); ws as for pyseqm_eigh_density. */
+ * nmax <= 192; ws as for pyseqm_eigh_density.  Where pyseqm_eigh_density_lds_ok(nmax, nmax) does not
+ * hold (above 139 orbitals) the vectors stand in Q while they are computed. */
 int pyseqm_eigh_vectors(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const double* F,
                         const long long* orb_off, double* evals, double* Q, double* ws, int* fail, void* stream);
 /* Fermi_Q (fermi_q.py:8-72) after the eigen-decomposition: the chemical potential by Newton steps
@@ -371,6 +372,8 @@ int pyseqm_small_solve(const int* idx, int nact, int r, const double* O, const d
  * pair_base [nmol]: pairs before each molecule.  pyseqm_pair_ref: reference pair index of every tile
  *   lane, -1 without a pair, out [ntiles_total*64].
  * pyseqm_w_reference: out [npairs][10][10], the dense integrals (hcore.py:9-179).
+ * pyseqm_evec_view: the eigenpairs of pyseqm_eigh_vectors as e [nmol][4 molsize] (zero-padded) and V
+ *   [nmol][nmax][nmax] (the identity beyond a block; nmax: at least the batch's largest block).
  * pyseqm_orbital_charges (scf_loop.py:2376-2387): out [nmol][4 molsize][molsize] from eigenvectors V with
  *   the given strides (doubles). */
 int pyseqm_to_padded(const pyseqm_layout_t* L, int molsize, int mode, const double* X, double* out, void* stream);
@@ -378,6 +381,8 @@ int pyseqm_from_padded(const pyseqm_layout_t* L, int molsize, const double* Xp, 
 int pyseqm_pair_ref(const pyseqm_layout_t* L, const long long* pair_base, int* out, void* stream);
 int pyseqm_w_reference(const pyseqm_layout_t* L, const long long* pair_base, const double* w_xx, const double* w_xh,
                        const double* w_hh, double* out, void* stream);
+int pyseqm_evec_view(const pyseqm_layout_t* L, int molsize, int nmax, const long long* orb_off,
+                     const double* lam, const double* Q, double* e, double* V, void* stream);
 int pyseqm_orbital_charges(const pyseqm_layout_t* L, int molsize, const double* V, long long stride_mol,
                            long long stride_row, long long stride_col, double* out, void* stream);
 

@@ -88,6 +88,7 @@ _SIGS = {
     "pyseqm_from_padded": [c_int, c_void_p, c_void_p, c_void_p],
     "pyseqm_pair_ref": [c_void_p, c_void_p, c_void_p],
     "pyseqm_w_reference": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
+    "pyseqm_evec_view": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
     "pyseqm_orbital_charges": [c_int, c_void_p, c_longlong, c_longlong, c_longlong, c_void_p, c_void_p],
     "pyseqm_xl_energy": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
 }

@@ -694,8 +694,12 @@ __device__ __forceinline__ void back_panels(doublex4 (&Cr)[S / 16], const double
 // EVEC = false: the density P = 2 C_occ C_occ^T of the nocc lowest vectors.  EVEC = true: every
 // eigenpair (nv = n vectors), written as Qout (packed layout, column j = eigenvector j) and evals
 // (orb_off[m] + j, the Rayleigh quotients of the final vectors: exact to rounding whatever the
-// multisection bracket width).
-template <int NW, int RR, int RC, bool EVEC>
+// multisection bracket width).  GZ (with EVEC): the vectors stand in Qout itself instead of LDS, for
+// blocks whose n x n vectors do not fit (140 to 192 orbitals): rows are read ahead of their use in every
+// sweep, and lanes run along a row, so the L2 serves them.
+// All pairs of 128 alkanes of 2-30 carbons: 0.72 ms for the blocks above 139 orbitals, 0.44 for the rest (6.5 ms
+// by the library's batched solver on padded stacks).
+template <int NW, int RR, int RC, bool EVEC, bool GZ>
 __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, const int* __restrict__ idx,
                                                        const double* __restrict__ F, double* __restrict__ P,
                                                        double* __restrict__ ws, int nmax,
@@ -714,9 +718,9 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
   double* U0 = HH + nm2;
   double* U1 = HH + 2 * nm2;
   double* U2 = HH + 3 * nm2;
-  const int ldz = zstride(n, nv);
-  double* Z = lds;  // eigenvectors: Z[k * ldz + j]
-  double2* de = reinterpret_cast<double2*>(Z + ((zregion(n, nv, S) + 1) & ~1));  // (d, e^2)
+  const int ldz = GZ ? n : zstride(n, nv);
+  double* Z = GZ ? P + mo : lds;  // eigenvectors: Z[k * ldz + j]
+  double2* de = reinterpret_cast<double2*>(lds + ((zregion(GZ ? 0 : n, nv, S) + 1) & ~1));  // (d, e^2)
   double* e = reinterpret_cast<double*>(de + n);
   double* lam = e + n;
   double* tau = lam + n;
@@ -728,8 +732,8 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
   // ---- 1. tridiagonal form
   {
     TriState t;
-    t.xb = Z;
-    t.pb = Z + S;
+    t.xb = lds;
+    t.pb = lds + S;
     t.de = de;
     t.e = e;
     t.tau = tau;
@@ -763,7 +767,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
   const double btol = 1.0e-11 * tnorm, ctol = 1.0e-9 * tnorm, dtol = 1.0e-10 * tnorm, gtol = 1.0e-3 * tnorm;
   {
     constexpr int M = 2 * NT;  // grid points
-    int* counts = reinterpret_cast<int*>(Z);
+    int* counts = reinterpret_cast<int*>(lds);
     const double step = (ghi - glo) / (double)(M + 1);
     {
       const double x[2] = {fma((double)(tid + 1), step, glo), fma((double)(tid + NT + 1), step, glo)};
@@ -1111,8 +1115,10 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
     __syncthreads();
   }
   if (EVEC) {
-    double* Qm = P + mo;
-    for (int t = tid; t < n * n; t += NT) Qm[t] = Z[(t / n) * ldz + t % n];  // row = orbital, column = vector
+    if (!GZ) {
+      double* Qm = P + mo;
+      for (int t = tid; t < n * n; t += NT) Qm[t] = Z[(t / n) * ldz + t % n];  // row = orbital, column = vector
+    }
     for (int j = tid; j < n; j += NT) evals[orb_off[m] + j] = lam[j];
     return;
   }
@@ -1167,11 +1173,11 @@ template <bool EVEC>
 void launch_eigh(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const double* F, double* out,
                  double* ws, int* fail, const long long* orb_off, double* evals, size_t lds, hipStream_t s) {
   if (nmax <= 48)
-    k_eigh_density<1, 12, 3, EVEC><<<nact, 64, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
+    k_eigh_density<1, 12, 3, EVEC, false><<<nact, 64, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
   else if (nmax <= 96)
-    k_eigh_density<4, 6, 6, EVEC><<<nact, 256, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
+    k_eigh_density<4, 6, 6, EVEC, false><<<nact, 256, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
   else
-    k_eigh_density<8, 6, 12, EVEC><<<nact, 512, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
+    k_eigh_density<8, 6, 12, EVEC, false><<<nact, 512, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
 }
 
 extern "C" int pyseqm_eigh_density_lds_ok(int norb, int nocc) {
@@ -1195,8 +1201,13 @@ extern "C" int pyseqm_eigh_vectors(const pyseqm_layout_t* L, const int* idx, int
                                    const long long* orb_off, double* evals, double* Q, double* ws, int* fail,
                                    void* stream) {
   if (!L || nact < 0 || nmax < 1 || nmax > kEighMaxN || !fail || !orb_off || !evals) return PYSEQM_EINVAL;
-  if (!pyseqm_eigh_density_lds_ok(nmax, nmax)) return PYSEQM_EINVAL;
   if (nact == 0) return PYSEQM_OK;
+  if (!pyseqm_eigh_density_lds_ok(nmax, nmax)) {  // above 139 orbitals: vectors in Q
+    const size_t lds = (size_t)(zregion(0, 0, 192) + 6 * nmax + kLdsExtra) * sizeof(double);
+    k_eigh_density<8, 6, 12, true, true>
+        <<<nact, 512, lds, (hipStream_t)stream>>>(*L, idx, F, Q, ws, nmax, fail, orb_off, evals);
+    return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
+  }
   const size_t lds = (size_t)lds_doubles(nmax, nmax) * sizeof(double);
   launch_eigh<true>(L, idx, nact, nmax, F, Q, ws, fail, orb_off, evals, lds, (hipStream_t)stream);
   return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;

@@ -143,6 +143,24 @@ __global__ __launch_bounds__(256) void k_orbital_charges(pyseqm_layout_t L, int 
     }
 }
 
+// Packed eigenpairs (column j of Q: vector j, lam[orb_off[m] + j]) as zero-padded eigenvalues e[m][w] and
+// vectors V[m][nmax][nmax], the identity beyond the block: the basis vectors of padding rows, as a padded
+// solve would return them.
+__global__ __launch_bounds__(256) void k_evec_view(pyseqm_layout_t L, int w, int nmax,
+                                                   const long long* __restrict__ orb_off,
+                                                   const double* __restrict__ lam, const double* __restrict__ Q,
+                                                   double* __restrict__ e, double* __restrict__ V) {
+  const int m = blockIdx.x, n = L.mol_norb[m];
+  const double* q = Q + L.mol_mat_off[m];
+  double* v = V + (size_t)m * nmax * nmax;
+  const int r1 = min(nmax, (int)(blockIdx.y + 1) * kViewRows);
+  for (int r = blockIdx.y * kViewRows; r < r1; ++r)
+    for (int c = threadIdx.x; c < nmax; c += 256)
+      v[(size_t)r * nmax + c] = (r < n && c < n) ? q[(size_t)r * n + c] : (r == c ? 1.0 : 0.0);
+  if (blockIdx.y == 0)
+    for (int c = threadIdx.x; c < w; c += 256) e[(size_t)m * w + c] = c < n ? lam[orb_off[m] + c] : 0.0;
+}
+
 dim3 view_grid(const pyseqm_layout_t& L, int molsize) { return dim3(L.nmol, (4 * molsize + kViewRows - 1) / kViewRows); }
 int launched() { return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH; }
 
@@ -187,6 +205,15 @@ extern "C" int pyseqm_w_reference(const pyseqm_layout_t* L, const long long* pai
   if (L->ntile[0]) k_w_reference<0><<<L->ntile[0], 256, 0, s>>>(*L, 0, pair_base, w_xx, out);
   if (L->ntile[1]) k_w_reference<1><<<L->ntile[1], 256, 0, s>>>(*L, t1, pair_base, w_xh, out);
   if (L->ntile[2]) k_w_reference<2><<<L->ntile[2], 256, 0, s>>>(*L, t2, pair_base, w_hh, out);
+  return launched();
+}
+
+extern "C" int pyseqm_evec_view(const pyseqm_layout_t* L, int molsize, int nmax, const long long* orb_off,
+                                const double* lam, const double* Q, double* e, double* V, void* stream) {
+  if (!L || molsize < 1 || nmax < 1 || !orb_off || nmax > 4 * molsize) return PYSEQM_EINVAL;
+  if (L->nmol == 0) return PYSEQM_OK;
+  const dim3 g(L->nmol, (nmax + kViewRows - 1) / kViewRows);
+  k_evec_view<<<g, 256, 0, (hipStream_t)stream>>>(*L, 4 * molsize, nmax, orb_off, lam, Q, e, V);
   return launched();
 }
 

@@ -65,6 +65,12 @@ def eigh_wg_ok(norb, nocc):
     return (n >= 1) & (n <= EIGH_WG_MAX_N) & (o <= n) & (eigh_wg_lds(n, o) <= EIGH_WG_LDS_DOUBLES)
 
 
+def eigh_pairs_ok(norb):
+    """Whether pyseqm_eigh_vectors takes every eigenpair of blocks of norb orbitals."""
+    n = np.asarray(norb, dtype=np.int64)
+    return (n >= 1) & (n <= EIGH_WG_MAX_N)
+
+
 def size_groups(norb, ratio=0.7, min_group=32, floor=EIGH_MIN_N):
     """Partition molecules (by position) into groups of similar orbital counts: sorted by size,
     a group takes molecules down to `ratio` of its largest; groups smaller than `min_group` join
@@ -493,19 +499,26 @@ class SCFEngine:
 
     def eigenpairs(self, F, orb_off, evals, Q, eig_ws, fail):
         """Every eigenpair of every block of F: Q in the packed layout (column j = eigenvector j,
-        ascending eigenvalues) and evals[orb_off[m] + j].  Blocks whose full decomposition fits the
-        workgroup eigensolver's LDS (at most 139 orbitals) take pyseqm_eigh_vectors; larger ones the
-        batched library eigensolver on Gershgorin-padded stacks per size group, scattered into the
-        same layout.  eig_ws holds 4 nmol n^2 doubles for the n of the workgroup blocks; fail counts
-        vectors the workgroup solver lost (read by the caller)."""
+        ascending eigenvalues) and evals[orb_off[m] + j].  Blocks of up to EIGH_WG_MAX_N orbitals take
+        pyseqm_eigh_vectors, in one launch for those whose vectors fit its LDS (at most 139 orbitals) and
+        one for the others; larger ones the batched library eigensolver on Gershgorin-padded stacks per
+        size group, scattered into the same layout.  eig_ws holds 4 nmol n^2 doubles for the n of the
+        workgroup blocks (allocated here where it is smaller); fail counts vectors the workgroup solver
+        lost (read by the caller)."""
         b = self.b
         norb = np.asarray(b.norb)
-        wg = eigh_wg_ok(norb, norb)
-        ids = np.nonzero(wg)[0]
-        if len(ids):
+        wg = eigh_pairs_ok(norb)
+        in_lds = eigh_wg_ok(norb, norb)
+        for ids in (np.nonzero(wg & ~in_lds)[0], np.nonzero(in_lds)[0]):
+            if len(ids) == 0:
+                continue
+            ids = ids[np.argsort(-norb[ids], kind="stable")]  # long solves first, as in density_eigh
+            top = int(norb[ids[0]])
+            ws = eig_ws if eig_ws.numel() >= 4 * len(ids) * top ** 2 else torch.empty(
+                4 * len(ids) * top ** 2, dtype=torch.float64, device=self.device)
             idx = torch.as_tensor(ids.astype(np.int32), device=self.device)
-            nat.call("pyseqm_eigh_vectors", b.L, nat.ptr(idx), len(ids), int(norb[ids].max()), nat.ptr(F),
-                     nat.ptr(orb_off), nat.ptr(evals), nat.ptr(Q), nat.ptr(eig_ws), nat.ptr(fail), self.stream)
+            nat.call("pyseqm_eigh_vectors", b.L, nat.ptr(idx), len(ids), top, nat.ptr(F), nat.ptr(orb_off),
+                     nat.ptr(evals), nat.ptr(Q), nat.ptr(ws), nat.ptr(fail), self.stream)
         rest = np.nonzero(~wg)[0]
         if len(rest) == 0:
             return
@@ -526,16 +539,33 @@ class SCFEngine:
 
     def eig(self, F):
         """Orbital energies in the reference layout e (nmol, 4*molsize), zero padded, and the packed
-        eigenvectors (nmol, nmax, nmax), sym_eig_trunc(eig_only=True) (diag.py:110-241)."""
+        eigenvectors (nmol, nmax, nmax), sym_eig_trunc(eig_only=True) (diag.py:110-241).  Batches of
+        blocks of up to EIGH_WG_MAX_N orbitals take the workgroup eigensolver (128 alkanes of 14-182
+        orbitals: 1.2 ms, 6.5 by the library's batched solver); those with a larger block, or where the
+        workgroup solver lost a vector or met a value that is not finite, the library's."""
         b = self.b
         self._idx_host = np.arange(b.nmol)
-        idx = torch.arange(b.nmol, dtype=torch.int32, device=self.device)
         nmax = b.nmax
-        Fp = torch.empty(b.nmol, nmax, nmax, dtype=torch.float64, device=self.device)
+        f64 = dict(dtype=torch.float64, device=self.device)
+        if eigh_pairs_ok(b.norb).all():
+            fail = torch.zeros(1, dtype=torch.int32, device=self.device)
+            orb_off = torch.as_tensor(np.concatenate([[0], np.cumsum(b.norb)[:-1]]).astype(np.int64),
+                                      device=self.device)
+            evals = torch.empty(int(b.norb.sum()), **f64)
+            Q = torch.empty(max(b.total, 1), **f64)
+            self.eigenpairs(F, orb_off, evals, Q, evals, fail)
+            e = torch.empty(b.nmol, 4 * b.molsize, **f64)
+            V = torch.empty(b.nmol, nmax, nmax, **f64)
+            nat.call("pyseqm_evec_view", b.L, b.molsize, nmax, nat.ptr(orb_off), nat.ptr(evals), nat.ptr(Q),
+                     nat.ptr(e), nat.ptr(V), self.stream)
+            if int((fail[0] + (~torch.isfinite(evals)).sum()).item()) == 0:
+                return e, V
+        idx = torch.arange(b.nmol, dtype=torch.int32, device=self.device)
+        Fp = torch.empty(b.nmol, nmax, nmax, **f64)
         nat.call("pyseqm_pad_for_eigh", b.L, nat.ptr(F), nat.ptr(idx), b.nmol, nmax, nat.ptr(Fp),
                  nat.ptr(self.red), nat.red_blocks(nmax), self.stream)
         e0, V = torch.linalg.eigh(Fp)
-        e = torch.zeros(b.nmol, 4 * b.molsize, dtype=torch.float64, device=self.device)
+        e = torch.zeros(b.nmol, 4 * b.molsize, **f64)
         mask = torch.arange(nmax, device=self.device)[None, :] < torch.as_tensor(b.norb, device=self.device)[:, None]
         e[:, :nmax] = torch.where(mask, e0, torch.zeros_like(e0))
         return e, V

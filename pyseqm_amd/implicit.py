@@ -11,7 +11,7 @@ with G the two-electron part of the Fock build (self-adjoint in the Frobenius pr
 first-order density response of D to a Fock perturbation,
 R(X) = C [M o (C^T X C)] C^T, M_ia = M_ai = 2 / (e_i - e_a) for occupied i and virtual a
 (self-adjoint as well).  Every piece is a device kernel: the eigenpairs (pyseqm_eigh_vectors; the
-batched library eigensolver for blocks above its 139-orbital all-eigenpairs limit),
+batched library eigensolver for blocks of more than 192 orbitals),
 the eigenbasis products (pyseqm_block_gemm), M (pyseqm_density_response_elem), G (pyseqm_fock
 with a zero core Hamiltonian) and the parameter contraction (pyseqm_fock_param_vjp).  The
 Anderson mixing of the adjoint iterates runs as per-molecule torch reductions on the packed
@@ -21,7 +21,7 @@ import numpy as np
 import torch
 
 from . import _native as nat
-from .engine import eigh_wg_ok
+from .engine import eigh_pairs_ok
 
 
 class ResponseWorkspace:
@@ -40,7 +40,7 @@ class ResponseWorkspace:
         self.orb_off = torch.as_tensor(np.concatenate([[0], np.cumsum(norb)[:-1]]).astype(np.int64), device=dev)
         self.evals = torch.zeros(max(int(norb.sum()), 1), **f64)
         self.Q = torch.zeros(total, **f64)
-        wg = norb[eigh_wg_ok(norb, norb)]
+        wg = norb[eigh_pairs_ok(norb)]
         self.eig_ws = torch.zeros(max(4 * b.nmol * int(wg.max()) ** 2 if len(wg) else 1, 1), **f64)
         self.fail = torch.zeros(1, dtype=torch.int32, device=dev)
         self.Hzero = torch.zeros(total, **f64)

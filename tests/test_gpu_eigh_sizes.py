@@ -106,3 +106,24 @@ def test_eigenpairs_at_grid_edges(grid, kind):
         assert np.abs(q.T @ q - np.eye(n)).max() < 1e-9, n
         assert np.abs(f @ q - q * e).max() < 1e-9 * scale, n
     assert int(fail.item()) == 0
+
+
+@pytest.mark.parametrize("kind", ["spread", "degenerate", "close", "diagonal", "blocks"])
+def test_eigenpairs_above_the_lds_limit(kind):
+    """140 to 192 orbitals: the vectors stand in the output; blocks on both sides of the limit in one batch, and
+    eig()'s padded view of the same pairs (the identity beyond a block, zero energies)."""
+    sizes = [140, 5, 141, 159, 160, 139, 161, 182, 191, 192]
+    eng = _engine(sizes, [n // 2 for n in sizes])
+    fs = _blocks(sizes, [n // 2 for n in sizes], kind, 7)
+    F = torch.as_tensor(np.concatenate([f.reshape(-1) for f in fs]), device=DEV)
+    e, V = (t.cpu().numpy() for t in eng.eig(F))
+    assert V.shape == (len(sizes), 192, 192) and e.shape == (len(sizes), 4 * eng.b.molsize)
+    for k, (f, n) in enumerate(zip(fs, sizes)):
+        scale = np.abs(f).max() * np.sqrt(n)
+        want = np.eye(192)
+        want[:n, :n] = V[k, :n, :n]
+        q = V[k, :n, :n]
+        assert np.array_equal(V[k], want) and not e[k, n:].any(), n
+        assert np.abs(e[k, :n] - np.linalg.eigvalsh(f)).max() < 1e-10 * scale, n
+        assert np.abs(q.T @ q - np.eye(n)).max() < 1e-9, n
+        assert np.abs(f @ q - q * e[k, :n]).max() < 1e-9 * scale, n
