@@ -279,6 +279,24 @@ int pyseqm_diis_dots(const pyseqm_layout_t* L, const int* idx, int nact, const d
  * (stride nfock) and reset[m] = 1 when max|lambda| / min|lambda| > 1e7. */
 int pyseqm_diis_solve(const pyseqm_layout_t* L, const int* idx, int nact, int nfock, int count, int slot,
                       const double* Bmat, double* coef, unsigned char* reset, void* stream);
+/* A Pulay iteration's device work around the density step, without a host step in between.
+ * pyseqm_pulay_pre: F's upper triangle into ring slot `slot` of Fring, the residual C = FP - PF into that of
+ * Cring with diis_err[m] = max|C| (residual == 0: both are there already), the B row (pyseqm_diis_dots), for
+ * count >= 2 the coefficients with reset[m] (pyseqm_diis_solve; count <= 15) and the extrapolated F
+ * (pyseqm_diis_combine).  X: FP64 scratch of the packed size; red: nact nb 16 doubles.
+ * pyseqm_pulay_post: P = alpha P + (1 - alpha) Pnew, the Fock build of the molecules marked in notconv (the
+ * listed ones), the convergence test of pyseqm_scf_check on that step, then a wait for the stream: host
+ * [2][nmol] in pinned memory then holds notconv and reset of the listed molecules. */
+int pyseqm_pulay_pre(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, double* F, const double* P,
+                     double* X, double* Fring, double* Cring, long long ring_stride, int slot, int count, int nfock,
+                     double* EMAT, double* coef, unsigned char* reset, double* diis_err, double* red, int nb,
+                     int residual, void* stream);
+int pyseqm_pulay_post(const pyseqm_layout_t* L, const int* idx, int nact, double alpha, double* P,
+                      const double* Pnew, const double* atom_par, const double* w_xx, const double* w_xh,
+                      const double* w_hh, const double* H, double* F, double* part, double* tile_v, double* atom_v,
+                      double* e_new, double* e_old, const double* diis_err, double eps, double diis_tol,
+                      unsigned char* notconv, double* metrics, double* red, int nb, const unsigned char* reset,
+                      unsigned char* host, void* stream);
 /* F = sum_j coef[j] ring[j] (scf_loop.py:1033-1035), full symmetric F formed from the ring
  * entries' upper triangles. */
 int pyseqm_diis_combine(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const double* ring,

@@ -69,6 +69,10 @@ _SIGS = {
                                       c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
     "pyseqm_sp2_iterate_many": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                 c_void_p, c_int, c_double, c_int, c_void_p, c_int, c_int, c_void_p],
+    "pyseqm_pulay_pre": [c_void_p, c_int, c_int] + [c_void_p] * 5 + [c_longlong, c_int, c_int, c_int]
+                        + [c_void_p] * 5 + [c_int, c_int, c_void_p],
+    "pyseqm_pulay_post": [c_void_p, c_int, c_double] + [c_void_p] * 14 + [c_double, c_double] + [c_void_p] * 3
+                         + [c_int] + [c_void_p] * 3,
     "pyseqm_diis_solve": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
     "pyseqm_diis_dots": [c_void_p, c_int, c_void_p, c_longlong, c_int, c_int, c_int, c_void_p, c_void_p, c_int,
                          c_void_p],

@@ -289,11 +289,52 @@ __global__ void k_check_partial(pyseqm_layout_t L, const int* __restrict__ idx, 
   }
 }
 
+// P = a P + (1 - a) Pnew and the partial sums of that step's dP, as k_mix then k_check_partial give them (the
+// same elements per thread in the same order, so the same bits), without Pold: 128 alkanes of 14-182
+// orbitals: 10.6 us (11.6 + 11.8 as two).
+__global__ __launch_bounds__(kEl) void k_mix_check(pyseqm_layout_t L, const int* __restrict__ idx, int nb, double a,
+                                                   double* __restrict__ P, const double* __restrict__ Pnew,
+                                                   double* __restrict__ red) {
+  __shared__ double sh[kEl / 64];
+  const int k = blockIdx.y;
+  const int m = idx[k];
+  const size_t n2 = (size_t)L.mol_norb[m] * L.mol_norb[m];
+  const size_t off = L.mol_mat_off[m], step = (size_t)nb * blockDim.x;
+  double ss = 0.0, mx = 0.0;
+  for (size_t e0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e0 < n2; e0 += 2 * kElPerThread * step) {
+    double p[2 * kElPerThread], q[2 * kElPerThread];
+#pragma unroll
+    for (int u = 0; u < 2 * kElPerThread; ++u) {
+      const size_t e = e0 + u * step;
+      p[u] = e < n2 ? P[off + e] : 0.0;
+      q[u] = e < n2 ? Pnew[off + e] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 2 * kElPerThread; ++u) {
+      const size_t e = e0 + u * step;
+      if (e < n2) {
+        const double v = a * p[u] + (1.0 - a) * q[u], d = v - p[u];
+        P[off + e] = v;
+        ss += d * d;
+        mx = fmax(mx, fabs(d));
+      }
+    }
+  }
+  const double s2 = block_sum(ss, sh);
+  const double m2 = block_max(mx, sh);
+  if (threadIdx.x == 0) {
+    red[((size_t)k * nb + blockIdx.x) * 2] = s2;
+    red[((size_t)k * nb + blockIdx.x) * 2 + 1] = m2;
+  }
+}
+
 __global__ __launch_bounds__(64) void k_check_final(pyseqm_layout_t L, const int* __restrict__ idx, int nact, int nb,
                                                    const double* __restrict__ red, const double* __restrict__ e_new,
                                                    double* __restrict__ e_old, const double* __restrict__ diis_err,
                                                    double eps, double diis_tol, unsigned char* __restrict__ notconv,
-                                                   double* __restrict__ metrics) {
+                                                   double* __restrict__ metrics,
+                                                   const unsigned char* __restrict__ reset,
+                                                   unsigned char* __restrict__ host) {
   // one wave per molecule: lanes take block partials b = lane, lane + 64, ... (fixed order)
   const int k = blockIdx.x;
   const int lane = threadIdx.x;
@@ -313,6 +354,10 @@ __global__ __launch_bounds__(64) void k_check_final(pyseqm_layout_t L, const int
   const bool bad = fabs(de) > eps || dd > diis_tol || dm > 2.0 * eps || m2 > 15.0 * eps;
   notconv[m] = bad ? 1 : 0;
   if (bad) e_old[m] = e_new[m];
+  if (host) {  // the caller's copy in pinned memory: read after a wait for the stream, without a copy command
+    host[m] = bad ? 1 : 0;
+    host[L.nmol + m] = reset ? reset[m] : 0;
+  }
   if (metrics) {
     metrics[4 * m + 0] = de;
     metrics[4 * m + 1] = dd;
@@ -371,13 +416,14 @@ __global__ __launch_bounds__(256) void k_gemm64(pyseqm_layout_t L, const int* __
     }
 }
 
-// C = X - X^T (X = F P, so C = FP - PF) into the ring slot, with per-block partial max|C|.
 // C = X - X^T and per-block max|C| over the active blocks.  Work unit: a pair of mirrored 32 x 32
 // tiles (I, J), I <= J, of one molecule; both are read as coalesced rows into LDS and both output
-// tiles are written as rows (C_JI = -C_IJ^T), so no element of X is read down a column of HBM.
+// tiles are written as rows (C_JI = -C_IJ^T), so no element of X is read down a column of HBM.  With Fsrc, the
+// same blocks copy F's upper tiles into its ring slot (the rings are read there only).
 __global__ __launch_bounds__(kEl) void k_antisym(pyseqm_layout_t L, const int* __restrict__ idx, int nb,
                                                  const double* __restrict__ X, double* __restrict__ Cout,
-                                                 double* __restrict__ red) {
+                                                 double* __restrict__ red, int rw, const double* __restrict__ Fsrc,
+                                                 double* __restrict__ Fdst) {
   __shared__ double A[32][33], B[32][33];
   __shared__ double sh[kEl / 64];
   const int k = blockIdx.y;
@@ -403,6 +449,10 @@ __global__ __launch_bounds__(kEl) void k_antisym(pyseqm_layout_t L, const int* _
       const double vb = Xm[(size_t)min(j0 + rr, n - 1) * n + min(i0 + tx, n - 1)];
       A[rr][tx] = (i0 + rr < n && j0 + tx < n) ? va : 0.0;
       B[rr][tx] = (j0 + rr < n && i0 + tx < n) ? vb : 0.0;
+      if (Fsrc && i0 + rr < n && j0 + tx < n && i0 + rr <= j0 + tx) {
+        const size_t e = L.mol_mat_off[m] + (size_t)(i0 + rr) * n + j0 + tx;
+        Fdst[e] = Fsrc[e];
+      }
     }
     __syncthreads();
 #pragma unroll
@@ -422,16 +472,7 @@ __global__ __launch_bounds__(kEl) void k_antisym(pyseqm_layout_t L, const int* _
     __syncthreads();
   }
   const double r = block_max(mx, sh);
-  if (threadIdx.x == 0) red[(size_t)k * nb + blockIdx.x] = r;
-}
-
-__global__ __launch_bounds__(64) void k_antisym_final(const int* __restrict__ idx, int nact, int nb,
-                                                     const double* __restrict__ red, double* __restrict__ diis_err) {
-  const int k = blockIdx.x;
-  double mx = 0.0;
-  for (int b = threadIdx.x; b < nb; b += 64) mx = fmax(mx, red[(size_t)k * nb + b]);
-  mx = wave_max(mx);
-  if (threadIdx.x == 0) diis_err[idx[k]] = mx;
+  if (threadIdx.x == 0) red[((size_t)k * nb + blockIdx.x) * rw + rw - 1] = r;
 }
 
 // B[m][slot][j] = <C_slot, C_j> over the strict upper triangle (= 0.5 * full Frobenius product: C is
@@ -478,75 +519,119 @@ __global__ __launch_bounds__(kEl) void k_diis_dots(pyseqm_layout_t L, const int*
   }
 }
 
-__global__ __launch_bounds__(64) void k_diis_dots_final(const int* __restrict__ idx, int nact, int nb, int slot,
-                                                       int count, int nfock, const double* __restrict__ red,
-                                                       double* __restrict__ Bmat) {
-  // one wave per (molecule, history entry): lanes take block partials b = lane, lane + 64, ...
-  const int k = blockIdx.x / count, j = blockIdx.x % count;
-  double s = 0.0;
-  for (int b = threadIdx.x; b < nb; b += 64) s += red[((size_t)k * nb + b) * 16 + j];
-  s = wave_sum(s);
-  if (threadIdx.x == 0) Bmat[((size_t)idx[k] * (nfock + 1) + slot) * (nfock + 1) + j] = s;
-}
-
-// DIIS coefficients from the bordered B matrix (scf_loop.py:1015-1031): the lower triangle of
-// EMAT[m][0..cF][0..cF] (mirrored), its cF x cF block divided by B[slot][slot], eigendecomposed by
-// cyclic Jacobi in FP64 (one 64-lane block per molecule, matrix and vectors in LDS, lane i owns
-// row / column i), then c_k = -sum_i Q[k][i] q_i Q[cF][i] with q_i = 1/lambda_i for |lambda_i| >
-// 1e-13 (else 0), and reset[m] = (max|lambda| / min|lambda| > 1e7).
+// What follows the partial sums of one molecule's Pulay step, in the order of `what`'s bits (one wave per
+// molecule; what bounds it is the latency of the Jacobi rotations, so nothing else gets a launch of its own):
+//   kDiisErr   diis_err[m] = max of the residual's partials (the last of each block's rw)
+//   kDiisRow   EMAT[m][slot][j] = <C_slot, C_j> from the products' partials (elements 0 .. count-1)
+//   kDiisSolve the coefficients from the bordered B matrix (scf_loop.py:1015-1031): the lower triangle of
+//              EMAT[m][0..cF][0..cF] (mirrored), its cF x cF block divided by B[slot][slot], eigendecomposed
+//              by Jacobi in FP64, then c_k = -sum_i Q[k][i] q_i Q[cF][i] with q_i = 1/lambda_i for
+//              |lambda_i| > 1e-13 (else 0), and reset[m] = (max|lambda| / min|lambda| > 1e7).
+// Jacobi runs in the round-robin order: a round's pairs are disjoint, so their rotations are formed at
+// once (a lane each) and applied at once, N - 1 rounds a sweep instead of N (N - 1) / 2 rotations one after
+// another.  One ethane: 13.6 us (as launches of their own: 1.9 + 2.0 for the sums, 19.0 for the solve).
 constexpr int kDiisMax = 16;
+enum { kDiisErr = 1, kDiisRow = 2, kDiisSolve = 4 };
 
-__global__ __launch_bounds__(64) void k_diis_solve(const int* __restrict__ idx, int nfock, int cF, int slot,
-                                                   const double* __restrict__ EMAT, double* __restrict__ coef,
-                                                   unsigned char* __restrict__ reset) {
-  __shared__ double A[kDiisMax][kDiisMax + 1], V[kDiisMax][kDiisMax + 1];
-  const int m = idx[blockIdx.x];
+__global__ __launch_bounds__(64) void k_diis_finish(const int* __restrict__ idx, int what, int nb, int rw, int nfock, int cF,
+                                                    int slot, const double* __restrict__ red,
+                                                    double* __restrict__ EMAT, double* __restrict__ diis_err,
+                                                    double* __restrict__ coef, unsigned char* __restrict__ reset) {
+  __shared__ double A[kDiisMax][kDiisMax + 1], V[kDiisMax][kDiisMax + 1], B[kDiisMax], rot[kDiisMax / 2][2];
+  __shared__ int pq[kDiisMax / 2][2];
+  const int k = blockIdx.x, m = idx[k];
   const int lane = threadIdx.x;
   const int n = cF + 1, nf1 = nfock + 1;
-  const double* E = EMAT + (size_t)m * nf1 * nf1;
-  const double den = fmax(E[slot * nf1 + slot], 1.0e-15);
-  for (int e = lane; e < n * n; e += 64) {
-    const int i = e / n, j = e % n;
-    double v = i >= j ? E[i * nf1 + j] : E[j * nf1 + i];
+  const double* part = red + (size_t)k * nb * rw;  // rw doubles per block of partials
+  double* E = EMAT + (size_t)m * nf1 * nf1;
+  if (what & kDiisErr) {
+    double mx = 0.0;
+    for (int b = lane; b < nb; b += 64) mx = fmax(mx, part[b * rw + rw - 1]);
+    mx = wave_max(mx);
+    if (lane == 0) diis_err[m] = mx;
+  }
+  if (what & kDiisRow) {
+    for (int j = 0; j < cF; ++j) {  // lanes take block partials b = lane, lane + 64, ... (fixed order)
+      double s = 0.0;
+      for (int b = lane; b < nb; b += 64) s += part[b * rw + j];
+      s = wave_sum(s);
+      if (lane == 0) {
+        B[j] = s;
+        E[slot * nf1 + j] = s;
+      }
+    }
+    __syncthreads();
+  }
+  if (!(what & kDiisSolve)) return;
+  const bool own = what & kDiisRow;  // row `slot` of E is in B
+  auto at = [&](int i, int j) { return own && i == slot && j < cF ? B[j] : E[i * nf1 + j]; };
+  const double den = fmax(at(slot, slot), 1.0e-15);
+  const int N = (n + 1) & ~1;  // an odd order gets a player that sits out: its pair is skipped
+  const int N2 = kDiisMax * n;
+  for (int e = lane; e < N2; e += 64) {
+    const int i = e / kDiisMax, j = e % kDiisMax;
+    if (j >= n) continue;
+    double v = i >= j ? at(i, j) : at(j, i);
     if (i < cF && j < cF) v /= den;
     A[i][j] = v;
     V[i][j] = i == j ? 1.0 : 0.0;
   }
   __syncthreads();
+  const int h = N / 2;
   for (int sweep = 0; sweep < 30; ++sweep) {
     double off = 0.0, tot = 0.0;
-    for (int i = 0; i < n; ++i)
-      for (int j = 0; j < n; ++j) {
-        const double a = A[i][j];
-        tot += a * a;
-        if (j > i) off += a * a;
-      }
-    if (off <= 1.0e-34 * tot) break;  // the same decision in every lane
-    for (int p = 0; p < n - 1; ++p)
-      for (int q = p + 1; q < n; ++q) {
-        const double apq = A[p][q];
-        if (fabs(apq) < 1.0e-300) continue;
-        const double tau = (A[q][q] - A[p][p]) / (2.0 * apq);
-        const double t = fabs(tau) < 1.0e150 ? (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau))
-                                             : 0.5 / tau;
-        const double c = 1.0 / sqrt(1.0 + t * t), sn = t * c;
-        __syncthreads();
-        if (lane < n) {
-          const double ap = A[lane][p], aq = A[lane][q];
-          A[lane][p] = c * ap - sn * aq;
-          A[lane][q] = sn * ap + c * aq;
+    for (int e = lane; e < N2; e += 64) {
+      const int i = e / kDiisMax, j = e % kDiisMax;
+      const double a = j < n ? A[i][j] : 0.0;
+      tot += a * a;
+      if (j > i) off += a * a;
+    }
+    off = wave_sum(off);
+    tot = wave_sum(tot);
+    if (!(off > 1.0e-34 * tot)) break;  // the same decision in every lane
+    for (int round = 0; round < N - 1; ++round) {
+      // circle method: player N - 1 stays, the others move on by one each round
+      if (lane < h) {
+        const int a = lane == 0 ? N - 1 : (round + lane) % (N - 1), b = (round + N - 1 - lane) % (N - 1);
+        const int p = min(a, b), q = max(a, b);
+        double c = 1.0, sn = 0.0;
+        if (q < n && fabs(A[p][q]) >= 1.0e-300) {
+          const double apq = A[p][q];
+          const double tau = (A[q][q] - A[p][p]) / (2.0 * apq);
+          const double t = fabs(tau) < 1.0e150 ? (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau))
+                                               : 0.5 / tau;
+          c = 1.0 / sqrt(1.0 + t * t);
+          sn = t * c;
         }
-        __syncthreads();
-        if (lane < n) {
-          const double ap = A[p][lane], aq = A[q][lane];
-          A[p][lane] = c * ap - sn * aq;
-          A[q][lane] = sn * ap + c * aq;
-          const double vp = V[lane][p], vq = V[lane][q];
-          V[lane][p] = c * vp - sn * vq;
-          V[lane][q] = sn * vp + c * vq;
-        }
-        __syncthreads();
+        rot[lane][0] = c;
+        rot[lane][1] = sn;
+        pq[lane][0] = p;
+        pq[lane][1] = q;
       }
+      __syncthreads();
+      for (int e = lane; e < n * (kDiisMax / 2); e += 64) {  // columns p, q of A and V
+        const int i = e / (kDiisMax / 2), t = min(e % (kDiisMax / 2), h - 1), p = pq[t][0], q = pq[t][1];
+        if (e % (kDiisMax / 2) < h && q < n) {
+          const double c = rot[t][0], sn = rot[t][1];
+          const double ap = A[i][p], aq = A[i][q], vp = V[i][p], vq = V[i][q];
+          A[i][p] = c * ap - sn * aq;
+          A[i][q] = sn * ap + c * aq;
+          V[i][p] = c * vp - sn * vq;
+          V[i][q] = sn * vp + c * vq;
+        }
+      }
+      __syncthreads();
+      for (int e = lane; e < n * (kDiisMax / 2); e += 64) {  // rows p, q of A
+        const int i = e / (kDiisMax / 2), t = min(e % (kDiisMax / 2), h - 1), p = pq[t][0], q = pq[t][1];
+        if (e % (kDiisMax / 2) < h && q < n) {
+          const double c = rot[t][0], sn = rot[t][1];
+          const double ap = A[p][i], aq = A[q][i];
+          A[p][i] = c * ap - sn * aq;
+          A[q][i] = sn * ap + c * aq;
+        }
+      }
+      __syncthreads();
+    }
   }
   if (lane < cF) {
     double ck = 0.0;
@@ -703,7 +788,7 @@ extern "C" int pyseqm_scf_check(const pyseqm_layout_t* L, const int* idx, int na
   hipStream_t s = (hipStream_t)stream;
   k_check_partial<<<dim3(nb, nact), kEl, 0, s>>>(*L, idx, nb, P, Pold, red);
   k_check_final<<<nact, 64, 0, s>>>(*L, idx, nact, nb, red, e_new, e_old, diis_err, eps, diis_tol,
-                                                  notconv, metrics);
+                                                  notconv, metrics, nullptr, nullptr);
   return status();
 }
 
@@ -734,8 +819,9 @@ extern "C" int pyseqm_diis_residual(const pyseqm_layout_t* L, const int* idx, in
                  : pyseqm_dgemm_sym(L, idx, nact, nmax, L->mol_mat_off, nullptr, F, P, X, 0, stream);
   if (rc != PYSEQM_OK || nact == 0) return rc;
   hipStream_t s = (hipStream_t)stream;
-  k_antisym<<<dim3(nb, nact), kEl, 0, s>>>(*L, idx, nb, X, Cout, red);
-  k_antisym_final<<<nact, 64, 0, s>>>(idx, nact, nb, red, diis_err);
+  k_antisym<<<dim3(nb, nact), kEl, 0, s>>>(*L, idx, nb, X, Cout, red, 1, nullptr, nullptr);
+  k_diis_finish<<<nact, 64, 0, s>>>(idx, kDiisErr, nb, 1, 1, 1, 0, red, nullptr, diis_err, nullptr,
+                                     nullptr);
   return status();
 }
 
@@ -748,8 +834,8 @@ extern "C" int pyseqm_diis_dots(const pyseqm_layout_t* L, const int* idx, int na
   if (nact == 0) return PYSEQM_OK;
   hipStream_t s = (hipStream_t)stream;
   k_diis_dots<<<dim3(nb, nact), kEl, 0, s>>>(*L, idx, nb, ring, (size_t)ring_stride, slot, count, red);
-  k_diis_dots_final<<<nact * count, 64, 0, s>>>(idx, nact, nb, slot, count, nfock, red,
-                                                                         Bmat);
+  k_diis_finish<<<nact, 64, 0, s>>>(idx, kDiisRow, nb, 16, nfock, count, slot, red, Bmat, nullptr, nullptr,
+                                     nullptr);
   return status();
 }
 
@@ -758,7 +844,8 @@ extern "C" int pyseqm_diis_solve(const pyseqm_layout_t* L, const int* idx, int n
   if (!L || nact < 0 || count < 1 || count + 1 > kDiisMax || count > nfock || slot < 0 || slot >= nfock)
     return PYSEQM_EINVAL;
   if (nact == 0) return PYSEQM_OK;
-  k_diis_solve<<<nact, 64, 0, (hipStream_t)stream>>>(idx, nfock, count, slot, Bmat, coef, reset);
+  k_diis_finish<<<nact, 64, 0, (hipStream_t)stream>>>(idx, kDiisSolve, 0, 16, nfock, count, slot, nullptr,
+                                                      const_cast<double*>(Bmat), nullptr, coef, reset);
   return status();
 }
 
@@ -771,4 +858,55 @@ extern "C" int pyseqm_diis_combine(const pyseqm_layout_t* L, const int* idx, int
   k_diis_combine<<<dim3(nb, nact), kEl, 0, (hipStream_t)stream>>>(*L, idx, nb, ring, (size_t)ring_stride, count, coef,
                                                                    cstride, F);
   return status();
+}
+
+// The Pulay step's device work before the density step: F's ring slot, the residual C = FP - PF (with
+// residual == 0 it is in its ring slot already, and diis_err), the B row, coefficients and extrapolated F.
+extern "C" int pyseqm_pulay_pre(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, double* F,
+                                const double* P, double* X, double* Fring, double* Cring, long long ring_stride,
+                                int slot, int count, int nfock, double* EMAT, double* coef, unsigned char* reset,
+                                double* diis_err, double* red, int nb, int residual, void* stream) {
+  if (!L || nact < 0 || nmax <= 0 || count < 1 || count + 1 > kDiisMax || count > nfock || nfock > 16 || slot < 0 ||
+      slot >= nfock || nb < 1 || nb > PYSEQM_MAX_RED_BLOCKS)
+    return PYSEQM_EINVAL;
+  if (nact == 0) return PYSEQM_OK;
+  hipStream_t s = (hipStream_t)stream;
+  const size_t at = (size_t)slot * ring_stride;
+  if (residual) {
+    const int rc = pyseqm_dgemm_sym(L, idx, nact, nmax, L->mol_mat_off, nullptr, F, P, X, 0, stream);
+    if (rc != PYSEQM_OK) return rc;
+    k_antisym<<<dim3(nb, nact), kEl, 0, s>>>(*L, idx, nb, X, Cring + at, red, 16, F, Fring + at);
+  } else {
+    k_copy_active<<<dim3(row_blocks(nmax), nact), kEl, 0, s>>>(*L, idx, row_blocks(nmax), F, Fring + at);
+  }
+  k_diis_dots<<<dim3(nb, nact), kEl, 0, s>>>(*L, idx, nb, Cring, (size_t)ring_stride, slot, count, red);
+  const int what = kDiisRow | (residual ? kDiisErr : 0) | (count >= 2 ? kDiisSolve : 0);
+  k_diis_finish<<<nact, 64, 0, s>>>(idx, what, nb, 16, nfock, count, slot, red, EMAT, diis_err, coef, reset);
+  if (count >= 2) {
+    const int nt = tile_pair_blocks(nmax);
+    k_diis_combine<<<dim3(nt, nact), kEl, 0, s>>>(*L, idx, nt, Fring, (size_t)ring_stride, count, coef, nfock, F);
+  }
+  return status();
+}
+
+// The Pulay step's device work after the density step: mixing, the Fock build of the listed molecules, the
+// convergence test; then a wait for the stream, after which host[0 .. nmol) holds the listed molecules'
+// notconv and host[nmol .. 2 nmol) their reset flags.
+extern "C" int pyseqm_pulay_post(const pyseqm_layout_t* L, const int* idx, int nact, double alpha, double* P,
+                                 const double* Pnew, const double* atom_par, const double* w_xx, const double* w_xh,
+                                 const double* w_hh, const double* H, double* F, double* part, double* tile_v,
+                                 double* atom_v, double* e_new, double* e_old, const double* diis_err, double eps,
+                                 double diis_tol, unsigned char* notconv, double* metrics, double* red, int nb,
+                                 const unsigned char* reset, unsigned char* host, void* stream) {
+  if (!L || nact < 0 || nb < 1 || nb > PYSEQM_MAX_RED_BLOCKS || !notconv || !host) return PYSEQM_EINVAL;
+  hipStream_t s = (hipStream_t)stream;
+  if (nact > 0) {
+    k_mix_check<<<dim3(nb, nact), kEl, 0, s>>>(*L, idx, nb, alpha, P, Pnew, red);
+    const int rc = pyseqm_fock(L, atom_par, w_xx, w_xh, w_hh, P, H, F, part, tile_v, atom_v, e_new, notconv, stream);
+    if (rc != PYSEQM_OK) return rc;
+    k_check_final<<<nact, 64, 0, s>>>(*L, idx, nact, nb, red, e_new, e_old, diis_err, eps, diis_tol, notconv, metrics,
+                                      reset, host);
+    if (status() != PYSEQM_OK) return PYSEQM_ELAUNCH;
+  }
+  return hipStreamSynchronize(s) == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
 }

@@ -233,8 +233,7 @@ class SCFEngine:
                 # one launch, largest blocks first: the long solves start at once and the short
                 # ones fill the CUs behind them (C2's density step: 5.2 ms against 8.4 ms for
                 # launches per size group, each of which waits for its own largest block)
-                ids = idx_h[wg]
-                self._eigh_wg(F, ids[np.argsort(-b.norb[ids], kind="stable")], Pout)
+                self._eigh_wg_run(F, *self._eigh_wg_order(idx_h[wg]), Pout)
             rest = idx_h[~wg]
             if len(rest) == 0:
                 return None
@@ -261,16 +260,26 @@ class SCFEngine:
             return e, V, nmax
         return None
 
+    def _eigh_wg_order(self, ids):
+        """(device index list, count, largest block, most occupied orbitals) of the molecules `ids`, largest first."""
+        b = self.b
+        ids = ids[np.argsort(-b.norb[ids], kind="stable")]
+        idx = torch.as_tensor(ids.astype(np.int32), device=self.device)
+        return idx, len(ids), int(b.norb[ids[0]]), int(b.nocc[ids].max())
+
+    def _eigh_wg_list(self, ids):
+        """_eigh_wg_order of the molecules `ids` if the workgroup eigensolver takes all of them, else None."""
+        return self._eigh_wg_order(ids) if eigh_wg_ok(self.b.norb[ids], self.b.nocc[ids]).all() else None
+
     def _eigh_wg(self, F, ids, Pout):
         """One launch of the workgroup eigensolver on the molecules `ids` (host int array)."""
-        b = self.b
-        nmax = int(b.norb[ids].max())
-        nocc_max = int(b.nocc[ids].max())
-        ws = torch.empty(max(4 * len(ids) * nmax * nmax, 1), dtype=torch.float64, device=self.device)
-        idx = torch.as_tensor(ids.astype(np.int32), device=self.device)
-        nat.call("pyseqm_eigh_density", b.L, nat.ptr(idx), len(ids), nmax, nocc_max, nat.ptr(F), nat.ptr(Pout),
+        self._eigh_wg_run(F, *self._eigh_wg_order(ids), Pout)
+
+    def _eigh_wg_run(self, F, idx, count, nmax, nocc_max, Pout):
+        ws = torch.empty(max(4 * count * nmax * nmax, 1), dtype=torch.float64, device=self.device)
+        nat.call("pyseqm_eigh_density", self.b.L, nat.ptr(idx), count, nmax, nocc_max, nat.ptr(F), nat.ptr(Pout),
                  nat.ptr(ws), nat.ptr(self.eigh_fail), self.stream)
-        self.eigh_log.append((len(ids), nmax, "workgroup"))
+        self.eigh_log.append((count, nmax, "workgroup"))
 
     def _sp2_workspace(self):
         ws = getattr(self, "_sp2ws", None)
@@ -309,7 +318,6 @@ class SCFEngine:
         self._metrics = torch.zeros(b.nmol, 4, **f64)
         F = torch.empty_like(P)
         Pnew = torch.zeros_like(P)
-        Pold = torch.zeros_like(P)
         e_old = torch.zeros(b.nmol, **f64)
         e_new = torch.zeros(b.nmol, **f64)
         self.fock(P, F, eelec=e_old)
@@ -318,9 +326,9 @@ class SCFEngine:
         kind = converger[0]
         it = 0
         if kind == 2:
-            res = self._pulay(P, F, Pnew, Pold, e_old, e_new, notconv, eps, max_iter)
+            res = self._pulay(P, F, Pnew, e_old, e_new, notconv, eps, max_iter)
         elif kind in (0, 1):
-            res = self._simple(kind, converger, P, F, Pnew, Pold, e_old, e_new, notconv, eps, max_iter)
+            res = self._simple(kind, converger, P, F, Pnew, torch.zeros_like(P), e_old, e_new, notconv, eps, max_iter)
         else:
             raise ValueError("scf_converger must be [0, alpha], [1] or [2]")
         P, it, nc_host = res
@@ -362,18 +370,14 @@ class SCFEngine:
             else:
                 nat.call("pyseqm_adaptive_mix", b.L, nat.ptr(idx), nact, nmax, int(k), nat.ptr(P), nat.ptr(Pnew),
                          nat.ptr(Pold), nat.ptr(old2), nat.ptr(orb_off), nat.ptr(fac), nat.ptr(mask), self.stream)
-            act = self._act_mask(nc_host)
-            self.fock(P, F, active=act, eelec=e_new)
+            self.fock(P, F, active=notconv, eelec=e_new)  # notconv marks the active molecules
             nat.call("pyseqm_scf_check", b.L, nat.ptr(idx), nact, nat.ptr(P), nat.ptr(Pold), nat.ptr(e_new),
                      nat.ptr(e_old), None, float(eps), 0.0, nat.ptr(notconv), None, nat.ptr(self.red),
                      nat.red_blocks(nmax), self.stream)
             nc_host = notconv.cpu().numpy().astype(bool)
         return P, it, nc_host
 
-    def _act_mask(self, nc_host):
-        return torch.as_tensor(nc_host.astype(np.uint8), device=self.device)
-
-    def _pulay(self, P, F, Pnew, Pold, e_old, e_new, notconv, eps, max_iter):
+    def _pulay(self, P, F, Pnew, e_old, e_new, notconv, eps, max_iter):
         """scf_forward2 (scf_loop.py:639-1132): Pulay DIIS on FP - PF with a 10-deep history,
         batch-global history counter and reset on ill-conditioning (cond > 1e7)."""
         b = self.b
@@ -390,58 +394,63 @@ class SCFEngine:
         EMAT = emat0.expand(b.nmol, -1, -1).clone()
         coef = torch.zeros(b.nmol, NFOCK, **f64)
         reset_flags = torch.zeros(b.nmol, dtype=torch.uint8, device=dev)
+        # notconv and reset flags of the last iteration: the device writes them here, pyseqm_pulay_post waits
+        host = torch.empty(2, b.nmol, dtype=torch.uint8, pin_memory=True)
+        status = host.numpy()
+        ptrs = {k: nat.ptr(t) for k, t in dict(
+            F=F, P=P, X=X, Fring=Fring, Cring=Cring, EMAT=EMAT, coef=coef, reset=reset_flags, diis=diis_err,
+            red=self.red, Pnew=Pnew, par=self.atom_par, xx=self.w_xx, xh=self.w_xh, hh=self.w_hh, H=self.H,
+            part=self.part, tile_v=self.tile_v, atom_v=self.atom_v, e_new=e_new, e_old=e_old, notconv=notconv,
+            metrics=self._metrics, host=host).items()}
         nc_host = np.ones(b.nmol, dtype=bool)
         counter, cF = -1, 0
         it = 0
+        idx = None
         for k in range(max_iter + 1):
-            idx, nact = self._active(nc_host)
-            if nact == 0:
-                break
+            if idx is None:  # the active molecules changed
+                idx, nact = self._active(nc_host)
+                if nact == 0:
+                    break
+                active = self._idx_host
+                nmax = int(b.norb[active].max())
+                nb = nat.red_blocks(nmax)
+                solver = self._eigh_wg_list(active) if self.density_kind == "eigh" else None
             it += 1
-            nmax = int(b.norb[self._idx_host].max())
             cF = min(cF + 1, NFOCK)
             counter = (counter + 1) % NFOCK
-            Fslot = Fring[counter]
-            nat.call("pyseqm_copy_active", b.L, nat.ptr(idx), nact, nmax, nat.ptr(F), nat.ptr(Fslot), self.stream)
-            nb = nat.red_blocks(nmax)
-            if self.density_kind == "sp2" and nmax > MIXED_DIIS_MIN_N:
+            mixed = self.density_kind == "sp2" and nmax > MIXED_DIIS_MIN_N
+            if mixed:
                 # bf16x3 commutator on the upper triangle (the ring is read there only), from FP32
                 # copies of F and P in the SP2 X buffers, which are free until the density step
                 ws = self._sp2_workspace()
                 nat.call("pyseqm_diis_commutator_bf16x3", b.L, nat.ptr(idx), nact, nmax, nat.ptr(F), nat.ptr(P),
                          nat.ptr(ws.xoff), nat.ptr(ws.xld), nat.ptr(ws.Xa), nat.ptr(ws.Xb), nat.ptr(Cring[counter]),
                          nat.ptr(diis_err), nat.ptr(self.red), nat.MAX_RED_BLOCKS * 16, self.stream)
+            # the coefficients from cF = 2 on: the reference's eigh reads only the lower triangle (stale upper
+            # entries included), the kernel mirrors it, normalises by B[slot][slot] and solves by FP64 Jacobi
+            nat.call("pyseqm_pulay_pre", b.L, nat.ptr(idx), nact, nmax, ptrs["F"], ptrs["P"], ptrs["X"],
+                     ptrs["Fring"], ptrs["Cring"], total, counter, cF, NFOCK, ptrs["EMAT"], ptrs["coef"],
+                     ptrs["reset"], ptrs["diis"], ptrs["red"], nb, 0 if mixed else 1, self.stream)
+            if cF >= 2 and self.diis_log is not None:
+                self.diis_log.append((cF, counter, EMAT.cpu().numpy().copy(), coef.cpu().numpy().copy(),
+                                      np.where(nc_host, reset_flags.cpu().numpy(), 0).astype(np.uint8),
+                                      diis_err.cpu().numpy().copy()))
+            if solver is not None:
+                self._eigh_wg_run(F, *solver, Pnew)
             else:
-                nat.call("pyseqm_diis_residual", b.L, nat.ptr(idx), nact, nmax, nat.ptr(F), nat.ptr(P), nat.ptr(X),
-                         nat.ptr(Cring[counter]), nat.ptr(diis_err), nat.ptr(self.red), nb, 0, self.stream)
-            nat.call("pyseqm_diis_dots", b.L, nat.ptr(idx), nact, nat.ptr(Cring), total, counter, cF, NFOCK,
-                     nat.ptr(EMAT), nat.ptr(self.red), nb, self.stream)
-            reset_t = None
-            if cF >= 2:
-                # the reference's eigh reads only the lower triangle (stale upper entries included):
-                # the kernel mirrors it, normalises by B[slot][slot] and solves by FP64 Jacobi
-                reset_flags.zero_()
-                nat.call("pyseqm_diis_solve", b.L, nat.ptr(idx), nact, NFOCK, cF, counter, nat.ptr(EMAT),
-                         nat.ptr(coef), nat.ptr(reset_flags), self.stream)
-                reset_t = reset_flags.any()  # read with the convergence flags (one host sync)
-                if self.diis_log is not None:
-                    self.diis_log.append((cF, counter, EMAT.cpu().numpy().copy(), coef.cpu().numpy().copy(),
-                                          reset_flags.cpu().numpy().copy(), diis_err.cpu().numpy().copy()))
-                nat.call("pyseqm_diis_combine", b.L, nat.ptr(idx), nact, nmax, nat.ptr(Fring), total, cF,
-                         nat.ptr(coef), NFOCK, nat.ptr(F), self.stream)
-            self.density(F, idx, nact, Pnew)
-            alpha = 0.5 if cF < 2 else 0.0
-            nat.call("pyseqm_mix", b.L, nat.ptr(idx), nact, nmax, alpha, nat.ptr(P), nat.ptr(Pnew),
-                     nat.ptr(Pold), self.stream)
-            act = self._act_mask(nc_host)
-            self.fock(P, F, active=act, eelec=e_new)
-            nat.call("pyseqm_scf_check", b.L, nat.ptr(idx), nact, nat.ptr(P), nat.ptr(Pold), nat.ptr(e_new),
-                     nat.ptr(e_old), nat.ptr(diis_err), float(eps), self.diis_tol, nat.ptr(notconv),
-                     nat.ptr(self._metrics), nat.ptr(self.red), nb, self.stream)
-            nc_host = notconv.cpu().numpy().astype(bool)
-            reset = bool(reset_t.item()) if reset_t is not None else False
+                self.density(F, idx, nact, Pnew)
+            nat.call("pyseqm_pulay_post", b.L, nat.ptr(idx), nact, 0.5 if cF < 2 else 0.0, ptrs["P"], ptrs["Pnew"],
+                     ptrs["par"], ptrs["xx"], ptrs["xh"], ptrs["hh"], ptrs["H"], ptrs["F"], ptrs["part"],
+                     ptrs["tile_v"], ptrs["atom_v"], ptrs["e_new"], ptrs["e_old"], ptrs["diis"], float(eps),
+                     self.diis_tol, ptrs["notconv"], ptrs["metrics"], ptrs["red"], nb, ptrs["reset"], ptrs["host"],
+                     self.stream)
             if self.trace is not None:
                 self.trace.append(self._metrics.cpu().numpy().copy())
+            reset = cF >= 2 and bool(status[1][active].any())
+            still = status[0][active]
+            if not still.all():
+                nc_host[active] = still.astype(bool)
+                idx = None
             if reset:
                 counter, cF = -1, 0
                 EMAT.copy_(emat0.expand(b.nmol, -1, -1))
