@@ -281,8 +281,8 @@ int pyseqm_diis_solve(const pyseqm_layout_t* L, const int* idx, int nact, int nf
                       const double* Bmat, double* coef, unsigned char* reset, void* stream);
 /* A Pulay iteration's device work around the density step, without a host step in between.
  * pyseqm_pulay_pre: F's upper triangle into ring slot `slot` of Fring, the residual C = FP - PF into that of
- * Cring with diis_err[m] = max|C| (residual == 0: both are there already), the B row (pyseqm_diis_dots), for
- * count >= 2 the coefficients with reset[m] (pyseqm_diis_solve; count <= 15) and the extrapolated F
+ * Cring with diis_err[m] = max|C| (residual == 0: both are there already), the B row (pyseqm_diis_dots; count ==
+ * 1 starts a history and sets EMAT up first), for count >= 2 the coefficients with reset[m] (pyseqm_diis_solve; count <= 15) and the extrapolated F
  * (pyseqm_diis_combine).  X: FP64 scratch of the packed size; red: nact nb 16 doubles.
  * pyseqm_pulay_post: P = alpha P + (1 - alpha) Pnew, the Fock build of the molecules marked in notconv (the
  * listed ones), the convergence test of pyseqm_scf_check on that step, then a wait for the stream: host
@@ -391,7 +391,8 @@ int pyseqm_small_solve(const int* idx, int nact, int r, const double* O, const d
  *   lane, -1 without a pair, out [ntiles_total*64].
  * pyseqm_w_reference: out [npairs][10][10], the dense integrals (hcore.py:9-179).
  * pyseqm_evec_view: the eigenpairs of pyseqm_eigh_vectors as e [nmol][4 molsize] (zero-padded) and V
- *   [nmol][nmax][nmax] (the identity beyond a block; nmax: at least the batch's largest block).
+ *   [nmol][nmax][nmax] (the identity beyond a block; nmax: at least the batch's largest block); *fail is
+ *   raised by the eigenvalues that are not finite.
  * pyseqm_orbital_charges (scf_loop.py:2376-2387): out [nmol][4 molsize][molsize] from eigenvectors V with
  *   the given strides (doubles). */
 int pyseqm_to_padded(const pyseqm_layout_t* L, int molsize, int mode, const double* X, double* out, void* stream);
@@ -400,7 +401,7 @@ int pyseqm_pair_ref(const pyseqm_layout_t* L, const long long* pair_base, int* o
 int pyseqm_w_reference(const pyseqm_layout_t* L, const long long* pair_base, const double* w_xx, const double* w_xh,
                        const double* w_hh, double* out, void* stream);
 int pyseqm_evec_view(const pyseqm_layout_t* L, int molsize, int nmax, const long long* orb_off,
-                     const double* lam, const double* Q, double* e, double* V, void* stream);
+                     const double* lam, const double* Q, double* e, double* V, int* fail, void* stream);
 int pyseqm_orbital_charges(const pyseqm_layout_t* L, int molsize, const double* V, long long stride_mol,
                            long long stride_row, long long stride_col, double* out, void* stream);
 

@@ -6,6 +6,7 @@ missing or the device is not a HIP GPU, every compute entry point raises.
 import ctypes
 import os
 
+import numpy as np
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -92,7 +93,7 @@ _SIGS = {
     "pyseqm_from_padded": [c_int, c_void_p, c_void_p, c_void_p],
     "pyseqm_pair_ref": [c_void_p, c_void_p, c_void_p],
     "pyseqm_w_reference": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
-    "pyseqm_evec_view": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
+    "pyseqm_evec_view": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
     "pyseqm_orbital_charges": [c_int, c_void_p, c_longlong, c_longlong, c_longlong, c_void_p, c_void_p],
     "pyseqm_xl_energy": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
 }
@@ -156,6 +157,22 @@ def exported_symbols():
 
 def stream_ptr(device=None):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+def upload(device, **arrays):
+    """Host arrays on the device in one copy: {name: tensor}, each at a 16-byte boundary of one buffer (a copy of
+    its own costs some 30 us of host time whatever its size)."""
+    arrays = {k: np.ascontiguousarray(a) for k, a in arrays.items()}
+    off, at = {}, 0
+    for k, a in arrays.items():
+        off[k] = at
+        at += -(-a.nbytes // 16) * 16
+    buf = np.zeros(max(at, 16), dtype=np.uint8)
+    for k, a in arrays.items():
+        buf[off[k]:off[k] + a.nbytes] = a.reshape(-1).view(np.uint8)
+    dev = torch.as_tensor(buf, device=device)
+    return {k: dev[off[k]:off[k] + a.nbytes].view(torch.from_numpy(a[:0].reshape(-1)).dtype).view(a.shape)
+            for k, a in arrays.items()}
 
 
 def ptr(t):

@@ -90,17 +90,18 @@ class Pack_Parameters(torch.nn.Module):
         dev = Z.device
         zc = Z.detach().cpu().numpy()
         out = dict(learned_params)
-        for name in self.parameters:
-            if name not in out:
-                out[name] = torch.as_tensor(self.tab[zc, COLUMNS.index(name)], dtype=torch.float64, device=dev)
+        names = [name for name in self.parameters if name not in out]
+        cols = torch.as_tensor(self.tab[zc][:, [COLUMNS.index(name) for name in names]].T.copy(), dtype=torch.float64,
+                               device=dev)  # one copy for all of them
+        out.update((name, cols[k]) for k, name in enumerate(names))
         out["beta"] = torch.stack((out["beta_s"], out["beta_p"]), dim=1)
         zeros = torch.zeros_like(out["U_ss"])
         for k in ("zeta_d", "s_orb_exp_tail", "p_orb_exp_tail", "d_orb_exp_tail", "U_dd", "F0SD", "G2SD",
                   "rho_core"):
             out[k] = zeros
         out["Kbeta"] = out.get("Kbeta", None)
-        alpha = torch.zeros(int(Z.max().item()) + 1 if len(Z) else 1, int(Z.max().item()) + 1 if len(Z) else 1,
-                            dtype=torch.float64, device=dev)
+        top = int(zc.max()) + 1 if len(zc) else 1
+        alpha = torch.zeros(top, top, dtype=torch.float64, device=dev)
         return out, alpha, alpha.clone()
 
 
@@ -199,7 +200,7 @@ class _ParamEnergies(torch.autograd.Function):
         P, atom_par, coords = ctx.state
         G = eng.param_grad(P, atom_par=atom_par, coords=coords)  # (natoms, 2, 24)
         dI = eng.eiso_grad()
-        mol = torch.as_tensor(eng.b.atom_mol, device=G.device).long()
+        mol = eng.atom_mol()
         dT = G[:, 0] + G[:, 1]
         tot = torch.zeros_like(dT)
         for g, d in ((gEelec, G[:, 0]), (gEnuc, G[:, 1]), (gEtot, dT), (gEiso, dI), (gHf, dT - dI)):
@@ -211,18 +212,17 @@ class _ParamEnergies(torch.autograd.Function):
 
 
 def eng_pair_enuc(eng):
-    """Per-pair core-core repulsion in reference pair order."""
-    eng.set_coordinates(eng.coords, enuc_pair=True)
+    """Per-pair core-core repulsion in reference pair order (from the last integrals where they kept it)."""
+    if eng.enuc_pair is None:
+        eng.set_coordinates(eng.coords, enuc_pair=True)
     return eng.enuc_pair[:eng.b.npairs].clone()
 
 
 def _run_scf(molecule, ham, P0):
-    from .seqm_functions.scf_loop import scf_loop
-    F, e, P, Hcore, w, charge, rho0xi, rho0xj, riXH, ri, notconverged, v = scf_loop(
-        molecule, eps=ham.eps, P=P0, sp2=ham.sp2, scf_converger=list(ham.converger), eig=ham.eig,
-        scf_backward=ham.scf_backward, scf_backward_eps=ham.scf_backward_eps)
-    eng = molecule.engine()
-    en = eng.energies(eng._last_P)
+    from .seqm_functions.scf_loop import run_scf
+    (F, e, P, Hcore, w, charge, rho0xi, rho0xj, riXH, ri, notconverged, v), en = run_scf(
+        molecule, ham.eps, P0, ham.sp2, list(ham.converger), ham.eig, ham.scf_backward, ham.scf_backward_eps,
+        enuc_pair=True)
     e_gap = None
     if e is not None:
         lumo = molecule.nocc.reshape(-1, 1)

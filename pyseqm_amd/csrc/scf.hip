@@ -521,6 +521,7 @@ __global__ __launch_bounds__(kEl) void k_diis_dots(pyseqm_layout_t L, const int*
 
 // What follows the partial sums of one molecule's Pulay step, in the order of `what`'s bits (one wave per
 // molecule; what bounds it is the latency of the Jacobi rotations, so nothing else gets a launch of its own):
+//   kDiisInit  EMAT[m] starts: -1 below the diagonal, else 0
 //   kDiisErr   diis_err[m] = max of the residual's partials (the last of each block's rw)
 //   kDiisRow   EMAT[m][slot][j] = <C_slot, C_j> from the products' partials (elements 0 .. count-1)
 //   kDiisSolve the coefficients from the bordered B matrix (scf_loop.py:1015-1031): the lower triangle of
@@ -531,7 +532,7 @@ __global__ __launch_bounds__(kEl) void k_diis_dots(pyseqm_layout_t L, const int*
 // once (a lane each) and applied at once, N - 1 rounds a sweep instead of N (N - 1) / 2 rotations one after
 // another.  One ethane: 13.6 us (as launches of their own: 1.9 + 2.0 for the sums, 19.0 for the solve).
 constexpr int kDiisMax = 16;
-enum { kDiisErr = 1, kDiisRow = 2, kDiisSolve = 4 };
+enum { kDiisErr = 1, kDiisRow = 2, kDiisSolve = 4, kDiisInit = 8 };
 
 __global__ __launch_bounds__(64) void k_diis_finish(const int* __restrict__ idx, int what, int nb, int rw, int nfock, int cF,
                                                     int slot, const double* __restrict__ red,
@@ -544,6 +545,10 @@ __global__ __launch_bounds__(64) void k_diis_finish(const int* __restrict__ idx,
   const int n = cF + 1, nf1 = nfock + 1;
   const double* part = red + (size_t)k * nb * rw;  // rw doubles per block of partials
   double* E = EMAT + (size_t)m * nf1 * nf1;
+  if (what & kDiisInit) {
+    for (int e = lane; e < nf1 * nf1; e += 64) E[e] = e % nf1 < e / nf1 ? -1.0 : 0.0;
+    __syncthreads();  // before the row
+  }
   if (what & kDiisErr) {
     double mx = 0.0;
     for (int b = lane; b < nb; b += 64) mx = fmax(mx, part[b * rw + rw - 1]);
@@ -861,7 +866,8 @@ extern "C" int pyseqm_diis_combine(const pyseqm_layout_t* L, const int* idx, int
 }
 
 // The Pulay step's device work before the density step: F's ring slot, the residual C = FP - PF (with
-// residual == 0 it is in its ring slot already, and diis_err), the B row, coefficients and extrapolated F.
+// residual == 0 it is in its ring slot already, and diis_err), the B row (count == 1 starts a history: EMAT
+// is set up), coefficients and extrapolated F.
 extern "C" int pyseqm_pulay_pre(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, double* F,
                                 const double* P, double* X, double* Fring, double* Cring, long long ring_stride,
                                 int slot, int count, int nfock, double* EMAT, double* coef, unsigned char* reset,
@@ -880,7 +886,7 @@ extern "C" int pyseqm_pulay_pre(const pyseqm_layout_t* L, const int* idx, int na
     k_copy_active<<<dim3(row_blocks(nmax), nact), kEl, 0, s>>>(*L, idx, row_blocks(nmax), F, Fring + at);
   }
   k_diis_dots<<<dim3(nb, nact), kEl, 0, s>>>(*L, idx, nb, Cring, (size_t)ring_stride, slot, count, red);
-  const int what = kDiisRow | (residual ? kDiisErr : 0) | (count >= 2 ? kDiisSolve : 0);
+  const int what = kDiisRow | (residual ? kDiisErr : 0) | (count >= 2 ? kDiisSolve : kDiisInit);
   k_diis_finish<<<nact, 64, 0, s>>>(idx, what, nb, 16, nfock, count, slot, red, EMAT, diis_err, coef, reset);
   if (count >= 2) {
     const int nt = tile_pair_blocks(nmax);

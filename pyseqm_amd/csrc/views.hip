@@ -149,7 +149,8 @@ __global__ __launch_bounds__(256) void k_orbital_charges(pyseqm_layout_t L, int 
 __global__ __launch_bounds__(256) void k_evec_view(pyseqm_layout_t L, int w, int nmax,
                                                    const long long* __restrict__ orb_off,
                                                    const double* __restrict__ lam, const double* __restrict__ Q,
-                                                   double* __restrict__ e, double* __restrict__ V) {
+                                                   double* __restrict__ e, double* __restrict__ V,
+                                                   int* __restrict__ fail) {
   const int m = blockIdx.x, n = L.mol_norb[m];
   const double* q = Q + L.mol_mat_off[m];
   double* v = V + (size_t)m * nmax * nmax;
@@ -158,7 +159,11 @@ __global__ __launch_bounds__(256) void k_evec_view(pyseqm_layout_t L, int w, int
     for (int c = threadIdx.x; c < nmax; c += 256)
       v[(size_t)r * nmax + c] = (r < n && c < n) ? q[(size_t)r * n + c] : (r == c ? 1.0 : 0.0);
   if (blockIdx.y == 0)
-    for (int c = threadIdx.x; c < w; c += 256) e[(size_t)m * w + c] = c < n ? lam[orb_off[m] + c] : 0.0;
+    for (int c = threadIdx.x; c < w; c += 256) {
+      const double x = c < n ? lam[orb_off[m] + c] : 0.0;
+      e[(size_t)m * w + c] = x;
+      if (!(fabs(x) < INFINITY)) atomicAdd(fail, 1);
+    }
 }
 
 dim3 view_grid(const pyseqm_layout_t& L, int molsize) { return dim3(L.nmol, (4 * molsize + kViewRows - 1) / kViewRows); }
@@ -209,11 +214,11 @@ extern "C" int pyseqm_w_reference(const pyseqm_layout_t* L, const long long* pai
 }
 
 extern "C" int pyseqm_evec_view(const pyseqm_layout_t* L, int molsize, int nmax, const long long* orb_off,
-                                const double* lam, const double* Q, double* e, double* V, void* stream) {
-  if (!L || molsize < 1 || nmax < 1 || !orb_off || nmax > 4 * molsize) return PYSEQM_EINVAL;
+                                const double* lam, const double* Q, double* e, double* V, int* fail, void* stream) {
+  if (!L || molsize < 1 || nmax < 1 || !orb_off || !fail || nmax > 4 * molsize) return PYSEQM_EINVAL;
   if (L->nmol == 0) return PYSEQM_OK;
   const dim3 g(L->nmol, (nmax + kViewRows - 1) / kViewRows);
-  k_evec_view<<<g, 256, 0, (hipStream_t)stream>>>(*L, 4 * molsize, nmax, orb_off, lam, Q, e, V);
+  k_evec_view<<<g, 256, 0, (hipStream_t)stream>>>(*L, 4 * molsize, nmax, orb_off, lam, Q, e, V, fail);
   return launched();
 }
 

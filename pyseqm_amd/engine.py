@@ -112,7 +112,20 @@ class SCFEngine:
         self.default_params = True  # atom_par holds the parameter file's values
         par = np.zeros((b.natoms, nat.NPAR))
         par[:, :len(COLUMNS)] = tab[b.Z]
-        self.atom_par = torch.as_tensor(par, **f64)
+        # isolated-atom energies and atomic heats of formation (geometry independent), initial diagonal density
+        Z = b.Z
+        eiso = (tab[Z, 0] * np.take(USSC, Z) + tab[Z, 1] * np.take(UPPC, Z) + tab[Z, 6] * np.take(GSSC, Z)
+                + tab[Z, 8] * np.take(GPPC, Z) + tab[Z, 7] * np.take(GSPC, Z) + tab[Z, 9] * np.take(GP2C, Z)
+                + tab[Z, 10] * np.take(HSPC, Z))
+        self.eiso_atom = eiso
+        # diag_index is molecule-major in orbital order, the same order as the atoms
+        guess = np.repeat(np.where(Z > 1, np.take(TORE, Z) / 4.0, 1.0), np.where(Z > 1, 4, 1))
+        up = nat.upload(dev, par=par, eiso=np.bincount(b.atom_mol, eiso, minlength=b.nmol),
+                        eheat=np.bincount(b.atom_mol, np.take(EHEAT, Z) / ev_kcalpmol, minlength=b.nmol),
+                        diag=b.diag_index()[0].astype(np.int64), guess=guess,
+                        orb_off=(np.cumsum(b.norb) - b.norb).astype(np.int64))
+        self.atom_par, self.eiso, self.eheat = up["par"], up["eiso"], up["eheat"]
+        self._diag, self._guess, self.orb_off = up["diag"], up["guess"], up["orb_off"]
         self.stream = nat.stream_ptr(dev)
         nat.call("pyseqm_atom_setup", b.L, nat.ptr(self.atom_par), self.stream)
         nt = b.ntiles
@@ -126,15 +139,7 @@ class SCFEngine:
         self.enuc = torch.zeros(b.nmol, **f64)
         self.red = torch.zeros(max(b.nmol, 1) * nat.MAX_RED_BLOCKS * 16, **f64)  # reduction scratch
         self.eelec = torch.zeros(b.nmol, **f64)
-        # isolated-atom energies and atomic heats of formation (geometry independent)
-        Z = b.Z
-        eiso = (tab[Z, 0] * np.take(USSC, Z) + tab[Z, 1] * np.take(UPPC, Z) + tab[Z, 6] * np.take(GSSC, Z)
-                + tab[Z, 8] * np.take(GPPC, Z) + tab[Z, 7] * np.take(GSPC, Z) + tab[Z, 9] * np.take(GP2C, Z)
-                + tab[Z, 10] * np.take(HSPC, Z))
-        self.eiso_atom = eiso
-        self.eiso = torch.as_tensor(np.bincount(b.atom_mol, eiso, minlength=b.nmol), **f64)
-        self.eheat = torch.as_tensor(np.bincount(b.atom_mol, np.take(EHEAT, Z) / ev_kcalpmol, minlength=b.nmol),
-                                     **f64)
+        self._atoms = None
         self.coords = None
         self.trace = None  # set to a list to collect per-iteration (dE, diis, dm, dm_max) metrics
         self.diis_log = None  # set to a list to collect (cF, slot, B matrices, coefficients, resets, errors)
@@ -159,25 +164,46 @@ class SCFEngine:
         kb = params.get("Kbeta", None)
         if torch.is_tensor(kb):
             raise NotImplementedError("per-pair Kbeta resonance scaling is not supported by the device engine")
+        values = {}
         for name, v in params.items():
             if name not in COLUMNS or v is None:
                 continue
             v = torch.as_tensor(v, dtype=torch.float64, device=self.device).detach().reshape(-1)
             if v.numel() != b.natoms:
                 raise ValueError(f"parameter {name!r}: {v.numel()} values for {b.natoms} atoms")
-            self.atom_par[:, COLUMNS.index(name)] = v
+            values[COLUMNS.index(name)] = v
+        if len(values) == len(COLUMNS):
+            self.atom_par[:, :len(COLUMNS)] = torch.stack([values[c] for c in range(len(COLUMNS))], dim=1)
+        else:
+            for c, v in values.items():
+                self.atom_par[:, c] = v
         self.default_params = False
         nat.call("pyseqm_atom_setup", b.L, nat.ptr(self.atom_par), self.stream)
-        Z = torch.as_tensor(b.Z, device=self.device).long()
         ap = self.atom_par
-        tab = lambda t: torch.as_tensor(t, dtype=torch.float64, device=self.device)[Z]
-        eiso = (ap[:, 0] * tab(USSC) + ap[:, 1] * tab(UPPC) + ap[:, 6] * tab(GSSC) + ap[:, 8] * tab(GPPC)
-                + ap[:, 7] * tab(GSPC) + ap[:, 9] * tab(GP2C) + ap[:, 10] * tab(HSPC))
+        eiso = sum(ap[:, c] * coef for c, coef in self._eiso_coef())
         self.eiso_atom = eiso.cpu().numpy()
         self.eiso = torch.zeros(b.nmol, dtype=torch.float64, device=self.device).index_add_(
-            0, torch.as_tensor(b.atom_mol, device=self.device).long(), eiso)
+            0, self.atom_mol(), eiso)
         if self.coords is not None:
             self.set_coordinates(self.coords)
+
+    def _atom_data(self):
+        """Per-atom constants on the device, uploaded on first use: molecule and Eiso coefficients."""
+        if self._atoms is None:
+            Z = self.b.Z
+            coef = [(c, np.take(t, Z).astype(np.float64)) for c, t in
+                    ((0, USSC), (1, UPPC), (6, GSSC), (8, GPPC), (7, GSPC), (9, GP2C), (10, HSPC))]
+            up = nat.upload(self.device, mol=self.b.atom_mol.astype(np.int64), coef=np.stack([t for _, t in coef]))
+            self._atoms = up["mol"], [(c, up["coef"][k]) for k, (c, _) in enumerate(coef)]
+        return self._atoms
+
+    def atom_mol(self):
+        """Molecule of each atom (int64, device)."""
+        return self._atom_data()[0]
+
+    def _eiso_coef(self):
+        """(parameter column, its coefficient per atom) of the isolated-atom energy (energy.py:8-23)."""
+        return self._atom_data()[1]
 
     # ------------------------------------------------------------- integrals
     def set_coordinates(self, coordinates, enuc_pair=False):
@@ -185,7 +211,7 @@ class SCFEngine:
         b = self.b
         c = torch.as_tensor(coordinates, dtype=torch.float64, device=self.device)
         if c.dim() == 3:
-            c = c.reshape(-1, 3)[torch.as_tensor(b.real_flat, device=self.device)]
+            c = c.reshape(-1, 3)[b.d["real_flat"]]
         self.coords = c.contiguous()
         self.enuc_pair = torch.zeros(max(b.npairs, 1), dtype=torch.float64, device=self.device) if enuc_pair \
             else None
@@ -205,14 +231,8 @@ class SCFEngine:
 
     def initial_density(self):
         """Diagonal guess (scf_loop.py:2066-2081): heavy atoms tore/4 on s and p, H 1.0."""
-        b = self.b
-        P = torch.zeros(max(b.total, 1), dtype=torch.float64, device=self.device)
-        didx, _ = b.diag_index()
-        # diag_index is molecule-major in orbital order, the same order as the atoms
-        k = np.where(b.Z > 1, 4, 1)
-        vals = np.repeat(np.where(b.Z > 1, np.take(TORE, b.Z) / 4.0, 1.0), k)
-        P[torch.as_tensor(didx, device=self.device)] = torch.as_tensor(vals, dtype=torch.float64,
-                                                                        device=self.device)
+        P = torch.zeros(max(self.b.total, 1), dtype=torch.float64, device=self.device)
+        P[self._diag] = self._guess
         return P
 
     # ---------------------------------------------------------- density step
@@ -317,9 +337,9 @@ class SCFEngine:
         P = self.initial_density() if P is None else P.clone()
         self._metrics = torch.zeros(b.nmol, 4, **f64)
         F = torch.empty_like(P)
-        Pnew = torch.zeros_like(P)
-        e_old = torch.zeros(b.nmol, **f64)
-        e_new = torch.zeros(b.nmol, **f64)
+        Pnew = torch.empty_like(P)
+        e_old = torch.empty(b.nmol, **f64)
+        e_new = torch.empty(b.nmol, **f64)
         self.fock(P, F, eelec=e_old)
         notconv = torch.ones(b.nmol, dtype=torch.uint8, device=dev)
         nc_host = np.ones(b.nmol, dtype=bool)
@@ -384,16 +404,15 @@ class SCFEngine:
         dev = self.device
         total = max(b.total, 1)
         f64 = dict(dtype=torch.float64, device=dev)
-        Fring = torch.zeros(NFOCK, total, **f64)
-        Cring = torch.zeros(NFOCK, total, **f64)
+        # every element that is read is written first: a history of cF entries reads those only, and
+        # pyseqm_pulay_pre starts EMAT at cF = 1
+        Fring = torch.empty(NFOCK, total, **f64)
+        Cring = torch.empty(NFOCK, total, **f64)
         X = torch.empty(total, **f64)
-        diis_err = torch.full((b.nmol,), torch.finfo(torch.float64).max, **f64)
-        emat0 = torch.tril(torch.eye(NFOCK + 1, **f64) - 1.0)
-        # clone, not contiguous(): for one molecule the expanded view already counts as contiguous and
-        # would alias emat0, so the reset below would copy the updated matrix onto itself
-        EMAT = emat0.expand(b.nmol, -1, -1).clone()
-        coef = torch.zeros(b.nmol, NFOCK, **f64)
-        reset_flags = torch.zeros(b.nmol, dtype=torch.uint8, device=dev)
+        diis_err = torch.empty(b.nmol, **f64)
+        EMAT = torch.empty(b.nmol, NFOCK + 1, NFOCK + 1, **f64)
+        coef = torch.empty(b.nmol, NFOCK, **f64)
+        reset_flags = torch.empty(b.nmol, dtype=torch.uint8, device=dev)
         # notconv and reset flags of the last iteration: the device writes them here, pyseqm_pulay_post waits
         host = torch.empty(2, b.nmol, dtype=torch.uint8, pin_memory=True)
         status = host.numpy()
@@ -453,7 +472,6 @@ class SCFEngine:
                 idx = None
             if reset:
                 counter, cF = -1, 0
-                EMAT.copy_(emat0.expand(b.nmol, -1, -1))
         return P, it, nc_host
 
     # -------------------------------------------------------------- results
@@ -498,12 +516,9 @@ class SCFEngine:
         """d(isolated-atom energy)/d(input parameter) per atom, (natoms, 24): the coefficients of
         U_ss, U_pp, g_ss, g_sp, g_pp, g_p2, h_sp in Eiso (energy.py:8-23)."""
         b = self.b
-        Z = torch.as_tensor(b.Z, device=self.device).long()
-        tab = lambda t: torch.as_tensor(t, dtype=torch.float64, device=self.device)[Z]
         g = torch.zeros(b.natoms, 24, dtype=torch.float64, device=self.device)
-        for name, coef in (("U_ss", USSC), ("U_pp", UPPC), ("g_ss", GSSC), ("g_sp", GSPC), ("g_pp", GPPC),
-                           ("g_p2", GP2C), ("h_sp", HSPC)):
-            g[:, COLUMNS.index(name)] = tab(coef)
+        for c, coef in self._eiso_coef():
+            g[:, c] = coef
         return g
 
     def eigenpairs(self, F, orb_off, evals, Q, eig_ws, fail):
@@ -558,16 +573,14 @@ class SCFEngine:
         f64 = dict(dtype=torch.float64, device=self.device)
         if eigh_pairs_ok(b.norb).all():
             fail = torch.zeros(1, dtype=torch.int32, device=self.device)
-            orb_off = torch.as_tensor(np.concatenate([[0], np.cumsum(b.norb)[:-1]]).astype(np.int64),
-                                      device=self.device)
             evals = torch.empty(int(b.norb.sum()), **f64)
             Q = torch.empty(max(b.total, 1), **f64)
-            self.eigenpairs(F, orb_off, evals, Q, evals, fail)
+            self.eigenpairs(F, self.orb_off, evals, Q, evals, fail)
             e = torch.empty(b.nmol, 4 * b.molsize, **f64)
             V = torch.empty(b.nmol, nmax, nmax, **f64)
-            nat.call("pyseqm_evec_view", b.L, b.molsize, nmax, nat.ptr(orb_off), nat.ptr(evals), nat.ptr(Q),
-                     nat.ptr(e), nat.ptr(V), self.stream)
-            if int((fail[0] + (~torch.isfinite(evals)).sum()).item()) == 0:
+            nat.call("pyseqm_evec_view", b.L, b.molsize, nmax, nat.ptr(self.orb_off), nat.ptr(evals),
+                     nat.ptr(Q), nat.ptr(e), nat.ptr(V), nat.ptr(fail), self.stream)
+            if int(fail.item()) == 0:
                 return e, V
         idx = torch.arange(b.nmol, dtype=torch.int32, device=self.device)
         Fp = torch.empty(b.nmol, nmax, nmax, **f64)

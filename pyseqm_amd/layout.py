@@ -325,31 +325,37 @@ class PackedBatch:
         return self.d["pair_ref"]
 
     def pair_base_device(self):
-        """Pairs before each molecule (int64) on the device, uploaded on first use."""
-        if "pair_base" not in self.d:
-            self.d["pair_base"] = torch.as_tensor(self.pair_base[:-1].copy(), dtype=torch.int64, device=self.device)
+        """Pairs before each molecule (int64) on the device."""
         return self.d["pair_base"]
 
     # ----------------------------------------------------------------- device
     def _to_device(self, device_tiles=False):
         dev = self.device
         i32 = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.int32, device=dev)
-        self.d = {
-            "mol_atom_off": i32(self.mol_atom_off), "mol_norb": i32(self.norb), "mol_nocc": i32(self.nocc),
-            "mol_mat_off": torch.as_tensor(self.mol_mat_off, dtype=torch.int64, device=dev),
-            "mol_tile_off": i32(self.mol_tile_off), "atom_mol": i32(self.atom_mol), "atom_ao": i32(self.atom_ao),
-            "atom_Z": i32(self.Z),
-        }
+        h32 = lambda a: np.asarray(a).astype(np.int32)
+        # per-molecule Fock build: its LDS slots and the launch order, heaviest molecule first
+        # (bytes of the build: 1184 per heavy-heavy pair, 176 heavy-H, 32 H-H, 240 per atom)
+        nh, nH = self.nheavy.astype(np.int64), self.nhydro.astype(np.int64)
+        work = 1184 * nh * (nh - 1) // 2 + 176 * nh * nH + 32 * nH * (nH - 1) // 2 + 240 * (nh + nH)
+        self.d = _native.upload(
+            dev, mol_atom_off=h32(self.mol_atom_off), mol_norb=h32(self.norb), mol_nocc=h32(self.nocc),
+            mol_mat_off=self.mol_mat_off.astype(np.int64), mol_tile_off=h32(self.mol_tile_off),
+            atom_mol=h32(self.atom_mol), atom_ao=h32(self.atom_ao), atom_Z=h32(self.Z), nheavy=h32(nh),
+            mol_order=h32(np.argsort(-work, kind="stable") if self.nmol else np.zeros(1)),
+            real_flat=self.real_flat.astype(np.int64), pair_base=self.pair_base[:-1].astype(np.int64))
         if device_tiles:
             nt = sum(self.ntile)
-            self.d["tiles"] = torch.zeros(max(4 * nt, 4), dtype=torch.int32, device=dev)
-            self.d["tile_woff"] = torch.zeros(max(nt, 1), dtype=torch.int64, device=dev)
-            self.d["csr_off"] = torch.zeros(self.natoms + 1, dtype=torch.int32, device=dev)
-            self.d["csr_idx"] = torch.zeros(max(self.nslots, 1), dtype=torch.int32, device=dev)
-            w_size = torch.zeros(3, dtype=torch.int64, device=dev)
+            sizes = dict(tile_woff=2 * max(nt, 1), w_size=6, tiles=max(4 * nt, 4), csr_off=self.natoms + 1,
+                         csr_idx=max(self.nslots, 1))  # in 32-bit words, 64-bit ones first
+            at = np.concatenate([[0], np.cumsum([-(-n // 4) * 4 for n in sizes.values()])])
+            words = torch.zeros(int(at[-1]), dtype=torch.int32, device=dev)
+            for o, (name, n) in zip(at, sizes.items()):
+                self.d[name] = words[int(o):int(o) + n]
+            self.d["tile_woff"] = self.d["tile_woff"].view(torch.int64)
+            w_size = self.d.pop("w_size").view(torch.int64)
             scratch = torch.empty(nt + (self.natoms + 1) // 2 + 1, dtype=torch.int64, device=dev)
             ntile = (ctypes.c_int * 3)(*self.ntile)
-            nheavy = i32(self.nheavy)
+            nheavy = self.d["nheavy"]
             _native.call_raw("pyseqm_build_tiles", self.nmol, self.natoms, _native.ptr(self.d["mol_atom_off"]),
                              _native.ptr(nheavy), _native.ptr(self.d["mol_tile_off"]), ntile,
                              _native.ptr(self.d["tiles"]), _native.ptr(self.d["tile_woff"]), _native.ptr(w_size),
@@ -376,11 +382,6 @@ class PackedBatch:
         for name in ("mol_atom_off", "mol_norb", "mol_nocc", "mol_mat_off", "mol_tile_off", "atom_mol",
                      "atom_ao", "atom_Z", "tiles", "csr_off", "csr_idx", "tile_woff"):
             setattr(L, name, self.d[name].data_ptr())
-        # per-molecule Fock build: its LDS slots and the launch order, heaviest molecule first
-        # (bytes of the build: 1184 per heavy-heavy pair, 176 heavy-H, 32 H-H, 240 per atom)
-        nh, nH = self.nheavy.astype(np.int64), self.nhydro.astype(np.int64)
-        work = 1184 * nh * (nh - 1) // 2 + 176 * nh * nH + 32 * nH * (nH - 1) // 2 + 240 * (nh + nH)
-        self.d["mol_order"] = i32(np.argsort(-work, kind="stable") if self.nmol else np.zeros(1, np.int64))
         L.max_mol_atoms = int(self.nat.max()) if self.nmol else 0
         L.max_mol_slots = int((10 * nh + nH).max()) if self.nmol else 0
         L.mol_order = self.d["mol_order"].data_ptr()
@@ -505,17 +506,21 @@ class PackedBatch:
         out[flat] = Xp[mm, rr, cc]
         return out
 
+    def _real_flat_on(self, device):
+        return self.d["real_flat"] if device == self.d["real_flat"].device else torch.as_tensor(self.real_flat,
+                                                                                                device=device)
+
     def atoms_from_padded(self, v):
         """(nmol, molsize, ...) reference layout -> per-atom (natoms, ...); (natoms, ...) passes through."""
         v = torch.as_tensor(v)
         if v.dim() >= 2 and tuple(v.shape[:2]) == (self.nmol, self.molsize) and not (
                 v.dim() == 2 and v.shape[0] == self.natoms):
-            return v.reshape((-1,) + tuple(v.shape[2:]))[torch.as_tensor(self.real_flat, device=v.device)]
+            return v.reshape((-1,) + tuple(v.shape[2:]))[self._real_flat_on(v.device)]
         return v
 
     def atom_to_padded(self, v, fill=0.0):
         """Per-atom (natoms, ...) -> (nmol, molsize, ...) in the reference's padded atom layout."""
         shape = (self.nmol * self.molsize,) + tuple(v.shape[1:])
         out = torch.full(shape, fill, dtype=v.dtype, device=v.device)
-        out[torch.as_tensor(self.real_flat, device=v.device)] = v
+        out[self._real_flat_on(v.device)] = v
         return out.reshape((self.nmol, self.molsize) + tuple(v.shape[1:]))

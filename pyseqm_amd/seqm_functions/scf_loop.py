@@ -35,11 +35,17 @@ def _check_pair_cutoff(molecule):
 
 def scf_loop(molecule, eps=1.0e-4, P=None, sp2=[False], scf_converger=[1], eig=False, scf_backward=0,
              scf_backward_eps=1.0e-2):
+    return run_scf(molecule, eps, P, sp2, scf_converger, eig, scf_backward, scf_backward_eps)[0]
+
+
+def run_scf(molecule, eps, P, sp2, scf_converger, eig, scf_backward, scf_backward_eps, enuc_pair=False):
+    """(scf_loop's 12-tuple, the energies of its density); enuc_pair: the integrals keep the per-pair core
+    repulsion too (eng.enuc_pair)."""
     if scf_backward not in (0, 1, 2):
         raise ValueError(f"scf_backward must be 0, 1 or 2 (got {scf_backward!r})")
     _check_pair_cutoff(molecule)
     eng = molecule.engine()
-    eng.set_coordinates(molecule.coordinates.detach())
+    eng.set_coordinates(molecule.coordinates.detach(), enuc_pair=enuc_pair)
     b = eng.b
     P0 = b.from_padded(P.detach().to(torch.float64)) if torch.is_tensor(P) else None
     eps = float(eps)
@@ -48,8 +54,8 @@ def scf_loop(molecule, eps=1.0e-4, P=None, sp2=[False], scf_converger=[1], eig=F
     r = eng.scf(eps=eps, converger=_converger(scf_converger), density=density, sp2_eps=sp2_eps, P=P0,
                 max_iter=MAX_ITER)
     nc = torch.as_tensor(r.notconverged, device=molecule.coordinates.device)
-    if nc.any():
-        nnot = int(nc.sum())
+    if r.notconverged.any():
+        nnot = int(r.notconverged.sum())
         warnings.warn("SCF for %d/%d molecules doesn't converge after %d iterations" % (nnot, b.nmol, MAX_ITER))
         if RAISE_ERROR_IF_SCF_FORWARD_FAILS:
             raise ValueError("SCF for some the molecules in the batch doesn't converge")
@@ -77,4 +83,4 @@ def scf_loop(molecule, eps=1.0e-4, P=None, sp2=[False], scf_converger=[1], eig=F
             out = SCFImplicit.apply(eng, r.P, en["F"], float(scf_backward_eps), r.notconverged,
                                     [n for n, _ in trained], Ppad, e, *[t for _, t in trained])
             Ppad, e = out if eig else (out, None)
-    return F, e, Ppad, Hcore, w, charge, rho0xi, rho0xj, None, None, nc, V
+    return (F, e, Ppad, Hcore, w, charge, rho0xi, rho0xj, None, None, nc, V), en
