@@ -380,6 +380,25 @@ int pyseqm_block_axpy(const pyseqm_layout_t* L, const int* idx, int nact, int nm
 int pyseqm_ksa_max_rank(void);
 int pyseqm_small_solve(const int* idx, int nact, int r, const double* O, const double* rhs, double* alpha,
                        void* stream);
+/* A Krylov vector of EnergyXL's rank-m fit (xlbomd.py:243-339) per listed molecule; V and W hold one packed batch
+ * per vector, `stride` doubles apart; O, rhs, alpha as for pyseqm_small_solve; k < pyseqm_ksa_max_rank().
+ * pyseqm_krylov_start: V_k from the residual (k == 0: D - P, also written to dDS; else W_{k-1}; D and P are read
+ *   for k == 0 only), modified Gram-Schmidt against V_0 .. V_{k-1}, normalised.
+ * pyseqm_krylov_fit: W_k (the response of V_k) -= V_k; row k of O and rhs; alpha of the first k + 1 responses.
+ * pyseqm_krylov_response: both from G = G(V_k): W_k = Q canon(Q^T G Q) Q^T (pyseqm_canon_prt) and the fit, for
+ *   blocks with pyseqm_krylov_response_ok(nmax, steps) (three blocks and the recursion's tables in LDS).
+ * pyseqm_krylov_combine: out = -sum_{i < r} alpha_i V_i. */
+int pyseqm_krylov_start(const pyseqm_layout_t* L, const int* idx, int nact, int k, const double* D, const double* P,
+                        double* dDS, double* V, const double* W, long long stride, void* stream);
+int pyseqm_krylov_fit(const pyseqm_layout_t* L, const int* idx, int nact, int k, const double* V, double* W,
+                      long long stride, const double* dDS, double* O, double* rhs, double* alpha, void* stream);
+int pyseqm_krylov_response_ok(int nmax, int steps);
+int pyseqm_krylov_response(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const long long* orb_off,
+                           const double* evals, const double* mu, double T, double kB, int steps, const double* Q,
+                           const double* G, int k, const double* V, double* W, long long stride, const double* dDS,
+                           double* O, double* rhs, double* alpha, void* stream);
+int pyseqm_krylov_combine(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, int r, const double* alpha,
+                          const double* V, long long stride, double* out, void* stream);
 
 /* ------------------------------------------------------------------ reference layouts
  * Views of the packed batch in the reference's padded layouts (rows of a molecule's 4 molsize x

@@ -53,6 +53,11 @@ _SIGS = {
     "pyseqm_block_gemm": [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
     "pyseqm_canon_prt": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_double, c_double, c_int, c_void_p,
                          c_void_p],
+    "pyseqm_krylov_start": [c_void_p, c_int, c_int] + [c_void_p] * 5 + [c_longlong, c_void_p],
+    "pyseqm_krylov_fit": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_longlong] + [c_void_p] * 5,
+    "pyseqm_krylov_response": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_double, c_double, c_int, c_void_p,
+                               c_void_p, c_int, c_void_p, c_void_p, c_longlong] + [c_void_p] * 5,
+    "pyseqm_krylov_combine": [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p],
     "pyseqm_block_dot": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
     "pyseqm_block_axpy": [c_void_p, c_int, c_int, c_int, c_double, c_void_p, c_int, c_void_p, c_void_p, c_void_p],
     "pyseqm_density_from_evecs": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p],
@@ -142,6 +147,8 @@ def lib():
         L.pyseqm_eigh_density_lds_ok.restype = c_int
         L.pyseqm_fermi_workspace.argtypes = [c_int]
         L.pyseqm_fermi_workspace.restype = c_longlong
+        L.pyseqm_krylov_response_ok.argtypes = [c_int, c_int]
+        L.pyseqm_krylov_response_ok.restype = c_int
         L.pyseqm_ksa_max_rank.argtypes = []
         L.pyseqm_ksa_max_rank.restype = c_int
         _lib = L
@@ -152,7 +159,7 @@ def exported_symbols():
     return list(_SIGS) + list(_RAW_SIGS) + ["pyseqm_fock_scratch_doubles", "pyseqm_param_grad_workspace",
                                             "pyseqm_eigh_density_workspace",
                                             "pyseqm_eigh_density_lds_ok", "pyseqm_fermi_workspace",
-                                            "pyseqm_ksa_max_rank"]
+                                            "pyseqm_krylov_response_ok", "pyseqm_ksa_max_rank"]
 
 
 def stream_ptr(device=None):

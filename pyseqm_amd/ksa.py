@@ -7,11 +7,12 @@ Per step, on the packed batch:
     Q, e = eigenpairs of F(P)                             (pyseqm_eigh_vectors)
     mu, f, D = 2 Q diag(f) Q^T, S                          (pyseqm_fermi_density)
     Krylov loop k = 0 .. rank-1 (while the fit's largest residual exceeds err_threshold):
-        V_k = W_{k-1} (W_{-1} = D - P), Gram-Schmidt against V_j, normalised   (block dot / axpy)
+        V_k = W_{k-1} (W_{-1} = D - P), Gram-Schmidt against V_j, normalised   (pyseqm_krylov_start)
         FO1 = G(V_k)                                     (the Fock kernels with H = 0)
-        W_k = Q canon(Q^T FO1 Q) Q^T - V_k               (block GEMMs, pyseqm_canon_prt)
-        alpha = argmin |sum_r alpha_r W_r - (D - P)|     (Frobenius products, pyseqm_small_solve)
-    dP2dt2 = -sum_r alpha_r V_r
+        W_k = Q canon(Q^T FO1 Q) Q^T - V_k               (pyseqm_krylov_response; larger blocks:
+                                                          block GEMMs, pyseqm_canon_prt)
+        alpha = argmin |sum_r alpha_r W_r - (D - P)|     (in the same launch, or pyseqm_krylov_fit)
+    dP2dt2 = -sum_r alpha_r V_r                          (pyseqm_krylov_combine)
 
 Every array stays on the device; with err_threshold <= 0 (the reference tests' setting) the loop
 length is fixed and nothing is read back.
@@ -24,7 +25,6 @@ from .engine import eigh_pairs_ok
 
 KB_EV = 8.61739e-5      # Boltzmann constant, eV/K (xlbomd.py:214)
 CANON_DM_PRT_ITER = 10  # recursion steps of Canon_DM_PRT in EnergyXL (xlbomd.py:55)
-K0 = 1.0                # xlbomd.py:248
 
 
 class KSAWorkspace:
@@ -45,6 +45,8 @@ class KSAWorkspace:
         f64 = dict(dtype=torch.float64, device=dev)
         total = max(b.total, 1)
         self.rank = int(rank)
+        # a whole response per launch where three blocks fit LDS (78 orbitals)
+        self.fused = bool(nat.lib().pyseqm_krylov_response_ok(int(norb.max()), CANON_DM_PRT_ITER))
         self.orb_off = torch.as_tensor(np.concatenate([[0], np.cumsum(norb)[:-1]]).astype(np.int64), device=dev)
         nsum = max(int(norb.sum()), 1)
         self.evals = torch.zeros(nsum, **f64)
@@ -122,43 +124,37 @@ def canon_response(eng, ks, FO1, out, T, kB=KB_EV, steps=CANON_DM_PRT_ITER):
     _gemm(eng, ks, 0, 1, ks.T1, ks.Q, out)       # (Q P1) Q^T
 
 
-def _fit(eng, ks, r):
-    """alpha = argmin over the first r responses: O alpha = rhs, O_ij = <W_i, W_j>, rhs_i = <W_i, D - P>."""
-    for i in range(r):
-        for j in range(r):
-            _dot(eng, ks, ks.W[i], ks.W[j], ks.dot)
-            ks.O[:, i, j].copy_(ks.dot)
-        _dot(eng, ks, ks.W[i], ks.dDS, ks.dot)
-        ks.rhs[:, i].copy_(ks.dot)
-    nat.call_raw("pyseqm_small_solve", nat.ptr(ks.idx), eng.b.nmol, int(r), nat.ptr(ks.O), nat.ptr(ks.rhs),
+def _response(eng, ks, k, T, kB, steps=CANON_DM_PRT_ITER):
+    """W_k = K0 (P1 - V_k) with P1 the response of V_k (its G in ks.G), and the fit over W_0 .. W_k."""
+    b = eng.b
+    stride = ks.V.stride(0)
+    if ks.fused:
+        nat.call("pyseqm_krylov_response", b.L, nat.ptr(ks.idx), b.nmol, int(b.nmax), nat.ptr(ks.orb_off),
+                 nat.ptr(ks.evals), nat.ptr(ks.mu), float(T), float(kB), int(steps), nat.ptr(ks.Q), nat.ptr(ks.G),
+                 k, nat.ptr(ks.V), nat.ptr(ks.W), stride, nat.ptr(ks.dDS), nat.ptr(ks.O), nat.ptr(ks.rhs),
                  nat.ptr(ks.alpha), eng.stream)
+        return
+    canon_response(eng, ks, ks.G, ks.W[k], T, kB, steps)
+    nat.call("pyseqm_krylov_fit", b.L, nat.ptr(ks.idx), b.nmol, k, nat.ptr(ks.V), nat.ptr(ks.W), stride,
+             nat.ptr(ks.dDS), nat.ptr(ks.O), nat.ptr(ks.rhs), nat.ptr(ks.alpha), eng.stream)
 
 
 def rank_kernel(eng, ks, D, P, T, err_threshold, dP2dt2, kB=KB_EV):
-    """The rank-m Krylov approximation dP2dt2 = -sum_r alpha_r V_r of EnergyXL (xlbomd.py:243-339)."""
-    R = ks.R
-    ks.dDS.copy_(D)
-    _axpy(eng, ks, 4, -K0, None, 0, P, ks.dDS)   # K0 (D - P), K0 = 1
-    dW = ks.dDS
+    """The rank-m Krylov approximation dP2dt2 = -sum_r alpha_r V_r of EnergyXL (xlbomd.py:243-339), with
+    K0 = 1 (xlbomd.py:248)."""
+    R, b = ks.R, eng.b
+    stride = ks.V.stride(0)
     k = -1
     err = None
-    if err_threshold > 0.0:
-        _dot(eng, ks, ks.dDS, ks.dDS, ks.nrm)
     while k < ks.rank - 1:
         k += 1
-        Vk = ks.V[k]
-        Vk.copy_(dW)
-        for j in range(k):  # modified Gram-Schmidt in the Frobenius product
-            _dot(eng, ks, Vk, ks.V[j], ks.dot)
-            _axpy(eng, ks, 0, -1.0, ks.dot, 1, ks.V[j], Vk)
-        _dot(eng, ks, Vk, Vk, ks.dot)
-        _axpy(eng, ks, 1, 1.0, ks.dot, 1, None, Vk)
-        g_matrix(eng, ks, Vk, ks.G)
-        canon_response(eng, ks, ks.G, ks.W[k], T, kB)
-        _axpy(eng, ks, 2, K0, None, 0, Vk, ks.W[k])  # W_k = K0 (P1 - V_k)
-        dW = ks.W[k]
-        _fit(eng, ks, k + 1)
+        nat.call("pyseqm_krylov_start", b.L, nat.ptr(ks.idx), b.nmol, k, nat.ptr(D), nat.ptr(P), nat.ptr(ks.dDS),
+                 nat.ptr(ks.V), nat.ptr(ks.W), stride, eng.stream)
+        g_matrix(eng, ks, ks.V[k], ks.G)
+        _response(eng, ks, k, T, kB)
         if err_threshold > 0.0:
+            if k == 0:
+                _dot(eng, ks, ks.dDS, ks.dDS, ks.nrm)
             _axpy(eng, ks, 3, 1.0, ks.alpha[:, 0], R, ks.W[0], ks.res)
             for r in range(1, k + 1):
                 _axpy(eng, ks, 0, 1.0, ks.alpha[:, r], R, ks.W[r], ks.res)
@@ -167,10 +163,8 @@ def rank_kernel(eng, ks, D, P, T, err_threshold, dP2dt2, kB=KB_EV):
             err = torch.sqrt(ks.dot / ks.nrm)
             if float(err.max()) <= err_threshold:  # the reference's loop test (host read only here)
                 break
-    # dP2dt2 = -sum_r alpha_r V_r with the last fit
-    _axpy(eng, ks, 3, -1.0, ks.alpha[:, 0], R, ks.V[0], dP2dt2)
-    for r in range(1, k + 1):
-        _axpy(eng, ks, 0, -1.0, ks.alpha[:, r], R, ks.V[r], dP2dt2)
+    nat.call("pyseqm_krylov_combine", b.L, nat.ptr(ks.idx), b.nmol, int(b.nmax), k + 1, nat.ptr(ks.alpha),
+             nat.ptr(ks.V), stride, nat.ptr(dP2dt2), eng.stream)
     ks.last_error = err
     ks.last_rank = k + 1
     return dP2dt2

@@ -116,9 +116,7 @@ class XLTrajectories:
         D, c = self.D, MIX_C
         if self.ksa and self.ksa["propagate"]:
             # KSA_XL_BOMD._propagate_P: kappa (dP2dt2 + P) + the history terms
-            from .ksa import _axpy
-            self.tmp.copy_(self.P)
-            _axpy(self.eng, self.ks, 4, 1.0, None, 0, self.dP2dt2, self.tmp)
+            torch.add(self.P, self.dP2dt2, out=self.tmp)
             D, c = self.tmp, 1.0
         nat.call_raw("pyseqm_xl_propagate", self.eng.b.total, nat.ptr(D), nat.ptr(self.P), nat.ptr(self.Pt),
                      self.Pt.shape[1], self.m, coef, self.coeff_D, c, self.m - 1 - cindx, self.eng.stream)
