@@ -48,17 +48,15 @@ __device__ inline void ld_tri10(const double* p, int n, double (&v)[10]) {
   v[9] = r3b[1];
 }
 
-// Heavy-H and H-H tiles, one wave per tile (heavy-heavy tiles: k_fock_xx2 below).
+// A heavy-H or H-H tile by one wave (heavy-heavy tiles: fock_xx_tile below).
 template <int KIND>
-__global__ __launch_bounds__(64) void k_fock_tiles(pyseqm_layout_t L, int tile_base, const double* __restrict__ w,
-                                                    const double* __restrict__ P, const double* __restrict__ H,
-                                                    double* __restrict__ F, double* __restrict__ part,
-                                                    double* __restrict__ etile,
-                                                    const unsigned char* __restrict__ active) {
-  static_assert(KIND == XH || KIND == HH, "heavy-heavy tiles run in k_fock_xx2");
-  const int tl = xcd_run(blockIdx.x, gridDim.x);
-  const int tile = tile_base + tl;
-  const int lane = threadIdx.x;
+__device__ __forceinline__ void fock_small_tile(const pyseqm_layout_t& L, int tile, const double* __restrict__ w,
+                                                const double* __restrict__ P, const double* __restrict__ H,
+                                                double* __restrict__ F, double* __restrict__ part,
+                                                double* __restrict__ etile,
+                                                const unsigned char* __restrict__ active) {
+  static_assert(KIND == XH || KIND == HH, "heavy-heavy tiles take two waves");
+  const int lane = threadIdx.x & 63;
   const Tile t = load_tile(L.tiles, tile);
   if (active && !active[t.mol]) return;  // uniform over the wave
   int i, j;
@@ -134,7 +132,7 @@ __global__ __launch_bounds__(64) void k_fock_tiles(pyseqm_layout_t L, int tile_b
   if (lane == 0) etile[tile] = es;
 }
 
-// The integral contraction of k_fock_xx2 for the (mu nu) pairs k = K0 .. K0+4 (static indices).
+// The integral contraction of fock_xx_tile for the (mu nu) pairs k = K0 .. K0+4 (static indices).
 template <int K0>
 __device__ inline void xx_half(const double* __restrict__ wt, int S, const double* Pm, int n, int ai, int aj,
                                const double (&pab)[4][4], double (&rowv)[5], double (&colv)[10], double (&K)[4][4]) {
@@ -166,18 +164,17 @@ __device__ inline void xx_half(const double* __restrict__ wt, int S, const doubl
   }
 }
 
-// Heavy-heavy tiles with two waves per tile: wave q contracts the integrals (kl) with k in its half
+// A heavy-heavy tile by the two waves of a workgroup: wave q contracts the integrals (kl) with k in its half
 // of the 10 (mu nu) pairs, so each wave streams 50 of the 100 integral columns; wave 1 hands its
 // partial Coulomb column sums, exchange block and row sums to wave 0 through LDS, and wave 0 writes
 // F, the tile partials and the energy.  Per pair: exchange block K from the 4 x 4 off-diagonal P
 // block, Coulomb row / column sums from the packed diagonal blocks of P (off-diagonal pairs doubled).
-__global__ __launch_bounds__(128) void k_fock_xx2(pyseqm_layout_t L, const double* __restrict__ w,
-                                                  const double* __restrict__ P, const double* __restrict__ H,
-                                                  double* __restrict__ F, double* __restrict__ part,
-                                                  double* __restrict__ etile,
-                                                  const unsigned char* __restrict__ active) {
+__device__ __forceinline__ void fock_xx_tile(const pyseqm_layout_t& L, int tile, const double* __restrict__ w,
+                                             const double* __restrict__ P, const double* __restrict__ H,
+                                             double* __restrict__ F, double* __restrict__ part,
+                                             double* __restrict__ etile,
+                                             const unsigned char* __restrict__ active) {
   __shared__ double xch[31][64];
-  const int tile = xcd_run(blockIdx.x, gridDim.x);
   const int q = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   const Tile t = load_tile(L.tiles, tile);
@@ -264,6 +261,34 @@ __global__ __launch_bounds__(128) void k_fock_xx2(pyseqm_layout_t L, const doubl
   write_partials_c(part, L, tile, lane, row10, colv);
   const double es = wave64(e);  // every lane active here
   if (lane == 0) etile[tile] = es;
+}
+
+// Every pair tile in one launch: a workgroup of two waves takes a heavy-heavy tile, or two heavy-H or H-H tiles, a
+// wave each, in that order of block ids, so that the light tiles fill the end of the heavy ones.  Each kind
+// keeps its own runs of neighbouring tiles per XCD.  As a launch per kind each waited out the last tiles of
+// the one before: 1024 alkanes of 2-30 carbons 121 -> 112 us, 8 clusters of 256 waters 151 -> 145.
+__global__ __launch_bounds__(128) void k_fock_pairs(pyseqm_layout_t L, const double* __restrict__ w_xx,
+                                                    const double* __restrict__ w_xh,
+                                                    const double* __restrict__ w_hh, const double* __restrict__ P,
+                                                    const double* __restrict__ H, double* __restrict__ F,
+                                                    double* __restrict__ part, double* __restrict__ etile,
+                                                    const unsigned char* __restrict__ active) {
+  const int nx = L.ntile[0], nh = (L.ntile[1] + 1) / 2, nhh = (L.ntile[2] + 1) / 2;
+  int b = blockIdx.x;
+  if (b < nx) {
+    fock_xx_tile(L, xcd_run(b, nx), w_xx, P, H, F, part, etile, active);
+    return;
+  }
+  b -= nx;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (b < nh) {
+    const int tl = 2 * xcd_run(b, nh) + wave;
+    if (tl < L.ntile[1]) fock_small_tile<XH>(L, nx + tl, w_xh, P, H, F, part, etile, active);
+    return;
+  }
+  b -= nh;
+  const int tl = 2 * xcd_run(b, nhh) + wave;
+  if (tl < L.ntile[2]) fock_small_tile<HH>(L, nx + L.ntile[1] + tl, w_hh, P, H, F, part, etile, active);
 }
 
 // One-center G(P_ii) of a heavy atom (fock.py:196-224) added to acc, which holds H_ii plus the
@@ -814,12 +839,8 @@ int launch_fock(const pyseqm_layout_t* L, const double* atom_par, const double* 
         *L, atom_par, w_xx, w_xh, w_hh, P, H, F, eelec, active, stride);
     return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
   }
-  int base = 0;
-  if (L->ntile[0]) k_fock_xx2<<<L->ntile[0], 128, 0, s>>>(*L, w_xx, P, H, F, part, etile, active);
-  base += L->ntile[0];
-  if (L->ntile[1]) k_fock_tiles<XH><<<L->ntile[1], 64, 0, s>>>(*L, base, w_xh, P, H, F, part, etile, active);
-  base += L->ntile[1];
-  if (L->ntile[2]) k_fock_tiles<HH><<<L->ntile[2], 64, 0, s>>>(*L, base, w_hh, P, H, F, part, etile, active);
+  const int blocks = L->ntile[0] + (L->ntile[1] + 1) / 2 + (L->ntile[2] + 1) / 2;
+  if (blocks) k_fock_pairs<<<blocks, 128, 0, s>>>(*L, w_xx, w_xh, w_hh, P, H, F, part, etile, active);
   if (L->natoms) {
     if (lanes_per_atom(L) == 64)
       k_fock_diag<64><<<(L->natoms + 3) / 4, 256, 0, s>>>(*L, atom_par, P, H, part, F, eatom, active);
