@@ -833,7 +833,10 @@ __global__ __launch_bounds__(64) void k_sp2_decide(const int* __restrict__ idx, 
 // C = A * B for symmetric B (B is read by rows, B[k][j] = B[j][k]); A read by rows.  Per active
 // molecule, square n x n, row-major with leading dimension n (packed layout) or ld (SP2 layout).
 // Tile DT x DT per 256-thread block (4 waves as 2x2), v_mfma_f64_16x16x4_f64, K slab 16 staged
-// through registers (prefetched during the MFMAs of the previous slab) and LDS.
+// through registers (prefetched during the MFMAs of the previous slab) and LDS.  What bounds it: the matrix
+// units, and how evenly the tiles fill 256 CUs.  Tiles of 64 at every size: with tiles of 128 above 256 orbitals
+// X^2 of 8 blocks of 1536 had 624 tiles, at two blocks a CU and 128 registers of sums a lane: 906 us, 593
+// with 2400 tiles of 64 (51 of the 73 TFLOP/s a large FP64 product reaches); one block of 300 to 3000: 1.4 to 2.5 times.
 // mode bit 0: McWeeny epilogue C <- 2 (3 A - 2 A B) (A = X^2, B = X); bit 1: the product is known
 // to be symmetric (X^2, X^2 X): only tiles ti <= tj are computed and mirrored.
 // AX / BX: the A / B operand is the final FP32 SP2 matrix X of each molecule (buffer Xa or Xb by
@@ -841,17 +844,19 @@ __global__ __launch_bounds__(64) void k_sp2_decide(const int* __restrict__ idx, 
 // to the packed layout (offset coff[m], leading dimension n) instead of the operands' layout.
 // DOUT (with AX, symmetric mode): the McWeeny first half; C = X^2 is written on the upper-triangle
 // tiles only, and D = C - X (FP32, both triangles) into the SP2 buffer that does not hold X.
+constexpr int kDgemmTile = 64;
 template <typename T>
 __device__ inline double ld64(const T* p) {
   return (double)*p;
 }
-template <int DT, bool AX, bool BX, bool CPACK, bool DOUT = false>
+template <bool AX, bool BX, bool CPACK, bool DOUT = false>
 __global__ __launch_bounds__(256, 2) void k_dgemm_sym(const int* __restrict__ idx, const int* __restrict__ norb,
                                                    const long long* __restrict__ off, const int* __restrict__ lds,
                                                    const double* __restrict__ A, const double* __restrict__ B,
                                                    double* __restrict__ C, int mode, int ntile_side,
                                                    float* Xa, float* Xb, const double* __restrict__ st,
                                                    const long long* __restrict__ coff) {
+  constexpr int DT = kDgemmTile;
   constexpr int WT = DT / 2;    // per-wave tile edge
   constexpr int NB = WT / 16;   // 16x16 MFMA blocks per wave side
   constexpr int NQ = DT * 16 / 256;
@@ -1080,15 +1085,9 @@ extern "C" int pyseqm_dgemm_sym(const pyseqm_layout_t* L, const int* idx, int na
   if (nact == 0) return PYSEQM_OK;
   hipStream_t s = (hipStream_t)stream;
   const bool symout = (mode & 2) != 0;
-  if (nmax <= 256) {
-    const int nt = (nmax + 63) / 64;
-    k_dgemm_sym<64, false, false, false><<<dim3(symout ? nt * (nt + 1) / 2 : nt * nt, nact), 256, 0, s>>>(
-        idx, L->mol_norb, off, lds, A, B, C, mode, nt, nullptr, nullptr, nullptr, nullptr);
-  } else {
-    const int nt = (nmax + 127) / 128;
-    k_dgemm_sym<128, false, false, false><<<dim3(symout ? nt * (nt + 1) / 2 : nt * nt, nact), 256, 0, s>>>(
-        idx, L->mol_norb, off, lds, A, B, C, mode, nt, nullptr, nullptr, nullptr, nullptr);
-  }
+  const int nt = (nmax + kDgemmTile - 1) / kDgemmTile;
+  k_dgemm_sym<false, false, false><<<dim3(symout ? nt * (nt + 1) / 2 : nt * nt, nact), 256, 0, s>>>(
+      idx, L->mol_norb, off, lds, A, B, C, mode, nt, nullptr, nullptr, nullptr, nullptr);
   return st_ok();
 }
 
@@ -1101,8 +1100,9 @@ static void launch_mcweeny(const pyseqm_layout_t* L, const int* idx, int nact, i
                            hipStream_t s) {
   const int nt = (nmax + DT - 1) / DT;
   const int ntri = nt * (nt + 1) / 2;
-  k_dgemm_sym<DT, true, true, false, true><<<dim3(ntri, nact), 256, 0, s>>>(
-      idx, L->mol_norb, xoff, xld, nullptr, nullptr, Y2, 2, nt, Xa, Xb, state, nullptr);
+  const int ntd = (nmax + kDgemmTile - 1) / kDgemmTile;
+  k_dgemm_sym<true, true, false, true><<<dim3(ntd * (ntd + 1) / 2, nact), 256, 0, s>>>(
+      idx, L->mol_norb, xoff, xld, nullptr, nullptr, Y2, 2, ntd, Xa, Xb, state, nullptr);
   k_mcw_bf16x3<DT><<<8 * ((nact * ntri + 7) / 8), 256, 0, s>>>(idx, nact, ntri, L->mol_norb, xoff, xld, Xa, Xb,
                                                                 state, Y2, L->mol_mat_off, P);
 }
