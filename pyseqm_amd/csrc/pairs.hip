@@ -13,6 +13,8 @@
 // fixed order (deterministic, no atomics).
 #include "common.h"
 
+#include <type_traits>
+
 using namespace pyseqm;
 
 namespace {
@@ -615,15 +617,39 @@ __device__ inline void core_block(const PairGeom& g, const double* pi, const dou
 
 // ------------------------------------------------------------------- tile kernels
 
+// The kernels over pair tiles come per kind of tile (first tile tile_base, its integrals or nothing in w) and as
+// ALL: one launch over the three kinds in that order.  A launch per kind lets light tiles run at their own
+// register count (up to 8 waves per SIMD, heavy-heavy ones 1); where all tiles fit the chip about at once
+// the launches only wait for each other.  Integrals and forces (us, per kind -> ALL) of n alkanes of 2-30 carbons:
+// n = 1 38.6 -> 25.0 and 28.7 -> 17.0; 64 (2116 tiles) 52.5 -> 31.1 and 36.5 -> 21.3; 128 (4270) 55.1 -> 47.5 and
+// 39.7 -> 35.0; 256 (8548) 91.7 -> 83.5 and 66.7 -> 63.6; 512 (17110) 137 -> 149 and 102 -> 119: ALL up to 8192.
+constexpr int ALL = 3;
+constexpr int kMergeTiles = 8192;
+inline bool merge_kinds(const pyseqm_layout_t* L) {
+  return (long long)L->ntile[0] + L->ntile[1] + L->ntile[2] <= kMergeTiles;
+}
+// f(kind as a constant, tile) for this block's tile
+template <int KIND, class Fn>
+__device__ __forceinline__ void for_tile(const pyseqm_layout_t& L, int tile_base, Fn f) {
+  if constexpr (KIND != ALL) {
+    f(std::integral_constant<int, KIND>(), tile_base + xcd_run(blockIdx.x, gridDim.x));
+  } else {
+    const int n0 = L.ntile[0], n1 = L.ntile[1], n2 = L.ntile[2], b = blockIdx.x;
+    if (b < n0)
+      f(std::integral_constant<int, XX>(), xcd_run(b, n0));
+    else if (b < n0 + n1)
+      f(std::integral_constant<int, XH>(), n0 + xcd_run(b - n0, n1));
+    else
+      f(std::integral_constant<int, HH>(), n0 + n1 + xcd_run(b - n0 - n1, n2));
+  }
+}
+
 template <int KIND>
-__global__ __launch_bounds__(64) void k_pair_tiles(pyseqm_layout_t L, int method, int tile_base,
-                                                    const double* __restrict__ coords,
-                                                    const double* __restrict__ par, double* __restrict__ wout,
-                                                    double* __restrict__ H, double* __restrict__ part,
-                                                    double* __restrict__ enuc_tile,
-                                                    double* __restrict__ enuc_pair,
-                                                    const int* __restrict__ pair_ref) {
-  const int tile = tile_base + xcd_run(blockIdx.x, gridDim.x);
+__device__ __forceinline__ void pair_tile(const pyseqm_layout_t& L, int method, int tile,
+                                          const double* __restrict__ coords, const double* __restrict__ par,
+                                          double* __restrict__ wout, double* __restrict__ H,
+                                          double* __restrict__ part, double* __restrict__ enuc_tile,
+                                          double* __restrict__ enuc_pair, const int* __restrict__ pair_ref) {
   const int lane = threadIdx.x;
   const Tile t = load_tile(L.tiles, tile);
   int i, j;
@@ -687,6 +713,21 @@ __global__ __launch_bounds__(64) void k_pair_tiles(pyseqm_layout_t L, int method
   write_partials_c(part, L, tile, lane, rowv, colv);
   const double es = wave64(en);  // every lane active here
   if (lane == 0) enuc_tile[tile] = es;
+}
+
+template <int KIND>
+__global__ __launch_bounds__(64) void k_pair_tiles(pyseqm_layout_t L, int method, int tile_base,
+                                                   const double* __restrict__ coords,
+                                                   const double* __restrict__ par, double* __restrict__ w_xx,
+                                                   double* __restrict__ w_xh, double* __restrict__ w_hh,
+                                                   double* __restrict__ H, double* __restrict__ part,
+                                                   double* __restrict__ enuc_tile, double* __restrict__ enuc_pair,
+                                                   const int* __restrict__ pair_ref) {
+  for_tile<KIND>(L, tile_base, [&](auto kind, int tile) {
+    constexpr int K = decltype(kind)::value;
+    pair_tile<K>(L, method, tile, coords, par, K == XX ? w_xx : (K == XH ? w_xh : w_hh), H, part, enuc_tile, enuc_pair,
+                 pair_ref);
+  });
 }
 
 // Hellmann-Feynman pair energy at fixed density: the part of 0.5 sum P (H + F) + E_nuc that
@@ -978,11 +1019,10 @@ __device__ inline void pair_gradient(int method, const double (&R0)[3], const do
 // Forces: +dE/dR on atom i, -dE/dR on atom j, reduced per tile.
 // XL: Dm is the density contracted with H (the XL-BOMD D), P the propagated field.
 template <int KIND, bool XL>
-__global__ __launch_bounds__(64) void k_pair_forces(pyseqm_layout_t L, int method, int tile_base,
-                                                     const double* __restrict__ coords,
-                                                     const double* __restrict__ par, const double* __restrict__ P,
-                                                     const double* __restrict__ Dm, double* __restrict__ part) {
-  const int tile = tile_base + xcd_run(blockIdx.x, gridDim.x);
+__device__ __forceinline__ void force_tile(const pyseqm_layout_t& L, int method, int tile,
+                                           const double* __restrict__ coords, const double* __restrict__ par,
+                                           const double* __restrict__ P, const double* __restrict__ Dm,
+                                           double* __restrict__ part) {
   const int lane = threadIdx.x;
   const Tile t = load_tile(L.tiles, tile);
   int i, j;
@@ -1006,6 +1046,16 @@ __global__ __launch_bounds__(64) void k_pair_forces(pyseqm_layout_t L, int metho
     for (int x = 0; x < 3; ++x) colv[x] = -rowv[x];
   }
   write_partials(part, tile, lane, rowv, colv);
+}
+
+template <int KIND, bool XL>
+__global__ __launch_bounds__(64) void k_pair_forces(pyseqm_layout_t L, int method, int tile_base,
+                                                    const double* __restrict__ coords,
+                                                    const double* __restrict__ par, const double* __restrict__ P,
+                                                    const double* __restrict__ Dm, double* __restrict__ part) {
+  for_tile<KIND>(L, tile_base, [&](auto kind, int tile) {
+    force_tile<decltype(kind)::value, XL>(L, method, tile, coords, par, P, Dm, part);
+  });
 }
 
 template <int G>
@@ -1591,15 +1641,15 @@ int launch_pair_forces(const pyseqm_layout_t* L, int method, const double* coord
                        const double* P, const double* D, double h, double* part, double* forces, void* stream) {
   if (!L || method < PYSEQM_MNDO || method > PYSEQM_PM3 || !(h > 0.0)) return PYSEQM_EINVAL;
   hipStream_t s = (hipStream_t)stream;
-  int base = 0;
-  if (L->ntile[0])
-    k_pair_forces<XX, XL><<<L->ntile[0], 64, 0, s>>>(*L, method, base, coords, atom_par, P, D, part);
-  base += L->ntile[0];
-  if (L->ntile[1])
-    k_pair_forces<XH, XL><<<L->ntile[1], 64, 0, s>>>(*L, method, base, coords, atom_par, P, D, part);
-  base += L->ntile[1];
-  if (L->ntile[2])
-    k_pair_forces<HH, XL><<<L->ntile[2], 64, 0, s>>>(*L, method, base, coords, atom_par, P, D, part);
+  const int n0 = L->ntile[0], n1 = L->ntile[1], n2 = L->ntile[2];
+  if (merge_kinds(L)) {
+    if (n0 + n1 + n2)
+      k_pair_forces<ALL, XL><<<n0 + n1 + n2, 64, 0, s>>>(*L, method, 0, coords, atom_par, P, D, part);
+  } else {
+    if (n0) k_pair_forces<XX, XL><<<n0, 64, 0, s>>>(*L, method, 0, coords, atom_par, P, D, part);
+    if (n1) k_pair_forces<XH, XL><<<n1, 64, 0, s>>>(*L, method, n0, coords, atom_par, P, D, part);
+    if (n2) k_pair_forces<HH, XL><<<n2, 64, 0, s>>>(*L, method, n0 + n1, coords, atom_par, P, D, part);
+  }
   if (L->natoms) {
     if (lanes_per_atom(L) == 64)
       k_atom_forces<64><<<(L->natoms + 3) / 4, 256, 0, s>>>(*L, part, forces);
@@ -1686,18 +1736,19 @@ extern "C" int pyseqm_pair_integrals(const pyseqm_layout_t* L, int method, const
   if (!L || method < PYSEQM_MNDO || method > PYSEQM_PM3) return PYSEQM_EINVAL;
   if (enuc_pair && !pair_ref) return PYSEQM_EINVAL;
   hipStream_t s = (hipStream_t)stream;
-  int base = 0;
-  if (L->ntile[0])
-    k_pair_tiles<XX><<<L->ntile[0], 64, 0, s>>>(*L, method, base, coords, atom_par, w_xx, H, part, enuc_tile,
-                                                enuc_pair, pair_ref);
-  base += L->ntile[0];
-  if (L->ntile[1])
-    k_pair_tiles<XH><<<L->ntile[1], 64, 0, s>>>(*L, method, base, coords, atom_par, w_xh, H, part, enuc_tile,
-                                                enuc_pair, pair_ref);
-  base += L->ntile[1];
-  if (L->ntile[2])
-    k_pair_tiles<HH><<<L->ntile[2], 64, 0, s>>>(*L, method, base, coords, atom_par, w_hh, H, part, enuc_tile,
-                                                enuc_pair, pair_ref);
+  const int n0 = L->ntile[0], n1 = L->ntile[1], n2 = L->ntile[2];
+  auto launch = [&](auto kind, int count, int base) {
+    if (count)
+      k_pair_tiles<decltype(kind)::value><<<count, 64, 0, s>>>(*L, method, base, coords, atom_par, w_xx, w_xh, w_hh, H,
+                                                               part, enuc_tile, enuc_pair, pair_ref);
+  };
+  if (merge_kinds(L)) {
+    launch(std::integral_constant<int, ALL>(), n0 + n1 + n2, 0);
+  } else {
+    launch(std::integral_constant<int, XX>(), n0, 0);
+    launch(std::integral_constant<int, XH>(), n1, n0);
+    launch(std::integral_constant<int, HH>(), n2, n0 + n1);
+  }
   if (L->natoms) {
     if (lanes_per_atom(L) == 64)
       k_hcore_diag<64><<<(L->natoms + 3) / 4, 256, 0, s>>>(*L, atom_par, part, H);
