@@ -76,14 +76,18 @@ __global__ void k_gersh(pyseqm_layout_t L, const double* __restrict__ F, const i
 }
 
 __device__ inline void gersh_bounds(const double* red, int k, int nb, double* sh2) {
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 64) {  // one wave: a thread alone waits for each of up to 256 pairs
     double a = -1.0e300, b = 1.0e300;
-    for (int q = 0; q < nb; ++q) {
+    for (int q = threadIdx.x; q < nb; q += 64) {
       a = fmax(a, red[((size_t)k * nb + q) * 4]);
       b = fmin(b, red[((size_t)k * nb + q) * 4 + 1]);
     }
-    sh2[0] = a;
-    sh2[1] = b;
+    a = wmax(a);
+    b = -wmax(-b);
+    if (threadIdx.x == 0) {
+      sh2[0] = a;
+      sh2[1] = b;
+    }
   }
   __syncthreads();
 }
@@ -128,17 +132,20 @@ __global__ void k_sp2_x0(pyseqm_layout_t L, const double* __restrict__ F, const 
   }
 }
 
-// Pass 3: per-molecule SP2 state (fixed-order sums of the partials).
-__global__ void k_sp2_state0(const int* __restrict__ idx, int nact, int nb, const int* __restrict__ nocc,
-                             const double* __restrict__ red, double* __restrict__ st) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nact) return;
+// Pass 3: per-molecule SP2 state, one wave per molecule (fixed-order sums of the partials).  One thread per
+// molecule took 33 us for 8 blocks of 1536 orbitals, this 4.7.
+__global__ __launch_bounds__(64) void k_sp2_state0(const int* __restrict__ idx, int nb, const int* __restrict__ nocc,
+                                                   const double* __restrict__ red, double* __restrict__ st) {
+  const int k = blockIdx.x;
   const int m = idx[k];
   double t = 0.0, f = 0.0;
-  for (int q = 0; q < nb; ++q) {
+  for (int q = threadIdx.x; q < nb; q += 64) {
     t += red[((size_t)k * nb + q) * 4 + 2];
     f += red[((size_t)k * nb + q) * 4 + 3];
   }
+  t = wsum(t);
+  f = wsum(f);
+  if (threadIdx.x != 0) return;
   double* s = st + (size_t)m * S_NST;
   const double N = nocc[m];
   s[S_TR] = t;
@@ -987,7 +994,7 @@ extern "C" int pyseqm_sp2_init(const pyseqm_layout_t* L, const double* F, const 
   hipStream_t s = (hipStream_t)stream;
   k_gersh<<<dim3(nb, nact), 256, 0, s>>>(*L, F, idx, nb, red);
   k_sp2_x0<<<dim3(nb, nact), 256, 0, s>>>(*L, F, idx, nb, xoff, xld, X, red);
-  k_sp2_state0<<<(nact + 63) / 64, 64, 0, s>>>(idx, nact, nb, L->mol_nocc, red, state);
+  k_sp2_state0<<<nact, 64, 0, s>>>(idx, nb, L->mol_nocc, red, state);
   return st_ok();
 }
 

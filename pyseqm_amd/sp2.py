@@ -32,7 +32,7 @@ class SP2Workspace:
         self.xld = torch.as_tensor(ld.astype(np.int32), device=dev)
         self.Xa = torch.zeros(max(self.xtotal, 1), dtype=torch.float32, device=dev)
         self.Xb = torch.zeros_like(self.Xa)
-        self.Y2 = torch.zeros(max(self.xtotal, 1), dtype=torch.float64, device=dev)  # McWeeny X^2
+        self.Y2 = torch.empty(max(self.xtotal, 1), dtype=torch.float64, device=dev)  # McWeeny X^2, written before read
         self.state = torch.zeros(b.nmol, NSTATE, dtype=torch.float64, device=dev)
         # per-tile (trace, Frobenius) partials; sized for the 64 x 64 tiles (the 128 x 128 tiles
         # used for large blocks need fewer)
