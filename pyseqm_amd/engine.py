@@ -45,6 +45,7 @@ MIXED_DIIS_MIN_N = 256
 EIGH_WG_MAX_N = 192
 EIGH_WG_LDS_DOUBLES = 20480
 EIGH_WG_CLASSES = (48, 96, 192)
+NUM_CU = 256  # compute units of an MI355X: the blocks of one workgroup each that run at once
 
 
 def eigh_wg_lds(norb, nvec):
@@ -525,7 +526,7 @@ class SCFEngine:
         """Every eigenpair of every block of F: Q in the packed layout (column j = eigenvector j,
         ascending eigenvalues) and evals[orb_off[m] + j].  Blocks of up to EIGH_WG_MAX_N orbitals take
         pyseqm_eigh_vectors, in one launch for those whose vectors fit its LDS (at most 139 orbitals) and
-        one for the others; larger ones the batched library eigensolver on Gershgorin-padded stacks per
+        one for the others, or in one for all where every block has a CU of its own; larger ones the batched library eigensolver on Gershgorin-padded stacks per
         size group, scattered into the same layout.  eig_ws holds 4 nmol n^2 doubles for the n of the
         workgroup blocks (allocated here where it is smaller); fail counts vectors the workgroup solver
         lost (read by the caller)."""
@@ -533,6 +534,10 @@ class SCFEngine:
         norb = np.asarray(b.norb)
         wg = eigh_pairs_ok(norb)
         in_lds = eigh_wg_ok(norb, norb)
+        if int(wg.sum()) <= NUM_CU and not in_lds[wg].all():
+            # the small blocks run beside the large ones (128 alkanes of 14-182 orbitals: a launch each took
+            # 0.72 and 0.44 ms, one for all 0.72)
+            in_lds = np.zeros_like(in_lds)
         for ids in (np.nonzero(wg & ~in_lds)[0], np.nonzero(in_lds)[0]):
             if len(ids) == 0:
                 continue
