@@ -694,9 +694,10 @@ __device__ __forceinline__ void back_panels(doublex4 (&Cr)[S / 16], const double
 // EVEC = false: the density P = 2 C_occ C_occ^T of the nocc lowest vectors.  EVEC = true: every
 // eigenpair (nv = n vectors), written as Qout (packed layout, column j = eigenvector j) and evals
 // (orb_off[m] + j, the Rayleigh quotients of the final vectors: exact to rounding whatever the
-// multisection bracket width).  GZ (with EVEC): the vectors stand in Qout itself instead of LDS, for
-// blocks whose n x n vectors do not fit (140 to 192 orbitals): rows are read ahead of their use in every
-// sweep, and lanes run along a row, so the L2 serves them.
+// multisection bracket width).  GZ: the vectors stand in memory instead of LDS, for blocks whose vectors do not
+// fit (all of 140 to 192 orbitals, or the occupied ones of clusters where they are most of the basis): with EVEC in
+// Qout itself, else in zbuf (nmax^2 doubles per slot).  Rows are read ahead of their use in every sweep, and
+// lanes run along a row, so the L2 serves them.
 // All pairs of 128 alkanes of 2-30 carbons: 0.72 ms for the blocks above 139 orbitals, 0.44 for the rest (6.5 ms
 // by the library's batched solver on padded stacks).
 template <int NW, int RR, int RC, bool EVEC, bool GZ>
@@ -704,7 +705,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
                                                        const double* __restrict__ F, double* __restrict__ P,
                                                        double* __restrict__ ws, int nmax,
                                                        int* __restrict__ fail, const long long* __restrict__ orb_off,
-                                                       double* __restrict__ evals) {
+                                                       double* __restrict__ evals, double* __restrict__ zbuf) {
   constexpr int NT = 64 * NW, S = 16 * RC;
   extern __shared__ __align__(16) double lds[];
   const int slot = blockIdx.x;
@@ -718,8 +719,8 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
   double* U0 = HH + nm2;
   double* U1 = HH + 2 * nm2;
   double* U2 = HH + 3 * nm2;
-  const int ldz = GZ ? n : zstride(n, nv);
-  double* Z = GZ ? P + mo : lds;  // eigenvectors: Z[k * ldz + j]
+  const int ldz = GZ ? nv : zstride(n, nv);
+  double* Z = GZ ? (EVEC ? P + mo : zbuf + (size_t)slot * nm2) : lds;  // eigenvectors: Z[k * ldz + j]
   double2* de = reinterpret_cast<double2*>(lds + ((zregion(GZ ? 0 : n, nv, S) + 1) & ~1));  // (d, e^2)
   double* e = reinterpret_cast<double*>(de + n);
   double* lam = e + n;
@@ -1173,11 +1174,14 @@ template <bool EVEC>
 void launch_eigh(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const double* F, double* out,
                  double* ws, int* fail, const long long* orb_off, double* evals, size_t lds, hipStream_t s) {
   if (nmax <= 48)
-    k_eigh_density<1, 12, 3, EVEC, false><<<nact, 64, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
+    k_eigh_density<1, 12, 3, EVEC, false><<<nact, 64, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals,
+                                                                  nullptr);
   else if (nmax <= 96)
-    k_eigh_density<4, 6, 6, EVEC, false><<<nact, 256, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
+    k_eigh_density<4, 6, 6, EVEC, false><<<nact, 256, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals,
+                                                                  nullptr);
   else
-    k_eigh_density<8, 6, 12, EVEC, false><<<nact, 512, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals);
+    k_eigh_density<8, 6, 12, EVEC, false><<<nact, 512, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals,
+                                                                   nullptr);
 }
 
 extern "C" int pyseqm_eigh_density_lds_ok(int norb, int nocc) {
@@ -1197,6 +1201,17 @@ extern "C" int pyseqm_eigh_density(const pyseqm_layout_t* L, const int* idx, int
   return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
 }
 
+extern "C" int pyseqm_eigh_density_large(const pyseqm_layout_t* L, const int* idx, int nact, int nmax,
+                                         const double* F, double* P, double* ws, double* Z, int* fail,
+                                         void* stream) {
+  if (!L || nact < 0 || nmax < 1 || nmax > kEighMaxN || !fail || !Z) return PYSEQM_EINVAL;
+  if (nact == 0) return PYSEQM_OK;
+  const size_t lds = (size_t)(zregion(0, 0, 192) + 6 * nmax + kLdsExtra) * sizeof(double);
+  k_eigh_density<8, 6, 12, false, true>
+      <<<nact, 512, lds, (hipStream_t)stream>>>(*L, idx, F, P, ws, nmax, fail, nullptr, nullptr, Z);
+  return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
+}
+
 extern "C" int pyseqm_eigh_vectors(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const double* F,
                                    const long long* orb_off, double* evals, double* Q, double* ws, int* fail,
                                    void* stream) {
@@ -1205,7 +1220,7 @@ extern "C" int pyseqm_eigh_vectors(const pyseqm_layout_t* L, const int* idx, int
   if (!pyseqm_eigh_density_lds_ok(nmax, nmax)) {  // above 139 orbitals: vectors in Q
     const size_t lds = (size_t)(zregion(0, 0, 192) + 6 * nmax + kLdsExtra) * sizeof(double);
     k_eigh_density<8, 6, 12, true, true>
-        <<<nact, 512, lds, (hipStream_t)stream>>>(*L, idx, F, Q, ws, nmax, fail, orb_off, evals);
+        <<<nact, 512, lds, (hipStream_t)stream>>>(*L, idx, F, Q, ws, nmax, fail, orb_off, evals, nullptr);
     return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
   }
   const size_t lds = (size_t)lds_doubles(nmax, nmax) * sizeof(double);

@@ -241,8 +241,9 @@ class SCFEngine:
         """FP64 density step by diagonalisation of the active Fock blocks -> Pout (diag.py:110-241).
 
         Blocks of up to EIGH_WG_MAX_N orbitals go to the one-workgroup-per-molecule solver
-        (pyseqm_eigh_density: Householder with the block in registers, multisection, inverse
-        iteration, cluster Gram-Schmidt, no padding) in one launch.  Larger blocks, and calls that
+        (pyseqm_eigh_density: Householder with the block in registers, multisection, twisted
+        factorisations, cluster Gram-Schmidt, no padding) in one launch, those whose occupied vectors do not
+        fit its LDS (28 to 32 waters) in one of their own.  Larger blocks, and calls that
         want the eigenvectors themselves, take the batched
         library eigensolver on Gershgorin-padded stacks, again per size group (the reference pads
         every molecule to the batch's largest, which for an uneven batch multiplies the O(n^3) work)."""
@@ -255,7 +256,10 @@ class SCFEngine:
                 # ones fill the CUs behind them (C2's density step: 5.2 ms against 8.4 ms for
                 # launches per size group, each of which waits for its own largest block)
                 self._eigh_wg_run(F, *self._eigh_wg_order(idx_h[wg]), Pout)
-            rest = idx_h[~wg]
+            large = ~wg & eigh_pairs_ok(b.norb[idx_h])
+            if large.any():
+                self._eigh_wg_run(F, *self._eigh_wg_order(idx_h[large]), Pout, large=True)
+            rest = idx_h[~wg & ~large]
             if len(rest) == 0:
                 return None
             groups = size_groups(b.norb[rest])
@@ -296,10 +300,14 @@ class SCFEngine:
         """One launch of the workgroup eigensolver on the molecules `ids` (host int array)."""
         self._eigh_wg_run(F, *self._eigh_wg_order(ids), Pout)
 
-    def _eigh_wg_run(self, F, idx, count, nmax, nocc_max, Pout):
-        ws = torch.empty(max(4 * count * nmax * nmax, 1), dtype=torch.float64, device=self.device)
-        nat.call("pyseqm_eigh_density", self.b.L, nat.ptr(idx), count, nmax, nocc_max, nat.ptr(F), nat.ptr(Pout),
-                 nat.ptr(ws), nat.ptr(self.eigh_fail), self.stream)
+    def _eigh_wg_run(self, F, idx, count, nmax, nocc_max, Pout, large=False):
+        ws = torch.empty((5 if large else 4) * count * nmax * nmax, dtype=torch.float64, device=self.device)
+        if large:
+            nat.call("pyseqm_eigh_density_large", self.b.L, nat.ptr(idx), count, nmax, nat.ptr(F), nat.ptr(Pout),
+                     nat.ptr(ws), nat.ptr(ws[4 * count * nmax * nmax:]), nat.ptr(self.eigh_fail), self.stream)
+        else:
+            nat.call("pyseqm_eigh_density", self.b.L, nat.ptr(idx), count, nmax, nocc_max, nat.ptr(F), nat.ptr(Pout),
+                     nat.ptr(ws), nat.ptr(self.eigh_fail), self.stream)
         self.eigh_log.append((count, nmax, "workgroup"))
 
     def _sp2_workspace(self):

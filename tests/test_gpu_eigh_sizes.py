@@ -127,3 +127,28 @@ def test_eigenpairs_above_the_lds_limit(kind):
         assert np.abs(e[k, :n] - np.linalg.eigvalsh(f)).max() < 1e-10 * scale, n
         assert np.abs(q.T @ q - np.eye(n)).max() < 1e-9, n
         assert np.abs(f @ q - q * e[k, :n]).max() < 1e-9 * scale, n
+
+
+@pytest.mark.parametrize("kind", ["spread", "degenerate", "close", "diagonal", "blocks"])
+def test_density_with_vectors_in_memory(kind):
+    """Blocks of up to 192 orbitals whose occupied vectors do not fit LDS, beside one that does, through the density step:
+    the bound of test_density_at_grid_edges."""
+    sizes, noccs = [168, 180, 40, 191, 192, 192, 175], [112, 120, 20, 191, 128, 192, 174]
+    eng = _engine(sizes, noccs)
+    assert eigh_wg_ok(sizes, noccs).tolist() == [n == 40 or n * o + 3 * n + 704 <= 20480 for n, o in zip(sizes, noccs)]
+    fs = _blocks(sizes, noccs, kind, 11)
+    F = torch.as_tensor(np.concatenate([f.reshape(-1) for f in fs]), device=DEV)
+    P = torch.full_like(F, float("nan"))
+    eng._idx_host = np.arange(len(sizes))
+    eng.eigh_log.clear()
+    eng.density_eigh(F, torch.arange(len(sizes), dtype=torch.int32, device=DEV), len(sizes), P)
+    assert all(how == "workgroup" for _, _, how in eng.eigh_log)
+    o = 0
+    for f, n, nocc in zip(fs, sizes, noccs):
+        p = P[o:o + n * n].view(n, n).cpu().numpy()
+        o += n * n
+        w, U = np.linalg.eigh(f)
+        ref = 2.0 * U[:, :nocc] @ U[:, :nocc].T
+        assert np.array_equal(p, p.T), n
+        assert np.abs(p - ref).max() < 1e-10, (n, nocc, np.abs(p - ref).max())
+    assert int(eng.eigh_fail.item()) == 0
