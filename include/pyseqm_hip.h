@@ -413,6 +413,10 @@ int pyseqm_krylov_combine(const pyseqm_layout_t* L, const int* idx, int nact, in
  * pair_base [nmol]: pairs before each molecule.  pyseqm_pair_ref: reference pair index of every tile
  *   lane, -1 without a pair, out [ntiles_total*64].
  * pyseqm_w_reference: out [npairs][10][10], the dense integrals (hcore.py:9-179).
+ * pyseqm_pair_lists: Parser's atom and pair lists (basics.py:199-403) of a padded batch species [nmol][molsize],
+ *   xyz [nmol][molsize][3] (rows sorted, padding last; nmol <= 65535) with every pair: atoms [3][natoms] = Z,
+ *   maskd, molecule; pairs [7][npairs] = molecule, ni, nj, idxi, idxj, mask, mask_l; xij [npairs][3] and rij in
+ *   Angstrom; *beyond is raised by the pairs not closer than cutoff.  atom_off / pair_off [nmol + 1].
  * pyseqm_evec_view: the eigenpairs of pyseqm_eigh_vectors as e [nmol][4 molsize] (zero-padded) and V
  *   [nmol][nmax][nmax] (the identity beyond a block; nmax: at least the batch's largest block); *fail is
  *   raised by the eigenvalues that are not finite.
@@ -423,6 +427,9 @@ int pyseqm_from_padded(const pyseqm_layout_t* L, int molsize, const double* Xp, 
 int pyseqm_pair_ref(const pyseqm_layout_t* L, const long long* pair_base, int* out, void* stream);
 int pyseqm_w_reference(const pyseqm_layout_t* L, const long long* pair_base, const double* w_xx, const double* w_xh,
                        const double* w_hh, double* out, void* stream);
+int pyseqm_pair_lists(int nmol, int molsize, const long long* species, const double* xyz, const long long* atom_off,
+                      const long long* pair_off, double cutoff, long long* atoms, long long natoms, long long* pairs,
+                      long long npairs, double* xij, double* rij, int* beyond, void* stream);
 int pyseqm_evec_view(const pyseqm_layout_t* L, int molsize, int nmax, const long long* orb_off,
                      const double* lam, const double* Q, double* e, double* V, int* fail, void* stream);
 int pyseqm_orbital_charges(const pyseqm_layout_t* L, int molsize, const double* V, long long stride_mol,

@@ -113,6 +113,8 @@ _RAW_SIGS = {
                          c_void_p],
     "pyseqm_build_tiles": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                            c_void_p, c_void_p, c_void_p, c_void_p],
+    "pyseqm_pair_lists": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_double, c_void_p, c_longlong,
+                          c_void_p, c_longlong, c_void_p, c_void_p, c_void_p, c_void_p],
     "pyseqm_small_solve": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
 }
 _lib = None

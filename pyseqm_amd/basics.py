@@ -7,6 +7,7 @@ builds, density steps, energies and forces are HIP kernels.
 import numpy as np
 import torch
 
+from . import _native as nat_lib
 from .seqm_functions.constants import ev
 from .seqm_functions.parameters import COLUMNS, METHODS, param_table
 
@@ -36,8 +37,6 @@ class Parser(torch.nn.Module):
         species = molecule.species
         nmol, molsize = species.shape
         nonblank = species > 0
-        flat = torch.nonzero(nonblank.reshape(-1), as_tuple=False).squeeze(1)
-        Z = species.reshape(-1)[flat]
         nHeavy = (species > 1).sum(dim=1)
         nHydro = (species == 1).sum(dim=1)
         nSuperHeavy = torch.zeros_like(nHeavy)
@@ -47,6 +46,16 @@ class Parser(torch.nn.Module):
         if ((n_el % 2) == 1).any():
             raise ValueError("RHF setting requires closed shell systems (even number of electrons)")
         nocc = n_el // 2
+        lists = self._lists_on_device(molecule)
+        if lists is not None:
+            Z, maskd, atom_molid, pm, ni, nj, idxi, idxj, mask, mask_l, xij, dist = lists
+            rij = dist * molecule.const.length_conversion_factor
+            out = [nmol, molsize, nSuperHeavy, nHeavy, nHydro, nocc, Z, maskd, atom_molid, mask]
+            if return_mask_l:
+                out.append(mask_l)
+            return tuple(out + [pm, ni, nj, idxi, idxj, xij, rij])
+        flat = torch.nonzero(nonblank.reshape(-1), as_tuple=False).squeeze(1)
+        Z = species.reshape(-1)[flat]
         maskd = (torch.arange(nmol, device=dev)[:, None] * molsize ** 2
                  + torch.arange(molsize, device=dev)[None, :] * (molsize + 1)).reshape(-1)[flat]
         atom_molid = flat // molsize
@@ -72,6 +81,38 @@ class Parser(torch.nn.Module):
             out.append(mask_l)
         out += [pm, ni, nj, idxi, idxj, xij, rij]
         return tuple(out)
+
+
+    def _lists_on_device(self, molecule):
+        """Atom and pair lists by pyseqm_pair_lists: Z, maskd, atom_molid, pair_molid, ni, nj, idxi, idxj, mask, mask_l,
+        xij, distance (Angstrom).  None where the general way below is needed: other types, layouts or devices, or
+        a pair at or beyond the cutoff (or at no finite distance)."""
+        sp, xyz = molecule.species, molecule.coordinates.detach()
+        if not (sp.is_cuda and xyz.device == sp.device and sp.dtype == torch.int64 and xyz.dtype == torch.float64
+                and xyz.shape == sp.shape + (3,) and sp.is_contiguous() and xyz.is_contiguous()
+                and 0 < sp.numel() and sp.shape[0] <= 65535):
+            return None
+        host = sp.cpu().numpy()
+        real = host > 0
+        nat = real.sum(1)
+        if (host < 0).any() or (real != (np.arange(sp.shape[1])[None] < nat[:, None])).any():
+            return None
+        dev = sp.device
+        up = nat_lib.upload(dev, atom_off=np.concatenate([[0], np.cumsum(nat)]).astype(np.int64),
+                            pair_off=np.concatenate([[0], np.cumsum(nat * (nat - 1) // 2)]).astype(np.int64),
+                            beyond=np.zeros(1, np.int32))
+        n, npairs = int(nat.sum()), int((nat * (nat - 1) // 2).sum())
+        atoms = torch.empty(3, n, dtype=torch.int64, device=dev)
+        pairs = torch.empty(7, npairs, dtype=torch.int64, device=dev)
+        xij = torch.empty(npairs, 3, dtype=torch.float64, device=dev)
+        dist = torch.empty(npairs, dtype=torch.float64, device=dev)
+        nat_lib.call_raw("pyseqm_pair_lists", sp.shape[0], sp.shape[1], nat_lib.ptr(sp), nat_lib.ptr(xyz),
+                         nat_lib.ptr(up["atom_off"]), nat_lib.ptr(up["pair_off"]), float(self.outercutoff),
+                         nat_lib.ptr(atoms), n, nat_lib.ptr(pairs), npairs, nat_lib.ptr(xij), nat_lib.ptr(dist),
+                         nat_lib.ptr(up["beyond"]), nat_lib.stream_ptr(dev))
+        if int(up["beyond"].item()):
+            return None
+        return (*atoms.unbind(0), *pairs.unbind(0), xij, dist)
 
 
 class Pack_Parameters(torch.nn.Module):

@@ -116,6 +116,47 @@ __global__ __launch_bounds__(256) void k_w_reference(pyseqm_layout_t L, int tile
   }
 }
 
+// The reference's atom and pair lists (Parser, basics.py:199-403) of a padded batch in which every pair of real atoms
+// counts: one block per padded atom (m, i), threads over the partners j > i.  Rows are sorted (padding last),
+// so atom i of molecule m is number atom_off[m] + i and its pairs are in row-major order.  As index arithmetic
+// on whole padded tensors this took some 35 launches, 10 to 15 us of host time each.  beyond: counts the pairs
+// that are not closer than `cutoff` (NaN included); the caller drops them.
+__global__ __launch_bounds__(64) void k_pair_lists(int molsize, const long long* __restrict__ species,
+                                                   const double* __restrict__ xyz,
+                                                   const long long* __restrict__ atom_off,
+                                                   const long long* __restrict__ pair_off, double cutoff,
+                                                   long long* __restrict__ atoms, long long natoms,
+                                                   long long* __restrict__ pairs, long long npairs,
+                                                   double* __restrict__ xij, double* __restrict__ rij,
+                                                   int* __restrict__ beyond) {
+  const long long m = blockIdx.y, i = blockIdx.x;
+  const long long a0 = atom_off[m], nat = atom_off[m + 1] - a0;
+  if (i >= nat) return;
+  const long long* z = species + m * molsize;
+  const double* x = xyz + m * molsize * 3;
+  const long long zi = z[i], w = molsize;
+  if (threadIdx.x == 0) {  // Z, maskd, atom_molid
+    atoms[a0 + i] = zi;
+    atoms[natoms + a0 + i] = m * w * w + i * (w + 1);
+    atoms[2 * natoms + a0 + i] = m;
+  }
+  const long long p0 = pair_off[m] + pair_index((int)i, (int)i + 1, (int)nat);
+  for (long long j = i + 1 + threadIdx.x; j < nat; j += 64) {
+#pragma clang fp contract(off)
+    const long long p = p0 + (j - i - 1);
+    const long long v[7] = {m, zi, z[j], a0 + i, a0 + j, m * w * w + i * w + j, m * w * w + j * w + i};
+#pragma unroll
+    for (int q = 0; q < 7; ++q) pairs[q * npairs + p] = v[q];  // molecule, ni, nj, idxi, idxj, mask, mask_l
+    const double d0 = x[3 * j] - x[3 * i], d1 = x[3 * j + 1] - x[3 * i + 1], d2 = x[3 * j + 2] - x[3 * i + 2];
+    const double r = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+    rij[p] = r;
+    xij[3 * p] = d0 / r;
+    xij[3 * p + 1] = d1 / r;
+    xij[3 * p + 2] = d2 / r;
+    if (!(r < cutoff)) atomicAdd(beyond, 1);
+  }
+}
+
 // charge[i][a] of the reference's per-orbital charges: with v row i of V squared, heavy atom a takes
 // v[a], v[nh + a], v[2 nh + a], v[3 nh + a] (the reference's reshape), hydrogen a takes its orbital
 __global__ __launch_bounds__(256) void k_orbital_charges(pyseqm_layout_t L, int molsize, const double* __restrict__ V,
@@ -210,6 +251,17 @@ extern "C" int pyseqm_w_reference(const pyseqm_layout_t* L, const long long* pai
   if (L->ntile[0]) k_w_reference<0><<<L->ntile[0], 256, 0, s>>>(*L, 0, pair_base, w_xx, out);
   if (L->ntile[1]) k_w_reference<1><<<L->ntile[1], 256, 0, s>>>(*L, t1, pair_base, w_xh, out);
   if (L->ntile[2]) k_w_reference<2><<<L->ntile[2], 256, 0, s>>>(*L, t2, pair_base, w_hh, out);
+  return launched();
+}
+
+extern "C" int pyseqm_pair_lists(int nmol, int molsize, const long long* species, const double* xyz,
+                                 const long long* atom_off, const long long* pair_off, double cutoff,
+                                 long long* atoms, long long natoms, long long* pairs, long long npairs, double* xij,
+                                 double* rij, int* beyond, void* stream) {
+  if (nmol < 0 || nmol > 65535 || molsize < 1 || natoms < 0 || npairs < 0 || !beyond) return PYSEQM_EINVAL;
+  if (nmol == 0 || natoms == 0) return PYSEQM_OK;
+  k_pair_lists<<<dim3(molsize, nmol), 64, 0, (hipStream_t)stream>>>(molsize, species, xyz, atom_off, pair_off, cutoff,
+                                                                    atoms, natoms, pairs, npairs, xij, rij, beyond);
   return launched();
 }
 
