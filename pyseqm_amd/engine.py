@@ -534,10 +534,11 @@ class SCFEngine:
         """Every eigenpair of every block of F: Q in the packed layout (column j = eigenvector j,
         ascending eigenvalues) and evals[orb_off[m] + j].  Blocks of up to EIGH_WG_MAX_N orbitals take
         pyseqm_eigh_vectors, in one launch for those whose vectors fit its LDS (at most 139 orbitals) and
-        one for the others, or in one for all where every block has a CU of its own; larger ones the batched library eigensolver on Gershgorin-padded stacks per
-        size group, scattered into the same layout.  eig_ws holds 4 nmol n^2 doubles for the n of the
-        workgroup blocks (allocated here where it is smaller); fail counts vectors the workgroup solver
-        lost (read by the caller)."""
+        one for the others, or in one for all where every block has a CU of its own; larger ones the
+        batched library eigensolver on Gershgorin-padded stacks per size group, scattered into the same
+        layout.  eig_ws: scratch that a launch may overwrite whole, of 4 nmol n^2 doubles for the n of the
+        workgroup blocks, or None to allocate each launch's here (as where it is smaller); fail counts
+        vectors the workgroup solver lost (read by the caller)."""
         b = self.b
         norb = np.asarray(b.norb)
         wg = eigh_pairs_ok(norb)
@@ -551,8 +552,9 @@ class SCFEngine:
                 continue
             ids = ids[np.argsort(-norb[ids], kind="stable")]  # long solves first, as in density_eigh
             top = int(norb[ids[0]])
-            ws = eig_ws if eig_ws.numel() >= 4 * len(ids) * top ** 2 else torch.empty(
-                4 * len(ids) * top ** 2, dtype=torch.float64, device=self.device)
+            need = 4 * len(ids) * top ** 2
+            ws = eig_ws if eig_ws is not None and eig_ws.numel() >= need else torch.empty(
+                need, dtype=torch.float64, device=self.device)
             idx = torch.as_tensor(ids.astype(np.int32), device=self.device)
             nat.call("pyseqm_eigh_vectors", b.L, nat.ptr(idx), len(ids), top, nat.ptr(F), nat.ptr(orb_off),
                      nat.ptr(evals), nat.ptr(Q), nat.ptr(ws), nat.ptr(fail), self.stream)
@@ -588,7 +590,7 @@ class SCFEngine:
             fail = torch.zeros(1, dtype=torch.int32, device=self.device)
             evals = torch.empty(int(b.norb.sum()), **f64)
             Q = torch.empty(max(b.total, 1), **f64)
-            self.eigenpairs(F, self.orb_off, evals, Q, evals, fail)
+            self.eigenpairs(F, self.orb_off, evals, Q, None, fail)
             e = torch.empty(b.nmol, 4 * b.molsize, **f64)
             V = torch.empty(b.nmol, nmax, nmax, **f64)
             nat.call("pyseqm_evec_view", b.L, b.molsize, nmax, nat.ptr(self.orb_off), nat.ptr(evals),
