@@ -28,6 +28,8 @@ namespace {
 
 constexpr int kEighMaxN = 192;      // largest block this solver takes
 constexpr int kLdsDoubles = 20480;  // 160 KiB of LDS
+constexpr int kLdsFixed = 32;       // of them the kernel's own 256 bytes (__syncthreads_or), beside what a launch asks for
+constexpr int kLdsLaunch = kLdsDoubles - kLdsFixed;
 constexpr int kTPanel = 256;        // doubles of one panel's 16 x 16 T factor
 constexpr int kLdsExtra = 25;       // doubles of the twist rows and of an alignment gap
 
@@ -43,11 +45,12 @@ constexpr int kLdsExtra = 25;       // doubles of the twist rows and of an align
 // multipliers.  The variant follows the launch's largest block nmax.
 __host__ __device__ inline int grid_slots(int nmax) { return nmax <= 48 ? 48 : (nmax <= 96 ? 96 : 192); }
 // The size rule of the entry points: n nocc + 3 n + 3 S + 128 doubles (S: the variant's 48 / 96 /
-// 192 grid rows).  lds_doubles, what a launch asks for, stays within it for every accepted block.
+// 192 grid rows) of the 20480.  lds_doubles, what a launch asks for, stays within kLdsLaunch for every
+// accepted block: with the even stride it is n nocc + 6 n + 25 <= 20480 + 3 n - 679 <= 20377.
 __host__ __device__ inline int rule_doubles(int n, int nv) { return n * nv + 3 * n + 3 * grid_slots(n) + 128; }
 // Row stride of the eigenvectors: odd where that fits (rows of 16 lanes then fall on distinct LDS
 // banks), else nv.
-__host__ __device__ inline int zstride(int n, int nv) { return n * (nv | 1) + 6 * n + kLdsExtra <= kLdsDoubles ? (nv | 1) : nv; }
+__host__ __device__ inline int zstride(int n, int nv) { return n * (nv | 1) + 6 * n + kLdsExtra <= kLdsLaunch ? (nv | 1) : nv; }
 // Doubles of the eigenvector region: also holds the Householder vectors (2 S) and the grid's counts
 // (two ints per thread) before.
 __host__ __device__ inline int zregion(int n, int nv, int S) {
@@ -57,7 +60,7 @@ __host__ __device__ inline int zregion(int n, int nv, int S) {
 inline int lds_doubles(int nmax, int nv) {
   const int S = grid_slots(nmax);
   // where the odd stride does not fit the largest block it may still fit a smaller one of the launch
-  if (zstride(nmax, nv) != (nv | 1)) return kLdsDoubles;
+  if (zstride(nmax, nv) != (nv | 1)) return kLdsLaunch;
   return zregion(nmax, nv, S) + 6 * nmax + kLdsExtra + (S == 48 ? 3 * kTPanel + nmax * (nv | 1) : 0);
 }
 
