@@ -243,23 +243,20 @@ class SCFEngine:
         Blocks of up to EIGH_WG_MAX_N orbitals go to the one-workgroup-per-molecule solver
         (pyseqm_eigh_density: Householder with the block in registers, multisection, twisted
         factorisations, cluster Gram-Schmidt, no padding) in one launch, those whose occupied vectors do not
-        fit its LDS (28 to 32 waters) in one of their own.  Larger blocks, and calls that
-        want the eigenvectors themselves, take the batched
-        library eigensolver on Gershgorin-padded stacks, again per size group (the reference pads
-        every molecule to the batch's largest, which for an uneven batch multiplies the O(n^3) work)."""
+        fit its LDS (28 to 32 waters; _eigh_wg_split) in one of their own.  Larger blocks, and calls
+        that want the eigenvectors themselves, take the batched library eigensolver on Gershgorin-padded
+        stacks, again per size group (the reference pads every molecule to the batch's largest, which for
+        an uneven batch multiplies the O(n^3) work)."""
         b = self.b
         if not want_evecs:
-            idx_h = np.asarray(self._idx_host)
-            wg = eigh_wg_ok(b.norb[idx_h], b.nocc[idx_h])
-            if wg.any():
+            lds, large, rest = self._eigh_wg_split(np.asarray(self._idx_host))
+            if len(lds):
                 # one launch, largest blocks first: the long solves start at once and the short
                 # ones fill the CUs behind them (C2's density step: 5.2 ms against 8.4 ms for
                 # launches per size group, each of which waits for its own largest block)
-                self._eigh_wg_run(F, *self._eigh_wg_order(idx_h[wg]), Pout)
-            large = ~wg & eigh_pairs_ok(b.norb[idx_h])
-            if large.any():
-                self._eigh_wg_run(F, *self._eigh_wg_order(idx_h[large]), Pout, large=True)
-            rest = idx_h[~wg & ~large]
+                self._eigh_wg_run(F, *self._eigh_wg_order(lds), Pout)
+            if len(large):
+                self._eigh_wg_run(F, *self._eigh_wg_order(large), Pout, large=True)
             if len(rest) == 0:
                 return None
             groups = size_groups(b.norb[rest])
@@ -285,6 +282,18 @@ class SCFEngine:
             return e, V, nmax
         return None
 
+    def _eigh_wg_split(self, ids):
+        """Molecules `ids` by the density step that takes them: the workgroup eigensolver with its vectors in LDS, with
+        its vectors in memory, the library's.  A launch asks for the LDS of its largest block and its
+        highest occupation, which may be two molecules' (30 carbons, 182 / 91, and 27 waters, 162 / 108):
+        blocks that fit alone but not beside the largest one go to the vectors in memory."""
+        norb, nocc = self.b.norb[ids], self.b.nocc[ids]
+        fits = eigh_wg_ok(norb, nocc)
+        if fits.any():
+            fits &= eigh_wg_ok(norb[fits].max(), nocc)
+        large = ~fits & eigh_pairs_ok(norb)
+        return ids[fits], ids[large], ids[~fits & ~large]
+
     def _eigh_wg_order(self, ids):
         """(device index list, count, largest block, most occupied orbitals) of the molecules `ids`, largest first."""
         b = self.b
@@ -293,8 +302,8 @@ class SCFEngine:
         return idx, len(ids), int(b.norb[ids[0]]), int(b.nocc[ids].max())
 
     def _eigh_wg_list(self, ids):
-        """_eigh_wg_order of the molecules `ids` if the workgroup eigensolver takes all of them, else None."""
-        return self._eigh_wg_order(ids) if eigh_wg_ok(self.b.norb[ids], self.b.nocc[ids]).all() else None
+        """_eigh_wg_order of the molecules `ids` if one launch of the workgroup eigensolver takes them, else None."""
+        return self._eigh_wg_order(ids) if eigh_wg_ok(self.b.norb[ids].max(), self.b.nocc[ids].max()) else None
 
     def _eigh_wg(self, F, ids, Pout):
         """One launch of the workgroup eigensolver on the molecules `ids` (host int array)."""
