@@ -209,8 +209,9 @@ long long pyseqm_eigh_density_workspace(int nact, int nmax);
 int pyseqm_eigh_density_lds_ok(int norb, int nocc);
 int pyseqm_eigh_density(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, int nocc_max,
                         const double* F, double* P, double* ws, int* fail, void* stream);
-/* The same for blocks of up to 192 orbitals at any occupation (those of pyseqm_eigh_density_lds_ok are faster there): the
- * occupied vectors stand in Z (nact nmax^2 doubles) instead of LDS. */
+/* The same for blocks of up to 192 orbitals at any occupation (those of pyseqm_eigh_density_lds_ok are faster
+ * there): the occupied vectors stand in Z (nact nmax^2 doubles) instead of LDS; not used for nmax <= 48,
+ * where they fit. */
 int pyseqm_eigh_density_large(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const double* F, double* P,
                               double* ws, double* Z, int* fail, void* stream);
 /* P = 2 C_occ C_occ^T from the padded eigenvectors (columns) (diag.py:230-232).  V holds nact

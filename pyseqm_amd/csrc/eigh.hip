@@ -1209,6 +1209,12 @@ extern "C" int pyseqm_eigh_density_large(const pyseqm_layout_t* L, const int* id
                                          void* stream) {
   if (!L || nact < 0 || nmax < 1 || nmax > kEighMaxN || !fail || !Z) return PYSEQM_EINVAL;
   if (nact == 0) return PYSEQM_OK;
+  if (nmax <= 48) {  // any occupation fits LDS; the 192-row variant's panel factors would not fit a slot below 32
+    launch_eigh<false>(L, idx, nact, nmax, F, P, ws, fail, nullptr, nullptr, lds_doubles(nmax, nmax) * sizeof(double),
+                       (hipStream_t)stream);
+    return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
+  }
+  static_assert(3 * 49 * 49 >= 12 * kTPanel, "the panel factors lie behind the reflectors in a molecule's slot");
   const size_t lds = (size_t)(zregion(0, 0, 192) + 6 * nmax + kLdsExtra) * sizeof(double);
   k_eigh_density<8, 6, 12, false, true>
       <<<nact, 512, lds, (hipStream_t)stream>>>(*L, idx, F, P, ws, nmax, fail, nullptr, nullptr, Z);
