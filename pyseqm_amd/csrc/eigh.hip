@@ -908,6 +908,8 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
         if (live) {
           double z = 0.0;
           if (side == 0) {
+            // rows up to the twist row only, read and written: the other wave writes those beyond it meanwhile
+            const int zr = r * ldz + j;
             auto row = [&](double* zk, double l, int k) {
               z = k == r ? 1.0 : -l * z;  // zero above the twist row, until it
               if (k <= r) {
@@ -917,22 +919,22 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
             };
             const int n8 = n & ~7;
             if (n > n8) row(Z + (n - 1) * ldz + j, 0.0, n - 1);
-            for (int k = n - 2; k >= n8; --k) row(Z + k * ldz + j, Z[k * ldz + j], k);
+            for (int k = n - 2; k >= n8; --k) row(Z + k * ldz + j, Z[min(k * ldz + j, zr)], k);
             if (n8) {
-              double* zk = Z + (n8 - 8) * ldz + j;
+              int zk = (n8 - 8) * ldz + j;
               double l[8];
 #pragma unroll
-              for (int t = 0; t < 8; ++t) l[t] = zk[t * ldz];
+              for (int t = 0; t < 8; ++t) l[t] = Z[min(zk + t * ldz, zr)];
               if (n8 == n) l[7] = 0.0;  // row n - 1 has no multiplier
 #pragma unroll 2
               for (int k0 = n8 - 8; k0 >= 0; k0 -= 8) {
                 double ln[8];
                 if (k0 >= 8) {
 #pragma unroll
-                  for (int t = 0; t < 8; ++t) ln[t] = zk[(t - 8) * ldz];
+                  for (int t = 0; t < 8; ++t) ln[t] = Z[min(zk + (t - 8) * ldz, zr)];
                 }
 #pragma unroll
-                for (int t = 7; t >= 0; --t) row(zk + t * ldz, l[t], k0 + t);
+                for (int t = 7; t >= 0; --t) row(Z + zk + t * ldz, l[t], k0 + t);
 #pragma unroll
                 for (int t = 0; t < 8; ++t) l[t] = ln[t];
                 zk -= 8 * ldz;
