@@ -66,6 +66,11 @@ def blocks_to_matrix(M, nmol, molsize):
     return Hp.triu() + Hp.triu(1).transpose(1, 2)
 
 
+def matrix_to_blocks(Hp, nmol, molsize):
+    """Symmetric (nmol, 4m, 4m) -> reference block array holding its upper triangle."""
+    return Hp.triu().reshape(nmol, molsize, 4, molsize, 4).transpose(2, 3).reshape(nmol * molsize * molsize, 4, 4)
+
+
 def fock(nmol, molsize, P0, M, maskd, mask, idxi, idxj, w, W, gss, gpp, gsp, gp2, hsp, themethod, zetas, zetap,
          zetad, Z, F0SD, G2SD):
     if P0.dim() == 4:

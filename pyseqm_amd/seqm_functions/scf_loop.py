@@ -18,6 +18,21 @@ def _converger(scf_converger):
     raise NotImplementedError("scf_converger [3] (KSA) is outside the closed-shell sp SCF path")
 
 
+def orbital_charges(molecule, v):
+    """Per-orbital charge on each atom from the eigenvectors (scf_loop.py:2376-2387), for tensors of any type and
+    device; the loop itself takes SCFEngine.orbital_charges."""
+    nmol = molecule.nmol
+    m = molecule.molsize
+    charge = torch.zeros(nmol, 4 * m, m, dtype=v.dtype, device=v.device)
+    v2 = v * v
+    for i in range(nmol):
+        nh, nH = int(molecule.nHeavy[i]), int(molecule.nHydro[i])
+        n = 4 * nh + nH
+        charge[i, :n, :nh] = v2[i][:n, :4 * nh].reshape(n, 4, nh).sum(dim=1)
+        charge[i, :n, nh:nh + nH] = v2[i][:n, 4 * nh:4 * nh + nH]
+    return charge
+
+
 def _check_pair_cutoff(molecule):
     """The device engine couples every atom pair of a molecule; a pair_outer_cutoff that would drop
     pairs (the reference's Parser keeps only r < cutoff, basics.py:313-328) is refused."""
