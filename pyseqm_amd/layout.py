@@ -314,11 +314,14 @@ class PackedBatch:
         return self._lane_arrays()[2]
 
     def pair_ref_device(self):
-        """Device copy of pair_ref_host (int32), made on first use."""
+        """Device copy of pair_ref_host (int32), made on first use and complete when this returns: engines on other
+        streams may share the batch."""
         if "pair_ref" not in self.d and self.device.type == "cuda":
-            self.d["pair_ref"] = torch.empty(max(64 * self.ntiles, 1), dtype=torch.int32, device=self.device)
-            _native.call("pyseqm_pair_ref", self.L, _native.ptr(self.pair_base_device()),
-                         _native.ptr(self.d["pair_ref"]), _native.stream_ptr(self.device))
+            ref = torch.empty(max(64 * self.ntiles, 1), dtype=torch.int32, device=self.device)
+            _native.call("pyseqm_pair_ref", self.L, _native.ptr(self.pair_base_device()), _native.ptr(ref),
+                         _native.stream_ptr(self.device))
+            torch.cuda.current_stream(self.device).synchronize()
+            self.d["pair_ref"] = ref
         elif "pair_ref" not in self.d:
             self.d["pair_ref"] = torch.as_tensor(np.ascontiguousarray(self.pair_ref_host), dtype=torch.int32,
                                                  device=self.device)
