@@ -11,6 +11,7 @@ import ctypes
 
 import numpy as np
 import torch
+from torch.autograd.forward_ad import unpack_dual
 
 from . import _native
 from .seqm_functions.constants import QN, TORE, MAX_Z
@@ -469,9 +470,10 @@ class PackedBatch:
 
     def _plain(self, X):
         """Whether a tensor can go to the view kernels as it is: FP64 on this batch's device, outside
-        autograd.  Others (host tensors, other types, tracked tensors) take index arrays."""
+        autograd (no gradient asked for, no forward-mode tangent).  Others (host tensors, other types,
+        tracked tensors) take index arrays."""
         return self.device.type == "cuda" and X.device == self.d["mol_norb"].device and X.dtype == torch.float64 \
-            and not X.requires_grad
+            and not X.requires_grad and unpack_dual(X).tangent is None
 
     def to_padded(self, X):
         """Packed matrices (flat) -> reference layout (nmol, 4*molsize, 4*molsize) on the device."""
