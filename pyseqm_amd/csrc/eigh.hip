@@ -14,7 +14,8 @@
 //      a cluster per wave.  Vectors further apart come out orthogonal to eps |T| / gap.  Where a
 //      neighbour is closer than 1e-10 |T| (a degenerate level, which a twisted factorisation would
 //      give the same vector twice) the vectors come from inverse iteration with different starts
-//      instead: they span the level's subspace (P depends on the occupied subspace only).
+//      instead, orthogonalised between its solves: they span the level's subspace (P depends on the
+//      occupied subspace only).
 //   5. Back-transformation C = Q Z by blocks of 16 reflectors and P = 2 C C^T, both on FP64 MFMA
 //      tiles.
 // Every reduction runs in a fixed order: reruns are bitwise identical.
@@ -265,14 +266,15 @@ __device__ __forceinline__ void twisted_sweep(const double2* d, const double* e,
     if (k + t + 1 < n) step(w[t], x[t]);
 }
 
-// Inverse iteration on T - sig I: three solves from a fixed pseudo-random start (of vector j), one
-// thread; z (stride ldz) ends scaled to a largest element of 1.  Returns 1 / |z|.
+// Inverse iteration on T - sig I, one thread: `solves` of them, from a fixed pseudo-random start (of
+// vector j) or from z as it is; z (stride ldz) ends scaled to a largest element of 1.  Returns 1 / |z|.
 __device__ __forceinline__ double inverse_iteration(const double2* de, const double* e, double* z, int ldz, double* U0,
                                                  double* U1, double* U2, int ldu, int n, int j, double sig,
-                                                 double tiny) {
+                                                 double tiny, bool start, int solves) {
   double nrm = 0.0;
-  for (int k = 0; k < n; ++k) z[k * ldz] = start_value(j, k);
-  for (int rep = 0; rep < 3; ++rep) {
+  if (start)
+    for (int k = 0; k < n; ++k) z[k * ldz] = start_value(j, k);
+  for (int rep = 0; rep < solves; ++rep) {
     // LU of T - sig I with partial pivoting, the right-hand side eliminated alongside; the
     // running row and right-hand side stay in registers, U goes to the workspace.  Each step
     // keeps one of two rows as the pivot row (its diagonal and sub-diagonal entries compared)
@@ -356,7 +358,7 @@ __device__ __forceinline__ double inverse_iteration(const double2* de, const dou
       nrm = fma(v, v, nrm);
     }
   }
-  return 1.0 / sqrt(nrm);
+  return nrm > 0.0 ? 1.0 / sqrt(nrm) : 0.0;
 }
 
 // ---- the thread grid of the Householder phase.  The lanes of a wave form 4 rows x 16 columns:
@@ -996,29 +998,37 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
       }
     }
   }
-  if (any_degenerate) {  // inverse iteration for the vectors of degenerate levels, one thread each
-    const double tiny = 2.2e-16 * fmax(tnorm, 1.0e-300);
-    for (int j = tid; j < nv; j += NT)
-      if (degenerate(j)) aux[j] = inverse_iteration(de, e, Z + j, ldz, U0 + j, U1 + j, U2 + j, nmax, n, j, lam[j], tiny);
-    __syncthreads();
-  }
-
-  // ---- 4. clusters (runs of eigenvalues closer than gtol): chain after chain per wave, each vector
+  // Vectors of degenerate levels (pass 0 and 1): two solves from different starts, orthogonalised within
+  // the level, one more solve, orthogonalised again.  At shifts equal to rounding a solve may favour one
+  // vector of the level a hundredfold, so that two starts come out nearly parallel; what the first
+  // orthogonalisation leaves of the second is small and carries the error of the rest of the spectrum
+  // magnified, which the third solve takes out again.  Density errors at such levels (14 to 192
+  // orbitals): 5e-14 at most; with three solves and one orthogonalisation after them 1e-13 to 1e-10.
+  // ---- 4. clusters (runs of eigenvalues closer than gtol; pass 2): chain after chain per wave, each vector
   //         against those before it within gtol, four at a time (their products are small, so that is
   //         the same to rounding as one by one); a second time where it lost half of its length.
   //         182 orbitals: 15-61 us by one thread per cluster at 1e-5 |T|, 13-26 here at 1e-3
-  {
+  for (int pass = any_degenerate ? 0 : 2; pass < 3; ++pass) {
+    const double tol = pass < 2 ? dtol : gtol;
+    if (pass < 2) {
+      const double tiny = 2.2e-16 * fmax(tnorm, 1.0e-300);
+      for (int j = tid; j < nv; j += NT)
+        if (degenerate(j))
+          aux[j] = inverse_iteration(de, e, Z + j, ldz, U0 + j, U1 + j, U2 + j, nmax, n, j, lam[j], tiny, pass == 0,
+                                     pass == 0 ? 2 : 1);
+      __syncthreads();
+    }
     constexpr int E = (S + 63) / 64;
     int chain = 0;
     for (int base = 0; base < nv; base += 64) {
       const int jl = base + lane;
-      const bool starts = jl + 1 < nv && (jl == 0 || lam[jl] - lam[jl - 1] > gtol) && lam[jl + 1] - lam[jl] <= gtol;
+      const bool starts = jl + 1 < nv && (jl == 0 || lam[jl] - lam[jl - 1] > tol) && lam[jl + 1] - lam[jl] <= tol;
       unsigned long long todo = __ballot(starts);
       for (; todo; todo &= todo - 1, ++chain) {
         if (chain % NW != wave) continue;
         const int first = base + __ffsll(todo) - 1;
         int p0 = first;
-        for (int q = first; q < nv && (q == first || lam[q] - lam[q - 1] <= gtol); ++q) {
+        for (int q = first; q < nv && (q == first || lam[q] - lam[q - 1] <= tol); ++q) {
           double zq[E];
           const double sc = aux[q];
 #pragma unroll
@@ -1026,7 +1036,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
             const int k = lane + 64 * i;
             zq[i] = k < n ? sc * Z[k * ldz + q] : 0.0;
           }
-          while (lam[q] - lam[p0] > gtol) ++p0;
+          while (lam[q] - lam[p0] > tol) ++p0;
           for (int rep = 0; rep < 2; ++rep) {
             for (int p = p0; p < q; p += 4) {
               double zp[4][E], dot[4];
@@ -1052,7 +1062,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
             for (int i = 0; i < E; ++i) nr = fma(zq[i], zq[i], nr);
             nr = wave64(nr);
             if (!(nr > 1.0e-200)) {  // lost to its cluster's span: flagged, left unscaled
-              if (lane == 0) atomicAdd(fail, 1);
+              if (lane == 0 && pass == 2) atomicAdd(fail, 1);
               break;
             }
             const double s = 1.0 / sqrt(nr);
@@ -1069,8 +1079,8 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
         }
       }
     }
+    __syncthreads();
   }
-  __syncthreads();
 
   if (EVEC) {  // Rayleigh quotients z^T T z of the normalised vectors (ascending to rounding)
     for (int j = tid; j < nv; j += NT) {
