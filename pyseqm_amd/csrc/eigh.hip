@@ -6,7 +6,7 @@
 //      matrix in registers (tridiagonalise below).  The reflectors go to the global workspace.
 //   2. The nocc lowest eigenvalues of T by Sturm counts: one evenly spaced grid over the whole
 //      spectrum for all of them, then multisection (a group of lanes per eigenvalue) to 1e-11 |T|,
-//      to rounding where a neighbour is closer than 1e-9 |T|.
+//      closer where a neighbour is within 1e-6 |T|, to rounding within 1e-9 |T|.
 //   3. Their eigenvectors from twisted factorisations of T - lambda I, two lanes per vector (one from
 //      each end), the vectors in LDS: one factorisation at the bracket's middle, whose Rayleigh
 //      correction is kept unrounded beside lambda, and one there.
@@ -770,7 +770,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
   ghi += slack;
   for (int k = tid; k + 1 < n; k += NT) de[k].y = fmax(e[k] * e[k], fmax(1.0e-60 * tnorm * tnorm, 1.0e-300));
   __syncthreads();
-  const double btol = 1.0e-11 * tnorm, ctol = 1.0e-9 * tnorm, dtol = 1.0e-10 * tnorm, gtol = 1.0e-3 * tnorm;
+  const double btol = 1.0e-11 * tnorm, ctol = 1.0e-6 * tnorm, dtol = 1.0e-10 * tnorm, gtol = 1.0e-3 * tnorm;
   {
     constexpr int M = 2 * NT;  // grid points
     int* counts = reinterpret_cast<int*>(lds);
@@ -817,10 +817,14 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
       if (gl == 0) lam[j] = 0.5 * (lo + hi);
     }
     __syncthreads();
-    const bool near = j < nvx && ((j > 0 && lam[j] - lam[j - 1] <= ctol) || (j + 1 < nvx && lam[j + 1] - lam[j] <= ctol));
+    // A bracket b leaves the Rayleigh correction b^2 / gap off, and the vector that over the other gaps: where a
+    // neighbour is closer than ctol the bracket shrinks until that is below 1e-16 |T|.
+    double gap = 2.0 * ctol;
+    if (j < nvx && j > 0) gap = fmin(gap, lam[j] - lam[j - 1]);
+    if (j + 1 < nvx) gap = fmin(gap, lam[j + 1] - lam[j]);
     __syncthreads();
-    if (near) {
-      narrow(0.0);
+    if (gap <= ctol) {
+      narrow(gap <= 1.0e-9 * tnorm ? 0.0 : 1.0e-8 * sqrt(gap * tnorm));
       if (gl == 0) lam[j] = 0.5 * (lo + hi);
     }
     __syncthreads();
