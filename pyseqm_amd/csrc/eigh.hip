@@ -1086,15 +1086,24 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
     __syncthreads();
   }
 
-  if (EVEC) {  // Rayleigh quotients z^T T z of the normalised vectors (ascending to rounding)
-    for (int j = tid; j < nv; j += NT) {
-      double rq = de[0].x * Z[j] * Z[j];
-      for (int k = 1; k < n; ++k) {
-        const double zk = Z[k * ldz + j], zk1 = Z[(k - 1) * ldz + j];
-        rq += de[k].x * zk * zk + 2.0 * e[k - 1] * zk * zk1;
+  if (EVEC) {
+    // Rayleigh quotients of the vectors (ascending to rounding) as lam + z^T (T - lam) z / z^T z, a group of
+    // lanes per vector: the rows of (T - lam) z are residuals, so their sum rounds at the size of those and not of T
+    int tg = 64;
+    while (nv * tg > NT) tg >>= 1;
+    const int j = tid / tg;
+    const double s = lam[min(j, nv - 1)];
+    double acc = 0.0;
+    if (j < nv)
+      for (int k = tid % tg; k < n; k += tg) {
+        const double* z = Z + k * ldz + j;
+        double row = (de[k].x - s) * z[0];
+        if (k > 0) row = fma(e[k - 1], z[-ldz], row);
+        if (k + 1 < n) row = fma(e[k], z[ldz], row);
+        acc = fma(z[0], row, acc);
       }
-      lam[j] = rq * aux[j] * aux[j];
-    }
+    acc = group_sum_t(acc, tg);
+    if (j < nv && tid % tg == 0) lam[j] = s + acc * aux[j] * aux[j];
     __syncthreads();
   }
   // ---- 5. C = Q Z: 16 columns per wave in registers, blocks of 16 reflectors last to first, each
