@@ -263,10 +263,12 @@ __device__ __forceinline__ void fock_xx_tile(const pyseqm_layout_t& L, int tile,
   if (lane == 0) etile[tile] = es;
 }
 
-// Every pair tile in one launch: a workgroup of two waves takes a heavy-heavy tile, or two heavy-H or H-H tiles, a
-// wave each, in that order of block ids, so that the light tiles fill the end of the heavy ones.  Each kind
-// keeps its own runs of neighbouring tiles per XCD.  As a launch per kind each waited out the last tiles of
-// the one before: 1024 alkanes of 2-30 carbons 121 -> 112 us, 8 clusters of 256 waters 151 -> 145.
+// Pair tiles of several kinds in one launch: a workgroup of two waves takes a heavy-heavy tile, or two heavy-H or H-H
+// tiles, a wave each, in that order of block ids, so that the light tiles fill the end of the heavy ones.  Each
+// kind keeps its own runs of neighbouring tiles per XCD.  As a launch per kind each waited out the last
+// tiles of the one before: 1024 alkanes of 2-30 carbons 121 -> 112 us, 8 clusters of 256 waters 151 -> 145.
+// Light tiles then run at the heavy ones' registers (3 waves per SIMD), which the many H-H tiles of a large batch
+// feel: launch_fock gives those a launch of their own.
 __global__ __launch_bounds__(128) void k_fock_pairs(pyseqm_layout_t L, const double* __restrict__ w_xx,
                                                     const double* __restrict__ w_xh,
                                                     const double* __restrict__ w_hh, const double* __restrict__ P,
@@ -289,6 +291,16 @@ __global__ __launch_bounds__(128) void k_fock_pairs(pyseqm_layout_t L, const dou
   b -= nh;
   const int tl = 2 * xcd_run(b, nhh) + wave;
   if (tl < L.ntile[2]) fock_small_tile<HH>(L, nx + L.ntile[1] + tl, w_hh, P, H, F, part, etile, active);
+}
+
+// Tiles of one light kind, a wave each
+template <int KIND>
+__global__ __launch_bounds__(64) void k_fock_tiles(pyseqm_layout_t L, int tile_base, const double* __restrict__ w,
+                                                   const double* __restrict__ P, const double* __restrict__ H,
+                                                   double* __restrict__ F, double* __restrict__ part,
+                                                   double* __restrict__ etile,
+                                                   const unsigned char* __restrict__ active) {
+  fock_small_tile<KIND>(L, tile_base + xcd_run(blockIdx.x, gridDim.x), w, P, H, F, part, etile, active);
 }
 
 // One-center G(P_ii) of a heavy atom (fock.py:196-224) added to acc, which holds H_ii plus the
@@ -828,6 +840,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(PYSEQM_
 
 namespace {
 
+// H-H tiles above this many take a launch of their own, and heavy-H tiles too where there are no heavy-heavy ones.
+// Tiles heavy-heavy / heavy-H / H-H: one launch, H-H apart, a launch per kind (us; same bits):
+//   0.5k / 3k / 8k   25.9  28.1  32.5      4.8k / 14k / 16k  134.0 134.1 142.8      8k / 33k / 33k   310.0 303.7 311.1
+//   4k / 12k / 12k   92.6  92.3 100.9      2k / 8k / 20k      54.9  54.1  59.1      5k / 33k / 70k   275.5 258.0 265.7
+//   0 / 4k / 10k     28.2  29.4  29.0      0 / 16k / 41k      75.4  69.4  68.3      1k / 13k / 93k   154.6 135.7 138.9
+//   0 / 0 / 5k       12.4  12.1  12.2      0 / 0 / 15k        24.6  21.3  21.4      0 / 0 / 20k       30.0  25.4  25.6
+constexpr int kApartTiles = 16384;
+
 int launch_fock(const pyseqm_layout_t* L, const double* atom_par, const double* w_xx, const double* w_xh,
                 const double* w_hh, const double* P, const double* H, double* F, double* part, double* etile,
                 double* eatom, double* eelec, const unsigned char* active, hipStream_t s) {
@@ -839,8 +859,12 @@ int launch_fock(const pyseqm_layout_t* L, const double* atom_par, const double* 
         *L, atom_par, w_xx, w_xh, w_hh, P, H, F, eelec, active, stride);
     return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
   }
-  const int blocks = L->ntile[0] + (L->ntile[1] + 1) / 2 + (L->ntile[2] + 1) / 2;
+  const int n0 = L->ntile[0], n1 = L->ntile[1], n2 = L->ntile[2];
+  const bool hh_apart = n2 > kApartTiles || n0 + n1 == 0, xh_apart = hh_apart && n0 == 0;
+  const int blocks = n0 + (xh_apart ? 0 : (n1 + 1) / 2) + (hh_apart ? 0 : (n2 + 1) / 2);
   if (blocks) k_fock_pairs<<<blocks, 128, 0, s>>>(*L, w_xx, w_xh, w_hh, P, H, F, part, etile, active);
+  if (xh_apart && n1) k_fock_tiles<XH><<<n1, 64, 0, s>>>(*L, n0, w_xh, P, H, F, part, etile, active);
+  if (hh_apart && n2) k_fock_tiles<HH><<<n2, 64, 0, s>>>(*L, n0 + n1, w_hh, P, H, F, part, etile, active);
   if (L->natoms) {
     if (lanes_per_atom(L) == 64)
       k_fock_diag<64><<<(L->natoms + 3) / 4, 256, 0, s>>>(*L, atom_par, P, H, part, F, eatom, active);
