@@ -622,11 +622,16 @@ __device__ inline void core_block(const PairGeom& g, const double* pi, const dou
 // register count (up to 8 waves per SIMD, heavy-heavy ones 1); where all tiles fit the chip about at once
 // the launches only wait for each other.  Integrals and forces (us, per kind -> ALL) of n alkanes of 2-30 carbons:
 // n = 1 38.6 -> 25.0 and 28.7 -> 17.0; 64 (2116 tiles) 52.5 -> 31.1 and 36.5 -> 21.3; 128 (4270) 55.1 -> 47.5 and
-// 39.7 -> 35.0; 256 (8548) 91.7 -> 83.5 and 66.7 -> 63.6; 512 (17110) 137 -> 149 and 102 -> 119: ALL up to 8192.
+// 39.7 -> 35.0; 256 (8548) 91.7 -> 83.5 and 66.7 -> 63.6; 512 (17110) 137 -> 149 and 102 -> 119: ALL up to 8192,
+// with at most 6144 light ones (800 / 2400 / 4800 tiles heavy-heavy / heavy-H / H-H 63.4 -> 65.7 and 48.3 -> 52.7;
+// 2700 each 132 -> 120 and 88 -> 84).  Without heavy-heavy tiles, whose latency the light ones fill, they lose
+// sooner: 500 + 500 25.2 -> 18.8 and 21.0 -> 15.8, 1500 + 1500 30.9 -> 30.3 and 24.3 -> 24.3, 4000 + 4000 39.7 ->
+// 59.9 and 33.7 -> 50.4; 8000 H-H alone 22.3 -> 40.1 and 21.4 -> 38.0.
 constexpr int ALL = 3;
-constexpr int kMergeTiles = 8192;
+constexpr int kMergeTiles = 8192, kMergeLight = 6144, kMergeNoHeavy = 3072;
 inline bool merge_kinds(const pyseqm_layout_t* L) {
-  return (long long)L->ntile[0] + L->ntile[1] + L->ntile[2] <= kMergeTiles;
+  const long long n0 = L->ntile[0], light = (long long)L->ntile[1] + L->ntile[2];
+  return n0 > 0 ? n0 + light <= kMergeTiles && light <= kMergeLight : L->ntile[1] > 0 && light <= kMergeNoHeavy;
 }
 // f(kind as a constant, tile) for this block's tile
 template <int KIND, class Fn>
