@@ -266,97 +266,94 @@ __device__ __forceinline__ void twisted_sweep(const double2* d, const double* e,
     if (k + t + 1 < n) step(w[t], x[t]);
 }
 
-// Inverse iteration on T - sig I, one thread: `solves` of them, from a fixed pseudo-random start (of
-// vector j) or from z as it is; z (stride ldz) ends scaled to a largest element of 1.  Returns 1 / |z|.
+// One step of inverse iteration on T - sig I, one thread, from a fixed pseudo-random start (of vector j) or from
+// z as it is; z (stride ldz) ends scaled to a largest element of 1.  Returns 1 / |z|.
 __device__ __forceinline__ double inverse_iteration(const double2* de, const double* e, double* z, int ldz, double* U0,
-                                                 double* U1, double* U2, int ldu, int n, int j, double sig,
-                                                 double tiny, bool start, int solves) {
-  double nrm = 0.0;
+                                                    double* U1, double* U2, int ldu, int n, int j, double sig,
+                                                    double tiny, bool start) {
   if (start)
     for (int k = 0; k < n; ++k) z[k * ldz] = start_value(j, k);
-  for (int rep = 0; rep < solves; ++rep) {
-    // LU of T - sig I with partial pivoting, the right-hand side eliminated alongside; the
-    // running row and right-hand side stay in registers, U goes to the workspace.  Each step
-    // keeps one of two rows as the pivot row (its diagonal and sub-diagonal entries compared)
-    // and eliminates the other, both cases as one select-based update (lanes differ in their
-    // choices); the next step's d, e and right-hand side are read from LDS one step ahead.
-    double diag = de[0].x - sig, sup = n > 1 ? e[0] : 0.0;
-    double yk = z[0];
-    double sub_n = n > 1 ? e[0] : 0.0, dn_n = n > 1 ? de[1].x : 0.0, ns_n = n > 2 ? e[1] : 0.0;
-    double y_n = n > 1 ? z[ldz] : 0.0;
-    for (int k = 0; k + 1 < n; ++k) {
-      const double sub = sub_n, nd = dn_n - sig, ns = ns_n, yk1 = y_n;
-      if (k + 2 < n) {
-        sub_n = ns_n;
-        dn_n = de[k + 2].x;
-        ns_n = k + 3 < n ? e[k + 2] : 0.0;
-        y_n = z[(k + 2) * ldz];
-      }
-      const size_t o = (size_t)k * ldu;
-      const bool keep = fabs(diag) >= fabs(sub);  // no row exchange
-      const double piv = keep ? (fabs(diag) < tiny ? copysign(tiny, diag) : diag) : sub;
-      const double rp = rcp_f64(piv);
-      const double mlt = (keep ? sub : diag) * rp;
-      const double p1 = keep ? sup : nd, p2 = keep ? 0.0 : ns, py = keep ? yk : yk1;
-      const double o1 = keep ? nd : sup, o2 = keep ? ns : 0.0, oy = keep ? yk1 : yk;
-      U0[o] = rp;
-      U1[o] = p1;
-      U2[o] = p2;
-      z[k * ldz] = py;
-      yk = fma(-mlt, py, oy);
-      diag = fma(-mlt, p1, o1);
-      sup = fma(-mlt, p2, o2);
+  // LU of T - sig I with partial pivoting, the right-hand side eliminated alongside; the
+  // running row and right-hand side stay in registers, U goes to the workspace.  Each step
+  // keeps one of two rows as the pivot row (its diagonal and sub-diagonal entries compared)
+  // and eliminates the other, both cases as one select-based update (lanes differ in their
+  // choices); the next step's d, e and right-hand side are read from LDS one step ahead.
+  double diag = de[0].x - sig, sup = n > 1 ? e[0] : 0.0;
+  double yk = z[0];
+  double sub_n = n > 1 ? e[0] : 0.0, dn_n = n > 1 ? de[1].x : 0.0, ns_n = n > 2 ? e[1] : 0.0;
+  double y_n = n > 1 ? z[ldz] : 0.0;
+  for (int k = 0; k + 1 < n; ++k) {
+    const double sub = sub_n, nd = dn_n - sig, ns = ns_n, yk1 = y_n;
+    if (k + 2 < n) {
+      sub_n = ns_n;
+      dn_n = de[k + 2].x;
+      ns_n = k + 3 < n ? e[k + 2] : 0.0;
+      y_n = z[(k + 2) * ldz];
     }
-    const double rlast = 1.0 / (fabs(diag) < tiny ? copysign(tiny, diag) : diag);
-    double x1 = yk * rlast, x2 = 0.0, xmax = fabs(x1);
-    z[(n - 1) * ldz] = x1;
-    // back substitution in blocks of kPF rows: the U factors of the next block are loaded while
-    // this block is solved (the loads come from L2; one row ahead left each row waiting on one)
-    constexpr int kPF = 8;
-    double c0[kPF], c1[kPF], c2[kPF];
+    const size_t o = (size_t)k * ldu;
+    const bool keep = fabs(diag) >= fabs(sub);  // no row exchange
+    const double piv = keep ? (fabs(diag) < tiny ? copysign(tiny, diag) : diag) : sub;
+    const double rp = rcp_f64(piv);
+    const double mlt = (keep ? sub : diag) * rp;
+    const double p1 = keep ? sup : nd, p2 = keep ? 0.0 : ns, py = keep ? yk : yk1;
+    const double o1 = keep ? nd : sup, o2 = keep ? ns : 0.0, oy = keep ? yk1 : yk;
+    U0[o] = rp;
+    U1[o] = p1;
+    U2[o] = p2;
+    z[k * ldz] = py;
+    yk = fma(-mlt, py, oy);
+    diag = fma(-mlt, p1, o1);
+    sup = fma(-mlt, p2, o2);
+  }
+  const double rlast = 1.0 / (fabs(diag) < tiny ? copysign(tiny, diag) : diag);
+  double x1 = yk * rlast, x2 = 0.0, xmax = fabs(x1);
+  z[(n - 1) * ldz] = x1;
+  // back substitution in blocks of kPF rows: the U factors of the next block are loaded while
+  // this block is solved (the loads come from L2; one row ahead left each row waiting on one)
+  constexpr int kPF = 8;
+  double c0[kPF], c1[kPF], c2[kPF];
+#pragma unroll
+  for (int t = 0; t < kPF; ++t) {
+    const int kk = n - 2 - t;
+    const size_t o = (size_t)(kk >= 0 ? kk : 0) * ldu;
+    c0[t] = U0[o];
+    c1[t] = U1[o];
+    c2[t] = U2[o];
+  }
+  for (int k0 = n - 2; k0 >= 0; k0 -= kPF) {
+    double n0[kPF], n1[kPF], n2[kPF];
 #pragma unroll
     for (int t = 0; t < kPF; ++t) {
-      const int kk = n - 2 - t;
+      const int kk = k0 - kPF - t;
       const size_t o = (size_t)(kk >= 0 ? kk : 0) * ldu;
-      c0[t] = U0[o];
-      c1[t] = U1[o];
-      c2[t] = U2[o];
+      n0[t] = U0[o];
+      n1[t] = U1[o];
+      n2[t] = U2[o];
     }
-    for (int k0 = n - 2; k0 >= 0; k0 -= kPF) {
-      double n0[kPF], n1[kPF], n2[kPF];
 #pragma unroll
-      for (int t = 0; t < kPF; ++t) {
-        const int kk = k0 - kPF - t;
-        const size_t o = (size_t)(kk >= 0 ? kk : 0) * ldu;
-        n0[t] = U0[o];
-        n1[t] = U1[o];
-        n2[t] = U2[o];
-      }
-#pragma unroll
-      for (int t = 0; t < kPF; ++t) {
-        const int k = k0 - t;
-        if (k >= 0) {
-          const double x = (z[k * ldz] - c1[t] * x1 - c2[t] * x2) * c0[t];
-          z[k * ldz] = x;
-          xmax = fmax(xmax, fabs(x));
-          x2 = x1;
-          x1 = x;
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < kPF; ++t) {
-        c0[t] = n0[t];
-        c1[t] = n1[t];
-        c2[t] = n2[t];
+    for (int t = 0; t < kPF; ++t) {
+      const int k = k0 - t;
+      if (k >= 0) {
+        const double x = (z[k * ldz] - c1[t] * x1 - c2[t] * x2) * c0[t];
+        z[k * ldz] = x;
+        xmax = fmax(xmax, fabs(x));
+        x2 = x1;
+        x1 = x;
       }
     }
-    const double sc = xmax > 0.0 ? 1.0 / xmax : 1.0;
-    nrm = 0.0;
-    for (int k = 0; k < n; ++k) {
-      const double v = z[k * ldz] * sc;
-      z[k * ldz] = v;
-      nrm = fma(v, v, nrm);
+#pragma unroll
+    for (int t = 0; t < kPF; ++t) {
+      c0[t] = n0[t];
+      c1[t] = n1[t];
+      c2[t] = n2[t];
     }
+  }
+  const double sc = xmax > 0.0 ? 1.0 / xmax : 1.0;
+  double nrm = 0.0;
+  for (int k = 0; k < n; ++k) {
+    const double v = z[k * ldz] * sc;
+    z[k * ldz] = v;
+    nrm = fma(v, v, nrm);
   }
   return nrm > 0.0 ? 1.0 / sqrt(nrm) : 0.0;
 }
@@ -834,8 +831,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
   auto degenerate = [&](int j) {
     return (j > 0 && lam[j] - lam[j - 1] <= dtol) || (j + 1 < nvx && lam[j + 1] - lam[j] <= dtol);
   };
-  bool mine = false;
-  for (int j = tid; j < nv; j += NT) mine = mine || degenerate(j);
+  const bool mine = tid < nv && degenerate(tid);  // nv <= NT in every variant
   const bool any_degenerate = __syncthreads_or(mine);
 
   // ---- 3. eigenvectors: NT / 2 vectors at a time, lane `side` 0 from the top, 1 from the bottom.
@@ -850,6 +846,9 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
     double* U = S == 48 ? T + 3 * kTPanel : U0;
     const int ldu = S == 48 ? ldz : nmax;
     const double tiny = 1.0e-40 * fmax(tnorm, 1.0e-200);
+    // levels degenerate to rounding keep their bisected eigenvalue: a twisted vector of theirs may be poor
+    static_assert(2 * kHalf >= S, "a thread has at most two vectors");
+    const bool keep[2] = {vec < nv && degenerate(vec), kHalf + vec < nv && degenerate(kHalf + vec)};
     for (int c0 = 0; c0 < nv; c0 += kHalf) {
       const int j = c0 + vec;
       const int nc = min(kHalf, nv - c0);
@@ -991,7 +990,7 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
         if (live && side == 1) {
           nrm += aux[j];
           aux[j] = 1.0 / sqrt(nrm);  // the vector's scale
-          if (pass == 0) {
+          if (pass == 0 && !keep[c0 > 0]) {
             const double corr = fmin(fmax(gam / nrm, -btol), btol);
             const double s = lam[j] + corr;
             de[j].y = corr - (s - lam[j]);
@@ -1006,8 +1005,8 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
   // the level, one more solve, orthogonalised again.  At shifts equal to rounding a solve may favour one
   // vector of the level a hundredfold, so that two starts come out nearly parallel; what the first
   // orthogonalisation leaves of the second is small and carries the error of the rest of the spectrum
-  // magnified, which the third solve takes out again.  Density errors at such levels (14 to 192
-  // orbitals): 5e-14 at most; with three solves and one orthogonalisation after them 1e-13 to 1e-10.
+  // magnified, which the third solve takes out again.  Density errors at such levels (8 to 192
+  // orbitals): 1e-14 to 1e-12; with three solves and one orthogonalisation after them up to 1e-10.
   // ---- 4. clusters (runs of eigenvalues closer than gtol; pass 2): chain after chain per wave, each vector
   //         against those before it within gtol, four at a time (their products are small, so that is
   //         the same to rounding as one by one); a second time where it lost half of its length.
@@ -1016,10 +1015,9 @@ __global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, con
     const double tol = pass < 2 ? dtol : gtol;
     if (pass < 2) {
       const double tiny = 2.2e-16 * fmax(tnorm, 1.0e-300);
-      for (int j = tid; j < nv; j += NT)
-        if (degenerate(j))
-          aux[j] = inverse_iteration(de, e, Z + j, ldz, U0 + j, U1 + j, U2 + j, nmax, n, j, lam[j], tiny, pass == 0,
-                                     pass == 0 ? 2 : 1);
+      for (int solve = pass; mine && solve < 2; ++solve)
+        aux[tid] = inverse_iteration(de, e, Z + tid, ldz, U0 + tid, U1 + tid, U2 + tid, nmax, n, tid, lam[tid], tiny,
+                                     pass + solve == 0);
       __syncthreads();
     }
     constexpr int E = (S + 63) / 64;
