@@ -702,8 +702,9 @@ __device__ __forceinline__ void back_panels(doublex4 (&Cr)[S / 16], const double
 // lanes run along a row, so the L2 serves them.
 // All pairs of 128 alkanes of 2-30 carbons: 0.72 ms for the blocks above 139 orbitals, 0.44 for the rest (6.5 ms
 // by the library's batched solver on padded stacks).
-template <int NW, int RR, int RC, bool EVEC, bool GZ>
-__global__ __launch_bounds__(64 * NW) void k_eigh_density(pyseqm_layout_t L, const int* __restrict__ idx,
+// WPS: waves per SIMD the registers are held to (launch_eigh).
+template <int NW, int RR, int RC, bool EVEC, bool GZ, int WPS>
+__global__ __launch_bounds__(64 * NW, WPS) void k_eigh_density(pyseqm_layout_t L, const int* __restrict__ idx,
                                                        const double* __restrict__ F, double* __restrict__ P,
                                                        double* __restrict__ ws, int nmax,
                                                        int* __restrict__ fail, const long long* __restrict__ orb_off,
@@ -1196,17 +1197,29 @@ extern "C" long long pyseqm_eigh_density_workspace(int nact, int nmax) {
 }
 
 // waves per workgroup and register slots per thread: the 4 NW x 16 thread grid covers 48, 96 or 192
+// orbitals.  The smaller two take 310 to 320 registers, one wave per SIMD; with more blocks than run so
+// at once they are held to 256, for two (some 30 spilled).  Blocks (us, one wave -> two): 4096 x 8 173 -> 126,
+// 4096 x 20 278 -> 198, 1024 x 50 402 -> 278, 512 x 96 414 -> 291; 1024 x 14 82 -> 88, 256 x 50 133 -> 132, and the
+// eigenpairs of 32 clusters of 3-12 waters 2 % slower: above the number of blocks that fills 256 CUs.
+template <int NW, int RR, int RC, bool EVEC>
+void launch_eigh_grid(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const double* F, double* out,
+                      double* ws, int* fail, const long long* orb_off, double* evals, size_t lds, hipStream_t s) {
+  if (nact <= 4 / NW * 256)
+    k_eigh_density<NW, RR, RC, EVEC, false, 1><<<nact, 64 * NW, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off,
+                                                                         evals, nullptr);
+  else
+    k_eigh_density<NW, RR, RC, EVEC, false, 2><<<nact, 64 * NW, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off,
+                                                                         evals, nullptr);
+}
 template <bool EVEC>
 void launch_eigh(const pyseqm_layout_t* L, const int* idx, int nact, int nmax, const double* F, double* out,
                  double* ws, int* fail, const long long* orb_off, double* evals, size_t lds, hipStream_t s) {
   if (nmax <= 48)
-    k_eigh_density<1, 12, 3, EVEC, false><<<nact, 64, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals,
-                                                                  nullptr);
+    launch_eigh_grid<1, 12, 3, EVEC>(L, idx, nact, nmax, F, out, ws, fail, orb_off, evals, lds, s);
   else if (nmax <= 96)
-    k_eigh_density<4, 6, 6, EVEC, false><<<nact, 256, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals,
-                                                                  nullptr);
+    launch_eigh_grid<4, 6, 6, EVEC>(L, idx, nact, nmax, F, out, ws, fail, orb_off, evals, lds, s);
   else
-    k_eigh_density<8, 6, 12, EVEC, false><<<nact, 512, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals,
+    k_eigh_density<8, 6, 12, EVEC, false, 2><<<nact, 512, lds, s>>>(*L, idx, F, out, ws, nmax, fail, orb_off, evals,
                                                                    nullptr);
 }
 
@@ -1239,7 +1252,7 @@ extern "C" int pyseqm_eigh_density_large(const pyseqm_layout_t* L, const int* id
   }
   static_assert(3 * 49 * 49 >= 12 * kTPanel, "the panel factors lie behind the reflectors in a molecule's slot");
   const size_t lds = (size_t)(zregion(0, 0, 192) + 6 * nmax + kLdsExtra) * sizeof(double);
-  k_eigh_density<8, 6, 12, false, true>
+  k_eigh_density<8, 6, 12, false, true, 2>
       <<<nact, 512, lds, (hipStream_t)stream>>>(*L, idx, F, P, ws, nmax, fail, nullptr, nullptr, Z);
   return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
 }
@@ -1251,7 +1264,7 @@ extern "C" int pyseqm_eigh_vectors(const pyseqm_layout_t* L, const int* idx, int
   if (nact == 0) return PYSEQM_OK;
   if (!pyseqm_eigh_density_lds_ok(nmax, nmax)) {  // above 139 orbitals: vectors in Q
     const size_t lds = (size_t)(zregion(0, 0, 192) + 6 * nmax + kLdsExtra) * sizeof(double);
-    k_eigh_density<8, 6, 12, true, true>
+    k_eigh_density<8, 6, 12, true, true, 2>
         <<<nact, 512, lds, (hipStream_t)stream>>>(*L, idx, F, Q, ws, nmax, fail, orb_off, evals, nullptr);
     return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH;
   }
