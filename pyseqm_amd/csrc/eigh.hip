@@ -1086,7 +1086,7 @@ __global__ __launch_bounds__(64 * NW, WPS) void k_eigh_density(pyseqm_layout_t L
   }
 
   if (EVEC) {
-    // Rayleigh quotients of the vectors (ascending to rounding) as lam + z^T (T - lam) z / z^T z, a group of
+    // Rayleigh quotients of the vectors as lam + z^T (T - lam) z / z^T z, a group of
     // lanes per vector: the rows of (T - lam) z are residuals, so their sum rounds at the size of those and not of T
     int tg = 64;
     while (nv * tg > NT) tg >>= 1;
@@ -1147,7 +1147,12 @@ __global__ __launch_bounds__(64 * NW, WPS) void k_eigh_density(pyseqm_layout_t L
       double* Qm = P + mo;
       for (int t = tid; t < n * n; t += NT) Qm[t] = Z[(t / n) * ldz + t % n];  // row = orbital, column = vector
     }
-    for (int j = tid; j < n; j += NT) evals[orb_off[m] + j] = lam[j];
+    for (int j = tid; j < n; j += NT) {  // ascending: the quotients of a degenerate level may differ by rounding
+      double v = lam[j];
+      for (int k = j - 1; k >= 0 && !(lam[j] - lam[k] > dtol); --k)
+        if (lam[k] > v) v = lam[k];
+      evals[orb_off[m] + j] = v;
+    }
     return;
   }
   // ---- P = 2 C C^T, a 16 x 16 tile of the upper triangle per wave at a time (two chains over the
