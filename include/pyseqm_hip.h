@@ -137,7 +137,8 @@ int pyseqm_param_grad(const pyseqm_layout_t* L, int method, const double* coords
  * d(sum Y F(theta; P))/d(slot k of atom a) at fixed P and symmetric Y (out[a][1][.] = 0), the
  * contraction (dP_out/dtheta)^T u of the SCF implicit backward after the density response
  * (scf_loop.py:1779-1993, agrad(Pout, gv, grad_outputs=u) over M, w, gss .. hsp and on to the
- * parameters).  Same kernels, steps and workspace as pyseqm_param_grad. */
+ * parameters).  Same kernels, steps and workspace as pyseqm_param_grad; part: no longer used (may be
+ * NULL). */
 int pyseqm_fock_param_vjp(const pyseqm_layout_t* L, int method, const double* coords, const double* atom_par,
                           const double* P, const double* Y, double hrel, double* rec, double* part, double* out,
                           void* stream);
@@ -150,7 +151,8 @@ int pyseqm_core_repulsion_pairs(long long npairs, int method, const int* idxi, c
 
 /* XL-BOMD forces: -d/dR of E(D, P) = sum D F(P) - 1/2 sum (F(P) - H) P + E_nuc at fixed D and P
  * (the energy of EnergyXL, energy.py:76-88, differentiated by ForceXL's backward,
- * seqm/dynamics/xlbomd.py:536-551).  D: density from F(P); P: propagated density field. */
+ * seqm/dynamics/xlbomd.py:536-551).  D: density from F(P); P: propagated density field; h as for
+ * pyseqm_pair_forces. */
 int pyseqm_pair_forces_xl(const pyseqm_layout_t* L, int method, const double* coords, const double* atom_par,
                           const double* D, const double* P, double h, double* part, double* forces,
                           void* stream);
@@ -287,8 +289,8 @@ int pyseqm_diis_solve(const pyseqm_layout_t* L, const int* idx, int nact, int nf
 /* A Pulay iteration's device work around the density step, without a host step in between.
  * pyseqm_pulay_pre: F's upper triangle into ring slot `slot` of Fring, the residual C = FP - PF into that of
  * Cring with diis_err[m] = max|C| (residual == 0: both are there already), the B row (pyseqm_diis_dots; count ==
- * 1 starts a history and sets EMAT up first), for count >= 2 the coefficients with reset[m] (pyseqm_diis_solve; count <= 15) and the extrapolated F
- * (pyseqm_diis_combine).  X: FP64 scratch of the packed size; red: nact nb 16 doubles.
+ * 1 starts a history and sets EMAT up first), for count >= 2 the coefficients with reset[m]
+ * (pyseqm_diis_solve; count <= 15) and the extrapolated F (pyseqm_diis_combine).  X: FP64 scratch of the packed size; red: nact nb 16 doubles.
  * pyseqm_pulay_post: P = alpha P + (1 - alpha) Pnew, the Fock build of the molecules marked in notconv (the
  * listed ones), the convergence test of pyseqm_scf_check on that step, then a wait for the stream: host
  * [2][nmol] in pinned memory then holds notconv and reset of the listed molecules. */

@@ -889,9 +889,9 @@ __device__ inline void axis_torque(const Dual* ri, const LocalDensity& M, const 
     }
 }
 
-// dE_pair/dR (R = r_j - r_i, Angstrom) of the pair energy above at fixed densities, in closed form.  In the frame of the pair axis the energy is sum_m c_m ri_m(r) (22 local integrals, c_m
-// bilinear in the local densities) + sum_m o_m S_m(r) (5 overlaps) + core repulsion(r): the
-// derivative along the axis takes each of those functions of r once with its derivative (Dual), and the
+// dE_pair/dR (R = r_j - r_i, Angstrom) of the pair energy above at fixed densities, in closed form.  In the
+// frame of the pair axis the energy is sum_m c_m ri_m(r) (22 local integrals, c_m bilinear in the local
+// densities) + sum_m o_m S_m(r) (5 overlaps) + core repulsion(r): the derivative along the axis takes each of those functions of r once with its derivative (Dual), and the
 // two derivatives across the axis are the turns of the local densities under the local potential.
 // Inside the antipodal fallback cone a frame is constant (the reference's autograd gives it no
 // derivative), which drops that frame's part across the axis; the overlaps keep their B-integral branch.
@@ -1455,7 +1455,8 @@ __global__ __launch_bounds__(256) void k_param_gather(pyseqm_layout_t L, int met
 #pragma unroll
   for (int k = 0; k < kJacSlots; ++k) {
     const double* J = jac + ((size_t)a * kJacSlots + k) * 5;
-    oe[kJacParam[k]] += acc[PV_DD] * J[0] + acc[PV_QQ] * J[1] + acc[PV_R0] * J[2] + acc[PV_R1] * J[3] + acc[PV_R2] * J[4];
+    oe[kJacParam[k]] +=
+        acc[PV_DD] * J[0] + acc[PV_QQ] * J[1] + acc[PV_R0] * J[2] + acc[PV_R1] * J[3] + acc[PV_R2] * J[4];
     on[kJacParam[k]] += acc[PV_REP] * J[2];
   }
   oe[PAR_ZS] += acc[PV_ZS];

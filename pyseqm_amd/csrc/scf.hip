@@ -548,8 +548,8 @@ __device__ inline double rsq_fast(double x) {
 }
 enum { kDiisErr = 1, kDiisRow = 2, kDiisSolve = 4, kDiisInit = 8 };
 
-__global__ __launch_bounds__(64) void k_diis_finish(const int* __restrict__ idx, int what, int nb, int rw, int nfock, int cF,
-                                                    int slot, const double* __restrict__ red,
+__global__ __launch_bounds__(64) void k_diis_finish(const int* __restrict__ idx, int what, int nb, int rw, int nfock,
+                                                    int cF, int slot, const double* __restrict__ red,
                                                     double* __restrict__ EMAT, double* __restrict__ diis_err,
                                                     double* __restrict__ coef, unsigned char* __restrict__ reset) {
   __shared__ double A[kDiisMax][kDiisMax + 1], V[kDiisMax][kDiisMax + 1], B[kDiisMax], rot[kDiisMax / 2][2];

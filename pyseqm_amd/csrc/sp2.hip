@@ -843,7 +843,8 @@ __global__ __launch_bounds__(64) void k_sp2_decide(const int* __restrict__ idx, 
 // through registers (prefetched during the MFMAs of the previous slab) and LDS.  What bounds it: the matrix
 // units, and how evenly the tiles fill 256 CUs.  Tiles of 64 at every size: with tiles of 128 above 256 orbitals
 // X^2 of 8 blocks of 1536 had 624 tiles, at two blocks a CU and 128 registers of sums a lane: 906 us, 593
-// with 2400 tiles of 64 (51 of the 73 TFLOP/s a large FP64 product reaches); one block of 300 to 3000: 1.4 to 2.5 times.
+// with 2400 tiles of 64 (51 of the 73 TFLOP/s a large FP64 product reaches); one block of 300 to 3000: 1.4 to
+// 2.5 times.
 // mode bit 0: McWeeny epilogue C <- 2 (3 A - 2 A B) (A = X^2, B = X); bit 1: the product is known
 // to be symmetric (X^2, X^2 X): only tiles ti <= tj are computed and mirrored.
 // AX / BX: the A / B operand is the final FP32 SP2 matrix X of each molecule (buffer Xa or Xb by

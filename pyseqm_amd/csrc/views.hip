@@ -60,7 +60,8 @@ __global__ __launch_bounds__(256) void k_from_padded(pyseqm_layout_t L, int mols
   const int r1 = min(n, (int)(blockIdx.y + 1) * kViewRows);
   for (int r = blockIdx.y * kViewRows; r < r1; ++r) {
     const int rp = r < 4 * nh ? r : 4 * (r - 3 * nh);
-    for (int c = threadIdx.x; c < n; c += 256) o[(size_t)r * n + c] = x[(size_t)rp * w + (c < 4 * nh ? c : 4 * (c - 3 * nh))];
+    for (int c = threadIdx.x; c < n; c += 256)
+      o[(size_t)r * n + c] = x[(size_t)rp * w + (c < 4 * nh ? c : 4 * (c - 3 * nh))];
   }
 }
 
@@ -229,7 +230,9 @@ __global__ __launch_bounds__(256) void k_evec_view(pyseqm_layout_t L, int w, int
     }
 }
 
-dim3 view_grid(const pyseqm_layout_t& L, int molsize) { return dim3(L.nmol, (4 * molsize + kViewRows - 1) / kViewRows); }
+dim3 view_grid(const pyseqm_layout_t& L, int molsize) {
+  return dim3(L.nmol, (4 * molsize + kViewRows - 1) / kViewRows);
+}
 int launched() { return hipGetLastError() == hipSuccess ? PYSEQM_OK : PYSEQM_ELAUNCH; }
 
 }  // namespace

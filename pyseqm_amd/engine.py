@@ -144,9 +144,9 @@ class SCFEngine:
         self.coords = None
         self.trace = None  # set to a list to collect per-iteration (dE, diis, dm, dm_max) metrics
         self.diis_log = None  # set to a list to collect (cF, slot, B matrices, coefficients, resets, errors)
-        self.eigh_log = collections.deque(maxlen=256)
+        self.eigh_log = collections.deque(maxlen=256)  # (blocks, largest, solver) of the recent eigensolves
         # vectors the workgroup eigensolver lost to Gram-Schmidt (stays 0 unless its vectors degenerate)
-        self.eigh_fail = torch.zeros(1, dtype=torch.int32, device=dev)  # (blocks, padded size) of the recent batched eigensolves
+        self.eigh_fail = torch.zeros(1, dtype=torch.int32, device=dev)
         if coordinates is not None:
             self.set_coordinates(coordinates)
 
@@ -553,8 +553,9 @@ class SCFEngine:
         wg = eigh_pairs_ok(norb)
         in_lds = eigh_wg_ok(norb, norb)
         if int(wg.sum()) <= NUM_CU and not in_lds[wg].all():
-            # the small blocks run beside the large ones (128 alkanes of 14-182 orbitals: a launch each took
-            # 0.72 and 0.44 ms, one for all 0.72)
+            # the small blocks run beside the large ones (us, two launches -> one: 128 alkanes of 14-182 orbitals
+            # 1020 -> 615, 255 blocks of 14 and one of 140 503 -> 439, of 192 747 -> 680, 250 of 139 and one of
+            # 140 892 -> 481, 200 of 50 and 56 of 182 745 -> 632, 250 of 96 and 6 of 140 686 -> 464)
             in_lds = np.zeros_like(in_lds)
         for ids in (np.nonzero(wg & ~in_lds)[0], np.nonzero(in_lds)[0]):
             if len(ids) == 0:
@@ -589,7 +590,8 @@ class SCFEngine:
         """Orbital energies in the reference layout e (nmol, 4*molsize), zero padded, and the packed
         eigenvectors (nmol, nmax, nmax), sym_eig_trunc(eig_only=True) (diag.py:110-241).  Batches of
         blocks of up to EIGH_WG_MAX_N orbitals take the workgroup eigensolver (128 alkanes of 14-182
-        orbitals: 1.2 ms, 6.5 by the library's batched solver); those with a larger block, or where the
+        orbitals: 1.2 ms, 6.5 by the library's batched solver; energies and squared vector elements are as
+        exact as the library's); those with a larger block, or where the
         workgroup solver lost a vector or met a value that is not finite, the library's."""
         b = self.b
         self._idx_host = np.arange(b.nmol)

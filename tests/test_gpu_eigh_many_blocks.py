@@ -1,6 +1,6 @@
-"""The workgroup eigensolver on more blocks than run at once (where the variants for up to 48 and up to 96 orbitals are held
-to two waves per SIMD), one block below and above that number: every block's density and eigenpairs against numpy's, with
-the bounds of test_gpu_eigh_sizes.py, plain and degenerate levels.
+"""The workgroup eigensolver on more blocks than run at once (where the variants for up to 48 and up to 96 orbitals are
+held to two waves per SIMD), and on as many as do: every block's density and eigenpairs against numpy's, with the
+bounds of test_gpu_eigh_sizes.py, plain and degenerate levels.
 """
 import numpy as np
 import pytest

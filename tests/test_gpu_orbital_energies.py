@@ -16,8 +16,8 @@ LD = np.longdouble
 
 
 def _refined(A):
-    """Eigenvalues of a symmetric float64 matrix with simple, separated levels, in extended precision: its float64 vectors
-    orthonormalised and corrected to first order until they stand."""
+    """Eigenvalues of a symmetric float64 matrix with simple, separated levels, in extended precision: its float64
+    vectors orthonormalised and corrected to first order until they stand."""
     n = len(A)
     V, A, one = np.linalg.eigh(A)[1].astype(LD), A.astype(LD), np.eye(n, dtype=LD)
     for _ in range(3):

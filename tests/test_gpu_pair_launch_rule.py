@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-# (heavy atoms, hydrogens), molecules: light tiles 3072 / 3074 without heavy-heavy ones, 6138 / 6160 with them; H-H alone
+# (heavy atoms, hydrogens), molecules: light tiles 3072 / 3074 without heavy-heavy ones, 6116 / 6160 with them, H-H
+# alone
 @pytest.mark.parametrize("heavy,hydro,nmol", [(1, 7, 1536), (1, 7, 1537), (2, 62, 139), (2, 62, 140), (0, 8, 9),
                                               (0, 8, 3100)])
 def test_launches_agree(heavy, hydro, nmol):

@@ -1,5 +1,5 @@
-"""Forward-mode derivatives through the padded views: a tensor that carries a tangent takes the index arrays, as one that
-requires grad does, and its tangent is viewed like its value (a view is linear)."""
+"""Forward-mode derivatives through the padded views: a tensor that carries a tangent takes the index arrays, as one
+that requires grad does, and its tangent is viewed like its value (a view is linear)."""
 import types
 
 import numpy as np
